@@ -253,6 +253,12 @@ int build_charge_plan(lgv_ctx *c) {
     xw = xw && (p.NH == 64 || p.NH == 128) && TXH == 64 && TQ == 4;
   }
   c->plan_charge.xwave = xw;
+  // the twelve half-planes of the charges in one buffer resource need 32-bit
+  // offsets (any size below 448^3 in FP64, 564^3 in FP32)
+  const uint64_t esz = c->fp32 ? sizeof(float) : sizeof(double);
+  c->plan_charge.far = c->wide;
+  for (const ReplicaParams &p : c->hp)
+    c->plan_charge.far = c->plan_charge.far || 12 * (uint64_t)p.half * esz > 0xFFFFFFFFull;
   return rc;
 }
 

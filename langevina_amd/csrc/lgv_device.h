@@ -69,15 +69,17 @@ __device__ __forceinline__ uint64_t rotr64_lt32(uint64_t x, int r) {
 // xoroshiro128plus::operator(), ModelG/xoroshiro128plus.h:97-107; on the
 // device the rotations by 55 and 36 are taken as rotations right by 9 and 28,
 // and the three-way xor of the new s0 as one v_bitop3_b32 per half (truth
-// table 0x96 = a ^ b ^ c): eleven instructions per step instead of twelve
-// (256^3 FP32 charge sweep about -3 %).
+// table 0x96 = a ^ b ^ c): ten instructions per step.
 LGV_HD uint64_t xoro_next(Xoro &g) {
   const uint64_t s0 = g.s0;
   uint64_t s1 = g.s1;
   const uint64_t result = s0 + s1;
   s1 ^= s0;
 #ifdef __HIP_DEVICE_COMPILE__
-  const uint64_t r = rotr64_lt32(s0, 9), t = s1 << 14;
+  const uint64_t r = rotr64_lt32(s0, 9);
+  // one v_lshlrev_b64 (the compiler shifts the halves apart, two instructions)
+  uint64_t t;
+  __asm__("v_lshlrev_b64 %0, 14, %1" : "=v"(t) : "v"(s1));
   const uint32_t lo = __builtin_amdgcn_bitop3_b32((uint32_t)r, (uint32_t)s1, (uint32_t)t, 0x96);
   const uint32_t hi = __builtin_amdgcn_bitop3_b32((uint32_t)(r >> 32), (uint32_t)(s1 >> 32),
                                                   (uint32_t)(t >> 32), 0x96);

@@ -28,6 +28,23 @@ __device__ __forceinline__ int live(const ReplicaState &s) {
   return s.cur_phi | (s.cur_chg << 1);
 }
 
+// Lane 0's value of v, uniform over the wave (v_readfirstlane per word).  Also
+// for values that are the same in every lane but were computed in vector
+// registers: the compiler would treat whatever follows from them (plane bases,
+// branches) as differing between lanes.
+__device__ __forceinline__ int first_lane(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ uint64_t first_lane(uint64_t v) {
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return ((uint64_t)hi << 32) | lo;
+}
+__device__ __forceinline__ float first_lane(float v) {
+  return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v)));
+}
+__device__ __forceinline__ double first_lane(double v) {
+  return __longlong_as_double((long long)first_lane((uint64_t)__double_as_longlong(v)));
+}
+
 // Global-memory view of one plane for the sweep kernels.  The base is
 // uniform over a block (it sits in SGPRs) and, with W == false, the element
 // offset is a 32-bit byte offset, so every access is one global load/store
@@ -98,6 +115,60 @@ __device__ __forceinline__ GPlane<T, W> gplane(const FieldBufs &fb, int cur, int
   return {(gbyte *)((buf ? fb.f1 : fb.f0) + (int64_t)(c * 2 + par) * fb.half_bytes)};
 }
 
+// The charge planes of a replica: reads from the live buffer, writes to the
+// other one.  W == false: the twelve half-planes of a buffer span less than 4
+// GiB and are one buffer resource, so an access is one buffer instruction with
+// the site's 32-bit byte offset in a vector register and the plane's offset
+// in a scalar one: no address arithmetic per access and no scalar pair per
+// plane (24 plane bases do not fit the scalar registers of the sweep).
+// W == true: 64-bit addresses.
+template <typename T, bool W>
+struct ChargePlanes {
+  FieldBufs fb;
+  int cur;
+  __device__ __forceinline__ ChargePlanes(const ReplicaParams &p, int cur_)
+      : fb(field_bufs<T>(p)), cur(cur_) {}
+  // component c of the six, parity par
+  __device__ __forceinline__ T ld(int c, int par, uint32_t i) const {
+    return gplane<T, true>(fb, cur, 4 + c, par).raw(i);
+  }
+  __device__ __forceinline__ void st(int c, int par, uint32_t i, T v) const {
+    gplane<T, true>(fb, cur ^ 2, 4 + c, par).template put_raw<false>(i, v);
+  }
+};
+template <typename T>
+struct ChargePlanes<T, false> {
+  __amdgpu_buffer_rsrc_t in, out;
+  uint32_t half_bytes;
+  __device__ __forceinline__ ChargePlanes(const ReplicaParams &p, int cur) {
+    const FieldBufs fb = field_bufs<T>(p);
+    half_bytes = first_lane((int)fb.half_bytes);
+    auto resource = [&](char *f) __attribute__((always_inline)) {
+      char *b = reinterpret_cast<char *>(
+          first_lane((uint64_t)reinterpret_cast<uintptr_t>(f + 8 * fb.half_bytes)));
+      // raw 32-bit format: reads past the twelve half-planes return zero
+      return __builtin_amdgcn_make_buffer_rsrc(b, 0, (int)(12u * half_bytes), 0x00027000);
+    };
+    in = resource(cur >> 1 ? fb.f1 : fb.f0);
+    out = resource(cur >> 1 ? fb.f0 : fb.f1);
+  }
+  __device__ __forceinline__ T ld(int c, int par, uint32_t i) const {
+    const uint32_t s = (uint32_t)(c * 2 + par) * half_bytes;
+    if constexpr (sizeof(T) == 4)
+      return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(in, i * 4u, s, 0));
+    else
+      return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(in, i * 8u, s, 0));
+  }
+  __device__ __forceinline__ void st(int c, int par, uint32_t i, T v) const {
+    const uint32_t s = (uint32_t)(c * 2 + par) * half_bytes;
+    typedef uint32_t b64 __attribute__((ext_vector_type(2)));
+    if constexpr (sizeof(T) == 4)
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), out, i * 4u, s, 0);
+    else
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(b64, v), out, i * 8u, s, 0);
+  }
+};
+
 // Block index of this workgroup within the launch plan.  (A renumbering that
 // gives each XCD a contiguous eighth of the plan was measured on MI355X and
 // made the ideal and charge sweeps slower; the ideal kernel and the phi march
@@ -108,87 +179,118 @@ __device__ __forceinline__ int xcd_block() { return blockIdx.x; }
 __device__ __forceinline__ int wrapp(int a, int N) { return a == N ? 0 : a; }
 __device__ __forceinline__ int wrapm(int a, int N) { return a < 0 ? N - 1 : a; }
 
-// Deterministic block reduction of the monitor increments; thread 0 adds the
-// block total into the block's own slot (stream order makes this race-free).
-// The three counts travel packed in one 64-bit word, 21 bits each (a block
-// counts at most 12 decisions per thread).
-__device__ __forceinline__ uint64_t mon_pack(uint64_t down, uint64_t upyes, uint64_t upno) {
-  return down | (upyes << 21) | (upno << 42);
+// The lanes of the wavefront that hold a predicate, and back.  (The builtin,
+// not __ballot, which rebuilds the mask with a select and a compare.)
+__device__ __forceinline__ uint64_t lanes(bool pred) {
+  return __builtin_amdgcn_ballot_w64(pred);
 }
-__device__ void block_monitor_add(MonSlot *slot, uint64_t cnt, double dSd, double dSu) {
-  __shared__ uint64_t sc[kBlock / 64];
+__device__ __forceinline__ bool in_lanes(uint64_t mask) {
+  return __builtin_amdgcn_inverse_ballot_w64(mask);
+}
+
+// A thread's share of the monitor (o4_stepper_monitor).  The counts are those
+// of the whole wavefront, popcounts of lane masks in scalar registers, so all
+// active lanes carry the same values; the sums of dS are the lane's own.
+struct Tally {
+  uint32_t all = 0, down = 0, yes = 0;  // decisions, dS < 0, accepted dS >= 0
+  double dSd = 0., dSu = 0.;
+};
+// n decisions of every lane that holds count
+__device__ __forceinline__ void tally_all(Tally &m, int n, bool count) {
+  m.all += n * __builtin_popcountll(lanes(count));
+}
+// One decision of the lanes in count: those in down had dS < 0, those in up
+// were accepted with dS >= 0.
+__device__ __forceinline__ void tally(Tally &m, double dS, uint64_t down, uint64_t up,
+                                      uint64_t count) {
+  uint32_t nd = __builtin_popcountll(down & count), ny = __builtin_popcountll(up & count);
+  if (in_lanes(down & count)) m.dSd += dS;
+  if (in_lanes(up & count)) m.dSu += dS;
+  // counted and summed here and now: otherwise the compiler keeps the masks
+  // and dS of a dozen decisions (in spilled registers) for later
+  __asm__ volatile("" : "+s"(nd), "+s"(ny), "+v"(m.dSd), "+v"(m.dSu));
+  m.down += nd;
+  m.yes += ny;
+}
+
+// Deterministic block reduction of the tallies; thread 0 adds the block
+// total into the block's own slot (stream order makes this race-free).  The
+// sums of dS are scaled by unit.
+__device__ void block_monitor_add(MonSlot *slot, const Tally &m, double unit = 1.) {
+  __shared__ uint32_t sc[3][kBlock / 64];
   __shared__ double sd[2][kBlock / 64];
+  double dSd = m.dSd, dSu = m.dSu;
+  uint32_t c[3] = {m.all, m.down, m.yes};
   for (int o = 32; o > 0; o >>= 1) {
-    cnt += __shfl_xor(cnt, o, 64);
     dSd += __shfl_xor(dSd, o, 64);
     dSu += __shfl_xor(dSu, o, 64);
+    // lanes without sites hold zeros, the others the wave's counts
+    for (int i = 0; i < 3; i++) c[i] |= __shfl_xor(c[i], o, 64);
   }
   const int w = threadIdx.x >> 6;
   if ((threadIdx.x & 63) == 0) {
-    sc[w] = cnt;
+    for (int i = 0; i < 3; i++) sc[i][w] = c[i];
     sd[0][w] = dSd; sd[1][w] = dSu;
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    uint64_t c = 0;
+    long long n[3] = {0, 0, 0};
     double d = 0, e = 0;
     for (int i = 0; i < kBlock / 64; i++) {
-      c += sc[i];
+      for (int k = 0; k < 3; k++) n[k] += sc[k][i];
       d += sd[0][i]; e += sd[1][i];
     }
-    const long long a = (long long)(c & 0x1fffff), b = (long long)((c >> 21) & 0x1fffff),
-                    n = (long long)(c >> 42);
-    slot->down_counts += a;
-    slot->up_counts += b + n;
-    slot->up_yes += b;
-    slot->up_no += n;
-    slot->down_dS += d;
-    slot->up_dS += e;
+    slot->down_counts += n[1];
+    slot->up_counts += n[0] - n[1];
+    slot->up_yes += n[2];
+    slot->up_no += n[0] - n[1] - n[2];
+    slot->down_dS += d * unit;
+    slot->up_dS += e * unit;
   }
 }
 
 // ------------------------------------------------------------------------
 // The Metropolis test canonical(u) < exp(x) for the draw u and x = -dS <= 0,
-// decided as the double test decides it.  Fast path (x > -11, exp(x) >
-// 1.6e-5): the draw's top 32 bits in single precision against single-
-// precision bounds e (1 -+ 1e-3) 2^32, e = __expf(x).  With r = 2^-32
-// float(u >> 32), |canonical(u) - r| <= 2^-32 + 2^-24 r, and e is within
-// 2e-6 of exp(x) relative (x and x log2(e) rounded to float, one-ulp
-// v_exp_f32), so a draw below the lower bound lies below exp(x) and one at
-// or above the upper bound does not: the margin, about 1e-3 exp(x), exceeds
-// the 2.4e-10 of the draw's rounding whenever exp(x) > 2.4e-7.  The double
-// draw and the double exp decide the rest (about 2e-3 of the tests).
-// The double test, out of line: it runs for about 2e-3 of the tests, and
-// inlined at every decision of a sweep kernel its exp makes up a sizeable
-// part of the kernel's code.
+// decided as the double test decides it: the lanes that accept.  e is exp(x)
+// in single precision: the callers round x log2(e) by at most three half-ulps
+// (4.2e-6 of exp(x) for x > -23) and v_exp_f32 by one ulp.  r = float(u >> 32)
+// is within 1 + 2^-24 r of canonical(u) 2^32, so D = e 2^32 - r in single
+// precision is within 2e4 of (exp(x) - canonical(u)) 2^32 and its sign decides
+// where |D| > 2^16.  The double draw and the double exp decide the rest (3e-5
+// of the tests; with the earlier band of 1e-3 exp(x), a wavefront went there
+// at every tenth decision).  Lanes that are in `sure` (dS < 0, e >= 1) accept;
+// a NaN does not.
+// The double test is out of line: inlined at every decision of a sweep
+// kernel its exp makes up a sizeable part of the kernel's code.
 __device__ __attribute__((noinline)) bool accept_exact(uint64_t u, double x) {
   return canonical(u) < exp(x);
 }
-__device__ __forceinline__ bool accept_draw(uint64_t u, double x) {
-  // the bounds are formed for every x (a very negative x gives e = 0, no
-  // NaN) and the test falls back to the double path outside x > -11; the
-  // empty asm keeps the draw's top half a 32-bit value (otherwise it is
+constexpr float kLog2e = 0x1.715476p+0f;
+template <typename X>
+__device__ __forceinline__ uint64_t accept_draw(uint64_t u, float e, uint64_t sure, X x) {
+  // the empty asm keeps the draw's top half a 32-bit value (otherwise it is
   // converted as a 64-bit one, six instructions instead of one)
   uint32_t h = (uint32_t)(u >> 32);
   __asm__("" : "+v"(h));
-  const float e = __expf((float)x);
-  const float r = (float)h;
-  const bool below = r < e * (0.999f * 0x1p32f);
-  const bool above = r >= e * (1.001f * 0x1p32f);
-  if (x > -11. && (below || above)) return below;
-  // the draw rebuilt from h (the same bits), so that u's top half need not
-  // be kept beside h
-  return accept_exact(((uint64_t)h << 32) | (uint32_t)u, x);
+  const float D = __builtin_fmaf(e, 0x1p32f, -(float)h);
+  uint64_t accept = lanes(D > 0.f);
+  const uint64_t near = lanes(fabsf(D) <= 0x1p16f);
+  if (__builtin_expect(near != 0, 0)) {
+    // the draw rebuilt from h (the same bits), so that u's top half need not
+    // be kept beside h
+    const uint64_t exact = lanes(accept_exact(((uint64_t)h << 32) | (uint32_t)u, x()));
+    accept = (accept & ~near) | ((exact | sure) & near);
+  }
+  return accept;
 }
 
 // The Metropolis decision of one phi site (Stepper.cxx:330-370) in the
 // reference's operand order: heff[l] is the neighbour sum of component l,
 // ((x+1 + x-1) + (y+1 + y-1)) + (z+1 + z-1).  Returns the new value (the
-// old one on reject) and adds the decision to the monitor when count.
+// old one on reject) and adds the decision to the monitor.
 __device__ __forceinline__ void hb_decide(const double phi_o[4], const double heff[4],
                                           double Lambda2, double lambda, double H, double rdtg,
-                                          Xoro &g, double phi_new[4], uint64_t &cnt,
-                                          double &dSd, double &dSu, bool count) {
+                                          Xoro &g, double phi_new[4], Tally &m) {
   double hphi_o = 0., hphi_n = 0., s_o = 0., s_n = 0.;
   double phi_n[4];
 #pragma unroll
@@ -203,18 +305,15 @@ __device__ __forceinline__ void hb_decide(const double phi_o[4], const double he
   hphi_n += (H * phi_n[0]);
   const double dS = -(hphi_n - hphi_o) + Lambda2 * (s_n - s_o) +
                     lambda / 4. * (s_n * s_n - s_o * s_o);
-  bool accept;
-  if (dS < 0) {
-    accept = true;
-    if (count) { cnt += mon_pack(1, 0, 0); dSd += dS; }
-  } else {
-    accept = accept_draw(xoro_next(g), -dS);
-    if (count) {
-      if (accept) { cnt += mon_pack(0, 1, 0); dSu += dS; } else { cnt += mon_pack(0, 0, 1); }
-    }
-  }
+  const uint64_t down = lanes(dS < 0);
+  // the site's last draw: taken whether or not it is needed
+  const uint64_t accept =
+      accept_draw(xoro_next(g), __builtin_amdgcn_exp2f((float)dS * -kLog2e), down,
+                  [&] { return -dS; });
+  tally_all(m, 1, true);
+  tally(m, dS, down, accept & ~down, ~0ull);
 #pragma unroll
-  for (int l = 0; l < 4; l++) phi_new[l] = accept ? phi_n[l] : phi_o[l];
+  for (int l = 0; l < 4; l++) phi_new[l] = in_lanes(accept) ? phi_n[l] : phi_o[l];
 }
 
 // One parity of EulerLangevinHB::step (ModelG/Stepper.cxx:309-386), one
@@ -237,8 +336,7 @@ __global__ __launch_bounds__(kBlock) void k_hb_phi(const ReplicaParams *__restri
       (int)gridDim.x == p.N * bpp)
     pb = band_block(pb, bpp);
   const uint32_t idx = (uint32_t)pb * kBlock + threadIdx.x;
-  uint64_t cnt = 0;
-  double dSd = 0., dSu = 0.;
+  Tally mt;
   if (idx < (uint64_t)p.half) {
     const uint32_t N = p.N, NH = p.NH;
     const uint32_t rowi = idx / NH, xh = idx - rowi * NH;
@@ -266,11 +364,11 @@ __global__ __launch_bounds__(kBlock) void k_hb_phi(const ReplicaParams *__restri
                 (fq.ld(nb[4]) + fq.ld(nb[5]));
       phi_o[l] = gplane<T, W>(p, cur, l, ieo).ld(idx);
     }
-    hb_decide(phi_o, heff, Lambda2, p.lambda, p.H, p.rdtg, g, phi_n, cnt, dSd, dSu, true);
+    hb_decide(phi_o, heff, Lambda2, p.lambda, p.H, p.rdtg, g, phi_n, mt);
 #pragma unroll
     for (int l = 0; l < 4; l++) gplane<T, W>(p, cur, l, ieo).st(idx, phi_n[l]);
   }
-  block_monitor_add(mon + bid, cnt, dSd, dSu);
+  block_monitor_add(mon + bid, mt);
 }
 
 __device__ __forceinline__ int wrapz(int z, int N) { return z < 0 ? z + N : (z >= N ? z - N : z); }
@@ -335,8 +433,7 @@ __global__ __launch_bounds__(kBlock) void k_hb_march(const ReplicaParams *__rest
   const double Lambda2 = 0.5 * (2. * 3. + mass);
   const double lambda = p.lambda, H = p.H, rdtg = p.rdtg;
   const uint64_t key = stream_key(p.base_key, s.sweep_ctr + ctr_off);
-  uint64_t cnt = 0;
-  double dSd = 0., dSu = 0.;
+  Tally mt;
   auto idx = [&](int xhh, int yy, int z) __attribute__((always_inline)) {
     return ((uint32_t)z * N + yy) * NH + xhh;
   };
@@ -439,7 +536,7 @@ __global__ __launch_bounds__(kBlock) void k_hb_march(const ReplicaParams *__rest
         heff[l] = (g[l][pos + o] + g[l][pos - 1 + o]) +
                   (g[l][pos + GW] + g[l][pos - GW]) + (qp[l] + qm[l]);
       Xoro gg = xoro_seeded(site_key(key, ((uint64_t)z * N + y) * N + 2 * xh + o));
-      hb_decide(phi_o, heff, Lambda2, lambda, H, rdtg, gg, phi_n, cnt, dSd, dSu, true);
+      hb_decide(phi_o, heff, Lambda2, lambda, H, rdtg, gg, phi_n, mt);
       pend_i = idx(xh, y, z);
 #pragma unroll
       for (int l = 0; l < 4; l++) {
@@ -458,51 +555,55 @@ __global__ __launch_bounds__(kBlock) void k_hb_march(const ReplicaParams *__rest
     }
   }
   if (own && tz > 0) store4(pend_i, pend);
-  block_monitor_add(mon + bid, cnt, dSd, dSu);
+  block_monitor_add(mon + bid, mt);
 }
 
 
 // ------------------------------------------------------------------------
 // modelg_update_charge_pair (Stepper.cxx:419-441) for one component of one
 // pair, applied as nA + (-q), nB + q; counts the decision when count.
-// The constants of a charge sweep: the proposal width and the divisor 2 chi
-// of dS with its rounded reciprocal.
+// The constants of a charge sweep: the proposal width, the divisor d = 2 chi
+// of dS with its rounded reciprocal, and -log2(e) / d in single precision.
 struct ChargeK {
   double rms, d, inv;
+  float l2;
 };
 __device__ __forceinline__ ChargeK charge_k(double rms, double chi) {
-  const double d = 2. * chi;
-  return {rms, d, 1. / d};
+  const double d = 2. * chi, inv = 1. / d;
+  return {rms, d, inv, (float)(-0x1.71547652b82fep+0 * inv)};
 }
 // x / d from the rounded reciprocal with one Markstein correction: q0 = x *
 // inv, the residual x - q0 d exact with one FMA, q0 + residual * inv rounded
 // once.  It equals the IEEE quotient for these divisors (no difference in
 // 1.6e8 random dividends over eight values of chi, including the defaults;
 // the CPU suite checks it); a one-ulp difference could only change a
-// decision if the uniform draw fell within that ulp of exp(-dS).  Three
-// instructions instead of the division's ten.
+// decision if the uniform draw fell within that ulp of exp(-dS).
 __device__ __forceinline__ double div_by(double x, const ChargeK &k) {
   const double q0 = x * k.inv;
   return fma(fma(-q0, k.d, x), k.inv, q0);
 }
 
+// The decision goes by X = dS d: its sign is that of dS, the single-precision
+// test needs exp2(X l2), the monitor sums X (scaled by inv at the end of the
+// launch), and only the double test divides.
 __device__ __forceinline__ void charge_pair(double nA, double nB, const ChargeK &k,
-                                            Xoro &g, double &outA, double &outB, uint64_t &cnt,
-                                            double &dSd, double &dSu, bool count) {
-  double q = k.rms * variance1(g);
-  const double dS = div_by((nA - q) * (nA - q) + (nB + q) * (nB + q) - nA * nA - nB * nB, k);
-  if (dS < 0) {
-    if (count) { cnt += mon_pack(1, 0, 0); dSd += dS; }
-  } else {
-    if (accept_draw(xoro_next(g), -dS)) {
-      if (count) { cnt += mon_pack(0, 1, 0); dSu += dS; }
-    } else {
-      if (count) cnt += mon_pack(0, 0, 1);
-      q = 0.;
-    }
+                                            Xoro &g, double &outA, double &outB, Tally &m,
+                                            bool count) {
+  const double q = k.rms * variance1(g);
+  const double X = (nA - q) * (nA - q) + (nB + q) * (nB + q) - nA * nA - nB * nB;
+  const uint64_t down = lanes(X < 0);
+  // the uniform draw: the engine advances where it is needed
+  const uint64_t u = g.s0 + g.s1;
+  if (!in_lanes(down)) (void)xoro_next(g);
+  const uint64_t accept = accept_draw(u, __builtin_amdgcn_exp2f((float)X * k.l2), down,
+                                      [&] { return -div_by(X, k); });
+  tally(m, X, down, accept & ~down, lanes(count));
+  outA = nA;
+  outB = nB;
+  if (in_lanes(accept)) {
+    outA = nA - q;
+    outB = nB + q;
   }
-  outA = nA + (-q);
-  outB = nB + q;
 }
 
 // The two sub-sweeps of one direction (the shuffled order always runs both
@@ -515,10 +616,9 @@ __device__ __forceinline__ void charge_pair(double nA, double nB, const ChargeK 
 // the monitor counts it once, from the thread on its right.  Reads the live
 // charge buffer, writes A' and B' into the other one.
 template <typename T, bool W>
-__device__ __forceinline__ void charge_line(const ReplicaParams &p, int cur, int nxt, int dir,
-                                            int e1, int e2, uint32_t xh, uint32_t y, uint32_t z,
-                                            uint64_t k1, uint64_t k2, uint64_t &cnt,
-                                            double &dSd, double &dSu) {
+__device__ __forceinline__ void charge_line(const ReplicaParams &p, const ChargePlanes<T, W> &f,
+                                            int dir, int e1, int e2, uint32_t xh, uint32_t y, uint32_t z,
+                                            uint64_t k1, uint64_t k2, Tally &m) {
   const uint32_t N = p.N, NH = p.NH;
   const uint32_t x = site_x(xh, y, z, e2);
   // the four sites along the direction: L, A', B', R (parities e1 e2 e1 e2)
@@ -535,50 +635,33 @@ __device__ __forceinline__ void charge_line(const ReplicaParams &p, int cur, int
     lin[k] = (zz * N + yy) * N + xx;
   }
   const ChargeK ck = charge_k(p.rms, p.chi);
-  const FieldBufs fb = field_bufs<T>(p);
   Xoro gL = xoro_seeded(site_key(k1, lin[0]));
   Xoro gB = xoro_seeded(site_key(k1, lin[2]));
   Xoro gA = xoro_seeded(site_key(k2, lin[1]));
-  uint64_t c0 = 0;
-  double sd0 = 0., su0 = 0.;
+  tally_all(m, 12, true);
   // every load of the line before the first store (see charge_column)
-  double w[6][4];
+  T w[6][4];
 #pragma unroll
-  for (int L = 4; L < 10; L++) {
-    const GPlane<T, W> f1 = gplane<T, W>(fb, cur, L, e1), f2 = gplane<T, W>(fb, cur, L, e2);
-    w[L - 4][0] = f1.ld(ii[0]);
-    w[L - 4][1] = f2.ld(ii[1]);
-    w[L - 4][2] = f1.ld(ii[2]);
-    w[L - 4][3] = f2.ld(ii[3]);
+  for (int c = 0; c < 6; c++) {
+    w[c][0] = f.ld(c, e1, ii[0]);
+    w[c][1] = f.ld(c, e2, ii[1]);
+    w[c][2] = f.ld(c, e1, ii[2]);
+    w[c][3] = f.ld(c, e2, ii[3]);
   }
 #pragma unroll
-  for (int L = 4; L < 10; L++) {
-    const double vL = w[L - 4][0];
-    const double vA = w[L - 4][1];
-    const double vB = w[L - 4][2];
-    const double vR = w[L - 4][3];
+  for (int c = 0; c < 6; c++) {
+    const double vL = w[c][0], vA = w[c][1], vB = w[c][2], vR = w[c][3];
     double tL, a1, b1, tR;
-    charge_pair(vL, vA, ck, gL, tL, a1, cnt, dSd, dSu, true);
-    charge_pair(vB, vR, ck, gB, b1, tR, c0, sd0, su0, false);
+    charge_pair(vL, vA, ck, gL, tL, a1, m, true);
+    charge_pair(vB, vR, ck, gB, b1, tR, m, false);
     // the first sub-sweep's results as stored (rounded in FP32 storage)
     a1 = (double)(T)a1;
     b1 = (double)(T)b1;
     double a2, b2;
-    charge_pair(a1, b1, ck, gA, a2, b2, cnt, dSd, dSu, true);
-    gplane<T, W>(fb, nxt, L, e2).st(ii[1], a2);
-    gplane<T, W>(fb, nxt, L, e1).st(ii[2], b2);
+    charge_pair(a1, b1, ck, gA, a2, b2, m, true);
+    f.st(c, e2, ii[1], (T)a2);
+    f.st(c, e1, ii[2], (T)b2);
   }
-}
-
-// Lane 0's value of v, uniform over the wave (v_readfirstlane per word).
-__device__ __forceinline__ float first_lane(float v) {
-  return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v)));
-}
-__device__ __forceinline__ double first_lane(double v) {
-  const long long bits = __double_as_longlong(v);
-  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)bits);
-  const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(bits >> 32));
-  return __longlong_as_double(((long long)hi << 32) | lo);
 }
 
 // The x direction with a whole row in one wavefront or in one aligned
@@ -593,15 +676,13 @@ __device__ __forceinline__ double first_lane(double v) {
 // same counter streams as charge_line.  Index logic checked on the CPU
 // against the plain two sub-sweeps (exact integer stand-in, N = 4 ... 256).
 template <typename T, bool W, int H>
-__device__ __forceinline__ void charge_row_wave(const ReplicaParams &p, int cur, int nxt, int e1,
-                                                int e2, uint32_t y, uint32_t z, int lane, int seg,
-                                                uint64_t k1, uint64_t k2, uint64_t &cnt,
-                                                double &dSd, double &dSu) {
+__device__ __forceinline__ void charge_row_wave(const ReplicaParams &p, const ChargePlanes<T, W> &f,
+                                                int e1, int e2, uint32_t y, uint32_t z, int lane, int seg,
+                                                uint64_t k1, uint64_t k2, Tally &m) {
   static_assert(H == 1 || H == 2, "rows of up to 128 half-columns");
   const uint32_t N = p.N, NH = p.NH;
   const uint32_t row = z * N + y;
   const ChargeK ck = charge_k(p.rms, p.chi);
-  const FieldBufs fb = field_bufs<T>(p);
   // a1: updated A'_h; r: updated L_{h+1} from lane + 1; l0: lane 0's updated
   // L (H = 2 only); all as stored (T), which is how the second sub-sweep reads
   // them, so that FP32 fields hold and shuffle half the registers
@@ -614,15 +695,16 @@ __device__ __forceinline__ void charge_row_wave(const ReplicaParams &p, int cur,
     const uint32_t iA = row * NH + h, iL = row * NH + (xl >> 1);
     T wl[6], wa[6];  // as stored: converted where used
 #pragma unroll
-    for (int L = 4; L < 10; L++) {
-      wl[L - 4] = gplane<T, W>(fb, cur, L, e1).raw(iL);
-      wa[L - 4] = gplane<T, W>(fb, cur, L, e2).raw(iA);
+    for (int c = 0; c < 6; c++) {
+      wl[c] = f.ld(c, e1, iL);
+      wa[c] = f.ld(c, e2, iA);
     }
     Xoro gL = xoro_seeded(site_key(k1, row * N + xl));
+    tally_all(m, 12, true);  // the six of this sub-sweep and the second's
 #pragma unroll
     for (int c = 0; c < 6; c++) {
       double tl, ta;
-      charge_pair((double)wl[c], (double)wa[c], ck, gL, tl, ta, cnt, dSd, dSu, true);
+      charge_pair((double)wl[c], (double)wa[c], ck, gL, tl, ta, m, true);
       // the first sub-sweep's results as stored (rounded in FP32 storage)
       const T tls = (T)tl;
       a1[j][c] = (T)ta;
@@ -645,9 +727,9 @@ __device__ __forceinline__ void charge_row_wave(const ReplicaParams &p, int cur,
       // H = 2: lane 63's B'_h is lane 0's L of the next j (wrapping to j = 0)
       const double nb = (double)((H > 1 && lane == 63) ? l0[(j + 1) % H][c] : r[j][c]);
       double a2, b2;
-      charge_pair((double)a1[j][c], nb, ck, gA, a2, b2, cnt, dSd, dSu, true);
-      gplane<T, W>(fb, nxt, 4 + c, e2).st(row * NH + h, a2);
-      gplane<T, W>(fb, nxt, 4 + c, e1).st(row * NH + (xb >> 1), b2);
+      charge_pair((double)a1[j][c], nb, ck, gA, a2, b2, m, true);
+      f.st(c, e2, row * NH + h, (T)a2);
+      f.st(c, e1, row * NH + (xb >> 1), (T)b2);
     }
   }
 }
@@ -665,13 +747,11 @@ __device__ __forceinline__ void charge_row_wave(const ReplicaParams &p, int cur,
 //  * d = x: pairs lie in rows; the thread runs charge_line for the row
 //    (y, z) of each z of its chunk.
 template <typename T, bool W, bool PIPE>
-__device__ __forceinline__ void charge_column(const ReplicaParams &p, int cur, int nxt, int dir,
-                                              int e1, int e2, uint32_t x, uint32_t q, int c0,
-                                              int c1, uint64_t k1, uint64_t k2, uint64_t &cnt,
-                                              double &dSd, double &dSu) {
+__device__ __forceinline__ void charge_column(const ReplicaParams &p, const ChargePlanes<T, W> &f,
+                                              int dir, int e1, int e2, uint32_t x, uint32_t q, int c0,
+                                              int c1, uint64_t k1, uint64_t k2, Tally &m) {
   const int N = p.N, NH = p.NH;
   const ChargeK ck = charge_k(p.rms, p.chi);
-  const FieldBufs fb = field_bufs<T>(p);
   // index / linear site of position m along the column
   auto at = [&](int m, uint32_t &ii, uint32_t &lin) __attribute__((always_inline)) {
     const uint32_t row = dir == 2 ? (uint32_t)m * N + q : q * N + (uint32_t)m;
@@ -697,16 +777,16 @@ __device__ __forceinline__ void charge_column(const ReplicaParams &p, int cur, i
   uint32_t si0 = 0, si1 = 0;
   auto load_pair = [&](uint32_t i1, uint32_t i2) __attribute__((always_inline)) {
 #pragma unroll
-    for (int L = 4; L < 10; L++) {
-      n1[L - 4] = gplane<T, W>(fb, cur, L, e1).raw(i1);
-      n2[L - 4] = gplane<T, W>(fb, cur, L, e2).raw(i2);
+    for (int c = 0; c < 6; c++) {
+      n1[c] = f.ld(c, e1, i1);
+      n2[c] = f.ld(c, e2, i2);
     }
   };
   auto store_pending = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int L = 4; L < 10; L++) {
-      gplane<T, W>(fb, nxt, L, e2).template put_raw<false>(si0, s0[L - 4]);
-      gplane<T, W>(fb, nxt, L, e1).template put_raw<false>(si1, s1[L - 4]);
+    for (int c = 0; c < 6; c++) {
+      f.st(c, e2, si0, s0[c]);
+      f.st(c, e1, si1, s1[c]);
     }
   };
   const int npair = (c1 - c0) / 2;
@@ -716,13 +796,15 @@ __device__ __forceinline__ void charge_column(const ReplicaParams &p, int cur, i
     pair_at(0, m1, i1, l1, i2, l2);
     load_pair(i1, i2);
   }
-  double up[6];  // upper site of the previous first-parity pair
+  T up[6];  // upper site of the previous first-parity pair, as stored
   for (int k = 0; k <= npair; k++) {
     const int mm = mm0 + 2 * k;
     int m1;
     uint32_t i1, l1, i2, l2;
     pair_at(k, m1, i1, l1, i2, l2);
     const bool own1 = mm >= c0 && mm < c1;
+    tally_all(m, 6, own1);
+    if (k > 0) tally_all(m, 6, true);
     Xoro g1 = xoro_seeded(site_key(k1, l1));
     Xoro g2;
     uint32_t i0 = 0, l0;
@@ -731,12 +813,12 @@ __device__ __forceinline__ void charge_column(const ReplicaParams &p, int cur, i
       at(m0, i0, l0);
       g2 = xoro_seeded(site_key(k2, l0));
     }
-    double w1[6], w2[6];
+    T w1[6], w2[6];  // as stored: converted where used
     if (PIPE) {
 #pragma unroll
-      for (int L = 4; L < 10; L++) {
-        w1[L - 4] = (double)n1[L - 4];
-        w2[L - 4] = (double)n2[L - 4];
+      for (int c = 0; c < 6; c++) {
+        w1[c] = n1[c];
+        w2[c] = n2[c];
       }
       if (k < npair) {
         int mn;
@@ -751,31 +833,29 @@ __device__ __forceinline__ void charge_column(const ReplicaParams &p, int cur, i
       // planes and would otherwise wait for each component's load after the
       // previous store
 #pragma unroll
-      for (int L = 4; L < 10; L++) {
-        w1[L - 4] = gplane<T, W>(fb, cur, L, e1).ld(i1);
-        w2[L - 4] = gplane<T, W>(fb, cur, L, e2).ld(i2);
+      for (int c = 0; c < 6; c++) {
+        w1[c] = f.ld(c, e1, i1);
+        w2[c] = f.ld(c, e2, i2);
       }
     }
 #pragma unroll
-    for (int L = 4; L < 10; L++) {
-      const double v1 = w1[L - 4];
-      const double v2 = w2[L - 4];
+    for (int c = 0; c < 6; c++) {
       double a, b;
-      charge_pair(v1, v2, ck, g1, a, b, cnt, dSd, dSu, own1);
-      a = (double)(T)a;
-      b = (double)(T)b;
+      charge_pair((double)w1[c], (double)w2[c], ck, g1, a, b, m, own1);
+      // as stored (rounded in FP32 storage)
+      const T as = (T)a, bs = (T)b;
       if (k > 0) {
         double o0, o1;
-        charge_pair(up[L - 4], a, ck, g2, o0, o1, cnt, dSd, dSu, true);
+        charge_pair((double)up[c], (double)as, ck, g2, o0, o1, m, true);
         if (PIPE) {
-          s0[L - 4] = (T)o0;
-          s1[L - 4] = (T)o1;
+          s0[c] = (T)o0;
+          s1[c] = (T)o1;
         } else {
-          gplane<T, W>(fb, nxt, L, e2).st(i0, o0);
-          gplane<T, W>(fb, nxt, L, e1).st(i1, o1);
+          f.st(c, e2, i0, (T)o0);
+          f.st(c, e1, i1, (T)o1);
         }
       }
-      up[L - 4] = b;
+      up[c] = bs;
     }
     if (PIPE && k > 0) {
       si0 = i0;
@@ -787,7 +867,7 @@ __device__ __forceinline__ void charge_column(const ReplicaParams &p, int cur, i
 
 template <typename T, bool W, bool XW>
 __global__ __launch_bounds__(kBlock)
-__attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && XW ? 4 : 1))) void k_charge_march(const ReplicaParams *__restrict__ P,
+__attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 && XW ? 3 : 4))) void k_charge_march(const ReplicaParams *__restrict__ P,
                                                          const ReplicaState *__restrict__ S,
                                                          const int *__restrict__ blk_rep,
                                                          const int *__restrict__ blk_first,
@@ -808,10 +888,9 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && XW ? 4 : 1))) void k_charge
   const int t = threadIdx.x;
   const uint32_t xh = bx * TXH + t % TXH, q = bq * TQ + t / TXH;
   const int c0 = bc * C, c1 = min(c0 + C, N);
-  uint64_t cnt = 0;
-  double dSd = 0., dSu = 0.;
+  Tally mt;
   if (xh < (uint32_t)NH && q < (uint32_t)N && t < TXH * TQ) {
-    const int cur = live(s) ^ flip, nxt = cur ^ 2;
+    const ChargePlanes<T, W> f(p, first_lane(live(s) ^ flip));
     // the shuffled sub-sweep order of ModelGChargeHB::step
     // (Stepper.cxx:461-468) from the sweep's shuffle stream, the counter
     // before the first direction's two; every thread draws the same order
@@ -820,10 +899,10 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && XW ? 4 : 1))) void k_charge
       Xoro g = xoro_seeded(site_key(stream_key(p.base_key, s.sweep_ctr + ctr_off - 1 - 2 * ixyz), 0));
       shuffle_orders(g, order);
     }
-    const int dir = order[ixyz];
-    const int e1 = order[3], e2 = order[4];
-    const uint64_t k1 = stream_key(p.base_key, s.sweep_ctr + ctr_off);
-    const uint64_t k2 = stream_key(p.base_key, s.sweep_ctr + ctr_off + 1);
+    const int dir = first_lane(ixyz == 0 ? order[0] : (ixyz == 1 ? order[1] : order[2]));
+    const int e1 = first_lane(order[3]), e2 = e1 ^ 1;
+    const uint64_t k1 = first_lane(stream_key(p.base_key, s.sweep_ctr + ctr_off));
+    const uint64_t k2 = first_lane(stream_key(p.base_key, s.sweep_ctr + ctr_off + 1));
     if (XW && dir == 0) {  // every replica of the launch has NH = 64 or 128
       // whole rows in one wavefront (TXH = 64, TQ = 4: wave w takes row q);
       // the chunk's planes are split over the nbx x-blocks
@@ -832,30 +911,26 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && XW ? 4 : 1))) void k_charge
       const int zs = c0 + bx * len / nbx, ze = c0 + (bx + 1) * len / nbx;
       for (int z = zs; z < ze; z++) {
         if (NH == 64)
-          charge_row_wave<T, W, 1>(p, cur, nxt, e1, e2, q, (uint32_t)z, lane, 64, k1, k2, cnt,
-                                   dSd, dSu);
+          charge_row_wave<T, W, 1>(p, f, e1, e2, q, (uint32_t)z, lane, 64, k1, k2, mt);
         else
-          charge_row_wave<T, W, 2>(p, cur, nxt, e1, e2, q, (uint32_t)z, lane, 64, k1, k2, cnt,
-                                   dSd, dSu);
+          charge_row_wave<T, W, 2>(p, f, e1, e2, q, (uint32_t)z, lane, 64, k1, k2, mt);
       }
     } else if (dir == 0 && TXH == NH && NH <= 64 && (NH & (NH - 1)) == 0) {
       // whole rows in aligned segments of NH lanes: with TXH = NH thread t
       // takes half-column t % NH of the tile's row t / NH, and NH divides
       // the wavefront, so a row never straddles two waves
       for (int z = c0; z < c1; z++)
-        charge_row_wave<T, W, 1>(p, cur, nxt, e1, e2, q, (uint32_t)z, (int)xh, NH, k1, k2, cnt,
-                                 dSd, dSu);
+        charge_row_wave<T, W, 1>(p, f, e1, e2, q, (uint32_t)z, (int)xh, NH, k1, k2, mt);
     } else if (dir == 0) {
       for (int z = c0; z < c1; z++)
-        charge_line<T, W>(p, cur, nxt, 0, e1, e2, xh, q, (uint32_t)z, k1, k2, cnt, dSd, dSu);
+        charge_line<T, W>(p, f, 0, e1, e2, xh, q, (uint32_t)z, k1, k2, mt);
     } else {
 #pragma unroll 1
       for (int sx = 0; sx < 2; sx++)
-        charge_column<T, W, XW>(p, cur, nxt, dir, e1, e2, 2 * xh + sx, q, c0, c1, k1, k2, cnt,
-                                dSd, dSu);
+        charge_column<T, W, XW>(p, f, dir, e1, e2, 2 * xh + sx, q, c0, c1, k1, k2, mt);
     }
   }
-  block_monitor_add(mon + bid, cnt, dSd, dSu);
+  block_monitor_add(mon + bid, mt, 1. / (2. * p.chi));
 }
 
 // ------------------------------------------------------------------------
@@ -1507,11 +1582,11 @@ void launch_charge_march(bool fp32, const Plan &plan, const ReplicaParams *P, Re
 #define LGV_CHARGE(TT, WW, XX)                                                         \
   k_charge_march<TT, WW, XX><<<g, kBlock, 0, st>>>(P, S, br, bf, ixyz, ctr_off, flip, mon)
   if (plan.xwave) {
-    if (fp32) { if (plan.wide) LGV_CHARGE(float, true, true); else LGV_CHARGE(float, false, true); }
-    else { if (plan.wide) LGV_CHARGE(double, true, true); else LGV_CHARGE(double, false, true); }
+    if (fp32) { if (plan.far) LGV_CHARGE(float, true, true); else LGV_CHARGE(float, false, true); }
+    else { if (plan.far) LGV_CHARGE(double, true, true); else LGV_CHARGE(double, false, true); }
   } else {
-    if (fp32) { if (plan.wide) LGV_CHARGE(float, true, false); else LGV_CHARGE(float, false, false); }
-    else { if (plan.wide) LGV_CHARGE(double, true, false); else LGV_CHARGE(double, false, false); }
+    if (fp32) { if (plan.far) LGV_CHARGE(float, true, false); else LGV_CHARGE(float, false, false); }
+    else { if (plan.far) LGV_CHARGE(double, true, false); else LGV_CHARGE(double, false, false); }
   }
 #undef LGV_CHARGE
 }
