@@ -318,7 +318,7 @@ def run_single(L, N, fp32, steps, warmup, graph=False, tune=True, ideal_tile=Non
         "value": value, "ms_per_step": el * 1e3 / steps, "steps": steps, "warmup": warmup,
         "dtype": "f32-storage/f64-arith" if fp32 else "f64",
         "workload": f"ModelG {N}^3 PV2HBSplit23 {'FP32 fields' if fp32 else 'FP64'}",
-        "ideal_tile": list(tuned[N][:2]) if tuned else "default (32, 16)",
+        "ideal_tile": list(tuned[N][:2]) if tuned else "default",
         "sweep_tiles": list(sweeps[N]) if sweeps else "default",
         "phi_kernel": kern["phi"],
         "kernel_timing": ("a pass of stream launches after the timed graph replays" if graph else

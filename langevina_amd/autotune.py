@@ -16,7 +16,7 @@ from .lgv import _check, lib
 CAPS = (8, 16, 32, 64)
 # short z chunks give a small lattice (one 64^3 replica: 32 blocks with the
 # default tile) more blocks than the march's depth costs it
-TZS = (2, 4, 8, 16, 32, 64)
+TZS = (1, 2, 4, 8, 16, 32, 64)
 CHARGE_CAPS = (16, 32, 64)
 CHARGE_CHUNKS = (2, 4, 8, 16, 32)
 HB_CAPS = (16, 32, 64)
@@ -29,11 +29,16 @@ def set_ideal_tile(ctx, replica, cap, tz):
     _check(L.lgv_set_ideal_tile(ctx.h, replica, cap, tz))
 
 
+def ideal_caps(N):
+    """Tile widths tried at side N: powers of two and even splits of the row."""
+    NH = N // 2
+    return sorted({c for c in CAPS if c <= max(NH, 2)} |
+                  {c for c in (-(-NH // k) for k in (1, 2, 3)) if 8 <= c <= 64})
+
+
 def charge_eff(N, cap, chunk):
-    """The charge tile (TXH, C) a (cap, chunk) request gives (0 = default)."""
-    c = cap or 64
-    ch = chunk or (16 if N >= 128 else 8)
-    return min(c, N // 2), min(ch, N)
+    """The charge tile (TXH, C) a (cap, chunk) request gives."""
+    return min(cap, N // 2), min(chunk, N)
 
 
 def hb_eff(N, cap, tz):
@@ -132,7 +137,7 @@ def autotune_sweeps(ctx, dt, march=None, steps=3, verbose=False):
             print(f"autotune phi kernel: {'march' if march else 'site'} {ms:.3f} ms/step",
                   flush=True)
     for N in sizes:
-        cands, seen = [(0, 0)], {charge_eff(N, 0, 0)}
+        cands, seen = [(0, 0)], set()
         for cap in CHARGE_CAPS:
             for ch in CHARGE_CHUNKS:
                 if ch <= N and charge_eff(N, cap, ch) not in seen:
@@ -196,8 +201,8 @@ def autotune_ideal(ctx, dt, steps=3, cache_path=None, verbose=False):
             for _ in range(WARMUP):
                 ctx.step(dt)
             warmed = True
-        cands = [(32, 16)] + [(cap, tz) for cap in CAPS for tz in TZS
-                              if cap <= max(N // 2, 2) and tz <= N and (cap, tz) != (32, 16)]
+        cands = [(32, 16)] + [(cap, tz) for cap in ideal_caps(N) for tz in TZS
+                              if tz <= N and (cap, tz) != (32, 16)]
         (cap, tz), ms = _search(ctx, dt, steps, "ideal", apply, cands)
         if verbose:
             print(f"autotune ideal N={N}: cap={cap} tz={tz} {ms * 1e3:.1f} us", flush=True)

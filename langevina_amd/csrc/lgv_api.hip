@@ -78,6 +78,11 @@ struct HostNoise {
 
 }  // namespace
 
+// Tiles a caller asked for; 0: the library's rule.
+struct TileRequest {
+  int ideal_cap = 0, ideal_tz = 0, hb_cap = 0, hb_tz = 0, chg_cap = 0, chg_chunk = 0;
+};
+
 struct lgv_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -92,6 +97,7 @@ struct lgv_ctx {
   int nrep = 0;
   std::vector<lgv_model_params> mp;
   std::vector<ReplicaParams> hp;
+  std::vector<TileRequest> tiles;  // per replica; hp holds the resolved tiles
   std::vector<HostNoise> noise;
   ReplicaParams *dP = nullptr;
   ReplicaState *dS = nullptr;
@@ -186,9 +192,75 @@ int free_plan(Plan &plan) {
   return LGV_OK;
 }
 
+constexpr int kCUs = 256;  // MI355X
+
+// Width of an x tile of at most cap half-columns that splits a row of NH
+// evenly: with a fixed width of 32 or 64 the last tile of a row whose length
+// is no multiple of it is mostly empty (NH = 75 in tiles of 64: 59 % of the
+// lanes at work; in two of 38, 99 %).
+int even_width(int NH, int cap) {
+  const int n = (NH + cap - 1) / cap;
+  return (NH + n - 1) / n;
+}
+
+// Blocks of one z plane of the ideal kernel with tiles of width cap.
+int64_t ideal_plane_blocks(const ReplicaParams &p, int cap) {
+  int TXH, TY, TZ;
+  ideal_tile(p.N, cap, 1, TXH, TY, TZ);
+  return (int64_t)((p.NH + TXH - 1) / TXH) * ((p.N + TY - 1) / TY);
+}
+
+// The ideal kernel's tiles where the caller asked for none.  Width: 32
+// half-columns where they divide the row (whole 128-byte lines of every
+// component: 256^3 FP64 541 us against 560 with 64) or need fewer tiles than
+// the alternative, which is the widest even split that the kernel's plane grid
+// holds (every ring column costs a line per row and component: 200^3 FP64 329
+// us with 50, 390 with 34, 435 with 25; 224^3 FP32 305 us with 32, 334 with
+// 38).  Depth: a block marches TZ planes and rotates one more on either side,
+// and the GPU holds `slots` blocks at a time, so a launch takes about
+// ceil(blocks / slots) rounds of TZ + 2.5 planes each; TZ minimises that, up to
+// 16 (from there on the planes above and below are a small share).  FP64 with
+// 32 x 16 tiles -> with the rule's: 32^3 54 -> 12 us (TZ 1), 64^3 60 -> 17
+// (TZ 1), 100^3 66 -> 41 (50 wide, TZ 4), 128^3 89 -> 79 (TZ 8), 150^3 215 ->
+// 153 (38 wide), 200^3 443 -> 320 (50 wide, TZ 8); 256^3 and the 96-replica
+// batch keep 32 x 16.
+void resolve_ideal_tiles(lgv_ctx *c) {
+  const int slots = kCUs * (c->fp32 ? 3 : 2);
+  for (int r = 0; r < c->nrep; r++) {
+    ReplicaParams &p = c->hp[r];
+    p.tile_cap = c->tiles[r].ideal_cap;
+    if (p.tile_cap) continue;
+    for (int cap = 64; cap >= 32 || !p.tile_cap; cap--) {
+      int TXH, TY, TZ;
+      ideal_tile(p.N, even_width(p.NH, cap), 1, TXH, TY, TZ);
+      if ((TY + 2) * (2 * TXH + 2) <= ideal_lds(c->fp32)) {
+        p.tile_cap = TXH;
+        break;
+      }
+    }
+    if (p.NH % 32 == 0 || ideal_plane_blocks(p, 32) < ideal_plane_blocks(p, p.tile_cap))
+      p.tile_cap = 32;
+  }
+  int best = 16;
+  double best_cost = 1e300;
+  for (int tz = 16; tz >= 1; tz--) {
+    int64_t blocks = 0;
+    for (const ReplicaParams &p : c->hp)
+      blocks += ideal_plane_blocks(p, p.tile_cap) * ((p.N + tz - 1) / tz);
+    const double cost = ((blocks + slots - 1) / slots) * (tz + 2.5);
+    if (cost < best_cost * 0.98) {
+      best = tz;
+      best_cost = cost;
+    }
+  }
+  for (int r = 0; r < c->nrep; r++)
+    c->hp[r].tile_tz = c->tiles[r].ideal_tz ? c->tiles[r].ideal_tz : best;
+}
+
 // Blocks of the fused ideal kernel: one per (x-tile, y-tile, z-chunk) of
 // every replica, with that replica's tile shape.
 int build_ideal_plan(lgv_ctx *c) {
+  resolve_ideal_tiles(c);
   std::vector<int64_t> work;
   for (int r = 0; r < c->nrep; r++) {
     const ReplicaParams &p = c->hp[r];
@@ -214,7 +286,9 @@ int build_ideal_plan(lgv_ctx *c) {
 int build_hb_plan(lgv_ctx *c) {
   std::vector<int64_t> work;
   for (int r = 0; r < c->nrep; r++) {
-    const ReplicaParams &p = c->hp[r];
+    ReplicaParams &p = c->hp[r];
+    p.hb_cap = c->tiles[r].hb_cap;
+    p.hb_tz = c->tiles[r].hb_tz;
     int TXH, TY, TZ;
     hb_tile(p.N, p.hb_cap, p.hb_tz, TXH, TY, TZ);
     if ((TY + 2) * (TXH + 2) > kHbMarchGrid || 2 * TY + 2 * TXH > kBlock)
@@ -229,30 +303,71 @@ int build_hb_plan(lgv_ctx *c) {
   return rc;
 }
 
+// Whether the x sub-sweeps of every replica run whole rows per wavefront
+// (charge_row_wave with two half-columns per lane or one): NH = 64 or 128 and
+// a tile of 64 half-columns x 4 lines.
+bool charge_rows(const lgv_ctx *c) {
+  bool rows = true;
+  for (const ReplicaParams &p : c->hp) {
+    int TXH, TQ, C;
+    charge_tile(p.N, p.chg_cap, 2, TXH, TQ, C);
+    rows = rows && (p.NH == 64 || p.NH == 128) && TXH == 64 && TQ == 4;
+  }
+  return rows;
+}
+
+// The charge march's tiles where the caller asked for none.  Width: an even
+// split of the row into at most 64 half-columns.  Chunk: a chunk of C sites
+// updates C/2 + 1 first-parity pairs for its C/2 second-parity ones, and the
+// GPU holds `slots` blocks at a time, so a launch takes about ceil(blocks /
+// slots) rounds of C/2 + 1.5 pairs; C of 16, 8, 4, 2 minimises that.  Measured
+// for C = 16, 8, 4, 2, FP64: 256^3 327, 329, 334, 462 us; 200^3 225, 213, 210,
+// 219; 160^3 114, 105, 106, 126; 128^3 49, 50, 50, 64; 100^3 36, 31, 29, 33;
+// 64^3 31, 21, 17, 16; FP32: 256^3 226, 242, 274, 401; 128^3 39, 36, 39, 50;
+// 32^3 29, 18, 13, 10.
+void resolve_charge_tiles(lgv_ctx *c) {
+  for (int r = 0; r < c->nrep; r++) {
+    ReplicaParams &p = c->hp[r];
+    p.chg_cap = c->tiles[r].chg_cap ? c->tiles[r].chg_cap : even_width(p.NH, 64);
+  }
+  const int slots = kCUs * (!c->fp32 && charge_rows(c) ? 3 : 4);
+  int best = 16;
+  double best_cost = 1e300;
+  for (int chunk = 16; chunk >= 2; chunk /= 2) {
+    int64_t blocks = 0;
+    for (const ReplicaParams &p : c->hp) {
+      int TXH, TQ, C;
+      charge_tile(p.N, p.chg_cap, chunk, TXH, TQ, C);
+      blocks += (int64_t)2 * ((p.NH + TXH - 1) / TXH) * ((p.N + TQ - 1) / TQ) *
+                ((p.N + C - 1) / C);
+    }
+    const double cost = ((blocks + slots - 1) / slots) * (chunk / 2 + 1.5);
+    if (cost < best_cost * 0.98) {
+      best = chunk;
+      best_cost = cost;
+    }
+  }
+  for (int r = 0; r < c->nrep; r++)
+    c->hp[r].chg_chunk = c->tiles[r].chg_chunk ? c->tiles[r].chg_chunk : best;
+}
+
 // Blocks of the charge march kernel: (x-tile, line tile, chunk) per replica.
 int build_charge_plan(lgv_ctx *c) {
+  resolve_charge_tiles(c);
   std::vector<int64_t> work;
   for (int r = 0; r < c->nrep; r++) {
     const ReplicaParams &p = c->hp[r];
     int TXH, TQ, C;
     charge_tile(p.N, p.chg_cap, p.chg_chunk, TXH, TQ, C);
     if (C % 2 != 0) return fail(LGV_ERR_ARG, "replica %d: charge chunk %d is odd", r, C);
-    work.push_back((int64_t)((p.NH + TXH - 1) / TXH) * ((p.N + TQ - 1) / TQ) *
+    // two blocks per tile: the even and the odd x of its half-columns
+    work.push_back((int64_t)2 * ((p.NH + TXH - 1) / TXH) * ((p.N + TQ - 1) / TQ) *
                    ((p.N + C - 1) / C) * kBlock);
   }
   int rc = free_plan(c->plan_charge);
   if (rc) return rc;
   rc = build_plan(c->plan_charge, work, c->wide);
-  // the x sub-sweeps with whole rows per wavefront need NH = 64 or 128 and
-  // a tile of 64 half-columns x 4 lines
-  bool xw = true;
-  for (int r = 0; r < c->nrep; r++) {
-    const ReplicaParams &p = c->hp[r];
-    int TXH, TQ, C;
-    charge_tile(p.N, p.chg_cap, p.chg_chunk, TXH, TQ, C);
-    xw = xw && (p.NH == 64 || p.NH == 128) && TXH == 64 && TQ == 4;
-  }
-  c->plan_charge.xwave = xw;
+  c->plan_charge.xwave = charge_rows(c);
   // the twelve half-planes of the charges in one buffer resource need 32-bit
   // offsets (any size below 448^3 in FP64, 564^3 in FP32)
   const uint64_t esz = c->fp32 ? sizeof(float) : sizeof(double);
@@ -500,6 +615,7 @@ int lgv_create(const lgv_config *cfg, lgv_ctx **out) {
   c->nrep = cfg->nreplicas;
   c->mp.assign(cfg->replicas, cfg->replicas + cfg->nreplicas);
   c->hp.resize(c->nrep);
+  c->tiles.resize(c->nrep);
   c->noise.resize(c->nrep);
   const size_t esz = c->fp32 ? sizeof(float) : sizeof(double);
   std::vector<int64_t> whalf, wfull;
@@ -518,9 +634,6 @@ int lgv_create(const lgv_config *cfg, lgv_ctx **out) {
       c->fields.push_back(field);
       p.fields[b] = field;
     }
-    p.tile_cap = 32;
-    p.tile_tz = 16;
-    p.hb_cap = p.hb_tz = p.chg_cap = p.chg_chunk = 0;
     p.N = N;
     p.NH = N / 2;
     p.half = half;
@@ -563,9 +676,6 @@ int lgv_create(const lgv_config *cfg, lgv_ctx **out) {
       return fail(LGV_ERR_ARG, "LGV_PHI_KERNEL=%s: expected site or march", pk);
     c->phi_march = k == "march";
   }
-  HIPCHECK(hipMalloc(&c->dP, c->nrep * sizeof(ReplicaParams)));
-  HIPCHECK(hipMemcpy(c->dP, c->hp.data(), c->nrep * sizeof(ReplicaParams),
-                     hipMemcpyHostToDevice));
   HIPCHECK(hipMalloc(&c->dS, c->nrep * sizeof(ReplicaState)));
   HIPCHECK(hipMemcpy(c->dS, hs.data(), c->nrep * sizeof(ReplicaState), hipMemcpyHostToDevice));
   int rc;
@@ -574,6 +684,10 @@ int lgv_create(const lgv_config *cfg, lgv_ctx **out) {
   if ((rc = build_ideal_plan(c.get())) != LGV_OK) return rc;
   if ((rc = build_charge_plan(c.get())) != LGV_OK) return rc;
   if ((rc = build_hb_plan(c.get())) != LGV_OK) return rc;
+  // the parameters as the plans' tile rules left them
+  HIPCHECK(hipMalloc(&c->dP, c->nrep * sizeof(ReplicaParams)));
+  HIPCHECK(hipMemcpy(c->dP, c->hp.data(), c->nrep * sizeof(ReplicaParams),
+                     hipMemcpyHostToDevice));
   HIPCHECK(hipMalloc(&c->mon_phi, hb_plan(c.get()).nblocks * sizeof(MonSlot)));
   HIPCHECK(hipMemset(c->mon_phi, 0, hb_plan(c.get()).nblocks * sizeof(MonSlot)));
   HIPCHECK(hipMalloc(&c->mon_charge, c->plan_charge.nblocks * sizeof(MonSlot)));
@@ -1087,15 +1201,15 @@ int lgv_set_ideal_tile(lgv_ctx *c, int r, int txh_cap, int tz) {
   if (txh_cap < 2 || txh_cap > 64 || tz < 1 || tz > 1024)
     return fail(LGV_ERR_ARG, "tile cap %d / tz %d out of range", txh_cap, tz);
   HIPCHECK(hipSetDevice(c->device));
-  std::vector<ReplicaParams> old = c->hp;
+  const std::vector<TileRequest> old = c->tiles;
   for (int i = 0; i < c->nrep; i++) {
     if (r >= 0 && i != r) continue;
-    c->hp[i].tile_cap = txh_cap;
-    c->hp[i].tile_tz = tz;
+    c->tiles[i].ideal_cap = txh_cap;
+    c->tiles[i].ideal_tz = tz;
   }
   int rc = build_ideal_plan(c);
   if (rc) {
-    c->hp = old;
+    c->tiles = old;
     build_ideal_plan(c);
     return rc;
   }
@@ -1118,18 +1232,18 @@ int lgv_set_sweep_tiles(lgv_ctx *c, int r, int hb_cap, int hb_tz, int chg_cap,
   HIPCHECK(hipSetDevice(c->device));
   HIPCHECK(hipStreamSynchronize(c->stream));
   if (int rm = fold_monitors(c)) return rm;
-  std::vector<ReplicaParams> old = c->hp;
+  const std::vector<TileRequest> old = c->tiles;
   for (int i = 0; i < c->nrep; i++) {
     if (r >= 0 && i != r) continue;
-    c->hp[i].hb_cap = hb_cap;
-    c->hp[i].hb_tz = hb_tz;
-    c->hp[i].chg_cap = chg_cap;
-    c->hp[i].chg_chunk = chg_chunk;
+    c->tiles[i].hb_cap = hb_cap;
+    c->tiles[i].hb_tz = hb_tz;
+    c->tiles[i].chg_cap = chg_cap;
+    c->tiles[i].chg_chunk = chg_chunk;
   }
   int rc = build_hb_plan(c);
   if (!rc) rc = build_charge_plan(c);
   if (rc) {
-    c->hp = old;
+    c->tiles = old;
     build_hb_plan(c);
     build_charge_plan(c);
   }

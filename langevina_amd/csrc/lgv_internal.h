@@ -43,9 +43,12 @@ struct ReplicaState {
   double E_old, E_new;
 };
 
+// The tile fields of ReplicaParams hold what a launch uses: the caller's
+// request, or where that is 0 the choice of the rules below (resolve_tiles in
+// lgv_api.hip, by replica size, storage type and the blocks of the launch).
+
 // Tile of the fused ideal kernel: TXH half-columns x TY rows in x-y,
-// marching over TZ planes in z.  txh_cap (8..64) and tz (4..64) are the
-// tunables (0 = defaults 32 and 16); (TY+2)(2 TXH+2) <= kIdealLds.  The
+// marching over TZ planes in z.  (TY+2)(2 TXH+2) <= kIdealLds.  The
 // one-site halo ring (2 TY + 4 TXH sites) may exceed the block's threads
 // (64 half-columns x 4 rows: 264); its remainder then takes a second pass.
 constexpr int kIdealLds = 800;
@@ -54,15 +57,12 @@ constexpr int kIdealLds = 800;
 // 660 entries) and three blocks still fit one CU's LDS.
 constexpr int kIdealLdsF32 = 660;
 __host__ __device__ constexpr int ideal_lds(bool fp32) { return fp32 ? kIdealLdsF32 : kIdealLds; }
-__host__ __device__ inline void ideal_tile(int N, int txh_cap, int tz, int &TXH, int &TY,
-                                           int &TZ) {
+__host__ __device__ inline void ideal_tile(int N, int cap, int tz, int &TXH, int &TY, int &TZ) {
   const int NH = N / 2;
-  const int cap = txh_cap > 0 ? txh_cap : 32;
-  const int zc = tz > 0 ? tz : 16;
   TXH = NH < cap ? NH : cap;
   TY = kBlock / TXH;
   if (TY > N) TY = N;
-  TZ = N < zc ? N : zc;
+  TZ = N < tz ? N : tz;
 }
 
 // Tile of the single-parity phi march: TXH half-columns x TY rows in x-y,
@@ -84,20 +84,15 @@ __host__ __device__ inline void hb_tile(int N, int cap, int tz, int &TXH, int &T
 constexpr int kHbMarchGrid = 400;
 
 // Tile of the charge march kernel: TXH half-columns x TQ lines of the
-// cross-section, chunks of C sites along the direction (C even).  Defaults
-// (cap, chunk = 0): TXH = min(NH, 64) and chunks of 16 from N = 128 on, 8
-// below, where the shorter chunks give small lattices (and batches of them)
-// enough blocks to fill the GPU (measured: 96-replica batch of 32^3-64^3,
-// charge 268 -> 252 us; at 256^3 16 is faster).  cap and chunk are tunables.
+// cross-section, chunks of C sites along the direction (C even), two blocks
+// per tile (the even and the odd x of its half-columns).
 __host__ __device__ inline void charge_tile(int N, int cap, int chunk, int &TXH, int &TQ,
                                             int &C) {
   const int NH = N / 2;
-  const int c = cap > 0 ? cap : 64;
-  TXH = NH < c ? NH : c;
+  TXH = NH < cap ? NH : cap;
   TQ = 256 / TXH;
   if (TQ > N) TQ = N;
-  const int ch = chunk > 0 ? chunk : (N >= 128 ? 16 : 8);
-  C = N < ch ? N : ch;
+  C = N < chunk ? N : chunk;
 }
 
 // Per-block monitor partials (o4_stepper_monitor counters).

@@ -204,11 +204,13 @@ __device__ __forceinline__ void tally_all(Tally &m, int n, bool count) {
 __device__ __forceinline__ void tally(Tally &m, double dS, uint64_t down, uint64_t up,
                                       uint64_t count) {
   uint32_t nd = __builtin_popcountll(down & count), ny = __builtin_popcountll(up & count);
-  if (in_lanes(down & count)) m.dSd += dS;
-  if (in_lanes(up & count)) m.dSu += dS;
+  // one masked add each; written in plain C++ they become an add and two
+  // selects
+  if (in_lanes(down & count)) __asm__ volatile("v_add_f64 %0, %0, %1" : "+v"(m.dSd) : "v"(dS));
+  if (in_lanes(up & count)) __asm__ volatile("v_add_f64 %0, %0, %1" : "+v"(m.dSu) : "v"(dS));
   // counted and summed here and now: otherwise the compiler keeps the masks
   // and dS of a dozen decisions (in spilled registers) for later
-  __asm__ volatile("" : "+s"(nd), "+s"(ny), "+v"(m.dSd), "+v"(m.dSu));
+  __asm__ volatile("" : "+s"(nd), "+s"(ny));
   m.down += nd;
   m.yes += ny;
 }
@@ -593,7 +595,8 @@ __device__ __forceinline__ void charge_pair(double nA, double nB, const ChargeK 
   const double X = (nA - q) * (nA - q) + (nB + q) * (nB + q) - nA * nA - nB * nB;
   const uint64_t down = lanes(X < 0);
   // the uniform draw: the engine advances where it is needed
-  const uint64_t u = g.s0 + g.s1;
+  uint64_t u = g.s0 + g.s1;
+  __asm__ volatile("" : "+v"(u));  // formed before the engine moves on: no copy of its state
   if (!in_lanes(down)) (void)xoro_next(g);
   const uint64_t accept = accept_draw(u, __builtin_amdgcn_exp2f((float)X * k.l2), down,
                                       [&] { return -div_by(X, k); });
@@ -882,6 +885,8 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 && XW ? 3 : 4))) void k_charge
   charge_tile(N, p.chg_cap, p.chg_chunk, TXH, TQ, C);
   const int nbx = (NH + TXH - 1) / TXH, nbq = (N + TQ - 1) / TQ;
   int b = bid - blk_first[r];
+  const int sx = b & 1;
+  b >>= 1;
   const int bx = b % nbx;
   b /= nbx;
   const int bq = b % nbq, bc = b / nbq;
@@ -903,31 +908,33 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 && XW ? 3 : 4))) void k_charge
     const int e1 = first_lane(order[3]), e2 = e1 ^ 1;
     const uint64_t k1 = first_lane(stream_key(p.base_key, s.sweep_ctr + ctr_off));
     const uint64_t k2 = first_lane(stream_key(p.base_key, s.sweep_ctr + ctr_off + 1));
+    // d = x: the chunk's planes, of which this block takes a share
+    const int len = c1 - c0;
     if (XW && dir == 0) {  // every replica of the launch has NH = 64 or 128
       // whole rows in one wavefront (TXH = 64, TQ = 4: wave w takes row q);
-      // the chunk's planes are split over the nbx x-blocks
-      const int lane = t & 63;
-      const int len = c1 - c0;
-      const int zs = c0 + bx * len / nbx, ze = c0 + (bx + 1) * len / nbx;
+      // the chunk's planes are split over the 2 nbx blocks of the row
+      const int lane = t & 63, part = 2 * bx + sx;
+      const int zs = c0 + part * len / (2 * nbx), ze = c0 + (part + 1) * len / (2 * nbx);
       for (int z = zs; z < ze; z++) {
         if (NH == 64)
           charge_row_wave<T, W, 1>(p, f, e1, e2, q, (uint32_t)z, lane, 64, k1, k2, mt);
         else
           charge_row_wave<T, W, 2>(p, f, e1, e2, q, (uint32_t)z, lane, 64, k1, k2, mt);
       }
-    } else if (dir == 0 && TXH == NH && NH <= 64 && (NH & (NH - 1)) == 0) {
-      // whole rows in aligned segments of NH lanes: with TXH = NH thread t
-      // takes half-column t % NH of the tile's row t / NH, and NH divides
-      // the wavefront, so a row never straddles two waves
-      for (int z = c0; z < c1; z++)
-        charge_row_wave<T, W, 1>(p, f, e1, e2, q, (uint32_t)z, (int)xh, NH, k1, k2, mt);
     } else if (dir == 0) {
-      for (int z = c0; z < c1; z++)
-        charge_line<T, W>(p, f, 0, e1, e2, xh, q, (uint32_t)z, k1, k2, mt);
+      const int zs = c0 + sx * len / 2, ze = c0 + (sx + 1) * len / 2;
+      if (TXH == NH && NH <= 64 && (NH & (NH - 1)) == 0) {
+        // whole rows in aligned segments of NH lanes: with TXH = NH thread t
+        // takes half-column t % NH of the tile's row t / NH, and NH divides
+        // the wavefront, so a row never straddles two waves
+        for (int z = zs; z < ze; z++)
+          charge_row_wave<T, W, 1>(p, f, e1, e2, q, (uint32_t)z, (int)xh, NH, k1, k2, mt);
+      } else {
+        for (int z = zs; z < ze; z++)
+          charge_line<T, W>(p, f, 0, e1, e2, xh, q, (uint32_t)z, k1, k2, mt);
+      }
     } else {
-#pragma unroll 1
-      for (int sx = 0; sx < 2; sx++)
-        charge_column<T, W, XW>(p, f, dir, e1, e2, 2 * xh + sx, q, c0, c1, k1, k2, mt);
+      charge_column<T, W, XW>(p, f, dir, e1, e2, 2 * xh + sx, q, c0, c1, k1, k2, mt);
     }
   }
   block_monitor_add(mon + bid, mt, 1. / (2. * p.chi));
