@@ -115,10 +115,11 @@ struct lgv_ctx {
   double coef_hb = NAN, coef_charge = NAN, coef_ideal = NAN;
   double *d_aos = nullptr;
   int maxN = 0;
-  double *d_partXZ = nullptr, *d_partXY = nullptr;
-  // walls, phase walls and their transforms of one measurement, packed for
-  // the current N (see MeasBuf) so that one copy brings them to the host
-  double *d_meas = nullptr;
+  double *d_part = nullptr;  // partial sums of a measurement (see MeasureShape)
+  double *d_meas = nullptr;  // walls and phase walls of one measurement (MeasBuf)
+  // the same and their transforms in pinned host memory, which the kernels
+  // write themselves
+  double *h_meas = nullptr;
   bool use_graph = false;
   int graph_steps = 1;                 // steps per captured graph
   hipGraphExec_t graph_exec = nullptr;  // graph_steps steps
@@ -149,18 +150,18 @@ int slab_planes(int N) {
 }
 
 // Layout of one measurement in a packed buffer for side N: walls [3][11][N],
-// phase walls [3][14][N], their transforms [3][11][nk][2] and [3][14][nk][2].
+// phase walls [3][14][N], their transforms [3][11][nk][2] and [3][14][nk][2]
+// (the device buffer holds the walls only).
 struct MeasBuf {
   double *wall, *wallphase, *wallk, *wallphasek;
-  int64_t total;  // doubles
-  static int64_t size(int N) { return 3 * 25 * (int64_t)N + 3 * 25 * (int64_t)(N / 2 + 1) * 2; }
+  static int64_t walls(int N) { return 3 * 25 * (int64_t)N; }
+  static int64_t size(int N) { return walls(N) + 3 * 25 * (int64_t)(N / 2 + 1) * 2; }
   MeasBuf(double *base, int N) {
     const int64_t nk = N / 2 + 1;
     wall = base;
     wallphase = wall + 3 * 11 * (int64_t)N;
     wallk = wallphase + 3 * 14 * (int64_t)N;
     wallphasek = wallk + 3 * 11 * nk * 2;
-    total = size(N);
   }
 };
 
@@ -559,6 +560,81 @@ int enqueue_step(lgv_ctx *c, int &flip) {
   return off;
 }
 
+// computeDerivedObs's OAverage (measurer.cxx:288-300): mean of wallX rows
+void volume_averages(const double *wall, int N, double *oavg) {
+  for (int l = 0; l < 11; l++) {
+    double s = 0.;
+    for (int i = 0; i < N; i++) s += wall[l * N + i];
+    oavg[l] = s / (double)N;
+  }
+}
+
+// Complex numbers of rotate_to_vev.  Products as std::complex forms them, whose
+// operator* also calls out of line to test every product for NaN (32 products
+// per k: 90 us of a 256^3 measurement); the test is made here, and a NaN goes
+// the library's way.
+struct Cplx {
+  double re, im;
+};
+inline Cplx operator*(const Cplx &a, const Cplx &b) {
+  const Cplx p{a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
+  if (__builtin_expect(p.re != p.re && p.im != p.im, 0)) {
+    const std::complex<double> q =
+        std::complex<double>(a.re, a.im) * std::complex<double>(b.re, b.im);
+    return {q.real(), q.imag()};
+  }
+  return p;
+}
+inline Cplx operator+(const Cplx &a, const Cplx &b) { return {a.re + b.re, a.im + b.im}; }
+inline Cplx operator-(const Cplx &a, const Cplx &b) { return {a.re - b.re, a.im - b.im}; }
+inline Cplx operator-(const Cplx &a) { return {-a.re, -a.im}; }
+
+// rotate_to_vev (measurer.cxx:231-286): rotates the k-space walls into the
+// frame of the k = 0 phi direction.  wk[11][nk][2] -> rot[14][nk][2].
+void rotate_to_vev(int nk, const double *wk, double *rot) {
+  auto W = [&](int a, int k) { return Cplx{wk[(a * nk + k) * 2], wk[(a * nk + k) * 2 + 1]}; };
+  auto contract = [](const Cplx *n, const Cplx *rho, Cplx *out) {
+    out[0] = -(n[1] * rho[0]) - n[2] * rho[1] - n[3] * rho[2];
+    out[1] = n[0] * rho[0] + n[3] * rho[4] - n[2] * rho[5];
+    out[2] = n[0] * rho[1] - n[3] * rho[3] + n[1] * rho[5];
+    out[3] = n[0] * rho[2] + n[2] * rho[3] - n[1] * rho[4];
+  };
+  Cplx n[4];
+  double norm = 0.;
+  for (int a = 0; a < 4; a++) {
+    n[a] = W(a, 0);
+    norm += n[a].re * n[a].re + n[a].im * n[a].im;
+  }
+  norm = std::sqrt(norm);
+  if (norm < std::numeric_limits<double>::min()) {
+    n[0] = {1, 0};
+    n[1] = n[2] = n[3] = {0, 0};
+  } else {
+    for (int a = 0; a < 4; a++) n[a] = {n[a].re / norm, n[a].im / norm};
+  }
+  for (int k = 0; k < nk; k++) {
+    Cplx phi[4], rho[6], drho[6], A[4], V[4];
+    for (int a = 0; a < 4; a++) phi[a] = W(a, k);
+    for (int ab = 0; ab < 6; ab++) rho[ab] = W(4 + ab, k);
+    for (int l = 0; l < 3; l++) { drho[l] = rho[l + 3]; drho[l + 3] = rho[l]; }
+    Cplx phis{0, 0};
+    for (int a = 0; a < 4; a++) phis = phis + n[a] * phi[a];
+    contract(n, rho, A);
+    contract(n, drho, V);
+    auto put = [&](int a, const Cplx &v) {
+      rot[(a * nk + k) * 2] = v.re;
+      rot[(a * nk + k) * 2 + 1] = v.im;
+    };
+    put(0, phis);
+    for (int a = 0; a < 4; a++) {
+      put(1 + a, phi[a] - n[a] * phis);
+      put(5 + a, A[a]);
+      put(9 + a, V[a]);
+    }
+    put(13, W(10, k));
+  }
+}
+
 int check_launch() {
   HIPCHECK(hipGetLastError());
   return LGV_OK;
@@ -698,10 +774,12 @@ int lgv_create(const lgv_config *cfg, lgv_ctx **out) {
   HIPCHECK(hipMalloc(&c->eslots, c->plan_full.nblocks * sizeof(EnergySlot)));
   HIPCHECK(hipMalloc(&c->d_aos, (int64_t)stage_planes(c->maxN) * c->maxN * c->maxN * 10 *
                                      sizeof(double)));
-  const int64_t part = 25 * std::max(kMeasureColumns, (int64_t)c->maxN * c->maxN);
-  HIPCHECK(hipMalloc(&c->d_partXZ, part * sizeof(double)));
-  HIPCHECK(hipMalloc(&c->d_partXY, part * sizeof(double)));
-  HIPCHECK(hipMalloc(&c->d_meas, MeasBuf::size(c->maxN) * sizeof(double)));
+  int64_t part = 0;
+  for (const ReplicaParams &p : c->hp)
+    part = std::max(part, measure_part(measure_shape(p.N), p.N));
+  HIPCHECK(hipMalloc(&c->d_part, part * sizeof(double)));
+  HIPCHECK(hipMalloc(&c->d_meas, MeasBuf::walls(c->maxN) * sizeof(double)));
+  HIPCHECK(hipHostMalloc(&c->h_meas, MeasBuf::size(c->maxN) * sizeof(double), 0));
   HIPCHECK(hipDeviceSynchronize());
   *out = c.release();
   return LGV_OK;
@@ -728,9 +806,10 @@ int lgv_destroy(lgv_ctx *c) {
     note(hipFree(pl->d_blk_first));
   }
   for (void *q : {(void *)c->mon_phi, (void *)c->mon_charge, (void *)c->mon_ideal,
-                  (void *)c->eslots, (void *)c->d_aos, (void *)c->d_partXZ, (void *)c->d_partXY,
+                  (void *)c->eslots, (void *)c->d_aos, (void *)c->d_part,
                   (void *)c->d_meas})
     note(hipFree(q));
+  if (c->h_meas) note(hipHostFree(c->h_meas));
   if (c->ev_fork) note(hipEventDestroy(c->ev_fork));
   if (c->ev_join) note(hipEventDestroy(c->ev_join));
   if (c->stream2) note(hipStreamDestroy(c->stream2));
@@ -1045,22 +1124,14 @@ int lgv_measure(lgv_ctx *c, int r, double *wall, double *wallphase, double *oavg
   if (!wall || !wallphase || !oavg) return fail(LGV_ERR_ARG, "null output");
   HIPCHECK(hipSetDevice(c->device));
   const int N = c->hp[r].N;
-  const MeasBuf mb(c->d_meas, N);
-  launch_measure(c->fp32, c->dP, c->dS, r, N, c->d_partXZ, c->d_partXY, mb.wall, mb.wallphase,
-                 c->stream);
+  const MeasBuf mb(c->d_meas, N), h(c->h_meas, N);
+  launch_measure(c->fp32, c->dP, c->dS, r, N, c->d_part, mb.wall, mb.wallphase, h.wall,
+                 h.wallphase, c->stream);
   if ((rc = check_launch())) return rc;
-  std::vector<double> h(3 * 25 * (size_t)N);  // walls and phase walls, one copy
-  HIPCHECK(hipMemcpyAsync(h.data(), mb.wall, h.size() * sizeof(double), hipMemcpyDeviceToHost,
-                          c->stream));
   HIPCHECK(hipStreamSynchronize(c->stream));
-  memcpy(wall, h.data(), 3 * 11 * N * sizeof(double));
-  memcpy(wallphase, h.data() + 3 * 11 * N, 3 * 14 * N * sizeof(double));
-  // computeDerivedObs's OAverage (measurer.cxx:288-300): mean of wallX rows
-  for (int l = 0; l < 11; l++) {
-    double s = 0.;
-    for (int i = 0; i < N; i++) s += wall[l * N + i];
-    oavg[l] = s / (double)N;
-  }
+  memcpy(wall, h.wall, 3 * 11 * N * sizeof(double));
+  memcpy(wallphase, h.wallphase, 3 * 14 * N * sizeof(double));
+  volume_averages(h.wall, N, oavg);
   return LGV_OK;
 }
 
@@ -1093,88 +1164,27 @@ int lgv_timing_get(lgv_ctx *c, double ms[LGV_NCLASS], long long launches[LGV_NCL
   return LGV_OK;
 }
 
-// rotate_to_vev (measurer.cxx:231-286): rotates the k-space walls into the
-// frame of the k = 0 phi direction.  wk[11][nk][2] -> rot[14][nk][2].
-static void rotate_to_vev(int nk, const double *wk, double *rot) {
-  using cd = std::complex<double>;
-  auto W = [&](int a, int k) { return cd(wk[(a * nk + k) * 2], wk[(a * nk + k) * 2 + 1]); };
-  auto contract = [](const cd *n, const cd *rho, cd *out) {
-    out[0] = -(n[1] * rho[0]) - n[2] * rho[1] - n[3] * rho[2];
-    out[1] = n[0] * rho[0] + n[3] * rho[4] - n[2] * rho[5];
-    out[2] = n[0] * rho[1] - n[3] * rho[3] + n[1] * rho[5];
-    out[3] = n[0] * rho[2] + n[2] * rho[3] - n[1] * rho[4];
-  };
-  cd n[4];
-  double norm = 0.;
-  for (int a = 0; a < 4; a++) {
-    n[a] = W(a, 0);
-    norm += std::norm(n[a]);
-  }
-  norm = std::sqrt(norm);
-  if (norm < std::numeric_limits<double>::min()) {
-    n[0] = 1; n[1] = n[2] = n[3] = 0;
-  } else {
-    for (int a = 0; a < 4; a++) n[a] /= norm;
-  }
-  for (int k = 0; k < nk; k++) {
-    cd phi[4], rho[6], drho[6], phir[4], A[4], V[4];
-    for (int a = 0; a < 4; a++) phi[a] = W(a, k);
-    for (int ab = 0; ab < 6; ab++) rho[ab] = W(4 + ab, k);
-    for (int l = 0; l < 3; l++) { drho[l] = rho[l + 3]; drho[l + 3] = rho[l]; }
-    const cd phi2k = W(10, k);
-    cd phis(0.);
-    for (int a = 0; a < 4; a++) phis += n[a] * phi[a];
-    for (int a = 0; a < 4; a++) phir[a] = phi[a] - n[a] * phis;
-    contract(n, rho, A);
-    contract(n, drho, V);
-    auto put = [&](int a, cd v) {
-      rot[(a * nk + k) * 2] = v.real();
-      rot[(a * nk + k) * 2 + 1] = v.imag();
-    };
-    put(0, phis);
-    for (int a = 0; a < 4; a++) {
-      put(1 + a, phir[a]);
-      put(5 + a, A[a]);
-      put(9 + a, V[a]);
-    }
-    put(13, phi2k);
-  }
-}
-
 int lgv_measure_full(lgv_ctx *c, int r, lgv_measurement *m) {
   int rc = check_replica(c, r);
   if (rc) return rc;
   if (!m) return fail(LGV_ERR_ARG, "null measurement");
   HIPCHECK(hipSetDevice(c->device));
   const int N = c->hp[r].N, nk = N / 2 + 1;
-  std::vector<double> wall(3 * 11 * N), wallphase(3 * 14 * N), oavg(11);
-  const MeasBuf mb(c->d_meas, N);
-  launch_measure(c->fp32, c->dP, c->dS, r, N, c->d_partXZ, c->d_partXY, mb.wall, mb.wallphase,
-                 c->stream);
-  launch_wall_dft(N, mb.wall, mb.wallphase, mb.wallk, mb.wallphasek, c->stream);
+  const MeasBuf mb(c->d_meas, N), h(c->h_meas, N);
+  launch_measure(c->fp32, c->dP, c->dS, r, N, c->d_part, mb.wall, mb.wallphase, h.wall,
+                 h.wallphase, c->stream);
+  launch_wall_dft(N, mb.wall, mb.wallphase, h.wallk, h.wallphasek, c->stream);
   if ((rc = check_launch())) return rc;
-  std::vector<double> h(mb.total);  // everything in one copy
-  HIPCHECK(hipMemcpyAsync(h.data(), mb.wall, h.size() * sizeof(double), hipMemcpyDeviceToHost,
-                          c->stream));
   HIPCHECK(hipStreamSynchronize(c->stream));
-  std::vector<double> wk(3 * 11 * nk * 2), wpk(3 * 14 * nk * 2);
-  memcpy(wall.data(), h.data(), wall.size() * sizeof(double));
-  memcpy(wallphase.data(), h.data() + (mb.wallphase - mb.wall), wallphase.size() * sizeof(double));
-  memcpy(wk.data(), h.data() + (mb.wallk - mb.wall), wk.size() * sizeof(double));
-  memcpy(wpk.data(), h.data() + (mb.wallphasek - mb.wall), wpk.size() * sizeof(double));
-  for (int l = 0; l < 11; l++) {
-    double s = 0.;
-    for (int i = 0; i < N; i++) s += wall[l * N + i];
-    oavg[l] = s / (double)N;
-  }
-  if (m->wall) memcpy(m->wall, wall.data(), wall.size() * sizeof(double));
-  if (m->wallphase) memcpy(m->wallphase, wallphase.data(), wallphase.size() * sizeof(double));
-  if (m->oavg) memcpy(m->oavg, oavg.data(), 11 * sizeof(double));
-  if (m->wall_k) memcpy(m->wall_k, wk.data(), wk.size() * sizeof(double));
-  if (m->wallphase_k) memcpy(m->wallphase_k, wpk.data(), wpk.size() * sizeof(double));
+  if (m->wall) memcpy(m->wall, h.wall, 3 * 11 * (size_t)N * sizeof(double));
+  if (m->wallphase) memcpy(m->wallphase, h.wallphase, 3 * 14 * (size_t)N * sizeof(double));
+  if (m->oavg) volume_averages(h.wall, N, m->oavg);
+  if (m->wall_k) memcpy(m->wall_k, h.wallk, 3 * 11 * (size_t)nk * 2 * sizeof(double));
+  if (m->wallphase_k)
+    memcpy(m->wallphase_k, h.wallphasek, 3 * 14 * (size_t)nk * 2 * sizeof(double));
   if (m->wall_k_rotated)
     for (int d = 0; d < 3; d++)
-      rotate_to_vev(nk, wk.data() + (size_t)d * 11 * nk * 2,
+      rotate_to_vev(nk, h.wallk + (size_t)d * 11 * nk * 2,
                     m->wall_k_rotated + (size_t)d * 14 * nk * 2);
   return LGV_OK;
 }

@@ -142,15 +142,50 @@ constexpr uint64_t kMarchBytesFp32 = 600ull << 20;
 // Largest side: N^3 must fit 32-bit site indices.
 constexpr int kMaxN = 1536;
 
-// Chunks of the measurement's column sums: about 2^19 column-chunks per
-// pass (8 chunks at N = 256, 1 from N = 724 on).  The partial buffers hold
-// 25 * measure_chunks(N) * N^2 <= 25 * max(2^19, N^2) doubles.
-constexpr int64_t kMeasureColumns = int64_t(1) << 19;
-__host__ __device__ inline int measure_chunks(int N) {
+// Shape of the measurement pass (k_measure_tile): TX x TZ columns per
+// wavefront, nz tiles in z taken in turn, chunks of CY rows in y; ntx, ntz
+// tiles and nch chunks.  The partial sums hold 25 N (nch ntz + nch ntx + ntx ntz)
+// doubles (with nz > 1 2 ntx ntz / nz in place of ntx ntz), at most 50 max(2^19,
+// N^2): nz grows with N for that.  Chunks are halved until the launch has 2048
+// wavefronts, which is what the GPU holds (256^3 FP64: 471 us with 1024, 385
+// with 2048, 383 with 4096); small lattices stop at 16 N, where more
+// partial sums cost as much as the shorter chunks give.
+struct MeasureShape {
+  int TX, TZ, nz, CY, ntx, ntz, nch;
+};
+constexpr int64_t kMeasurePart = int64_t(1) << 19;
+__host__ __device__ inline int64_t measure_part_limit(int N) {
   const int64_t n2 = (int64_t)N * N;
-  int c = 1;
-  while (c < 8 && 2 * c * n2 <= kMeasureColumns) c *= 2;
-  return c;
+  return 50 * (n2 > kMeasurePart ? n2 : kMeasurePart);
+}
+__host__ __device__ inline int64_t measure_part(const MeasureShape &s, int N) {
+  const int64_t groups = (int64_t)s.ntx * ((s.ntz + s.nz - 1) / s.nz);
+  return 25 * (int64_t)N *
+         ((int64_t)s.nch * (s.ntz + s.ntx) + (s.nz > 1 ? 2 : 1) * groups);
+}
+inline MeasureShape measure_shape(int N) {
+  MeasureShape s;
+  s.ntx = (N + 63) / 64;
+  s.TX = (N + s.ntx - 1) / s.ntx;
+  s.TZ = 64 / s.TX;
+  if (s.TZ > N) s.TZ = N;
+  s.ntz = (N + s.TZ - 1) / s.TZ;
+  s.nz = 1;
+  s.CY = N;
+  s.nch = 1;
+  while (measure_part(s, N) > measure_part_limit(N)) s.nz *= 2;
+  const int64_t waves = N < 128 ? 16 * N : 2048;
+  // more chunks while the launch leaves the GPU idle and the sums have room
+  while (s.CY > 1) {
+    MeasureShape h = s;
+    h.CY = (s.CY + 1) / 2;
+    h.nch = (N + h.CY - 1) / h.CY;
+    if ((int64_t)s.ntx * ((s.ntz + s.nz - 1) / s.nz) * s.nch >= waves ||
+        measure_part(h, N) > measure_part_limit(N))
+      break;
+    s = h;
+  }
+  return s;
 }
 
 // Kernel launchers (lgv_kernels.hip).  fp32 selects the storage type.
@@ -185,10 +220,12 @@ void launch_aos_to_rb(bool fp32, const ReplicaParams *P, const ReplicaState *S, 
                       int N, int z0, int nz, const double *aos, hipStream_t st);
 void launch_rb_to_aos(bool fp32, const ReplicaParams *P, const ReplicaState *S, int replica,
                       int N, int z0, int nz, double *aos, hipStream_t st);
-void launch_wall_dft(int N, const double *wall, const double *wallphase, double *wall_k,
-                     double *wallphase_k, hipStream_t st);
+// host_*: pinned host memory, written beside the device copies (launch_measure)
+// or alone (launch_wall_dft), so that no transfer follows the kernels.
+void launch_wall_dft(int N, const double *wall, const double *wallphase, double *host_wall_k,
+                     double *host_wallphase_k, hipStream_t st);
 void launch_measure(bool fp32, const ReplicaParams *P, const ReplicaState *S, int replica,
-                    int N, double *partXZ, double *partXY, double *wall, double *wallphase,
-                    hipStream_t st);
+                    int N, double *part, double *wall, double *wallphase, double *host_wall,
+                    double *host_wallphase, hipStream_t st);
 
 }  // namespace lgv

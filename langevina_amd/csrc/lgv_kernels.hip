@@ -1370,166 +1370,318 @@ __device__ __forceinline__ void contract_rho(const double n[4], const double rho
 }
 
 template <typename T>
-__device__ __forceinline__ void site_obs_add(const ReplicaParams &p, int cur, int par, int64_t i,
-                                             KSum acc[25]) {
+__device__ __forceinline__ void site_obs(const T raw[10], double o[25]) {
   double f[10];
-  for (int c = 0; c < 10; c++) f[c] = (double)plane<T>(p, cur, c, par)[i];
+#pragma unroll
+  for (int c = 0; c < 10; c++) o[c] = f[c] = (double)raw[c];
   double phi2 = 0.0;
+#pragma unroll
   for (int l = 0; l < 4; l++) phi2 += f[l] * f[l];
-  for (int c = 0; c < 10; c++) ksum_add(acc[c], f[c]);
-  ksum_add(acc[10], phi2);
   const double sigma = sqrt(phi2);
   double n[4];
   if (phi2 > 100. * DBL_MIN) {
-    for (int l = 0; l < 4; l++) n[l] = f[l] / sigma;
+    // f / sigma from the reciprocal with one Markstein correction: the
+    // quotient rounded once, three instructions instead of ten
+    const double inv = 1. / sigma;
+#pragma unroll
+    for (int l = 0; l < 4; l++) {
+      const double q = f[l] * inv;
+      n[l] = fma(fma(-q, sigma, f[l]), inv, q);
+    }
   } else {
     n[0] = 1; n[1] = 0; n[2] = 0; n[3] = 0;
   }
   const double rho[6] = {f[4], f[5], f[6], f[7], f[8], f[9]};
   const double drho[6] = {f[7], f[8], f[9], f[4], f[5], f[6]};
-  double A[4], V[4];
-  contract_rho(n, rho, A);
-  contract_rho(n, drho, V);
-  ksum_add(acc[11], sigma);
-  for (int l = 0; l < 4; l++) {
-    ksum_add(acc[12 + l], n[l]);
-    ksum_add(acc[16 + l], A[l]);
-    ksum_add(acc[20 + l], V[l]);
-  }
-  ksum_add(acc[24], sigma * sigma);
+  o[10] = phi2;
+  o[11] = sigma;
+#pragma unroll
+  for (int l = 0; l < 4; l++) o[12 + l] = n[l];
+  contract_rho(n, rho, o + 16);
+  contract_rho(n, drho, o + 20);
+  o[24] = sigma * sigma;
 }
 
-// Per (x, z): compensated sum over y of the 25 site observables ->
-// partXZ[ch][o][z][x]; per (x, y): sum over z -> partXY[ch][o][y][x].  The
-// summed axis is split into nch chunks (measure_chunks) so that a 256^3
-// lattice runs 8 N^2 threads instead of N^2; k_measure_fold adds the chunks.
+// a += x with the rounding error of the addition collected in a.c: Knuth's
+// two-sum, six additions and no comparison (ksum_add takes a branch or
+// selects).  The same error term as ksum_add's.
+__device__ __forceinline__ void two_sum_add(KSum &a, double x) {
+  const double s = a.s + x;
+  const double bx = s - a.s;
+  a.c += (a.s - (s - bx)) + (x - bx);
+  a.s = s;
+}
+__device__ __forceinline__ void ksum_xor_merge(KSum &a, int o) {
+  KSum b;
+  b.s = __shfl_xor(a.s, o, 64);
+  b.c = __shfl_xor(a.c, o, 64);
+  two_sum_add(a, b.s);
+  a.c += b.c;
+}
+// The same for sums that start at a bias B, a power of two: while |x| stays
+// below |a.s|, Dekker's two-sum, three additions, gives the error exactly.  B
+// is 2^14 .. 2^15 times the largest magnitude of a first sample, so that holds
+// as long as the values and their sum stay below 2^13 times the sample's;
+// beyond that the additions round as plain FP64 ones.
+__device__ __forceinline__ void biased_add(KSum &a, double x) {
+  const double s = a.s + x;
+  a.c += x - (s - a.s);
+  a.s = s;
+}
+__device__ __forceinline__ double bias_of(double largest) {
+  const uint64_t e = (uint64_t)__double_as_longlong(largest) >> 52;  // largest >= 0
+  return largest > 0. ? __longlong_as_double((long long)((e < 1900 ? e + 15 : 1915) << 52)) : 1.;
+}
+
+// The three walls' slice sums in one pass over the fields (measurer.cxx:
+// 10-229).  A wavefront takes 64 columns (x, z), TX x TZ of them in use, and
+// marches y through a chunk of CY rows: a lane keeps the 25 observables of its
+// column summed over y in registers (from which the x and z walls follow), and
+// each row's sums over the columns (the y wall) are taken through the
+// wavefront's own LDS table, two lanes to an observable.  No wavefront waits
+// for another.  All sums are compensated.  Partial sums:
+//   px[(chunk, z tile)][25][N]  over the tile's planes and the chunk's rows,
+//   pz[(chunk, x tile)][25][N]  over the tile's columns and the chunk's rows,
+//   py[(x tile, z group)][25][N][nz > 1 ? 2 : 1]  over the columns of the
+//     group's nz z tiles, which one wavefront takes in turn (sum, correction).
+// What bounds it is bytes in flight: two rows' loads ahead of the sums at two
+// wavefronts per SIMD keep 80 KB per CU under way.
+constexpr int kMeasureCols = 64;
+// the padding puts the rows that a half-wavefront reads at once on different banks
+typedef double MeasureTable[25][kMeasureCols + 2];
+
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_measure_cols(const ReplicaParams *P,
-                                                         const ReplicaState *S, int replica,
-                                                         int along_z, int nch, double *part) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2)))
+void k_measure_tile(const ReplicaParams *__restrict__ P, const ReplicaState *__restrict__ S,
+                    int replica, MeasureShape sh, double *__restrict__ px,
+                    double *__restrict__ py, double *__restrict__ pz) {
+  __shared__ MeasureTable tab[kBlock / 64];
   const ReplicaParams &p = P[replica];
-  const int cur = live(S[replica]);
-  const int N = p.N;
-  const int64_t N2 = (int64_t)N * N;
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= N2 * nch) return;
-  const int ch = (int)(t / N2);
-  const int64_t col = t - (int64_t)ch * N2;
-  const int x = (int)(col % N), w = (int)(col / N);
-  const int v0 = (int)((int64_t)ch * N / nch), v1 = (int)((int64_t)(ch + 1) * N / nch);
-  KSum acc[25];
-  for (int o = 0; o < 25; o++) acc[o] = KSum{0., 0.};
-  for (int v = v0; v < v1; v++) {
-    const int y = along_z ? w : v;
-    const int z = along_z ? v : w;
-    const int par = (x + y + z) & 1;
-    const int64_t i = ((int64_t)z * N + y) * p.NH + (x >> 1);
-    site_obs_add<T>(p, cur, par, i, acc);
+  const int cur = first_lane(live(S[replica]));
+  const gbyte *phi = (const gbyte *)(cur & 1 ? p.fields[1] : p.fields[0]),
+              *chg = (const gbyte *)(cur >> 1 ? p.fields[1] : p.fields[0]);
+  const int N = p.N, NH = p.NH;
+  const int64_t half = p.half;
+  const int wave = first_lane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+  MeasureTable &q = tab[wave];
+  int b = (int)blockIdx.x * (kBlock / 64) + wave;
+  const int ngz = (sh.ntz + sh.nz - 1) / sh.nz;
+  if (b >= sh.ntx * ngz * sh.nch) return;  // whole wavefronts; no barrier follows
+  const int bx = b % sh.ntx;
+  b /= sh.ntx;
+  const int gz = b % ngz, by = b / ngz;
+  const int tx = lane % sh.TX, tz = lane / sh.TX;
+  const int x0 = bx * sh.TX, tw = min(sh.TX, N - x0);
+  const int y0 = by * sh.CY, y1 = min(y0 + sh.CY, N);
+  const int yw = sh.nz > 1 ? 2 : 1;
+  double *yrow = py + (int64_t)(bx * ngz + gz) * 25 * N * yw;
+  // this lane's part in the table's row sums: row k, entries s, s + 2, ...
+  const int k = lane >> 1, s = lane & 1;
+  // the table is written and read by one wavefront: its LDS operations stay
+  // in order, and the compiler must keep them so
+  auto table_ready = [] __attribute__((always_inline)) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  for (int bz = gz * sh.nz; bz < min((gz + 1) * sh.nz, sh.ntz); bz++) {
+    const int z0 = bz * sh.TZ, th = min(sh.TZ, N - z0);
+    const int x = x0 + tx, z = z0 + tz;
+    const bool own = tx < tw && tz < th, ragged = !__all(own);
+    T raw[2][10];
+    auto load = [&](int y, T *r) __attribute__((always_inline)) {
+      // lanes without a column read site 0 and count zero
+      const int64_t i = own ? ((x + y + z) & 1) * half + ((int64_t)z * N + y) * NH + (x >> 1) : 0;
+#pragma unroll
+      for (int c = 0; c < 10; c++)
+        r[c] = reinterpret_cast<const __attribute__((address_space(1))) T *>(
+            c < 4 ? phi : chg)[c * 2 * half + i];
+    };
+    auto observe = [&](const T *r, double *o) __attribute__((always_inline)) {
+      site_obs(r, o);
+      if (ragged) {
+#pragma unroll
+        for (int i = 0; i < 25; i++) o[i] = own ? o[i] : 0.;
+      }
+    };
+    load(y0, raw[0]);
+    if (y0 + 1 < y1) load(y0 + 1, raw[1]);
+    KSum acc[25];
+    {
+      // the biases from the first row's largest magnitudes
+      double o[25];
+      observe(raw[0], o);
+#pragma unroll
+      for (int i = 0; i < 25; i++) q[i][lane] = o[i];
+      table_ready();
+      double m = 0.;
+      if (k < 25)
+        for (int i = s; i < kMeasureCols; i += 2) m = fmax(m, fabs(q[k][i]));
+      m = fmax(m, __shfl_xor(m, 1, 64));
+      table_ready();
+      if (k < 25 && s == 0) q[k][kMeasureCols] = bias_of(m);  // kept in the padding
+      table_ready();
+#pragma unroll
+      for (int i = 0; i < 25; i++) acc[i] = KSum{q[i][kMeasureCols], 0.};
+    }
+    const double yb = k < 25 ? q[k][kMeasureCols] : 1.;
+    auto take = [&](int y, T *r) __attribute__((always_inline)) {
+      double o[25];
+      observe(r, o);
+      if (y + 2 < y1) load(y + 2, r);
+#pragma unroll
+      for (int i = 0; i < 25; i++) {
+        q[i][lane] = o[i];
+        biased_add(acc[i], o[i]);
+      }
+      table_ready();
+      if (k < 25) {
+        KSum a{yb, 0.};
+        const double *row = &q[k][s];
+#pragma unroll
+        for (int i = 0; i < kMeasureCols; i += 2) biased_add(a, row[i]);
+        a.s -= yb;
+        ksum_xor_merge(a, 1);
+        if (s == 0) {
+          double *w = yrow + ((int64_t)k * N + y) * yw;
+          if (yw == 1) {
+            w[0] = ksum_value(a);
+          } else {
+            if (bz > gz * sh.nz) {  // the group's earlier tiles: this lane's own stores
+              two_sum_add(a, w[0]);
+              a.c += w[1];
+            }
+            w[0] = a.s;
+            w[1] = a.c;
+          }
+        }
+      }
+      table_ready();
+    };
+    for (int y = y0; y < y1; y += 2) {
+      take(y, raw[0]);
+      if (y + 1 < y1) take(y + 1, raw[1]);
+    }
+    // the columns' sums over the chunk, then over the tile's planes / columns
+#pragma unroll
+    for (int i = 0; i < 25; i++) q[i][lane] = (acc[i].s - q[i][kMeasureCols]) + acc[i].c;
+    table_ready();
+    double *xrow = px + (int64_t)(by * sh.ntz + bz) * 25 * N;
+    if (tz == 0 && tx < tw) {
+      for (int i = 0; i < 25; i++) {
+        KSum a{0., 0.};
+        for (int r = 0; r < th; r++) two_sum_add(a, q[i][r * sh.TX + tx]);
+        xrow[(int64_t)i * N + x] = ksum_value(a);
+      }
+    }
+    double *zrow = pz + (int64_t)(by * sh.ntx + bx) * 25 * N;
+    for (int j = lane >> 3; j < 25 * th; j += 8) {  // eight lanes to a row sum
+      const int i = j / th, r = j - i * th;
+      KSum a{0., 0.};
+      for (int c = lane & 7; c < tw; c += 8) two_sum_add(a, q[i][r * sh.TX + c]);
+      ksum_xor_merge(a, 1);
+      ksum_xor_merge(a, 2);
+      ksum_xor_merge(a, 4);
+      if ((lane & 7) == 0) zrow[(int64_t)i * N + z0 + r] = ksum_value(a);
+    }
+    table_ready();
   }
-  double *out = part + (int64_t)ch * 25 * N2;
-  for (int k = 0; k < 25; k++) out[((int64_t)k * N + w) * N + x] = ksum_value(acc[k]);
 }
 
-// Folds the chunk partials into chunk 0: part[0][j] = compensated sum over
-// ch of part[ch][j], j < 25 N^2 (one thread per element, coalesced).
-__global__ void k_measure_fold(int64_t n, int nch, double *part) {
-  const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= n) return;
-  KSum acc{0., 0.};
-  for (int ch = 0; ch < nch; ch++) ksum_add(acc, part[(int64_t)ch * n + j]);
-  part[j] = ksum_value(acc);
-}
-
-// Walls, x direction: wall_x[k][n] = (compensated sum over z of
-// partXZ[k][z][n]) / N^2.  A block takes 64 consecutive n (coalesced) of one
-// k; its 8 thread groups sum z = g, g + 8, ... and the 8 partials are merged
-// in group order.
-__global__ __launch_bounds__(512) void k_measure_reduce_x(int N, const double *partXZ,
-                                                          double *wall, double *wallphase) {
-  __shared__ KSum part[8][64];
+// wall_d[k][n] = (compensated sum of the partial sums of (d, k, n)) / N^2.  A
+// block takes 64 consecutive n (coalesced) of one (d, k); its thread groups g
+// take the partial sums g, g + kReduceGroups, ... and are merged in group order.
+constexpr int kReduceGroups = 16;
+__global__ __launch_bounds__(64 * kReduceGroups) void k_measure_reduce(int N, MeasureShape sh,
+                                                        const double *__restrict__ px,
+                                                        const double *__restrict__ py,
+                                                        const double *__restrict__ pz,
+                                                        double *__restrict__ wall,
+                                                        double *__restrict__ wallphase,
+                                                        double *__restrict__ host_wall,
+                                                        double *__restrict__ host_wallphase) {
+  __shared__ KSum part[kReduceGroups][64];
   const int nb = (N + 63) / 64;
-  const int k = blockIdx.x / nb;
-  const int n = (blockIdx.x % nb) * 64 + (threadIdx.x & 63);
-  const int g = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, g = threadIdx.x >> 6;
+  const int k = blockIdx.x / nb % 25, d = blockIdx.x / nb / 25;
+  const int n = (blockIdx.x % nb) * 64 + lane;
+  const int ngz = (sh.ntz + sh.nz - 1) / sh.nz;
+  const int entries = d == 0 ? sh.nch * sh.ntz : (d == 1 ? sh.ntx * ngz : sh.nch * sh.ntx);
+  const int64_t stride = 25 * (int64_t)N, at = (int64_t)k * N + n;
   KSum acc{0., 0.};
-  if (n < N)
-    for (int m = g; m < N; m += 8) ksum_add(acc, partXZ[((int64_t)k * N + m) * N + n]);
-  part[g][threadIdx.x & 63] = acc;
+  if (n < N) {
+    if (d == 1 && sh.nz > 1) {
+#pragma unroll 8
+      for (int e = g; e < entries; e += kReduceGroups) {
+        two_sum_add(acc, py[(e * stride + at) * 2]);
+        acc.c += py[(e * stride + at) * 2 + 1];
+      }
+    } else {
+      const double *src = d == 0 ? px : (d == 1 ? py : pz);
+#pragma unroll 8
+      for (int e = g; e < entries; e += kReduceGroups) two_sum_add(acc, src[e * stride + at]);
+    }
+  }
+  part[g][lane] = acc;
   __syncthreads();
   if (g == 0 && n < N) {
-    for (int i = 1; i < 8; i++) ksum_merge(acc, part[i][threadIdx.x]);
-    const double val = ksum_value(acc) / (double)(N * N);
-    if (k < 11) wall[(int64_t)k * N + n] = val;
-    else wallphase[(int64_t)(k - 11) * N + n] = val;
-  }
-}
-
-// Walls, y and z directions: row sums, one wave per (d, k, n) row (lanes
-// read consecutive x; lane partials merged by a fixed shuffle tree).
-//   d = 1: wall_y[k][n] = sum_x partXY[k][n][x] / N^2
-//   d = 2: wall_z[k][n] = sum_x partXZ[k][n][x] / N^2
-__global__ __launch_bounds__(256) void k_measure_reduce_rows(int N, const double *partXZ,
-                                                             const double *partXY,
-                                                             double *wall, double *wallphase) {
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (row >= 2 * 25 * N) return;  // whole waves exit together
-  const int n = row % N, k = (row / N) % 25, d = 1 + row / (25 * N);
-  const double *src = (d == 1 ? partXY : partXZ) + ((int64_t)k * N + n) * N;
-  KSum acc{0., 0.};
-  for (int x = lane; x < N; x += 64) ksum_add(acc, src[x]);
-  for (int o = 32; o > 0; o >>= 1) {
-    KSum t;
-    t.s = __shfl_xor(acc.s, o, 64);
-    t.c = __shfl_xor(acc.c, o, 64);
-    ksum_merge(acc, t);
-  }
-  if (lane == 0) {
-    const double val = ksum_value(acc) / (double)(N * N);
-    if (k < 11) wall[((int64_t)d * 11 + k) * N + n] = val;
-    else wallphase[((int64_t)d * 14 + (k - 11)) * N + n] = val;
+    for (int i = 1; i < kReduceGroups; i++) ksum_merge(acc, part[i][lane]);
+    const double val = ksum_value(acc) / (double)((int64_t)N * N);
+    const int64_t at_wall = ((int64_t)d * 11 + k) * N + n,
+                  at_phase = ((int64_t)d * 14 + (k - 11)) * N + n;
+    if (k < 11) wall[at_wall] = host_wall[at_wall] = val;
+    else wallphase[at_phase] = host_wallphase[at_phase] = val;
   }
 }
 
 // measurer_fft::execute_row (measurer.h:33-41): FFTW's r2c forward
 // transform divided by N, out[k] = (1/N) sum_x in[x] e^{-2 pi i k x / N},
 // k = 0..N/2, as a direct DFT with exactly reduced twiddles and compensated
-// sums.  One thread per (row, k); rows = 3 x 25 walls.
-__global__ __launch_bounds__(256) void k_wall_dft(int N, const double *wall,
-                                                  const double *wallphase, double *wall_k,
-                                                  double *wallphase_k) {
+// sums.  A block takes kDftK values of k of one row (3 x 25 rows), 16 lanes
+// to each: one thread per k was a chain of N dependent sums (256^3: 24 us).
+constexpr int kDftK = 16;
+__global__ __launch_bounds__(256) void k_wall_dft(int N, const double *__restrict__ wall,
+                                                  const double *__restrict__ wallphase,
+                                                  double *__restrict__ wall_k,
+                                                  double *__restrict__ wallphase_k) {
   // twiddles cos/sin(2 pi m / N), m = 0 .. N-1, once per block
   __shared__ double tc[kMaxN], ts[kMaxN];
   for (int m = threadIdx.x; m < N; m += blockDim.x) sincospi(2.0 * m / N, &ts[m], &tc[m]);
   __syncthreads();
-  const int nk = N / 2 + 1;
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= 3 * 25 * nk) return;
-  const int k = t % nk;
-  const int row = t / nk;  // d*25 + obs
+  const int nk = N / 2 + 1, nkb = (nk + kDftK - 1) / kDftK;
+  const int row = blockIdx.x / nkb;  // d*25 + obs
+  const int k = (blockIdx.x % nkb) * kDftK + (threadIdx.x >> 4), l = threadIdx.x & 15;
   const int d = row / 25, o = row % 25;
   const double *in = o < 11 ? wall + ((int64_t)d * 11 + o) * N
                             : wallphase + ((int64_t)d * 14 + (o - 11)) * N;
   KSum re{0., 0.}, im{0., 0.};
-  int m = 0;  // k x mod N
-  for (int x = 0; x < N; x++) {
-    ksum_add(re, in[x] * tc[m]);
-    ksum_add(im, -(in[x] * ts[m]));
-    m += k;
-    if (m >= N) m -= N;
+  if (k < nk) {
+    const int step = (int)((int64_t)k * 16 % N);
+    int m = (int)((int64_t)k * l % N);  // k x mod N
+    for (int x = l; x < N; x += 16) {
+      two_sum_add(re, in[x] * tc[m]);
+      two_sum_add(im, -(in[x] * ts[m]));
+      m += step;
+      if (m >= N) m -= N;
+    }
   }
-  double *out = o < 11 ? wall_k + (((int64_t)d * 11 + o) * nk + k) * 2
-                       : wallphase_k + (((int64_t)d * 14 + (o - 11)) * nk + k) * 2;
-  out[0] = ksum_value(re) / N;
-  out[1] = ksum_value(im) / N;
+  for (int b = 1; b < 16; b *= 2) {
+    ksum_xor_merge(re, b);
+    ksum_xor_merge(im, b);
+  }
+  if (k < nk && l == 0) {
+    double *out = o < 11 ? wall_k + (((int64_t)d * 11 + o) * nk + k) * 2
+                         : wallphase_k + (((int64_t)d * 14 + (o - 11)) * nk + k) * 2;
+    out[0] = ksum_value(re) / N;
+    out[1] = ksum_value(im) / N;
+  }
 }
 
 // ======================================================================== launchers
 
 void launch_wall_dft(int N, const double *wall, const double *wallphase, double *wall_k,
                      double *wallphase_k, hipStream_t st) {
-  const int n = 3 * 25 * (N / 2 + 1);
-  k_wall_dft<<<(n + 255) / 256, 256, 0, st>>>(N, wall, wallphase, wall_k, wallphase_k);
+  const int nkb = (N / 2 + 1 + kDftK - 1) / kDftK;
+  k_wall_dft<<<3 * 25 * nkb, 256, 0, st>>>(N, wall, wallphase, wall_k, wallphase_k);
 }
 
 static inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
@@ -1644,25 +1796,17 @@ void launch_rb_to_aos(bool fp32, const ReplicaParams *P, const ReplicaState *S, 
 }
 
 void launch_measure(bool fp32, const ReplicaParams *P, const ReplicaState *S, int replica,
-                    int N, double *partXZ, double *partXY, double *wall, double *wallphase,
-                    hipStream_t st) {
-  const int nch = measure_chunks(N);
-  const int64_t threads = (int64_t)N * N * nch;
-  if (fp32) {
-    k_measure_cols<float><<<nblk(threads, kBlock), kBlock, 0, st>>>(P, S, replica, 0, nch, partXZ);
-    k_measure_cols<float><<<nblk(threads, kBlock), kBlock, 0, st>>>(P, S, replica, 1, nch, partXY);
-  } else {
-    k_measure_cols<double><<<nblk(threads, kBlock), kBlock, 0, st>>>(P, S, replica, 0, nch, partXZ);
-    k_measure_cols<double><<<nblk(threads, kBlock), kBlock, 0, st>>>(P, S, replica, 1, nch, partXY);
-  }
-  if (nch > 1) {
-    const int64_t n = (int64_t)25 * N * N;
-    k_measure_fold<<<nblk(n, 256), 256, 0, st>>>(n, nch, partXZ);
-    k_measure_fold<<<nblk(n, 256), 256, 0, st>>>(n, nch, partXY);
-  }
-  k_measure_reduce_x<<<25 * ((N + 63) / 64), 512, 0, st>>>(N, partXZ, wall, wallphase);
-  k_measure_reduce_rows<<<nblk(2 * 25 * N, 4), 256, 0, st>>>(N, partXZ, partXY, wall,
-                                                             wallphase);
+                    int N, double *part, double *wall, double *wallphase, double *host_wall,
+                    double *host_wallphase, hipStream_t st) {
+  const MeasureShape sh = measure_shape(N);
+  double *px = part, *pz = px + (int64_t)sh.nch * sh.ntz * 25 * N,
+         *py = pz + (int64_t)sh.nch * sh.ntx * 25 * N;
+  const unsigned tiles = (unsigned)(sh.ntx * ((sh.ntz + sh.nz - 1) / sh.nz) * sh.nch);
+  const unsigned blocks = nblk(tiles, kBlock / 64);  // a wavefront to a tile
+  if (fp32) k_measure_tile<float><<<blocks, kBlock, 0, st>>>(P, S, replica, sh, px, py, pz);
+  else k_measure_tile<double><<<blocks, kBlock, 0, st>>>(P, S, replica, sh, px, py, pz);
+  k_measure_reduce<<<3 * 25 * ((N + 63) / 64), 64 * kReduceGroups, 0, st>>>(
+      N, sh, px, py, pz, wall, wallphase, host_wall, host_wallphase);
 }
 
 }  // namespace lgv

@@ -272,9 +272,9 @@ class Context:
 
     def measure(self, replica=0):
         N = self.N[replica]
-        wall = np.zeros((3, 11, N))
-        wallphase = np.zeros((3, 14, N))
-        oavg = np.zeros(11)
+        wall = np.empty((3, 11, N))
+        wallphase = np.empty((3, 14, N))
+        oavg = np.empty(11)
         _check(lib().lgv_measure(self.h, replica, wall.reshape(-1), wallphase.reshape(-1), oavg))
         return wall, wallphase, oavg
 
@@ -283,13 +283,12 @@ class Context:
         (wall_k, wall_k_rotated, wallphase_k as complex arrays, k = 0..N/2)."""
         N = self.N[replica]
         K = N // 2 + 1
-        out = {"wall": np.zeros((3, 11, N)), "wallphase": np.zeros((3, 14, N)),
-               "oavg": np.zeros(11), "wall_k": np.zeros((3, 11, K, 2)),
-               "wall_k_rotated": np.zeros((3, 14, K, 2)), "wallphase_k": np.zeros((3, 14, K, 2))}
+        c = np.complex128
+        out = {"wall": np.empty((3, 11, N)), "wallphase": np.empty((3, 14, N)),
+               "oavg": np.empty(11), "wall_k": np.empty((3, 11, K), c),
+               "wall_k_rotated": np.empty((3, 14, K), c), "wallphase_k": np.empty((3, 14, K), c)}
         m = Measurement(*[v.ctypes.data_as(C.POINTER(C.c_double)) for v in out.values()])
         _check(lib().lgv_measure_full(self.h, replica, C.byref(m)))
-        for k in ("wall_k", "wall_k_rotated", "wallphase_k"):
-            out[k] = out[k][..., 0] + 1j * out[k][..., 1]
         return out
 
     def set_mass(self, mass0, dmassdt=0.0, replica=-1):
