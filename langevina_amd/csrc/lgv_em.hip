@@ -36,27 +36,41 @@ constexpr uint64_t kEmTag = 0x4000000000000000ULL;
 // Tile of the two stencil marches: TX sites in x by TY rows in y, chunks of
 // TZ planes in z.  A block's plane (tile plus a one-site ring, no corners)
 // sits in LDS; each thread keeps its own column's planes z-1, z, z+1 in
-// registers.
+// registers.  TX splits the row evenly into at most 64.  A block marches TZ
+// planes after loading two, and the GPU holds about 1024 blocks: TZ of 8, 4, 2,
+// 1 minimises the rounds of TZ + 2 planes (per step with 8 -> with the rule's:
+// 33^3 Gaussian noise 24 -> 7.5 us (TZ 1), 64^3 15 -> 8.8 (TZ 1); 128^3 keeps 8).
 constexpr int kEmGrid = 400;  // (TY+2)(TX+2) <= 6 * 66
+__host__ __device__ inline int em_div(int a, int b) { return (a + b - 1) / b; }
 __host__ __device__ inline void em_tile(int N, int &TX, int &TY, int &TZ) {
-  TX = N < 64 ? N : 64;
+  TX = em_div(N, em_div(N, 64));
   TY = kEmBlock / TX;
   if (TY > N) TY = N;
-  TZ = N < 8 ? N : 8;
+  const int tiles = em_div(N, TX) * em_div(N, TY);
+  TZ = 8;
+  for (int tz = 4; tz >= 1; tz /= 2)
+    if (em_div(tiles * em_div(N, tz), 1024) * (tz + 2) <
+        em_div(tiles * em_div(N, TZ), 1024) * (TZ + 2))
+      TZ = tz;
+  if (TZ > N) TZ = N;
 }
 __host__ __device__ inline int em_blocks(int N) {
   int TX, TY, TZ;
   em_tile(N, TX, TY, TZ);
-  return ((N + TX - 1) / TX) * ((N + TY - 1) / TY) * ((N + TZ - 1) / TZ);
+  return em_div(N, TX) * em_div(N, TY) * em_div(N, TZ);
 }
 
 struct GradSlot {
   double m2_s, m2_c, h_s, h_c, l_s, l_c;
 };
 
-__device__ __forceinline__ void em_noise(uint64_t skey, int64_t s, int kind, double xi[4]) {
+// GAUSS: Box-Muller pairs, otherwise variance1 draws.  A template argument:
+// as a run-time choice the transcendental functions' registers cost the
+// uniform noise a wave per SIMD.
+template <bool GAUSS>
+__device__ __forceinline__ void em_noise(uint64_t skey, int64_t s, double xi[4]) {
   Xoro g = xoro_seeded(site_key(skey, (uint64_t)s));
-  if (kind == 0) {
+  if (!GAUSS) {
     for (int a = 0; a < 4; a++) xi[a] = variance1(g);
   } else {
     for (int a = 0; a < 4; a += 2) {
@@ -64,8 +78,10 @@ __device__ __forceinline__ void em_noise(uint64_t skey, int64_t s, int kind, dou
       const double u2 = canonical(xoro_next(g));
       const double r = sqrt(-2.0 * log(1.0 - u1));
       const double th = 6.283185307179586 * u2;
-      xi[a] = r * cos(th);
-      xi[a + 1] = r * sin(th);
+      double sn, cs;
+      sincos(th, &sn, &cs);  // one range reduction for both
+      xi[a] = r * cs;
+      xi[a + 1] = r * sn;
     }
   }
 }
@@ -182,6 +198,7 @@ __global__ void k_em_zero(double *__restrict__ p, int64_t n) {
 // and its ring site.
 struct EmMarch {
   int N, x0, y0, z0, tw, th, tz, GW;
+  int zs, dz;  // first plane and direction of the march
   int tx, ty, x, y;
   bool own, halo;
   int hx, hy, hpos, pos;
@@ -197,6 +214,11 @@ struct EmMarch {
     tw = min(TX, N - x0);
     th = min(TY, N - y0);
     tz = min(TZ, N - z0);
+    // odd chunks march downwards: two neighbouring chunks then start, or end,
+    // at their common boundary at the same time, and the plane that each
+    // reads from the other is still in the XCD's L2
+    dz = bz & 1 ? -1 : 1;
+    zs = bz & 1 ? z0 + tz - 1 : z0;
     GW = tw + 2;
     const int t = threadIdx.x;
     tx = t % TX;
@@ -217,6 +239,11 @@ struct EmMarch {
     hy = hy < 0 ? hy + N : (hy >= N ? hy - N : hy);
     hpos = (hly + 1) * GW + (hlx + 1);
   }
+  // the plane after z in the march's direction (d = 1) or before it (-1)
+  __device__ int next(int z, int d) const {
+    z += d * dz;
+    return z < 0 ? N - 1 : (z == N ? 0 : z);
+  }
   __device__ uint32_t site(int xx, int yy, int z) const {
     return ((uint32_t)z * N + yy) * N + xx;
   }
@@ -224,30 +251,30 @@ struct EmMarch {
 
 // One forward step in -> out, marching z with the plane in LDS; the NS
 // volume sums of `out` go to `red`.
-template <int NS>
+template <int NS, bool GAUSS>
 __global__ __launch_bounds__(kEmBlock) void k_em_step(const double *__restrict__ in,
                                                       double *__restrict__ out, int N,
                                                       double m2, double lam, double H,
                                                       double gdt, double amp, uint64_t skey,
-                                                      int kind, double *slots, EmMerge prev) {
+                                                      double *slots, EmMerge prev) {
   __shared__ double Q[2][4][kEmGrid];
   const int64_t V = (int64_t)N * N * N;
   if (prev.slots && blockIdx.x == 0) em_merge(prev, V);
   const EmMarch m(N);
   KSum acc[NS > 0 ? NS : 1];
   for (int i = 0; i < NS; i++) acc[i] = KSum{0., 0.};
-  double cm[4], cc[4], cp[4];  // own column at z-1, z, z+1
+  double cm[4], cc[4], cp[4];  // own column behind z, at z, ahead of z
   if (m.own) {
-    const int zm = m.z0 == 0 ? N - 1 : m.z0 - 1;
+    const int zm = m.next(m.zs, -1);
 #pragma unroll
     for (int a = 0; a < 4; a++) {
       cm[a] = in[a * V + m.site(m.x, m.y, zm)];
-      cc[a] = in[a * V + m.site(m.x, m.y, m.z0)];
+      cc[a] = in[a * V + m.site(m.x, m.y, m.zs)];
     }
   }
   for (int j = 0; j < m.tz; j++) {
-    const int z = m.z0 + j;
-    const int zp = z + 1 == N ? 0 : z + 1;
+    const int z = m.zs + j * m.dz;
+    const int zp = m.next(z, 1);
     double(*g)[kEmGrid] = Q[j & 1];
     if (m.own) {
 #pragma unroll
@@ -265,7 +292,7 @@ __global__ __launch_bounds__(kEmBlock) void k_em_step(const double *__restrict__
       const uint32_t s = m.site(m.x, m.y, z);
       const double s2 = cc[0] * cc[0] + cc[1] * cc[1] + cc[2] * cc[2] + cc[3] * cc[3];
       double xi[4], o[4];
-      em_noise(skey, s, kind, xi);
+      em_noise<GAUSS>(skey, s, xi);
 #pragma unroll
       for (int a = 0; a < 4; a++) {
         const double nb = (g[a][m.pos + 1] + g[a][m.pos - 1]) +
@@ -323,18 +350,18 @@ __global__ __launch_bounds__(kEmBlock) void k_em_adjoint(const double *__restric
   const int64_t V = (int64_t)N * N * N;
   const EmMarch m(N);
   KSum ga{0., 0.}, gb{0., 0.}, gc{0., 0.};  // d/d m2, d/d H, d/d lambda
-  double lm[4], lc[4], lp[4];  // lam_in of the own column at z-1, z, z+1
+  double lm[4], lc[4], lp[4];  // lam_in of the own column behind z, at z, ahead
   if (m.own) {
-    const int zm = m.z0 == 0 ? N - 1 : m.z0 - 1;
+    const int zm = m.next(m.zs, -1);
 #pragma unroll
     for (int a = 0; a < 4; a++) {
       lm[a] = lin[a * V + m.site(m.x, m.y, zm)];
-      lc[a] = lin[a * V + m.site(m.x, m.y, m.z0)];
+      lc[a] = lin[a * V + m.site(m.x, m.y, m.zs)];
     }
   }
   for (int j = 0; j < m.tz; j++) {
-    const int z = m.z0 + j;
-    const int zp = z + 1 == N ? 0 : z + 1;
+    const int z = m.zs + j * m.dz;
+    const int zp = m.next(z, 1);
     double(*g)[kEmGrid] = Q[j & 1];
     double c[4];
     if (m.own) {
@@ -342,7 +369,8 @@ __global__ __launch_bounds__(kEmBlock) void k_em_adjoint(const double *__restric
 #pragma unroll
       for (int a = 0; a < 4; a++) {
         lp[a] = lin[a * V + m.site(m.x, m.y, zp)];
-        c[a] = phi[a * V + s];
+        // streamed through once: kept out of the caches that hold lam_in, lam_out
+        c[a] = __builtin_nontemporal_load(phi + a * V + s);
         g[a][m.pos] = lc[a];
       }
     }
@@ -437,6 +465,9 @@ struct lgv_em {
   GradSlot *gslots = nullptr;
   std::vector<double> phibar_host;
   bool have_forward = false;
+  // seg holds the inner states of the last segment, as the forward run (or a
+  // recomputation) left them
+  bool seg_last = false;
 };
 
 namespace {
@@ -448,43 +479,40 @@ void launch_step(int NS, const lgv_em_params &p, uint64_t base, int nblocks, con
   const double gdt = p.gamma * p.dt;
   const double amp = std::sqrt(2.0 * gdt);
   const uint64_t skey = stream_key(base, kEmTag | (uint64_t)n);
-  if (NS == 0)
-    k_em_step<0><<<nblocks, kEmBlock, 0, st>>>(in, out, p.N, p.m2, p.lambda, p.H, gdt, amp,
-                                               skey, p.noise_kind, slots, prev);
-  else if (NS == 1)
-    k_em_step<1><<<nblocks, kEmBlock, 0, st>>>(in, out, p.N, p.m2, p.lambda, p.H, gdt, amp,
-                                               skey, p.noise_kind, slots, prev);
+  auto launch = [&](auto kernel) {
+    kernel<<<nblocks, kEmBlock, 0, st>>>(in, out, p.N, p.m2, p.lambda, p.H, gdt, amp, skey,
+                                         slots, prev);
+  };
+  if (p.noise_kind)
+    launch(NS == 0 ? k_em_step<0, true> : (NS == 1 ? k_em_step<1, true> : k_em_step<kObsSums, true>));
   else
-    k_em_step<kObsSums><<<nblocks, kEmBlock, 0, st>>>(in, out, p.N, p.m2, p.lambda, p.H, gdt,
-                                                      amp, skey, p.noise_kind, slots, prev);
+    launch(NS == 0 ? k_em_step<0, false>
+                   : (NS == 1 ? k_em_step<1, false> : k_em_step<kObsSums, false>));
 }
 
-// Steps n0..n1-1 starting from `start`.  Forward mode (states == nullptr):
-// records phibar of every step, ping-pongs through the work buffers and
-// leaves phi_{n1} in `last`; with every > 0 it also writes the observables
-// of the states every, 2 every, ... below nsteps into rows (row = state /
-// every).  `pending` (may be nullptr) is a merge an earlier launch left for
-// the first step.  Recompute mode: states[i] = phi_{n0+i} for i = 0..n1-n0
-// (start is copied to states[0]), no sums; the work buffers, which hold
-// the adjoint state during the backward pass, are not touched.
+// Steps n0..n1-1 starting from `start`, leaving phi_{n1} in `last` (nullptr:
+// not needed, the last step is left out).  The states between go to
+// states[i] = phi_{n0+i}, i >= 1, or with states == nullptr ping-pong through
+// the work buffers, which hold the adjoint state during the backward pass and
+// are then not touched.  sums: records phibar of every step; with every > 0
+// also writes the observables of the states every, 2 every, ... below nsteps
+// into rows (row = state / every).  `pending` (may be nullptr) is a merge an
+// earlier launch left for the first step.
 int em_run_segment(lgv_em *h, const double *start, int n0, int n1, double *states,
-                   double *last, int every = 0, double *rows = nullptr,
+                   double *last, bool sums, int every = 0, double *rows = nullptr,
                    const EmMerge *pending = nullptr) {
   const size_t st = 4 * h->V * sizeof(double);
   const double *in = start;
-  if (states) {
-    EMCHECK(hipMemcpyAsync(states, start, st, hipMemcpyDeviceToDevice, h->stream));
-    in = states;
-  }
   EmMerge prev{nullptr, 1, h->nblocks, nullptr, nullptr};
   if (pending) prev = *pending;
-  for (int n = n0; n < n1; n++) {
-    double *out = states ? states + (int64_t)(n - n0 + 1) * 4 * h->V
-                         : ((n + 1 == n1) ? last : h->work[(n - n0) & 1]);
+  for (int n = n0; n < (last ? n1 : n1 - 1); n++) {
+    double *out = n + 1 == n1 ? last
+                  : states    ? states + (int64_t)(n - n0 + 1) * 4 * h->V
+                              : h->work[(n - n0) & 1];
     double *slots = h->part + (size_t)(n & 1) * h->nblocks * kPartStride;
     EmMerge mine{slots, 1, h->nblocks, nullptr, nullptr};
     int NS = 0;
-    if (!states) {  // the reverse pass uses the forward's phibar
+    if (sums) {  // the reverse pass uses the forward's phibar
       NS = 1;
       mine.phibar = h->phibar + n;
       if (every > 0 && (n + 1) % every == 0 && n + 1 < h->nsteps) {
@@ -497,7 +525,7 @@ int em_run_segment(lgv_em *h, const double *start, int n0, int n1, double *state
     in = out;
   }
   if (prev.slots) k_em_merge<<<1, kEmBlock, 0, h->stream>>>(prev, h->V);
-  if (!states && n1 == n0 && last != start)
+  if (last && n1 == n0 && last != start)
     EMCHECK(hipMemcpyAsync(last, start, st, hipMemcpyDeviceToDevice, h->stream));
   EMCHECK(hipGetLastError());
   return LGV_OK;
@@ -617,16 +645,22 @@ int lgv_em_forward(lgv_em *h, const double *phi0, int window, double *phi_final,
   if (window <= 0 || window > h->nsteps) return em_fail(LGV_ERR_ARG, "window outside [1,nsteps]");
   EMCHECK(hipSetDevice(h->device));
   h->window = window;
+  h->seg_last = false;
   const size_t st = 4 * h->V * sizeof(double);
   EMCHECK(hipMemcpyAsync(h->ckpt, phi0, st, hipMemcpyDeviceToDevice, h->stream));
   int rc;
   for (int j = 0; j < h->nseg; j++) {
     const int n0 = j * h->K, n1 = std::min(h->nsteps, n0 + h->K);
-    double *last = (j + 1 < h->nseg) ? h->ckpt + (int64_t)(j + 1) * 4 * h->V
-                                     : (phi_final ? phi_final : h->seg);
-    if ((rc = em_run_segment(h, h->ckpt + (int64_t)j * 4 * h->V, n0, n1, nullptr, last)))
+    // the last segment's states stay in seg: the backward pass, which starts
+    // there, then need not recompute them
+    const bool end = j + 1 == h->nseg;
+    double *last = !end ? h->ckpt + (int64_t)(j + 1) * 4 * h->V
+                        : (phi_final ? phi_final : h->work[0]);
+    if ((rc = em_run_segment(h, h->ckpt + (int64_t)j * 4 * h->V, n0, n1, end ? h->seg : nullptr,
+                             last, true)))
       return rc;
   }
+  h->seg_last = true;
   h->phibar_host.resize(h->nsteps);
   EMCHECK(hipMemcpyAsync(h->phibar_host.data(), h->phibar, h->nsteps * sizeof(double),
                          hipMemcpyDeviceToHost, h->stream));
@@ -663,18 +697,20 @@ int lgv_em_backward(lgv_em *h, double *grad_phi0, double grad_params[3]) {
   int rc;
   for (int j = h->nseg - 1; j >= 0; j--) {
     const int n0 = j * h->K, n1 = std::min(h->nsteps, n0 + h->K);
-    // recompute phi_{n0} .. phi_{n1-1} into seg (the forward noise is
+    // recompute phi_{n0+1} .. phi_{n1-1} into seg (the forward noise is
     // replayed from the same counters)
-    if ((rc = em_run_segment(h, h->ckpt + (int64_t)j * 4 * h->V, n0, n1 - 1, h->seg,
-                             nullptr)))
-      return rc;
+    const double *first = h->ckpt + (int64_t)j * 4 * h->V;
+    if (!(j + 1 == h->nseg && h->seg_last)) {
+      if ((rc = em_run_segment(h, first, n0, n1, h->seg, nullptr, false))) return rc;
+      h->seg_last = j + 1 == h->nseg;
+    }
     for (int n = n1 - 1; n >= n0; n--) {
       double dl = 0.;
       if (n >= h->nsteps - W)
         dl = (1.0 / W + (double)h->V * 2.0 * (h->phibar_host[n] - (double)mean) / W) /
              (double)h->V;
       k_em_adjoint<<<h->nblocks, kEmBlock, 0, h->stream>>>(
-          h->seg + (int64_t)(n - n0) * 4 * h->V, lam, nxt, h->p.N, h->p.m2, h->p.lambda, gdt,
+          n == n0 ? first : h->seg + (int64_t)(n - n0) * 4 * h->V, lam, nxt, h->p.N, h->p.m2, h->p.lambda, gdt,
           dl, h->gslots);
       std::swap(lam, nxt);
     }
@@ -714,7 +750,8 @@ int lgv_em_series(lgv_em *h, const double *phi0, int every, double *phi_final,
   EMCHECK(hipGetLastError());
   const EmMerge row0{slots, kObsSums, h->nblocks, nullptr, h->rows};
   int rc;
-  if ((rc = em_run_segment(h, phi0, 0, h->nsteps, nullptr, phi_final ? phi_final : h->seg,
+  if (!phi_final) h->seg_last = false;  // the final state takes seg's room
+  if ((rc = em_run_segment(h, phi0, 0, h->nsteps, nullptr, phi_final ? phi_final : h->seg, true,
                            every, h->rows, &row0)))
     return rc;
   EMCHECK(hipMemcpyAsync(rows_host, h->rows, (size_t)nrows * kNobs * sizeof(double),
