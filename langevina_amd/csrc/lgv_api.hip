@@ -219,8 +219,8 @@ int64_t ideal_plane_blocks(const ReplicaParams &p, int cap) {
 // us with 50, 390 with 34, 435 with 25; 224^3 FP32 305 us with 32, 334 with
 // 38).  Depth: a block marches TZ planes and rotates one more on either side,
 // and the GPU holds `slots` blocks at a time, so a launch takes about
-// ceil(blocks / slots) rounds of TZ + 2.5 planes each; TZ minimises that, up to
-// 16 (from there on the planes above and below are a small share).  FP64 with
+// ceil(blocks / slots) rounds of TZ + 2.5 planes each; TZ of 16, 8, 4, 2, 1
+// minimises that (above 16 the planes on either side are a small share).  FP64 with
 // 32 x 16 tiles -> with the rule's: 32^3 54 -> 12 us (TZ 1), 64^3 60 -> 17
 // (TZ 1), 100^3 66 -> 41 (50 wide, TZ 4), 128^3 89 -> 79 (TZ 8), 150^3 215 ->
 // 153 (38 wide), 200^3 443 -> 320 (50 wide, TZ 8); 256^3 and the 96-replica
@@ -244,7 +244,7 @@ void resolve_ideal_tiles(lgv_ctx *c) {
   }
   int best = 16;
   double best_cost = 1e300;
-  for (int tz = 16; tz >= 1; tz--) {
+  for (int tz = 16; tz >= 1; tz /= 2) {
     int64_t blocks = 0;
     for (const ReplicaParams &p : c->hp)
       blocks += ideal_plane_blocks(p, p.tile_cap) * ((p.N + tz - 1) / tz);

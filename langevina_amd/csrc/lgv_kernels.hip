@@ -1080,15 +1080,20 @@ void k_ideal_fused(const ReplicaParams *__restrict__ P, const ReplicaState *__re
     }
   };
 
-  rotate_own((z0 - 1 + N) % N, nex, chn);
+  // Odd chunks march downwards: two neighbouring chunks then start, or end, at
+  // their common boundary at the same time, and the planes that each reads
+  // from the other are still in the XCD's L2 (256^3 FP64 555 -> 540 us, 200^3
+  // 320 -> 308).  Below, planes "z-1" and "z+1" are those behind and ahead of z.
+  const int dz = bz & 1 ? -1 : 1, zs = bz & 1 ? z0 + tz - 1 : z0;
+  rotate_own(wrapz(zs - dz, N), nex, chn);
   if (own) {
 #pragma unroll
     for (int s = 0; s < 2; s++)
 #pragma unroll
       for (int c = 0; c < 4; c++) lprv[s][c][t] = nex[s][c];
   }
-  rotate_own(z0, cen, chn);
-  // the charges of plane z0: registers (FP64) or the thread's LDS slots (FP32)
+  rotate_own(zs, cen, chn);
+  // the charges of the first plane: registers (FP64) or the thread's LDS slots (FP32)
   if (own) {
 #pragma unroll
     for (int s = 0; s < 2; s++)
@@ -1100,15 +1105,15 @@ void k_ideal_fused(const ReplicaParams *__restrict__ P, const ReplicaState *__re
   }
   if (kEarlyRing && t < nh) {
     double f[10];
-    load_site<T, W>(p, cur, rgx, rgy, z0, f);
+    load_site<T, W>(p, cur, rgx, rgy, zs, f);
     rotate_site_fast(f, f + 4, f + 7, h);
 #pragma unroll
     for (int c = 0; c < 4; c++) lds[c][rpos] = f[c];
   }
-  fill_lds(z0, cen);
+  fill_lds(zs, cen);
   for (int k = 0; k < tz; k++) {
-    const int z = z0 + k;
-    const int zn = (z + 1) % N;
+    const int z = zs + k * dz;
+    const int zn = wrapz(z + dz, N);
     rotate_own(zn, nex, chn);
     T rraw[10];  // the ring site's raw fields of plane z+1, as stored
     const bool ring1 = kEarlyRing && t < nh && k + 1 < tz;
