@@ -20,7 +20,7 @@ TZS = (1, 2, 4, 8, 16, 32, 64)
 CHARGE_CAPS = (16, 32, 64)
 CHARGE_CHUNKS = (2, 4, 8, 16, 32)
 HB_CAPS = (16, 32, 64)
-HB_TZS = (8, 16, 32)
+HB_TZS = (4, 8, 16, 32)
 
 
 def set_ideal_tile(ctx, replica, cap, tz):
@@ -42,8 +42,8 @@ def charge_eff(N, cap, chunk):
 
 
 def hb_eff(N, cap, tz):
-    """The phi-march tile (TXH, TZ) a (cap, tz) request gives (0 = default)."""
-    return min(cap or 64, N // 2), min(tz or 16, N)
+    """The phi-march tile (TXH, TZ) a (cap, tz) request gives."""
+    return min(cap, N // 2), min(tz, N)
 
 
 def set_sweep_tiles(ctx, replica, hb_cap, hb_tz, chg_cap, chg_chunk):
@@ -150,7 +150,7 @@ def autotune_sweeps(ctx, dt, march=None, steps=3, verbose=False):
             print(f"autotune charge N={N}: cap={cap} chunk={ch} {ms * 1e3:.1f} us", flush=True)
         if not march:
             continue
-        cands, seen = [(0, 0)], {hb_eff(N, 0, 0)}
+        cands, seen = [(0, 0)], set()
         for cap in HB_CAPS:
             for tz in HB_TZS:
                 if hb_eff(N, cap, tz) not in seen:

@@ -1,6 +1,7 @@
 // lgv_api.hip -- the C ABI of include/lgv.h: context, replica storage,
 // composition of PV2HBSplit::step from the kernels, host-side global engine
 // (initial charges), monitors and measurement.
+#include <algorithm>
 #include <cfloat>
 #include <array>
 #include <cmath>
@@ -104,7 +105,8 @@ struct lgv_ctx {
   std::vector<void *> fields;
   Plan plan_half, plan_full, plan_ideal, plan_charge, plan_hb;
   bool wide = false;    // some plane is >= 4 GiB: kernels use 64-bit offsets
-  bool nt_stores = false;  // one buffer's fields exceed kStreamBytes
+  uint64_t buffer_bytes = 0;  // one buffer's fields, all replicas
+  int nt_stores = -1;  // non-temporal stores: -1 by the rule, 0 / 1 forced
   bool phi_march = false;  // the phi half-sweep runs the z-march kernel
   bool phi_march_auto = false;  // the size rule's choice (LGV_PHI_AUTO)
   MonSlot *mon_phi = nullptr, *mon_charge = nullptr, *mon_ideal = nullptr;
@@ -165,30 +167,98 @@ struct MeasBuf {
   }
 };
 
-int build_plan(Plan &plan, const std::vector<int64_t> &work, bool wide) {
+// A launch's work on one replica: its blocks, numbered plane after plane of
+// `plane` blocks each (0: in no such order).
+struct PlanWork {
+  int64_t blocks;
+  double plane;
+};
+
+// The order of a launch's blocks.  The dispatcher deals workgroups round-robin
+// over the eight XCDs, each with its own L2, so workgroup b runs on XCD b % 8:
+// blocks that read each other's edges are put on one XCD, close in time.
+//  * A replica of at most a sixteenth of the launch goes to one XCD as a whole
+//    (the largest first, each to the XCD with the least work).
+//  * A larger one is cut into eight bands of every plane, each XCD taking its
+//    band of plane after plane (where a plane's blocks don't divide by eight,
+//    the band edges move by an eighth of a block from plane to plane, so that
+//    the XCDs' shares even out); with fewer than eight blocks per plane into
+//    eight slabs of planes.
+// XCDs that run out of blocks take over the last ones of the longest list.
+// local: block within its replica.
+void xcd_order(const std::vector<PlanWork> &work, std::vector<int> &rep, std::vector<int> &local) {
+  int64_t total = 0;
+  for (const PlanWork &w : work) total += w.blocks;
+  std::vector<std::pair<int, int>> list[8];
+  std::vector<int> by_size(work.size());
+  for (size_t r = 0; r < work.size(); r++) by_size[r] = (int)r;
+  std::stable_sort(by_size.begin(), by_size.end(),
+                   [&](int a, int b) { return work[a].blocks > work[b].blocks; });
+  for (int r : by_size) {
+    const PlanWork &w = work[r];
+    if (16 * w.blocks <= total) {
+      auto *least = &list[0];
+      for (auto &l : list)
+        if (l.size() < least->size()) least = &l;
+      for (int64_t j = 0; j < w.blocks; j++) least->push_back({r, (int)j});
+      continue;
+    }
+    const double span = w.plane >= 8. ? w.plane : (double)w.blocks;
+    for (int64_t j = 0; j < w.blocks; j++) {
+      const int64_t z = (int64_t)((double)j / span);
+      const double u = (double)j - (double)z * span + .125 * (double)(5 * z & 7);
+      const int x = w.plane > 0. ? (int)(8. * u / span) : (int)(j & 7);
+      list[std::min(std::max(x, 0), 7)].push_back({r, (int)j});
+    }
+  }
+  size_t head[8] = {0}, tail[8];
+  for (int x = 0; x < 8; x++) tail[x] = list[x].size();
+  rep.resize(total);
+  local.resize(total);
+  for (int64_t b = 0; b < total; b++) {
+    int x = (int)(b & 7);
+    std::pair<int, int> e;
+    if (head[x] < tail[x]) {
+      e = list[x][head[x]++];
+    } else {
+      for (int k = 0; k < 8; k++)
+        if (tail[k] - head[k] > tail[x] - head[x]) x = k;
+      e = list[x][--tail[x]];
+    }
+    rep[b] = e.first;
+    local[b] = e.second;
+  }
+}
+
+int upload(int **dev, const std::vector<int> &v) {
+  HIPCHECK(hipMalloc(dev, v.size() * sizeof(int)));
+  HIPCHECK(hipMemcpy(*dev, v.data(), v.size() * sizeof(int), hipMemcpyHostToDevice));
+  return LGV_OK;
+}
+
+// ordered: the blocks in xcd_order, otherwise replica after replica.
+int build_plan(Plan &plan, const std::vector<PlanWork> &work, bool wide, bool ordered = true) {
   plan.wide = wide;
   plan.first.clear();
-  std::vector<int> rep, first;
+  std::vector<int> rep, local;
+  int64_t total = 0;
   for (size_t r = 0; r < work.size(); r++) {
-    first.push_back((int)rep.size());
-    const int64_t nb = (work[r] + kBlock - 1) / kBlock;
-    for (int64_t b = 0; b < nb; b++) rep.push_back((int)r);
+    plan.first.push_back((int)total);
+    total += work[r].blocks;
+    if (!ordered) rep.resize(total, (int)r);
   }
-  plan.nblocks = (int)rep.size();
-  plan.first = first;
-  HIPCHECK(hipMalloc(&plan.d_blk_rep, rep.size() * sizeof(int)));
-  HIPCHECK(hipMalloc(&plan.d_blk_first, first.size() * sizeof(int)));
-  HIPCHECK(hipMemcpy(plan.d_blk_rep, rep.data(), rep.size() * sizeof(int),
-                     hipMemcpyHostToDevice));
-  HIPCHECK(hipMemcpy(plan.d_blk_first, first.data(), first.size() * sizeof(int),
-                     hipMemcpyHostToDevice));
-  return LGV_OK;
+  plan.nblocks = (int)total;
+  if (ordered) xcd_order(work, rep, local);
+  int rc = upload(&plan.blocks.rep, rep);
+  if (!rc) rc = upload(&plan.blocks.first, plan.first);
+  if (!rc && ordered) rc = upload(&plan.blocks.local, local);
+  return rc;
 }
 
 // Releases a plan's device arrays (the stream must be idle).
 int free_plan(Plan &plan) {
-  if (plan.d_blk_rep) HIPCHECK(hipFree(plan.d_blk_rep));
-  if (plan.d_blk_first) HIPCHECK(hipFree(plan.d_blk_first));
+  for (int *p : {plan.blocks.rep, plan.blocks.local, plan.blocks.first})
+    if (p) HIPCHECK(hipFree(p));
   plan = Plan{};
   return LGV_OK;
 }
@@ -214,17 +284,16 @@ int64_t ideal_plane_blocks(const ReplicaParams &p, int cap) {
 // The ideal kernel's tiles where the caller asked for none.  Width: 32
 // half-columns where they divide the row (whole 128-byte lines of every
 // component: 256^3 FP64 541 us against 560 with 64) or need fewer tiles than
-// the alternative, which is the widest even split that the kernel's plane grid
-// holds (every ring column costs a line per row and component: 200^3 FP64 329
-// us with 50, 390 with 34, 435 with 25; 224^3 FP32 305 us with 32, 334 with
-// 38).  Depth: a block marches TZ planes and rotates one more on either side,
-// and the GPU holds `slots` blocks at a time, so a launch takes about
-// ceil(blocks / slots) rounds of TZ + 2.5 planes each; TZ of 16, 8, 4, 2, 1
-// minimises that (above 16 the planes on either side are a small share).  FP64 with
-// 32 x 16 tiles -> with the rule's: 32^3 54 -> 12 us (TZ 1), 64^3 60 -> 17
-// (TZ 1), 100^3 66 -> 41 (50 wide, TZ 4), 128^3 89 -> 79 (TZ 8), 150^3 215 ->
-// 153 (38 wide), 200^3 443 -> 320 (50 wide, TZ 8); 256^3 and the 96-replica
-// batch keep 32 x 16.
+// the alternative; 16 for FP64 rows of several tiles that those divide (160^3
+// 174 -> 148 us, 224^3 443 -> 398; a FP32 row of 16 is half a line); otherwise
+// the widest even split that the kernel's plane grid holds (every ring column
+// costs a line per row and component: 200^3 FP64 329 us with 50, 390 with 34,
+// 435 with 25).  Depth: a block marches TZ planes and rotates one more on
+// either side, and the GPU holds `slots` blocks at a time.  A launch of up to
+// two rounds takes whole rounds of TZ planes, a longer one its blocks' share
+// and a tail; TZ of 16, 8, 4, and 2, 1 within one round, minimises that (FP64, TZ 16, 8, 4: 256^3
+// 537, 546, 575 us; 240^3 558, 522, 523; 192^3 261, 245, 249; 144^3 140, 125,
+// 123; 100^3 63, 42, 38; 64^3 TZ 1 17 us, TZ 16 60).
 void resolve_ideal_tiles(lgv_ctx *c) {
   const int slots = kCUs * (c->fp32 ? 3 : 2);
   for (int r = 0; r < c->nrep; r++) {
@@ -241,15 +310,19 @@ void resolve_ideal_tiles(lgv_ctx *c) {
     }
     if (p.NH % 32 == 0 || ideal_plane_blocks(p, 32) < ideal_plane_blocks(p, p.tile_cap))
       p.tile_cap = 32;
+    if (!c->fp32 && p.NH % 32 == 16 && p.NH > p.tile_cap) p.tile_cap = 16;
   }
   int best = 16;
   double best_cost = 1e300;
+  const double tail = c->fp32 ? .15 : .25;
   for (int tz = 16; tz >= 1; tz /= 2) {
     int64_t blocks = 0;
     for (const ReplicaParams &p : c->hp)
       blocks += ideal_plane_blocks(p, p.tile_cap) * ((p.N + tz - 1) / tz);
-    const double cost = ((blocks + slots - 1) / slots) * (tz + 2.5);
-    if (cost < best_cost * 0.98) {
+    const double rounds = (double)blocks / slots;
+    if (tz < 4 && rounds > 1.) break;
+    const double cost = (rounds <= 2. ? std::ceil(rounds) : rounds + tail) * (tz + .5);
+    if (cost < best_cost) {
       best = tz;
       best_cost = cost;
     }
@@ -258,49 +331,92 @@ void resolve_ideal_tiles(lgv_ctx *c) {
     c->hp[r].tile_tz = c->tiles[r].ideal_tz ? c->tiles[r].ideal_tz : best;
 }
 
+// Whether rows of NH half-columns and of tiles of TXH are whole units of bytes.
+bool whole_rows(const lgv_ctx *c, int NH, int TXH, int bytes) {
+  const int esz = c->fp32 ? 4 : 8;
+  return NH * esz % bytes == 0 && TXH * esz % bytes == 0;
+}
+
 // Blocks of the fused ideal kernel: one per (x-tile, y-tile, z-chunk) of
 // every replica, with that replica's tile shape.
 int build_ideal_plan(lgv_ctx *c) {
   resolve_ideal_tiles(c);
-  std::vector<int64_t> work;
+  std::vector<PlanWork> work;
+  bool stream = c->buffer_bytes > 2 * kCacheBytes;
   for (int r = 0; r < c->nrep; r++) {
     const ReplicaParams &p = c->hp[r];
     int TXH, TY, TZ;
     ideal_tile(p.N, p.tile_cap, p.tile_tz, TXH, TY, TZ);
     if ((TY + 2) * (2 * TXH + 2) > ideal_lds(c->fp32))
       return fail(LGV_ERR_ARG, "replica %d: ideal tile %dx%d exceeds the LDS plane", r, TXH, TY);
-    work.push_back((int64_t)((p.NH + TXH - 1) / TXH) * ((p.N + TY - 1) / TY) *
-                   ((p.N + TZ - 1) / TZ) * kBlock);
+    stream = stream && whole_rows(c, p.NH, TXH, 128);
+    const int64_t plane = (int64_t)((p.NH + TXH - 1) / TXH) * ((p.N + TY - 1) / TY);
+    work.push_back({plane * ((p.N + TZ - 1) / TZ), (double)plane});
   }
-  if (c->plan_ideal.d_blk_rep) {
-    HIPCHECK(hipStreamSynchronize(c->stream));
-    HIPCHECK(hipFree(c->plan_ideal.d_blk_rep));
-    HIPCHECK(hipFree(c->plan_ideal.d_blk_first));
-    c->plan_ideal = Plan{};
-  }
-  const int rc = build_plan(c->plan_ideal, work, c->wide);
-  c->plan_ideal.stream = c->nt_stores;
+  if (c->plan_ideal.nblocks) HIPCHECK(hipStreamSynchronize(c->stream));
+  int rc = free_plan(c->plan_ideal);
+  if (rc) return rc;
+  rc = build_plan(c->plan_ideal, work, c->wide);
+  c->plan_ideal.stream = c->nt_stores < 0 ? stream : c->nt_stores;
   return rc;
+}
+
+// The phi march's tiles where the caller asked for none.  Width: an even split
+// of the row into at most 64 half-columns (wide rows keep the x-halo columns a
+// small share of the lines that a plane touches), rounded up to a multiple of
+// 16 where the tile keeps as many rows, so that tiles begin on whole lines
+// (FP64 224^3 56 wide 120 us, 64 wide 119 and with non-temporal stores 106;
+// 272^3 46 wide 215, 48 wide 206 and 198).  Depth: TZ of 16, 8, 4 that minimises
+// the planes moved, blocks times TZ and the chunk's extra loads, over the GPU's
+// 1024 resident blocks, plus half a block's time for the launch's end (FP64 TZ
+// 16, 8, 4: 256^3 147, 144, 150 us; 128^3 26.4, 23.7, 24.2; 100^3 24.8, 16.8,
+// 15.5).
+void resolve_hb_tiles(lgv_ctx *c) {
+  for (int r = 0; r < c->nrep; r++) {
+    ReplicaParams &p = c->hp[r];
+    const int w = even_width(p.NH, 64), w16 = (w + 15) / 16 * 16;
+    p.hb_cap = c->tiles[r].hb_cap ? c->tiles[r].hb_cap
+               : w < p.NH && kBlock / w16 == kBlock / w ? w16 : w;
+  }
+  int best = 16;
+  double best_cost = 1e300;
+  for (int tz = 16; tz >= 4; tz /= 2) {
+    int64_t blocks = 0;
+    for (const ReplicaParams &p : c->hp) {
+      int TXH, TY, TZ;
+      hb_tile(p.N, p.hb_cap, tz, TXH, TY, TZ);
+      blocks += (int64_t)((p.NH + TXH - 1) / TXH) * ((p.N + TY - 1) / TY) * ((p.N + tz - 1) / tz);
+    }
+    const double cost = (tz + (c->fp32 ? 2 : 1)) * ((double)blocks / (4 * kCUs) + .5);
+    if (cost < best_cost * 0.98) {
+      best = tz;
+      best_cost = cost;
+    }
+  }
+  for (int r = 0; r < c->nrep; r++)
+    c->hp[r].hb_tz = c->tiles[r].hb_tz ? c->tiles[r].hb_tz : best;
 }
 
 // Blocks of the phi march kernel: (x-tile, y-tile, z-chunk) per replica.
 int build_hb_plan(lgv_ctx *c) {
-  std::vector<int64_t> work;
+  resolve_hb_tiles(c);
+  std::vector<PlanWork> work;
+  bool wide = c->wide, stream = c->buffer_bytes / 10 * 4 > kCacheBytes;
   for (int r = 0; r < c->nrep; r++) {
-    ReplicaParams &p = c->hp[r];
-    p.hb_cap = c->tiles[r].hb_cap;
-    p.hb_tz = c->tiles[r].hb_tz;
+    const ReplicaParams &p = c->hp[r];
+    wide = wide || 2 * (uint64_t)p.half * (c->fp32 ? 4 : 8) > 0xFFFFFFFFull;
     int TXH, TY, TZ;
     hb_tile(p.N, p.hb_cap, p.hb_tz, TXH, TY, TZ);
     if ((TY + 2) * (TXH + 2) > kHbMarchGrid || 2 * TY + 2 * TXH > kBlock)
       return fail(LGV_ERR_ARG, "replica %d: phi tile %dx%d does not fit", r, TXH, TY);
-    work.push_back((int64_t)((p.NH + TXH - 1) / TXH) * ((p.N + TY - 1) / TY) *
-                   ((p.N + TZ - 1) / TZ) * kBlock);
+    stream = stream && whole_rows(c, p.NH, TXH, 64);
+    const int64_t plane = (int64_t)((p.NH + TXH - 1) / TXH) * ((p.N + TY - 1) / TY);
+    work.push_back({plane * ((p.N + TZ - 1) / TZ), (double)plane});
   }
   int rc = free_plan(c->plan_hb);
   if (rc) return rc;
-  rc = build_plan(c->plan_hb, work, c->wide);
-  c->plan_hb.stream = c->nt_stores;
+  rc = build_plan(c->plan_hb, work, wide);
+  c->plan_hb.stream = c->nt_stores < 0 ? stream : c->nt_stores;
   return rc;
 }
 
@@ -355,15 +471,16 @@ void resolve_charge_tiles(lgv_ctx *c) {
 // Blocks of the charge march kernel: (x-tile, line tile, chunk) per replica.
 int build_charge_plan(lgv_ctx *c) {
   resolve_charge_tiles(c);
-  std::vector<int64_t> work;
+  std::vector<PlanWork> work;
   for (int r = 0; r < c->nrep; r++) {
     const ReplicaParams &p = c->hp[r];
     int TXH, TQ, C;
     charge_tile(p.N, p.chg_cap, p.chg_chunk, TXH, TQ, C);
     if (C % 2 != 0) return fail(LGV_ERR_ARG, "replica %d: charge chunk %d is odd", r, C);
     // two blocks per tile: the even and the odd x of its half-columns
-    work.push_back((int64_t)2 * ((p.NH + TXH - 1) / TXH) * ((p.N + TQ - 1) / TQ) *
-                   ((p.N + C - 1) / C) * kBlock);
+    work.push_back({(int64_t)2 * ((p.NH + TXH - 1) / TXH) * ((p.N + TQ - 1) / TQ) *
+                        ((p.N + C - 1) / C),
+                    0.});
   }
   int rc = free_plan(c->plan_charge);
   if (rc) return rc;
@@ -479,14 +596,11 @@ int enqueue_ideal(lgv_ctx *c, int off, int flip) {
 
 // EulerLangevinHB::step (counters off, off+1 for the two parities), one
 // in-place launch per parity: the z-march with the other parity's plane in
-// LDS or the one-thread-per-site kernel, by the size rule (the march for
-// FP64 fields above 1 GiB and FP32 fields above 600 MiB) unless
-// lgv_set_phi_kernel chose.  Measured per half-sweep before the march's
-// prefetch, FP64: 256^3 march 157 us against 204 us per site; 192^3 85
-// against 75 (70 in plane bands), 128^3 35 against 29 (26), 64^3 30 against
-// 9 (below 1 GiB the fields stay largely cache-resident and the per-site
-// kernel's 8 waves per SIMD win); FP32 256^3 110 against 109, but the
-// march's lower traffic speeds up the kernels that follow (kMarchBytesFp32).
+// LDS or the one-thread-per-site kernel, by the size rule (the march from
+// kMarchSites on) unless lgv_set_phi_kernel chose.  Per half-sweep, site
+// against march, FP64: 64^3 8.9, 9.5 us; 100^3 16.8, 15.5; 160^3 42, 44; 192^3
+// 67, 66; 224^3 147, 109; 256^3 221, 147; FP32: 160^3 33, 33; 224^3 79, 70;
+// 256^3 116, 86.
 bool use_march(const lgv_ctx *c) { return c->phi_march; }
 const Plan &hb_plan(const lgv_ctx *c) { return use_march(c) ? c->plan_hb : c->plan_half; }
 int enqueue_hb(lgv_ctx *c, int off, int flip) {
@@ -694,7 +808,7 @@ int lgv_create(const lgv_config *cfg, lgv_ctx **out) {
   c->tiles.resize(c->nrep);
   c->noise.resize(c->nrep);
   const size_t esz = c->fp32 ? sizeof(float) : sizeof(double);
-  std::vector<int64_t> whalf, wfull;
+  std::vector<PlanWork> whalf, wfull;
   uint64_t buffer_bytes = 0;  // one buffer: 10 planes x 2 parities
   std::vector<ReplicaState> hs(c->nrep);
   for (int r = 0; r < c->nrep; r++) {
@@ -725,24 +839,28 @@ int lgv_create(const lgv_config *cfg, lgv_ctx **out) {
     c->noise[r].g = xoro_seeded((uint64_t)s32);
     hs[r] = ReplicaState{};
     hs[r].t = m.initialtime;
-    whalf.push_back(half);
-    wfull.push_back(2 * half);
+    whalf.push_back({(half + kBlock - 1) / kBlock, (double)N * p.NH / kBlock});
+    wfull.push_back({(2 * half + kBlock - 1) / kBlock, 0.});
     if ((uint64_t)half * esz > 0xFFFFFFFFull) c->wide = true;
     buffer_bytes += (uint64_t)20 * half * esz;
     // test hook: LGV_FORCE_WIDE=1 runs the 64-bit-offset kernels on any size
     if (const char *fw = getenv("LGV_FORCE_WIDE")) c->wide = c->wide || atoi(fw) != 0;
     c->maxN = std::max(c->maxN, N);
   }
-  c->nt_stores = buffer_bytes > kStreamBytes;
-  // test hook: LGV_NT_STORES=0/1 forces the store mode on any size
-  if (const char *nt = getenv("LGV_NT_STORES")) c->nt_stores = atoi(nt) != 0;
-  c->phi_march = c->fp32 ? buffer_bytes > kMarchBytesFp32 : c->nt_stores;
-  c->phi_march_auto = c->phi_march;
+  c->buffer_bytes = buffer_bytes;
+  c->phi_march_auto = buffer_bytes / (10 * esz) >= kMarchSites;
+  // test hook: LGV_NT_STORES=0/1 forces the store mode on any size, and with
+  // FP64 fields the phi kernel that goes with it (1: the march)
+  if (const char *nt = getenv("LGV_NT_STORES")) {
+    c->nt_stores = atoi(nt) != 0;
+    if (!c->fp32) c->phi_march_auto = c->nt_stores;
+  }
+  c->phi_march = c->phi_march_auto;
   // one lattice whose launches each fill the GPU many times over gains
   // nothing from running the charge sweep beside the phi sweeps (256^3:
   // 1 % slower); smaller and batched lattices do (128^3 FP64 2.53e9 ->
   // 2.67e9 site-updates/s, the 96-replica FP32 batch +2 %)
-  c->overlap = !(cfg->nreplicas == 1 && buffer_bytes > kMarchBytesFp32);
+  c->overlap = !(cfg->nreplicas == 1 && buffer_bytes > kOverlapBytes);
   // test hook: LGV_OVERLAP=0/1 forces the sequential / concurrent order
   if (const char *ov = getenv("LGV_OVERLAP")) c->overlap = atoi(ov) != 0;
   // test hook: LGV_PHI_KERNEL=site/march forces the phi half-sweep kernel
@@ -756,7 +874,7 @@ int lgv_create(const lgv_config *cfg, lgv_ctx **out) {
   HIPCHECK(hipMemcpy(c->dS, hs.data(), c->nrep * sizeof(ReplicaState), hipMemcpyHostToDevice));
   int rc;
   if ((rc = build_plan(c->plan_half, whalf, c->wide)) != LGV_OK) return rc;
-  if ((rc = build_plan(c->plan_full, wfull, c->wide)) != LGV_OK) return rc;
+  if ((rc = build_plan(c->plan_full, wfull, c->wide, false)) != LGV_OK) return rc;
   if ((rc = build_ideal_plan(c.get())) != LGV_OK) return rc;
   if ((rc = build_charge_plan(c.get())) != LGV_OK) return rc;
   if ((rc = build_hb_plan(c.get())) != LGV_OK) return rc;
@@ -802,8 +920,7 @@ int lgv_destroy(lgv_ctx *c) {
   note(hipFree(c->dP));
   note(hipFree(c->dS));
   for (Plan *pl : {&c->plan_half, &c->plan_full, &c->plan_ideal, &c->plan_charge, &c->plan_hb}) {
-    note(hipFree(pl->d_blk_rep));
-    note(hipFree(pl->d_blk_first));
+    for (int *q : {pl->blocks.rep, pl->blocks.local, pl->blocks.first}) note(hipFree(q));
   }
   for (void *q : {(void *)c->mon_phi, (void *)c->mon_charge, (void *)c->mon_ideal,
                   (void *)c->eslots, (void *)c->d_aos, (void *)c->d_part,

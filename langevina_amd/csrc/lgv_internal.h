@@ -66,18 +66,14 @@ __host__ __device__ inline void ideal_tile(int N, int cap, int tz, int &TXH, int
 }
 
 // Tile of the single-parity phi march: TXH half-columns x TY rows in x-y,
-// chunks of TZ planes in z.  Defaults (cap, tz = 0): 64 x 4 x 16 from
-// N = 128 on (wide rows keep the x-halo columns a small share of the lines
-// each plane touches); cap and tz are tunables, valid while the packed grid
-// fits (TY+2)(TXH+2) <= kHbMarchGrid and the ring 2 TY + 2 TXH <= kBlock.
+// chunks of TZ planes in z, valid while the packed grid fits
+// (TY+2)(TXH+2) <= kHbMarchGrid and the ring 2 TY + 2 TXH <= kBlock.
 __host__ __device__ inline void hb_tile(int N, int cap, int tz, int &TXH, int &TY, int &TZ) {
   const int NH = N / 2;
-  const int c = cap > 0 ? cap : 64;
-  TXH = NH < c ? NH : c;
+  TXH = NH < cap ? NH : cap;
   TY = 256 / TXH;
   if (TY > N) TY = N;
-  const int zc = tz > 0 ? tz : 16;
-  TZ = N < zc ? N : zc;
+  TZ = N < tz ? N : tz;
 }
 
 // Its packed LDS grid: (TY+2)(TXH+2) entries.
@@ -105,39 +101,52 @@ struct EnergySlot {
   double g_s, g_c, h_s, h_c, n_s, n_c;
 };
 
-// A launch over several replicas: block b belongs to replica blk_rep[b] and
-// is its (b - blk_first[replica])-th block.
+// The blocks of a launch over several replicas, on the device: workgroup b is
+// block local[b] of replica rep[b] (local == nullptr: block b - first[rep[b]]),
+// and a replica's monitor slots start at first[replica].
+struct LaunchBlocks {
+  int *rep = nullptr, *local = nullptr, *first = nullptr;
+};
 struct Plan {
   int nblocks = 0;
-  int *d_blk_rep = nullptr;
-  int *d_blk_first = nullptr;
-  bool wide = false;    // some plane of the launch is >= 4 GiB (64-bit offsets)
-  bool stream = false;  // outputs written with non-temporal stores (see kStreamBytes)
+  LaunchBlocks blocks;
+  bool wide = false;    // 64-bit offsets: some plane of the launch (phi march: pair of planes)
+                        // is >= 4 GiB
+  bool stream = false;  // outputs written with non-temporal stores (see kCacheBytes)
   bool far = false;     // some replica's charge planes span >= 4 GiB (charge launch)
   bool xwave = false;   // charge launch: every replica has N = 128 or 256 (x rows per wave)
-  std::vector<int> first;  // host copy of d_blk_first
+  std::vector<int> first;  // host copy of blocks.first
 };
 
 // The phi march and the ideal kernel write their outputs with non-temporal
-// stores when one buffer's fields (all replicas) exceed this: the outputs
-// are next read by a later launch, after the whole lattice has been swept,
-// so caching them only evicts the lines that neighbouring tiles still read.
-// Measured at 256^3 FP64 (1.3 GB): ideal 602 -> 586 us, phi 175 -> 168 us;
-// at 64^3-128^3 and for FP32 256^3 (0.7 GB) the plain stores are as fast or
-// faster.
-constexpr uint64_t kStreamBytes = 1ull << 30;
+// stores where the outputs are next read by a later launch, after planes that
+// together exceed the last-level cache have been swept, so that caching them
+// only evicts lines that neighbouring tiles still read; and only where a tile's
+// rows are whole lines (a non-temporal store of part of a line costs more than
+// a cached one).  Ideal: fields (one buffer) above twice the cache, rows and
+// tile rows of whole 128-byte lines; FP64 192^3 263 -> 259 us, 224^3 449 ->
+// 437, 256^3 556 -> 534, FP32 256^3 324 -> 318, but 208^3 FP64 (rows of 6.5
+// lines) 384 -> 413, 200^3 308 -> 377, 288^3 FP32 644 -> 956.  Phi march: phi
+// planes (one buffer) above the cache, rows and tile rows of whole 64-byte
+// halves; FP64 208^3 94.5 -> 90.8 us, 224^3 119 -> 106, 256^3 170 -> 148,
+// FP32 384^3 302 -> 291, but 256^3 FP32 (phi planes of just 256 MB) 86 -> 92,
+// 280^3 FP64 (rows of 8.75 lines) 228 -> 242, 320^3 in tiles of 54 342 -> 394.
+constexpr uint64_t kCacheBytes = 256ull << 20;
 
-// FP32 fields above this (one buffer, all replicas) also take the phi
-// z-march: its own launch is no faster than the one-thread-per-site kernel
-// (256^3: 110 against 109 us), but it moves 1.09x instead of 1.36x the
-// algorithmic bytes and leaves more of the charge and phi planes in the
-// 256 MB last-level cache for the kernels that follow (256^3 FP32 step
-// 3.72 -> 3.61 ms: charge 337 -> 317 us, ideal 429 -> 414 us).  Below it
-// the size rule takes the per-site kernel (single 128^3-192^3 lattices run
-// faster with it); the autotuner may choose the march instead (the
-// 96-replica FP32 batch does).  A context of one lattice above this size
-// also keeps the charge sweep after the phi sweeps rather than beside them.
-constexpr uint64_t kMarchBytesFp32 = 600ull << 20;
+// From this many sites on (all replicas) the phi half-sweeps run the z-march:
+// it reads each value of the other parity once per launch where the
+// one-thread-per-site kernel reads it up to four times, which costs that
+// kernel traffic once the fields outgrow the 256 MB last-level cache; below,
+// the per-site kernel's eight waves per SIMD (the march has four) count more.
+// Whole steps, per site -> march: FP64 100^3 328 -> 332 us, 150^3 1134 -> 1169,
+// 180^3 2058 -> 2070, 192^3 2124 -> 2082, 224^3 3840 -> 3636, 256^3 5006 ->
+// 4371; FP32 128^3 410 -> 411, 180^3 1219 -> 1229, 192^3 1328 -> 1304, 224^3
+// 2253 -> 2214, 256^3 2949 -> 2708.
+constexpr uint64_t kMarchSites = 7000000;
+
+// A context of one lattice whose fields (one buffer) exceed this keeps the
+// charge sweep after the phi sweeps rather than beside them.
+constexpr uint64_t kOverlapBytes = 600ull << 20;
 
 // Largest side: N^3 must fit 32-bit site indices.
 constexpr int kMaxN = 1536;

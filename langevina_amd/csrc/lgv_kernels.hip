@@ -169,12 +169,76 @@ struct ChargePlanes<T, false> {
   }
 };
 
-// Block index of this workgroup within the launch plan.  (A renumbering that
-// gives each XCD a contiguous eighth of the plan was measured on MI355X and
-// made the ideal and charge sweeps slower; the ideal kernel and the phi march
-// map one-replica launches with yband_tile instead, the charge sweep keeps
-// dispatch order.)
-__device__ __forceinline__ int xcd_block() { return blockIdx.x; }
+// The phi planes of a replica's live buffer for a march in z: an access names
+// a component, a parity, a plane z and the lane's offset within the plane.
+// W == false: one buffer resource per component (its two half-planes, less
+// than 4 GiB); the plane's offset is scalar and the lane's stays in one vector
+// register for the whole march.  That leaves no vector address arithmetic, and
+// no address temporary that would first have to wait for a pending load into
+// its register (measured in the FP32 march, where such waits for the loads of
+// the plane after next come and go with the register allocation).
+// W == true: 64-bit addresses.
+// NT: a value no other thread reads, not kept in the caches.
+template <typename T, bool W>
+struct PhiPlanes {
+  GPlane<T, true> f[4];
+  int64_t half_bytes;
+  uint32_t plane;
+  __device__ __forceinline__ PhiPlanes(const ReplicaParams &p, int cur) {
+    const FieldBufs fb = field_bufs<T>(p);
+    half_bytes = fb.half_bytes;
+    plane = (uint32_t)p.N * p.NH;
+#pragma unroll
+    for (int l = 0; l < 4; l++) f[l] = gplane<T, true>(fb, cur, l, 0);
+  }
+  __device__ __forceinline__ GPlane<T, true> half(int l, int par) const {
+    return {f[l].b + (par ? half_bytes : 0)};
+  }
+  template <bool NT>
+  __device__ __forceinline__ T ld(int l, int par, int z, uint32_t i) const {
+    return half(l, par).template get_raw<NT>((uint32_t)z * plane + i);
+  }
+  template <bool NT>
+  __device__ __forceinline__ void st(int l, int par, int z, uint32_t i, T v) const {
+    half(l, par).template put_raw<NT>((uint32_t)z * plane + i, v);
+  }
+};
+template <typename T>
+struct PhiPlanes<T, false> {
+  __amdgpu_buffer_rsrc_t f[4];
+  uint32_t half_bytes, plane_bytes;
+  __device__ __forceinline__ PhiPlanes(const ReplicaParams &p, int cur) {
+    const FieldBufs fb = field_bufs<T>(p);
+    half_bytes = first_lane((int)fb.half_bytes);
+    plane_bytes = (uint32_t)p.N * p.NH * (uint32_t)sizeof(T);
+    char *b = cur & 1 ? fb.f1 : fb.f0;
+#pragma unroll
+    for (int l = 0; l < 4; l++)
+      f[l] = __builtin_amdgcn_make_buffer_rsrc(
+          reinterpret_cast<char *>(
+              first_lane((uint64_t)reinterpret_cast<uintptr_t>(b + 2 * l * fb.half_bytes))),
+          0, (int)(2u * half_bytes), 0x00027000);
+  }
+  template <bool NT>
+  __device__ __forceinline__ T ld(int l, int par, int z, uint32_t i) const {
+    const uint32_t s = (uint32_t)z * plane_bytes + (par ? half_bytes : 0u);
+    if constexpr (sizeof(T) == 4)
+      return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(f[l], i * 4u, s, NT ? 2 : 0));
+    else
+      return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(f[l], i * 8u, s, NT ? 2 : 0));
+  }
+  template <bool NT>
+  __device__ __forceinline__ void st(int l, int par, int z, uint32_t i, T v) const {
+    const uint32_t s = (uint32_t)z * plane_bytes + (par ? half_bytes : 0u);
+    typedef uint32_t b64 __attribute__((ext_vector_type(2)));
+    if constexpr (sizeof(T) == 4)
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), f[l], i * 4u, s,
+                                            NT ? 2 : 0);
+    else
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(b64, v), f[l], i * 8u, s,
+                                            NT ? 2 : 0);
+  }
+};
 
 __device__ __forceinline__ int wrapp(int a, int N) { return a == N ? 0 : a; }
 __device__ __forceinline__ int wrapm(int a, int N) { return a < 0 ? N - 1 : a; }
@@ -323,21 +387,13 @@ __device__ __forceinline__ void hb_decide(const double phi_o[4], const double he
 template <typename T, bool W>
 __global__ __launch_bounds__(kBlock) void k_hb_phi(const ReplicaParams *__restrict__ P,
                                                    const ReplicaState *__restrict__ S,
-                                                   const int *__restrict__ blk_rep,
-                                                   const int *__restrict__ blk_first, int ieo,
+                                                   LaunchBlocks blk, int ieo,
                                                    int ctr_off, int flip,
                                                    MonSlot *__restrict__ mon) {
-  const int bid = xcd_block();
-  const int r = blk_rep[bid];
+  const int r = blk.rep[blockIdx.x], b = blk.local[blockIdx.x];
+  MonSlot *slot = mon + blk.first[r] + b;
   const ReplicaParams &p = P[r];
-  // FP64 one-replica launches sweep plane bands per XCD (measured: 128^3
-  // 29.0 -> 26.3 us, 192^3 74.4 -> 70.1 us; FP32 256^3 1 % slower)
-  int pb = bid - blk_first[r];
-  const int bpp = p.N * p.NH / kBlock;  // blocks per plane
-  if (sizeof(T) == 8 && (p.N * p.NH) % kBlock == 0 && (bpp & 7) == 0 &&
-      (int)gridDim.x == p.N * bpp)
-    pb = band_block(pb, bpp);
-  const uint32_t idx = (uint32_t)pb * kBlock + threadIdx.x;
+  const uint32_t idx = (uint32_t)b * kBlock + threadIdx.x;
   Tally mt;
   if (idx < (uint64_t)p.half) {
     const uint32_t N = p.N, NH = p.NH;
@@ -370,7 +426,7 @@ __global__ __launch_bounds__(kBlock) void k_hb_phi(const ReplicaParams *__restri
 #pragma unroll
     for (int l = 0; l < 4; l++) gplane<T, W>(p, cur, l, ieo).st(idx, phi_n[l]);
   }
-  block_monitor_add(mon + bid, mt);
+  block_monitor_add(slot, mt);
 }
 
 __device__ __forceinline__ int wrapz(int z, int N) { return z < 0 ? z + N : (z >= N ? z - N : z); }
@@ -386,16 +442,15 @@ __device__ __forceinline__ int wrapz(int z, int N) { return z < 0 ? z + N : (z >
 template <typename T, bool W, bool NTS>
 __global__ __launch_bounds__(kBlock) void k_hb_march(const ReplicaParams *__restrict__ P,
                                                      const ReplicaState *__restrict__ S,
-                                                     const int *__restrict__ blk_rep,
-                                                     const int *__restrict__ blk_first, int ieo,
+                                                     LaunchBlocks blk, int ieo,
                                                      int ctr_off, int flip,
                                                      MonSlot *__restrict__ mon) {
   constexpr int kGrid = kHbMarchGrid;
   // values held widened to FP64 (exact for FP32 fields): each is read by up
   // to four sites, so one conversion on the way in replaces four on the way out
   __shared__ double Q[2][4][kGrid];
-  const int bid = xcd_block();
-  const int r = blk_rep[bid];
+  const int r = blk.rep[blockIdx.x], tile = blk.local[blockIdx.x];
+  MonSlot *slot = mon + blk.first[r] + tile;
   const ReplicaParams &p = P[r];
   const ReplicaState &s = S[r];
   const int cur = s.cur_phi ^ (flip & 1);  // phi planes only
@@ -404,16 +459,7 @@ __global__ __launch_bounds__(kBlock) void k_hb_march(const ReplicaParams *__rest
   int TXH, TY, TZ;
   hb_tile(N, p.hb_cap, p.hb_tz, TXH, TY, TZ);
   const int ntx = (NH + TXH - 1) / TXH, nty = (N + TY - 1) / TY;
-  int b = bid - blk_first[r];
-  int bx, by, bz;
-  if ((int)gridDim.x == ntx * nty * ((N + TZ - 1) / TZ)) {
-    yband_tile(b, ntx, nty, bx, by, bz);  // one replica
-  } else {
-    bx = b % ntx;
-    b /= ntx;
-    by = b % nty;
-    bz = b / nty;
-  }
+  const int bx = tile % ntx, by = tile / ntx % nty, bz = tile / ntx / nty;
   const int xh0 = bx * TXH, y0 = by * TY, z0 = bz * TZ;
   const int tw = min(TXH, NH - xh0), th = min(TY, N - y0), tz = min(TZ, N - z0);
   const int GW = tw + 2;  // grid row width: half-columns xh0-1 .. xh0+tw
@@ -436,33 +482,24 @@ __global__ __launch_bounds__(kBlock) void k_hb_march(const ReplicaParams *__rest
   const double lambda = p.lambda, H = p.H, rdtg = p.rdtg;
   const uint64_t key = stream_key(p.base_key, s.sweep_ctr + ctr_off);
   Tally mt;
-  auto idx = [&](int xhh, int yy, int z) __attribute__((always_inline)) {
-    return ((uint32_t)z * N + yy) * NH + xhh;
-  };
-  // the eight plane bases, formed once (a store would otherwise force
-  // p.fields to be reloaded)
-  GPlane<T, W> gq[4], go[4];
+  const PhiPlanes<T, W> f(p, first_lane(cur));
+  const uint32_t i_own = (uint32_t)y * NH + xh, i_halo = (uint32_t)hgy * NH + hgxh;
+  auto ld4 = [&](uint32_t i, int zz, double v[4]) __attribute__((always_inline)) {
 #pragma unroll
-  for (int l = 0; l < 4; l++) {
-    gq[l] = gplane<T, W>(p, cur, l, q);
-    go[l] = gplane<T, W>(p, cur, l, ieo);
-  }
-  auto ld4 = [&](uint32_t i, double v[4]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int l = 0; l < 4; l++) v[l] = gq[l].ld(i);
+    for (int l = 0; l < 4; l++) v[l] = f.template ld<false>(l, q, zz, i);
   };
   // The loads of plane z+1 (the own half-column's q values at z+2, its own
   // update-parity value at z+1, the ring entry at z+1) are issued before
   // plane z's barrier, into the registers nq, nphi, nh as stored, so that
   // they are in flight during plane z's decisions.
-  auto raw4 = [&](uint32_t i, T v[4]) __attribute__((always_inline)) {
+  auto raw4 = [&](uint32_t i, int zz, T v[4]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int l = 0; l < 4; l++) v[l] = gq[l].raw(i);
+    for (int l = 0; l < 4; l++) v[l] = f.template ld<false>(l, q, zz, i);
   };
   // the update parity's own value: read by this thread only
-  auto own4 = [&](uint32_t i, T v[4]) __attribute__((always_inline)) {
+  auto own4 = [&](int zz, T v[4]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int l = 0; l < 4; l++) v[l] = go[l].template get_raw<NTS>(i);
+    for (int l = 0; l < 4; l++) v[l] = f.template ld<NTS>(l, ieo, zz, i_own);
   };
   // Plane z's new values are stored in iteration z+1, after the loads of
   // plane z+2 are issued and before the barrier: one in-order counter covers
@@ -470,9 +507,9 @@ __global__ __launch_bounds__(kBlock) void k_hb_march(const ReplicaParams *__rest
   // waits for these stores, which have had the decisions of plane z+1 to
   // complete (a store at the end of an iteration would be waited for at
   // once).  Only this thread reads its own sites.
-  auto store4 = [&](uint32_t i, const T v[4]) __attribute__((always_inline)) {
+  auto store4 = [&](int zz, const T v[4]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int l = 0; l < 4; l++) go[l].template put_raw<NTS>(i, v[l]);
+    for (int l = 0; l < 4; l++) f.template st<NTS>(l, ieo, zz, i_own, v[l]);
   };
   // FP32 fields: the loads run two planes ahead in two register sets (a
   // set holds half the bytes of an FP64 one, so one set in flight per wave
@@ -484,20 +521,19 @@ __global__ __launch_bounds__(kBlock) void k_hb_march(const ReplicaParams *__rest
   // ring entry at z, for the planes z = z0 + s, z0 + s + kDepth, ...
   T nq[kDepth][4], nphi[kDepth][4], nh[kDepth][4];
   T pend[4];         // plane z-1's new values, stored at the top of iteration z
-  uint32_t pend_i = 0;
   if (own) {
-    ld4(idx(xh, y, wrapz(z0 - 1, N)), qm);
-    ld4(idx(xh, y, z0), qc);
+    ld4(i_own, wrapz(z0 - 1, N), qm);
+    ld4(i_own, z0, qc);
   }
 #pragma unroll
   for (int sidx = 0; sidx < kDepth; sidx++) {
     if (sidx < tz) {  // plane z0 + sidx < z0 + tz <= N
       const int zs = z0 + sidx;
       if (own) {
-        raw4(idx(xh, y, zs + 1 == N ? 0 : zs + 1), nq[sidx]);
-        own4(idx(xh, y, zs), nphi[sidx]);
+        raw4(i_own, zs + 1 == N ? 0 : zs + 1, nq[sidx]);
+        own4(zs, nphi[sidx]);
       }
-      if (halo) raw4(idx(hgxh, hgy, zs), nh[sidx]);
+      if (halo) raw4(i_halo, zs, nh[sidx]);
     }
   }
   // plane z0 + j from register set sq / sphi / sh, which then takes the
@@ -522,12 +558,12 @@ __global__ __launch_bounds__(kBlock) void k_hb_march(const ReplicaParams *__rest
     if (j + kDepth < tz) {  // plane zn = z + kDepth < z0 + tz <= N
       const int zn = z + kDepth;
       if (own) {
-        raw4(idx(xh, y, zn + 1 == N ? 0 : zn + 1), sq);
-        own4(idx(xh, y, zn), sphi);
+        raw4(i_own, zn + 1 == N ? 0 : zn + 1, sq);
+        own4(zn, sphi);
       }
-      if (halo) raw4(idx(hgxh, hgy, zn), sh);
+      if (halo) raw4(i_halo, zn, sh);
     }
-    if (own && j > 0) store4(pend_i, pend);
+    if (own && j > 0) store4(z - 1, pend);
     __syncthreads();
     if (own) {
       const int o = (ieo + y + z) & 1;  // x = 2 xh + o
@@ -539,7 +575,6 @@ __global__ __launch_bounds__(kBlock) void k_hb_march(const ReplicaParams *__rest
                   (g[l][pos + GW] + g[l][pos - GW]) + (qp[l] + qm[l]);
       Xoro gg = xoro_seeded(site_key(key, ((uint64_t)z * N + y) * N + 2 * xh + o));
       hb_decide(phi_o, heff, Lambda2, lambda, H, rdtg, gg, phi_n, mt);
-      pend_i = idx(xh, y, z);
 #pragma unroll
       for (int l = 0; l < 4; l++) {
         pend[l] = (T)phi_n[l];
@@ -556,8 +591,8 @@ __global__ __launch_bounds__(kBlock) void k_hb_march(const ReplicaParams *__rest
       if (j + 1 < tz) plane(j + 1, nq[kDepth - 1], nphi[kDepth - 1], nh[kDepth - 1]);
     }
   }
-  if (own && tz > 0) store4(pend_i, pend);
-  block_monitor_add(mon + bid, mt);
+  if (own && tz > 0) store4(z0 + tz - 1, pend);
+  block_monitor_add(slot, mt);
 }
 
 
@@ -872,21 +907,19 @@ template <typename T, bool W, bool XW>
 __global__ __launch_bounds__(kBlock)
 __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 && XW ? 3 : 4))) void k_charge_march(const ReplicaParams *__restrict__ P,
                                                          const ReplicaState *__restrict__ S,
-                                                         const int *__restrict__ blk_rep,
-                                                         const int *__restrict__ blk_first,
+                                                         LaunchBlocks blk,
                                                          int ixyz, int ctr_off, int flip,
                                                          MonSlot *__restrict__ mon) {
-  const int bid = xcd_block();
-  const int r = blk_rep[bid];
+  const int r = blk.rep[blockIdx.x], tile = blk.local[blockIdx.x];
+  MonSlot *slot = mon + blk.first[r] + tile;
   const ReplicaParams &p = P[r];
   const ReplicaState &s = S[r];
   const int N = p.N, NH = p.NH;
   int TXH, TQ, C;
   charge_tile(N, p.chg_cap, p.chg_chunk, TXH, TQ, C);
   const int nbx = (NH + TXH - 1) / TXH, nbq = (N + TQ - 1) / TQ;
-  int b = bid - blk_first[r];
-  const int sx = b & 1;
-  b >>= 1;
+  const int sx = tile & 1;
+  int b = tile >> 1;
   const int bx = b % nbx;
   b /= nbx;
   const int bq = b % nbq, bc = b / nbq;
@@ -937,7 +970,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 && XW ? 3 : 4))) void k_charge
       charge_column<T, W, XW>(p, f, dir, e1, e2, 2 * xh + sx, q, c0, c1, k1, k2, mt);
     }
   }
-  block_monitor_add(mon + bid, mt, 1. / (2. * p.chi));
+  block_monitor_add(slot, mt, 1. / (2. * p.chi));
 }
 
 // ------------------------------------------------------------------------
@@ -962,13 +995,11 @@ __device__ __forceinline__ void load_site(const ReplicaParams &p, int cur, int x
 template <typename T, bool W, bool NTS>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 3 : 1)))
 void k_ideal_fused(const ReplicaParams *__restrict__ P, const ReplicaState *__restrict__ S,
-                   const int *__restrict__ blk_rep, const int *__restrict__ blk_first,
-                   int flip) {
+                   LaunchBlocks blk, int flip) {
   __shared__ double lds[4][ideal_lds(sizeof(T) == 4)];
   // rotated phi of plane z-1 at the thread's own sites: thread-private slots
   __shared__ double lprv[2][4][kBlock];
-  const int bid = xcd_block();
-  const int r = blk_rep[bid];
+  const int r = blk.rep[blockIdx.x], tile = blk.local[blockIdx.x];
   // a reference, not a copy: a private copy would be staged in scratch memory
   const ReplicaParams &p = P[r];
   const int cur = live(S[r]) ^ flip, nxt = cur ^ 3;
@@ -976,16 +1007,7 @@ void k_ideal_fused(const ReplicaParams *__restrict__ P, const ReplicaState *__re
   int TXH, TY, TZ;
   ideal_tile(N, p.tile_cap, p.tile_tz, TXH, TY, TZ);
   const int ntx = (NH + TXH - 1) / TXH, nty = (N + TY - 1) / TY;
-  int b = bid - blk_first[r];
-  int bx, by, bz;
-  if ((int)gridDim.x == ntx * nty * ((N + TZ - 1) / TZ)) {
-    yband_tile(b, ntx, nty, bx, by, bz);  // one replica
-  } else {
-    bx = b % ntx;
-    b /= ntx;
-    by = b % nty;
-    bz = b / nty;
-  }
+  const int bx = tile % ntx, by = tile / ntx % nty, bz = tile / ntx / nty;
   const int xh0 = bx * TXH, y0 = by * TY, z0 = bz * TZ;
   const int tw = min(TXH, NH - xh0), th = min(TY, N - y0), tz = min(TZ, N - z0);
   const int LW = 2 * tw + 2;  // LDS row width
@@ -1208,14 +1230,13 @@ void k_ideal_fused(const ReplicaParams *__restrict__ P, const ReplicaState *__re
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_energy(const ReplicaParams *__restrict__ P,
                                                    const ReplicaState *__restrict__ S,
-                                                   const int *__restrict__ blk_rep,
-                                                   const int *__restrict__ blk_first,
+                                                   LaunchBlocks blk,
                                                    int flip, EnergySlot *__restrict__ slots) {
-  const int bid = xcd_block();
-  const int r = blk_rep[bid];
+  const int bid = blockIdx.x;
+  const int r = blk.rep[bid];
   const ReplicaParams p = P[r];
   const int cur = live(S[r]) ^ flip;
-  int64_t idx = (int64_t)(bid - blk_first[r]) * kBlock + threadIdx.x;
+  int64_t idx = (int64_t)(bid - blk.first[r]) * kBlock + threadIdx.x;
   double g2 = 0., hE = 0., n2 = 0.;
   if (idx < 2 * p.half) {
     const int par = idx >= p.half;
@@ -1727,13 +1748,13 @@ static inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / 
 
 void launch_hb_phi(bool fp32, const Plan &plan, const ReplicaParams *P, ReplicaState *S,
                    int ieo, int ctr_off, int flip, MonSlot *mon, hipStream_t st) {
-  LGV_DISPATCH(k_hb_phi, plan.nblocks, st, P, S, plan.d_blk_rep, plan.d_blk_first, ieo,
+  LGV_DISPATCH(k_hb_phi, plan.nblocks, st, P, S, plan.blocks, ieo,
                ctr_off, flip, mon);
 }
 
 void launch_hb_march(bool fp32, const Plan &plan, const ReplicaParams *P, ReplicaState *S,
                      int ieo, int ctr_off, int flip, MonSlot *mon, hipStream_t st) {
-  LGV_DISPATCH_S(k_hb_march, plan.nblocks, st, P, S, plan.d_blk_rep, plan.d_blk_first, ieo,
+  LGV_DISPATCH_S(k_hb_march, plan.nblocks, st, P, S, plan.blocks, ieo,
                ctr_off, flip, mon);
 }
 
@@ -1741,10 +1762,9 @@ void launch_charge_march(bool fp32, const Plan &plan, const ReplicaParams *P, Re
                          int ixyz, int ctr_off, int flip, MonSlot *mon, hipStream_t st) {
   // the row-per-wavefront x path costs registers (3 waves per SIMD instead of
   // 4), so it is compiled in only for launches whose replicas all use it
-  const int *br = plan.d_blk_rep, *bf = plan.d_blk_first;
   const int g = plan.nblocks;
 #define LGV_CHARGE(TT, WW, XX)                                                         \
-  k_charge_march<TT, WW, XX><<<g, kBlock, 0, st>>>(P, S, br, bf, ixyz, ctr_off, flip, mon)
+  k_charge_march<TT, WW, XX><<<g, kBlock, 0, st>>>(P, S, plan.blocks, ixyz, ctr_off, flip, mon)
   if (plan.xwave) {
     if (fp32) { if (plan.far) LGV_CHARGE(float, true, true); else LGV_CHARGE(float, false, true); }
     else { if (plan.far) LGV_CHARGE(double, true, true); else LGV_CHARGE(double, false, true); }
@@ -1757,23 +1777,21 @@ void launch_charge_march(bool fp32, const Plan &plan, const ReplicaParams *P, Re
 
 void launch_ideal(bool fp32, const Plan &plan, const ReplicaParams *P, ReplicaState *S,
                   int flip, hipStream_t st) {
-  LGV_DISPATCH_S(k_ideal_fused, plan.nblocks, st, P, S, plan.d_blk_rep, plan.d_blk_first, flip);
+  LGV_DISPATCH_S(k_ideal_fused, plan.nblocks, st, P, S, plan.blocks, flip);
 }
 
 void launch_energy(bool fp32, const Plan &plan, const ReplicaParams *P,
                    const ReplicaState *S, int flip, EnergySlot *slots, hipStream_t st) {
   if (fp32)
-    k_energy<float><<<plan.nblocks, kBlock, 0, st>>>(P, S, plan.d_blk_rep, plan.d_blk_first,
-                                                     flip, slots);
+    k_energy<float><<<plan.nblocks, kBlock, 0, st>>>(P, S, plan.blocks, flip, slots);
   else
-    k_energy<double><<<plan.nblocks, kBlock, 0, st>>>(P, S, plan.d_blk_rep, plan.d_blk_first,
-                                                      flip, slots);
+    k_energy<double><<<plan.nblocks, kBlock, 0, st>>>(P, S, plan.blocks, flip, slots);
 }
 
 void launch_energy_finish(int nrep, const Plan &plan, const ReplicaParams *P,
                           ReplicaState *S, const EnergySlot *slots, int which,
                           int ctr_off, MonSlot *mon_ideal, hipStream_t st) {
-  k_energy_finish<<<nrep, 64, 0, st>>>(P, S, plan.d_blk_first, nrep, plan.nblocks, slots,
+  k_energy_finish<<<nrep, 64, 0, st>>>(P, S, plan.blocks.first, nrep, plan.nblocks, slots,
                                        which, ctr_off, mon_ideal);
 }
 

@@ -58,3 +58,49 @@ def test_default_tiles_of_a_mixed_batch_keep_results(L):
         np.testing.assert_array_equal(ctx.get_field(r), one.get_field(), err_msg=str(sizes[r]))
         one.close()
     ctx.close()
+
+
+# The phi march's own tiles against the per-site kernel: 34: one row of 17
+# half-columns in tiles of 15 rows; 66, 90: rows of 33 and 45, not a multiple
+# of eight blocks per plane; 140: two tiles of 35; 208: two of 64, the second
+# 40 wide, and (FP64) large enough for non-temporal stores
+@pytest.mark.parametrize("N,prec", [(34, 0), (66, 1), (90, 0), (140, 1), (208, 0)])
+def test_phi_kernels_agree_on_default_tiles(L, N, prec):
+    print(f"[gpu-test] phi kernels {N} {prec}", flush=True)
+    u = np.random.default_rng(N).normal(size=(N, N, N, 10)) * 0.5
+    out = []
+    for kernel in (L.PHI_SITE, L.PHI_MARCH):
+        ctx = L.Context(L.model_params(N, seed=5), precision=prec)
+        ctx.set_phi_kernel(kernel)
+        ctx.set_field(u)
+        ctx.run(0.04, 1)
+        out.append((ctx.get_field(), ctx.monitors()["phi"]))
+        ctx.close()
+    np.testing.assert_array_equal(out[0][0], out[1][0])
+    for k in ("down_counts", "up_counts", "up_yes", "up_no"):
+        assert out[0][1][k] == out[1][1][k], k
+
+
+def test_phi_march_of_a_mixed_batch_keeps_results(L):
+    """Replicas that go to one XCD as a whole and replicas that are cut into
+    bands in one launch."""
+    print("[gpu-test] phi march, batch", flush=True)
+    sizes = [66] + [12] * 30 + [34]
+    us = [np.random.default_rng(i).normal(size=(N, N, N, 10)) * 0.5 for i, N in enumerate(sizes)]
+    out = []
+    for kernel in (L.PHI_SITE, L.PHI_MARCH):
+        ctx = L.Context([L.model_params(N, seed=7 + i) for i, N in enumerate(sizes)])
+        ctx.set_phi_kernel(kernel)
+        for r, u in enumerate(us):
+            ctx.set_field(u, r)
+        ctx.run(0.04, 1)
+        out.append([ctx.get_field(r) for r in range(len(sizes))])
+        ctx.close()
+    for r, N in enumerate(sizes):
+        np.testing.assert_array_equal(out[0][r], out[1][r], err_msg=f"{r}: {N}")
+    for r in (0, 5, 31):
+        one = L.Context(L.model_params(sizes[r], seed=7 + r))
+        one.set_field(us[r])
+        one.run(0.04, 1)
+        np.testing.assert_array_equal(out[1][r], one.get_field(), err_msg=str(r))
+        one.close()
