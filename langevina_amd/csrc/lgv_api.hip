@@ -103,17 +103,24 @@ struct lgv_ctx {
   ReplicaParams *dP = nullptr;
   ReplicaState *dS = nullptr;
   std::vector<void *> fields;
-  Plan plan_half, plan_full, plan_ideal, plan_charge, plan_hb;
+  Plan plan_half, plan_full, plan_ideal, plan_charge, plan_hb, plan_brick;
   bool wide = false;    // some plane is >= 4 GiB: kernels use 64-bit offsets
   uint64_t buffer_bytes = 0;  // one buffer's fields, all replicas
   int nt_stores = -1;  // non-temporal stores: -1 by the rule, 0 / 1 forced
   bool phi_march = false;  // the phi half-sweep runs the z-march kernel
   bool phi_march_auto = false;  // the size rule's choice (LGV_PHI_AUTO)
-  MonSlot *mon_phi = nullptr, *mon_charge = nullptr, *mon_ideal = nullptr;
+  // the per-site kernel's sweeps come in pairs of two-parity launches
+  bool phi_bricks = false;
+  int brick_lds = 0;  // bytes of LDS of such a launch
+  MonSlot *mon_phi = nullptr, *mon_brick = nullptr, *mon_charge = nullptr, *mon_ideal = nullptr;
   // monitor counts folded out of the per-block slots when a retile
   // reallocated them: [replica][phi, charge]
   std::vector<std::array<lgv_monitor, 2>> mon_carry;
   EnergySlot *eslots = nullptr;
+  // Sweeps counted here and not yet in the replicas' sweep_ctr: a launch's
+  // counter offset starts from it, so that a lone phi sweep needs no launch to
+  // advance the state (six sweeps of 32^3: 70.8 -> 51.8 us).
+  uint64_t ctr = 0;
   double coef_hb = NAN, coef_charge = NAN, coef_ideal = NAN;
   double *d_aos = nullptr;
   int maxN = 0;
@@ -134,7 +141,11 @@ struct lgv_ctx {
   uint64_t timing_ctr = 0;
   std::vector<hipEvent_t> ev_pool;
   size_t ev_used = 0;
-  std::vector<std::pair<int, std::pair<hipEvent_t, hipEvent_t>>> ev_pairs;
+  struct TimedLaunch {
+    int cls, count;  // the launch counts as `count` of its class
+    hipEvent_t e0, e1;
+  };
+  std::vector<TimedLaunch> ev_pairs;
   double t_ms[LGV_NCLASS] = {0};
   long long t_launch[LGV_NCLASS] = {0};
 };
@@ -249,8 +260,8 @@ int build_plan(Plan &plan, const std::vector<PlanWork> &work, bool wide, bool or
   }
   plan.nblocks = (int)total;
   if (ordered) xcd_order(work, rep, local);
-  int rc = upload(&plan.blocks.rep, rep);
-  if (!rc) rc = upload(&plan.blocks.first, plan.first);
+  int rc = upload(&plan.blocks.first, plan.first);
+  if (!rc && work.size() > 1) rc = upload(&plan.blocks.rep, rep);
   if (!rc && ordered) rc = upload(&plan.blocks.local, local);
   return rc;
 }
@@ -420,6 +431,52 @@ int build_hb_plan(lgv_ctx *c) {
   return rc;
 }
 
+// Rows of even sites that k_hb_brick decides for a brick of BY x BZ rows.
+int brick_rows(int N, int by, int bz) {
+  const int y = std::min(by, N), z = std::min(bz, N);
+  return y * z + 2 * y + 2 * z;
+}
+
+// The bricks of the two-parity phi sweep: of the BY x BZ rows whose even sites
+// fit kBrickLds, those with the fewest decisions per CU, in wavefronts and
+// whole rounds of 256 blocks (64^3 FP64: 4 x 4 rows, 256 blocks, 24 wavefronts
+// against the 16 that have no facing rows).
+int build_brick_plan(lgv_ctx *c) {
+  const int esz = c->fp32 ? 4 : 8;
+  int best_y = 0, best_z = 0;
+  double best = 1e300;
+  for (int by = 1; by <= 16; by++)
+    for (int bz = 1; bz <= by; bz++) {
+      double blocks = 0., waves = 0.;
+      bool fits = true;
+      for (const ReplicaParams &p : c->hp) {
+        const int rows = brick_rows(p.N, by, bz);
+        fits = fits && rows * p.NH * 4 * esz <= kBrickLds;
+        const double n = (double)((p.N + by - 1) / by) * ((p.N + bz - 1) / bz);
+        blocks += n;
+        waves += n * ((rows * p.NH + 63) / 64 + (std::min(by, p.N) * std::min(bz, p.N) * p.NH + 63) / 64);
+      }
+      const double cost = waves / blocks * std::ceil(blocks / kCUs);
+      if (fits && cost < best) {
+        best = cost;
+        best_y = by;
+        best_z = bz;
+      }
+    }
+  if (!best_y) c->phi_bricks = false;  // rows longer than the LDS holds
+  if (!c->phi_bricks) return LGV_OK;
+  std::vector<PlanWork> work;
+  bool wide = c->wide;
+  for (ReplicaParams &p : c->hp) {
+    p.brick_y = best_y;
+    p.brick_z = best_z;
+    c->brick_lds = std::max(c->brick_lds, brick_rows(p.N, best_y, best_z) * p.NH * 4 * esz);
+    const int64_t plane = (p.N + best_y - 1) / best_y;
+    work.push_back({plane * ((p.N + best_z - 1) / best_z), (double)plane});
+  }
+  return build_plan(c->plan_brick, work, wide);
+}
+
 // Whether the x sub-sweeps of every replica run whole rows per wavefront
 // (charge_row_wave with two half-columns per lane or one): NH = 64 or 128 and
 // a tile of 64 half-columns x 4 lines.
@@ -527,7 +584,7 @@ struct Timed {
   lgv_ctx *c;
   int cls;
   hipEvent_t e1 = nullptr;
-  Timed(lgv_ctx *cc, int k) : c(cc), cls(k) {
+  Timed(lgv_ctx *cc, int k, int count = 1) : c(cc), cls(k) {
     if (!c->timing_now) return;
     if (c->ev_used + 2 > c->ev_pool.size()) {
       for (int i = 0; i < 64; i++) {
@@ -542,7 +599,7 @@ struct Timed {
       return;
     }
     e1 = c->ev_pool[c->ev_used++];
-    c->ev_pairs.push_back({cls, {e0, e1}});
+    c->ev_pairs.push_back({cls, count, e0, e1});
   }
   ~Timed() {
     if (!e1) return;
@@ -559,9 +616,9 @@ int drain_timing(lgv_ctx *c) {
   HIPCHECK(hipStreamSynchronize(c->stream));
   for (auto &pr : c->ev_pairs) {
     float ms = 0.f;
-    HIPCHECK(hipEventElapsedTime(&ms, pr.second.first, pr.second.second));
-    c->t_ms[pr.first] += ms;
-    c->t_launch[pr.first] += 1;
+    HIPCHECK(hipEventElapsedTime(&ms, pr.e0, pr.e1));
+    c->t_ms[pr.cls] += ms;
+    c->t_launch[pr.cls] += pr.count;
   }
   c->ev_pairs.clear();
   c->ev_used = 0;
@@ -616,6 +673,21 @@ int enqueue_hb(lgv_ctx *c, int off, int flip) {
   return 0;  // in place
 }
 
+// n sweeps of EulerLangevinHB::step: pairs of out-of-place two-parity launches
+// where the context has them (a pair leaves the live buffer where it was, as
+// the in-place sweeps do), the others in place.
+void enqueue_phi_sweeps(lgv_ctx *c, int n, int off, int flip) {
+  int i = 0;
+  if (c->phi_bricks && !use_march(c)) {
+    for (; i < n - n % 2; i++) {
+      Timed tm(c, LGV_CLASS_PHI, 2);  // two half-sweeps
+      launch_hb_brick(c->fp32, c->plan_brick, c->brick_lds, c->dP, c->dS, off + 2 * i,
+                      flip ^ (i & 1), c->mon_brick, c->stream);
+    }
+  }
+  for (; i < n; i++) enqueue_hb(c, off + 2 * i, flip);
+}
+
 // ModelGChargeHB::step: the shuffle (counter off, drawn by every charge
 // launch), then per direction both parities in one pass (counters
 // off+1+2*ixyz and off+2+2*ixyz, as the unfused order), each launch writing
@@ -629,8 +701,20 @@ int enqueue_charge(lgv_ctx *c, int off, int flip, hipStream_t st) {
   return 2;  // three flips of the charge buffers
 }
 
+// The sweeps counted on the host, for a launch sequence whose k_advance adds
+// them to the replicas' counters.
+int take_ctr(lgv_ctx *c) {
+  const int n = (int)c->ctr;
+  c->ctr = 0;
+  return n;
+}
+// Adds them by a launch of their own (before a graph, whose offsets start at 0).
+void flush_ctr(lgv_ctx *c) {
+  if (const int n = take_ctr(c)) launch_advance(c->nrep, c->dS, 0., 0, (uint64_t)n, 0, c->stream);
+}
+
 // PV2HBSplit::step (Stepper.cxx:542-580); returns the number of stream
-// counters consumed.  The charge sweep reads and writes only the charges
+// counters consumed, and those taken from the host's count.  The charge sweep reads and writes only the charges
 // and the phi sweeps only phi, so after the last ideal substep the charge
 // sweep runs on the second stream while the phi sweeps run on the first
 // (fork and join by events, which a graph capture records as well).  Every
@@ -640,7 +724,7 @@ int enqueue_charge(lgv_ctx *c, int off, int flip, hipStream_t st) {
 // GPU on their own), and so do timed steps (events on one stream).  flip
 // returns the step's net live-buffer flip.
 int enqueue_step(lgv_ctx *c, int &flip) {
-  int off = 0;
+  int off = take_ctr(c);
   flip = 0;
   bool charge_queued = false, join_event = false;
   c->timing_now = c->timing && c->timing_ctr++ % c->timing_every == 0;
@@ -657,10 +741,8 @@ int enqueue_step(lgv_ctx *c, int &flip) {
         charge_queued = true;
         join_event = hipEventRecord(c->ev_join, c->stream2) == hipSuccess;
       }
-      for (unsigned i0 = 0; i0 < c->s0; i0++) {
-        flip ^= enqueue_hb(c, off, flip);
-        off += 2;
-      }
+      enqueue_phi_sweeps(c, (int)c->s0, off, flip);
+      off += 2 * (int)c->s0;
     }
   }
   if (!c->nodiffuse) {
@@ -870,6 +952,9 @@ int lgv_create(const lgv_config *cfg, lgv_ctx **out) {
       return fail(LGV_ERR_ARG, "LGV_PHI_KERNEL=%s: expected site or march", pk);
     c->phi_march = k == "march";
   }
+  c->phi_bricks = buffer_bytes / (10 * esz) < kBrickSites;
+  // test hook: LGV_PHI_BRICKS=0/1 forces the two-parity launches off / on
+  if (const char *pb = getenv("LGV_PHI_BRICKS")) c->phi_bricks = atoi(pb) != 0;
   HIPCHECK(hipMalloc(&c->dS, c->nrep * sizeof(ReplicaState)));
   HIPCHECK(hipMemcpy(c->dS, hs.data(), c->nrep * sizeof(ReplicaState), hipMemcpyHostToDevice));
   int rc;
@@ -878,12 +963,17 @@ int lgv_create(const lgv_config *cfg, lgv_ctx **out) {
   if ((rc = build_ideal_plan(c.get())) != LGV_OK) return rc;
   if ((rc = build_charge_plan(c.get())) != LGV_OK) return rc;
   if ((rc = build_hb_plan(c.get())) != LGV_OK) return rc;
+  if ((rc = build_brick_plan(c.get())) != LGV_OK) return rc;
   // the parameters as the plans' tile rules left them
   HIPCHECK(hipMalloc(&c->dP, c->nrep * sizeof(ReplicaParams)));
   HIPCHECK(hipMemcpy(c->dP, c->hp.data(), c->nrep * sizeof(ReplicaParams),
                      hipMemcpyHostToDevice));
   HIPCHECK(hipMalloc(&c->mon_phi, hb_plan(c.get()).nblocks * sizeof(MonSlot)));
   HIPCHECK(hipMemset(c->mon_phi, 0, hb_plan(c.get()).nblocks * sizeof(MonSlot)));
+  if (c->phi_bricks) {
+    HIPCHECK(hipMalloc(&c->mon_brick, c->plan_brick.nblocks * sizeof(MonSlot)));
+    HIPCHECK(hipMemset(c->mon_brick, 0, c->plan_brick.nblocks * sizeof(MonSlot)));
+  }
   HIPCHECK(hipMalloc(&c->mon_charge, c->plan_charge.nblocks * sizeof(MonSlot)));
   HIPCHECK(hipMemset(c->mon_charge, 0, c->plan_charge.nblocks * sizeof(MonSlot)));
   HIPCHECK(hipMalloc(&c->mon_ideal, c->nrep * sizeof(MonSlot)));
@@ -919,10 +1009,11 @@ int lgv_destroy(lgv_ctx *c) {
   for (void *f : c->fields) note(hipFree(f));
   note(hipFree(c->dP));
   note(hipFree(c->dS));
-  for (Plan *pl : {&c->plan_half, &c->plan_full, &c->plan_ideal, &c->plan_charge, &c->plan_hb}) {
+  for (Plan *pl : {&c->plan_half, &c->plan_full, &c->plan_ideal, &c->plan_charge, &c->plan_hb,
+                   &c->plan_brick}) {
     for (int *q : {pl->blocks.rep, pl->blocks.local, pl->blocks.first}) note(hipFree(q));
   }
-  for (void *q : {(void *)c->mon_phi, (void *)c->mon_charge, (void *)c->mon_ideal,
+  for (void *q : {(void *)c->mon_phi, (void *)c->mon_brick, (void *)c->mon_charge, (void *)c->mon_ideal,
                   (void *)c->eslots, (void *)c->d_aos, (void *)c->d_part,
                   (void *)c->d_meas})
     note(hipFree(q));
@@ -1033,6 +1124,7 @@ static int realloc_monitors(lgv_ctx *c) {
   HIPCHECK(hipMemset(c->mon_phi, 0, hb_plan(c).nblocks * sizeof(MonSlot)));
   HIPCHECK(hipMalloc(&c->mon_charge, c->plan_charge.nblocks * sizeof(MonSlot)));
   HIPCHECK(hipMemset(c->mon_charge, 0, c->plan_charge.nblocks * sizeof(MonSlot)));
+  if (c->mon_brick) HIPCHECK(hipMemset(c->mon_brick, 0, c->plan_brick.nblocks * sizeof(MonSlot)));
   return LGV_OK;
 }
 
@@ -1063,6 +1155,7 @@ int lgv_run(lgv_ctx *c, double dt, int nsteps) {
     }
     return check_launch();
   }
+  flush_ctr(c);
   if (!c->graph_exec || c->graph_dt != dt) {
     if ((rc = drop_graphs(c))) return rc;
     // graph_steps steps in one graph, and (when that is more than one) one
@@ -1101,8 +1194,8 @@ int lgv_ideal_step(lgv_ctx *c, double dt) {
   int rc = ensure_coeffs(c, c->coef_hb, c->coef_charge, dt);
   if (rc) return rc;
   c->timing_now = c->timing;  // single sweeps are always timed
-  const int flip = enqueue_ideal(c, 0, 0);
-  launch_advance(c->nrep, c->dS, 0., 0, 1, flip, c->stream);
+  const int off = take_ctr(c), flip = enqueue_ideal(c, off, 0);
+  launch_advance(c->nrep, c->dS, 0., 0, (uint64_t)off + 1, flip, c->stream);
   return check_launch();
 }
 
@@ -1112,8 +1205,9 @@ int lgv_hb_phi_step(lgv_ctx *c, double dt) {
   int rc = ensure_coeffs(c, dt, c->coef_charge, c->coef_ideal);
   if (rc) return rc;
   c->timing_now = c->timing;  // single sweeps are always timed
-  const int flip = enqueue_hb(c, 0, 0);
-  launch_advance(c->nrep, c->dS, 0., 0, 2, flip, c->stream);
+  if (c->ctr >> 20) flush_ctr(c);
+  enqueue_hb(c, (int)c->ctr, 0);  // in place: the live buffers stay
+  c->ctr += 2;
   return check_launch();
 }
 
@@ -1123,8 +1217,8 @@ int lgv_charge_step(lgv_ctx *c, double dt) {
   int rc = ensure_coeffs(c, c->coef_hb, dt, c->coef_ideal);
   if (rc) return rc;
   c->timing_now = c->timing;  // single sweeps are always timed
-  const int flip = enqueue_charge(c, 0, 0, c->stream);
-  launch_advance(c->nrep, c->dS, 0., 0, 7, flip, c->stream);
+  const int off = take_ctr(c), flip = enqueue_charge(c, off, 0, c->stream);
+  launch_advance(c->nrep, c->dS, 0., 0, (uint64_t)off + 7, flip, c->stream);
   return check_launch();
 }
 
@@ -1167,15 +1261,18 @@ int lgv_monitor_get(lgv_ctx *c, int r, lgv_monitor out[3]) {
   if (rc) return rc;
   HIPCHECK(hipSetDevice(c->device));
   HIPCHECK(hipStreamSynchronize(c->stream));
-  MonSlot *src[2] = {c->mon_phi, c->mon_charge};
-  const Plan *plan[2] = {&hb_plan(c), &c->plan_charge};
-  for (int k = 0; k < 2; k++) {
+  // phi half-sweeps, charge sweeps, two-parity phi sweeps
+  MonSlot *src[3] = {c->mon_phi, c->mon_charge, c->mon_brick};
+  const Plan *plan[3] = {&hb_plan(c), &c->plan_charge, &c->plan_brick};
+  for (int k = 0; k < 2; k++) out[k] = c->mon_carry[r][k];
+  for (int k = 0; k < 3; k++) {
+    if (!src[k]) continue;
     const int b0 = plan[k]->first[r];
     const int b1 = r + 1 < c->nrep ? plan[k]->first[r + 1] : plan[k]->nblocks;
     std::vector<MonSlot> slots(b1 - b0);
     HIPCHECK(hipMemcpy(slots.data(), src[k] + b0, slots.size() * sizeof(MonSlot),
                        hipMemcpyDeviceToHost));
-    lgv_monitor m = c->mon_carry[r][k];
+    lgv_monitor &m = out[k % 2];
     for (const MonSlot &s : slots) {
       m.down_counts += s.down_counts;
       m.up_counts += s.up_counts;
@@ -1184,7 +1281,6 @@ int lgv_monitor_get(lgv_ctx *c, int r, lgv_monitor out[3]) {
       m.down_dS += s.down_dS;
       m.up_dS += s.up_dS;
     }
-    out[k] = m;
   }
   MonSlot mi;
   HIPCHECK(hipMemcpy(&mi, c->mon_ideal + r, sizeof mi, hipMemcpyDeviceToHost));
@@ -1215,7 +1311,7 @@ int lgv_rng_get_state(lgv_ctx *c, int r, lgv_rng_state *st) {
   st->s1 = c->noise[r].g.s1;
   st->saved_normal = c->noise[r].saved;
   st->has_saved_normal = c->noise[r].has_saved;
-  st->sweep_ctr = s.sweep_ctr;
+  st->sweep_ctr = s.sweep_ctr + c->ctr;
   return LGV_OK;
 }
 
@@ -1230,7 +1326,7 @@ int lgv_rng_set_state(lgv_ctx *c, int r, const lgv_rng_state *st) {
   c->noise[r].has_saved = st->has_saved_normal;
   ReplicaState s;
   HIPCHECK(hipMemcpy(&s, c->dS + r, sizeof s, hipMemcpyDeviceToHost));
-  s.sweep_ctr = st->sweep_ctr;
+  s.sweep_ctr = st->sweep_ctr - c->ctr;
   HIPCHECK(hipMemcpy(c->dS + r, &s, sizeof s, hipMemcpyHostToDevice));
   return LGV_OK;
 }
@@ -1409,6 +1505,7 @@ int lgv_monitor_reset(lgv_ctx *c) {
   HIPCHECK(hipStreamSynchronize(c->stream));
   HIPCHECK(hipMemset(c->mon_phi, 0, hb_plan(c).nblocks * sizeof(MonSlot)));
   HIPCHECK(hipMemset(c->mon_charge, 0, c->plan_charge.nblocks * sizeof(MonSlot)));
+  if (c->mon_brick) HIPCHECK(hipMemset(c->mon_brick, 0, c->plan_brick.nblocks * sizeof(MonSlot)));
   HIPCHECK(hipMemset(c->mon_ideal, 0, c->nrep * sizeof(MonSlot)));
   HIPCHECK(hipDeviceSynchronize());
   for (auto &cr : c->mon_carry) cr = {lgv_monitor{}, lgv_monitor{}};

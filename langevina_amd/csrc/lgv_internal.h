@@ -9,7 +9,8 @@
 
 namespace lgv {
 
-constexpr int kBlock = 256;  // threads per block of every sweep kernel
+constexpr int kBlock = 256;  // threads per block of every sweep kernel but k_hb_brick
+constexpr int kBrickBlock = 1024;
 
 // Read-only (for the kernels) description of one replica.  The step
 // coefficients (rdtg, rms, dt_ideal, tau) are computed on the host with the
@@ -29,8 +30,9 @@ struct ReplicaParams {
   double tau_ideal;   // dt_ideal / 2.0
   uint64_t base_key;
   int tile_cap, tile_tz;   // ideal-kernel tile (see ideal_tile)
-  int hb_cap, hb_tz;       // phi-march tile (see hb_tile; 0 = default)
-  int chg_cap, chg_chunk;  // charge-march tile (see charge_tile; 0 = default)
+  int hb_cap, hb_tz;       // phi-march tile (see hb_tile)
+  int chg_cap, chg_chunk;  // charge-march tile (see charge_tile)
+  int brick_y, brick_z;    // rows of a brick of the two-parity phi sweep
 };
 
 // Device-written state of one replica (clock, counters, per-step data).
@@ -103,7 +105,8 @@ struct EnergySlot {
 
 // The blocks of a launch over several replicas, on the device: workgroup b is
 // block local[b] of replica rep[b] (local == nullptr: block b - first[rep[b]]),
-// and a replica's monitor slots start at first[replica].
+// and a replica's monitor slots start at first[replica].  rep == nullptr: all
+// of replica 0.
 struct LaunchBlocks {
   int *rep = nullptr, *local = nullptr, *first = nullptr;
 };
@@ -143,6 +146,16 @@ constexpr uint64_t kCacheBytes = 256ull << 20;
 // 4371; FP32 128^3 410 -> 411, 180^3 1219 -> 1229, 192^3 1328 -> 1304, 224^3
 // 2253 -> 2214, 256^3 2949 -> 2708.
 constexpr uint64_t kMarchSites = 7000000;
+
+// Below this many sites (all replicas) the per-site phi sweeps of a step run as
+// two-parity launches (k_hb_brick), in bricks that fit kBrickLds bytes of LDS
+// (two blocks of a CU).  Whole steps, half-sweeps -> two-parity launches: FP64
+// 16^3 100 -> 88 us, 32^3 106 -> 93, 64^3 151 -> 144, 80^3 231 -> 226, 84^3 248
+// -> 275, 5 x 48^3 230 -> 229; FP32 64^3 138 -> 128, 80^3 193 -> 189, 84^3 207
+// -> 209, 16 x 32^3 174 -> 165, 32 x 32^3 251 -> 246, 64 x 32^3 422 -> 457:
+// above, the facing rows' extra decisions cost more than the launches saved.
+constexpr uint64_t kBrickSites = 560000;
+constexpr int kBrickLds = 64 << 10;
 
 // A context of one lattice whose fields (one buffer) exceed this keeps the
 // charge sweep after the phi sweeps rather than beside them.
@@ -203,6 +216,8 @@ inline MeasureShape measure_shape(int N) {
 // step's net flip.
 void launch_hb_phi(bool fp32, const Plan &plan, const ReplicaParams *P, ReplicaState *S,
                    int ieo, int ctr_off, int flip, MonSlot *mon, hipStream_t st);
+void launch_hb_brick(bool fp32, const Plan &plan, int lds, const ReplicaParams *P,
+                     ReplicaState *S, int ctr_off, int flip, MonSlot *mon, hipStream_t st);
 void launch_hb_march(bool fp32, const Plan &plan, const ReplicaParams *P, ReplicaState *S,
                      int ieo, int ctr_off, int flip, MonSlot *mon, hipStream_t st);
 void launch_charge_march(bool fp32, const Plan &plan, const ReplicaParams *P, ReplicaState *S,

@@ -240,6 +240,17 @@ struct PhiPlanes<T, false> {
   }
 };
 
+// Replica r and block b of it that this workgroup is; returns the block's
+// number in the launch (its monitor slot).  A launch of one replica reads
+// nothing before the replica's parameters: a chain of loads at the start of a
+// launch costs about 0.7 us a link.
+__device__ __forceinline__ int block_of(const LaunchBlocks &blk, int &r, int &b) {
+  r = blk.rep ? blk.rep[blockIdx.x] : 0;
+  const int first = blk.rep ? blk.first[r] : 0;
+  b = blk.local ? blk.local[blockIdx.x] : (int)blockIdx.x - first;
+  return first + b;
+}
+
 __device__ __forceinline__ int wrapp(int a, int N) { return a == N ? 0 : a; }
 __device__ __forceinline__ int wrapm(int a, int N) { return a < 0 ? N - 1 : a; }
 
@@ -282,9 +293,10 @@ __device__ __forceinline__ void tally(Tally &m, double dS, uint64_t down, uint64
 // Deterministic block reduction of the tallies; thread 0 adds the block
 // total into the block's own slot (stream order makes this race-free).  The
 // sums of dS are scaled by unit.
+template <int B = kBlock>
 __device__ void block_monitor_add(MonSlot *slot, const Tally &m, double unit = 1.) {
-  __shared__ uint32_t sc[3][kBlock / 64];
-  __shared__ double sd[2][kBlock / 64];
+  __shared__ uint32_t sc[3][B / 64];
+  __shared__ double sd[2][B / 64];
   double dSd = m.dSd, dSu = m.dSu;
   uint32_t c[3] = {m.all, m.down, m.yes};
   for (int o = 32; o > 0; o >>= 1) {
@@ -302,7 +314,7 @@ __device__ void block_monitor_add(MonSlot *slot, const Tally &m, double unit = 1
   if (threadIdx.x == 0) {
     long long n[3] = {0, 0, 0};
     double d = 0, e = 0;
-    for (int i = 0; i < kBlock / 64; i++) {
+    for (int i = 0; i < B / 64; i++) {
       for (int k = 0; k < 3; k++) n[k] += sc[k][i];
       d += sd[0][i]; e += sd[1][i];
     }
@@ -353,10 +365,11 @@ __device__ __forceinline__ uint64_t accept_draw(uint64_t u, float e, uint64_t su
 // The Metropolis decision of one phi site (Stepper.cxx:330-370) in the
 // reference's operand order: heff[l] is the neighbour sum of component l,
 // ((x+1 + x-1) + (y+1 + y-1)) + (z+1 + z-1).  Returns the new value (the
-// old one on reject) and adds the decision to the monitor.
+// old one on reject) and adds the decision to the monitor where count.
 __device__ __forceinline__ void hb_decide(const double phi_o[4], const double heff[4],
                                           double Lambda2, double lambda, double H, double rdtg,
-                                          Xoro &g, double phi_new[4], Tally &m) {
+                                          Xoro &g, double phi_new[4], Tally &m,
+                                          bool count = true) {
   double hphi_o = 0., hphi_n = 0., s_o = 0., s_n = 0.;
   double phi_n[4];
 #pragma unroll
@@ -376,8 +389,8 @@ __device__ __forceinline__ void hb_decide(const double phi_o[4], const double he
   const uint64_t accept =
       accept_draw(xoro_next(g), __builtin_amdgcn_exp2f((float)dS * -kLog2e), down,
                   [&] { return -dS; });
-  tally_all(m, 1, true);
-  tally(m, dS, down, accept & ~down, ~0ull);
+  tally_all(m, 1, count);
+  tally(m, dS, down, accept & ~down, lanes(count));
 #pragma unroll
   for (int l = 0; l < 4; l++) phi_new[l] = in_lanes(accept) ? phi_n[l] : phi_o[l];
 }
@@ -390,8 +403,8 @@ __global__ __launch_bounds__(kBlock) void k_hb_phi(const ReplicaParams *__restri
                                                    LaunchBlocks blk, int ieo,
                                                    int ctr_off, int flip,
                                                    MonSlot *__restrict__ mon) {
-  const int r = blk.rep[blockIdx.x], b = blk.local[blockIdx.x];
-  MonSlot *slot = mon + blk.first[r] + b;
+  int r, b;
+  MonSlot *slot = mon + block_of(blk, r, b);
   const ReplicaParams &p = P[r];
   const uint32_t idx = (uint32_t)b * kBlock + threadIdx.x;
   Tally mt;
@@ -431,6 +444,134 @@ __global__ __launch_bounds__(kBlock) void k_hb_phi(const ReplicaParams *__restri
 
 __device__ __forceinline__ int wrapz(int z, int N) { return z < 0 ? z + N : (z >= N ? z - N : z); }
 
+// Both parities of EulerLangevinHB::step (Stepper.cxx:309-386) in one launch,
+// out of place: a block updates a brick of whole x rows, BY in y and BZ in z.
+// It first decides the even sites of the brick and of the rows that face it
+// (the neighbours of its odd sites; each decision has its own random stream,
+// so the blocks that share a row make the same one), keeps them in LDS, and
+// then decides its odd sites from there.  Small lattices spend most of a
+// half-sweep on the launch and on one round of loads, so half the launches
+// count more than deciding the facing rows again (a half-sweep of 32^3 6.6 ->
+// 4.6 us, of 64^3 8.6 -> 7.1, half of a launch; 100^3 15.9 -> 16.7: kBrickSites).
+// The first round of odd values is loaded before the even sites' decisions.
+template <typename T, bool W>
+__global__ __launch_bounds__(kBrickBlock) void k_hb_brick(const ReplicaParams *__restrict__ P,
+                                                          const ReplicaState *__restrict__ S,
+                                                          LaunchBlocks blk, int ctr_off, int flip,
+                                                          MonSlot *__restrict__ mon) {
+  extern __shared__ double brick_lds[];
+  T *even = reinterpret_cast<T *>(brick_lds);  // [4][rows][NH]
+  int r, b;
+  MonSlot *slot = mon + block_of(blk, r, b);
+  const ReplicaParams &p = P[r];
+  const ReplicaState &s = S[r];
+  const int cur = s.cur_phi ^ (flip & 1), nxt = cur ^ 1;  // phi planes only
+  const uint32_t N = p.N, NH = p.NH;
+  const int nby = (N + p.brick_y - 1) / p.brick_y;
+  const int y0 = b % nby * p.brick_y, z0 = b / nby * p.brick_z;
+  const int h = min(p.brick_y, (int)N - y0), d = min(p.brick_z, (int)N - z0);
+  // rows: the brick's, then the facing ones at y0 - 1, y0 + h, z0 - 1, z0 + d
+  const int ni = h * d, fy0 = ni, fy1 = ni + d, fz0 = ni + 2 * d, fz1 = fz0 + h;
+  const int rows = fz1 + h;
+  const int comp = rows * (int)NH;
+  const double mass = p.mass0 + p.dmassdt * s.t;
+  const double Lambda2 = 0.5 * (2. * 3. + mass);
+  const double lambda = p.lambda, H = p.H, rdtg = p.rdtg;
+  const uint64_t key_e = stream_key(p.base_key, s.sweep_ctr + ctr_off);
+  const uint64_t key_o = stream_key(p.base_key, s.sweep_ctr + ctr_off + 1);
+  // i / NH for i < 2^16 as a multiplication (exact while i NH < 2^32)
+  const uint32_t inv = 0xFFFFFFFFu / NH + 1;
+  const int wave0 = first_lane((int)(threadIdx.x & ~63u)), lane = threadIdx.x & 63;
+  Tally mt;
+  // the odd site of round i0 and its value, loaded a round ahead (before the
+  // even sites for the first one)
+  const int odd = ni * (int)NH;
+  T odd_o[4];
+  auto odd_site = [&](int i0, uint32_t &rid, uint32_t &xh, int &dy, int &dz)
+      __attribute__((always_inline)) {
+    const uint32_t i = i0 + lane < odd ? i0 + lane : odd - 1;
+    rid = __umulhi(i, inv);
+    xh = i - rid * NH;
+    dz = (int)rid / h;
+    dy = (int)rid - dz * h;
+    return ((z0 + dz) * N + y0 + dy) * NH + xh;
+  };
+  auto odd_load = [&](int i0) __attribute__((always_inline)) {
+    uint32_t rid, xh;
+    int dy, dz;
+    const uint32_t idx = odd_site(i0, rid, xh, dy, dz);
+#pragma unroll
+    for (int l = 0; l < 4; l++) odd_o[l] = gplane<T, W>(p, cur, l, 1).raw(idx);
+  };
+  if (wave0 < odd) odd_load(wave0);
+  // Every lane of a wavefront takes part in each of its rounds (the tallies
+  // are the wavefront's): lanes past the end repeat the last site.
+  for (int i0 = wave0; i0 < comp; i0 += kBrickBlock) {
+    const bool in = i0 + lane < comp;
+    const uint32_t i = in ? i0 + lane : comp - 1;
+    const uint32_t rid = __umulhi(i, inv), xh = i - rid * NH;
+    int dy, dz;
+    if ((int)rid < ni) { dz = (int)rid / h; dy = (int)rid - dz * h; }
+    else if ((int)rid < fz0) { const bool up = (int)rid >= fy1; dz = (int)rid - (up ? fy1 : fy0); dy = up ? h : -1; }
+    else { const bool up = (int)rid >= fz1; dy = (int)rid - (up ? fz1 : fz0); dz = up ? d : -1; }
+    const uint32_t y = wrapz(y0 + dy, N), z = wrapz(z0 + dz, N);
+    const uint32_t x = site_x(xh, y, z, 0);
+    const uint32_t rowi = z * N + y, row = rowi * NH;
+    const uint32_t xp = x + 1 == N ? 0 : x + 1, xm = x == 0 ? N - 1 : x - 1;
+    const uint32_t yp = y + 1 == N ? 0 : y + 1, ym = y == 0 ? N - 1 : y - 1;
+    const uint32_t zp = z + 1 == N ? 0 : z + 1, zm = z == 0 ? N - 1 : z - 1;
+    const uint32_t nb[6] = {row + (xp >> 1), row + (xm >> 1), (z * N + yp) * NH + xh,
+                            (z * N + ym) * NH + xh, (zp * N + y) * NH + xh,
+                            (zm * N + y) * NH + xh};
+    double phi_o[4], heff[4], phi_n[4];
+#pragma unroll
+    for (int l = 0; l < 4; l++) {
+      const GPlane<T, W> f = gplane<T, W>(p, cur, l, 1);
+      heff[l] = (f.ld(nb[0]) + f.ld(nb[1])) + (f.ld(nb[2]) + f.ld(nb[3])) +
+                (f.ld(nb[4]) + f.ld(nb[5]));
+      phi_o[l] = gplane<T, W>(p, cur, l, 0).ld(row + xh);
+    }
+    const bool mine = in && (int)rid < ni;
+    Xoro g = xoro_seeded(site_key(key_e, (uint64_t)rowi * N + x));
+    hb_decide(phi_o, heff, Lambda2, lambda, H, rdtg, g, phi_n, mt, mine);
+#pragma unroll
+    for (int l = 0; l < 4; l++) {
+      even[l * comp + i] = (T)phi_n[l];
+      if (mine) gplane<T, W>(p, nxt, l, 0).st(row + xh, phi_n[l]);
+    }
+  }
+  __syncthreads();
+  for (int i0 = wave0; i0 < odd; i0 += kBrickBlock) {
+    const bool in = i0 + lane < odd;
+    uint32_t rid, xh;
+    int dy, dz;
+    const uint32_t idx = odd_site(i0, rid, xh, dy, dz);
+    const uint32_t y = y0 + dy, z = z0 + dz;
+    const uint32_t x = site_x(xh, y, z, 1);
+    const uint32_t xp = x + 1 == N ? 0 : x + 1, xm = x == 0 ? N - 1 : x - 1;
+    const uint32_t ryp = dy + 1 < h ? rid + 1 : fy1 + dz, rym = dy > 0 ? rid - 1 : fy0 + dz;
+    const uint32_t rzp = dz + 1 < d ? rid + h : fz1 + dy, rzm = dz > 0 ? rid - h : fz0 + dy;
+    double phi_o[4], heff[4], phi_n[4];
+#pragma unroll
+    for (int l = 0; l < 4; l++) phi_o[l] = odd_o[l];
+    if (i0 + kBrickBlock < odd) odd_load(i0 + kBrickBlock);
+#pragma unroll
+    for (int l = 0; l < 4; l++) {
+      const T *f = even + l * comp;
+      heff[l] = ((double)f[rid * NH + (xp >> 1)] + (double)f[rid * NH + (xm >> 1)]) +
+                ((double)f[ryp * NH + xh] + (double)f[rym * NH + xh]) +
+                ((double)f[rzp * NH + xh] + (double)f[rzm * NH + xh]);
+    }
+    Xoro g = xoro_seeded(site_key(key_o, ((uint64_t)z * N + y) * N + x));
+    hb_decide(phi_o, heff, Lambda2, lambda, H, rdtg, g, phi_n, mt, in);
+    if (in) {
+#pragma unroll
+      for (int l = 0; l < 4; l++) gplane<T, W>(p, nxt, l, 1).st(idx, phi_n[l]);
+    }
+  }
+  block_monitor_add<kBrickBlock>(slot, mt);
+}
+
 // One parity of EulerLangevinHB::step (Stepper.cxx:309-386), in place, by
 // marching z through a TXH x TY tile of half-columns (the tile of hb_tile).
 // The update parity ieo reads only the other parity q, which no thread of
@@ -449,8 +590,8 @@ __global__ __launch_bounds__(kBlock) void k_hb_march(const ReplicaParams *__rest
   // values held widened to FP64 (exact for FP32 fields): each is read by up
   // to four sites, so one conversion on the way in replaces four on the way out
   __shared__ double Q[2][4][kGrid];
-  const int r = blk.rep[blockIdx.x], tile = blk.local[blockIdx.x];
-  MonSlot *slot = mon + blk.first[r] + tile;
+  int r, tile;
+  MonSlot *slot = mon + block_of(blk, r, tile);
   const ReplicaParams &p = P[r];
   const ReplicaState &s = S[r];
   const int cur = s.cur_phi ^ (flip & 1);  // phi planes only
@@ -910,8 +1051,8 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 && XW ? 3 : 4))) void k_charge
                                                          LaunchBlocks blk,
                                                          int ixyz, int ctr_off, int flip,
                                                          MonSlot *__restrict__ mon) {
-  const int r = blk.rep[blockIdx.x], tile = blk.local[blockIdx.x];
-  MonSlot *slot = mon + blk.first[r] + tile;
+  int r, tile;
+  MonSlot *slot = mon + block_of(blk, r, tile);
   const ReplicaParams &p = P[r];
   const ReplicaState &s = S[r];
   const int N = p.N, NH = p.NH;
@@ -999,7 +1140,8 @@ void k_ideal_fused(const ReplicaParams *__restrict__ P, const ReplicaState *__re
   __shared__ double lds[4][ideal_lds(sizeof(T) == 4)];
   // rotated phi of plane z-1 at the thread's own sites: thread-private slots
   __shared__ double lprv[2][4][kBlock];
-  const int r = blk.rep[blockIdx.x], tile = blk.local[blockIdx.x];
+  int r, tile;
+  block_of(blk, r, tile);
   // a reference, not a copy: a private copy would be staged in scratch memory
   const ReplicaParams &p = P[r];
   const int cur = live(S[r]) ^ flip, nxt = cur ^ 3;
@@ -1233,10 +1375,11 @@ __global__ __launch_bounds__(kBlock) void k_energy(const ReplicaParams *__restri
                                                    LaunchBlocks blk,
                                                    int flip, EnergySlot *__restrict__ slots) {
   const int bid = blockIdx.x;
-  const int r = blk.rep[bid];
+  int r, b;
+  block_of(blk, r, b);
   const ReplicaParams p = P[r];
   const int cur = live(S[r]) ^ flip;
-  int64_t idx = (int64_t)(bid - blk.first[r]) * kBlock + threadIdx.x;
+  int64_t idx = (int64_t)b * kBlock + threadIdx.x;
   double g2 = 0., hE = 0., n2 = 0.;
   if (idx < 2 * p.half) {
     const int par = idx >= p.half;
@@ -1750,6 +1893,15 @@ void launch_hb_phi(bool fp32, const Plan &plan, const ReplicaParams *P, ReplicaS
                    int ieo, int ctr_off, int flip, MonSlot *mon, hipStream_t st) {
   LGV_DISPATCH(k_hb_phi, plan.nblocks, st, P, S, plan.blocks, ieo,
                ctr_off, flip, mon);
+}
+
+void launch_hb_brick(bool fp32, const Plan &plan, int lds, const ReplicaParams *P,
+                     ReplicaState *S, int ctr_off, int flip, MonSlot *mon, hipStream_t st) {
+#define LGV_BRICK(TT, WW) \
+  k_hb_brick<TT, WW><<<plan.nblocks, kBrickBlock, lds, st>>>(P, S, plan.blocks, ctr_off, flip, mon)
+  if (fp32) { if (plan.wide) LGV_BRICK(float, true); else LGV_BRICK(float, false); }
+  else { if (plan.wide) LGV_BRICK(double, true); else LGV_BRICK(double, false); }
+#undef LGV_BRICK
 }
 
 void launch_hb_march(bool fp32, const Plan &plan, const ReplicaParams *P, ReplicaState *S,

@@ -104,3 +104,89 @@ def test_phi_march_of_a_mixed_batch_keeps_results(L):
         one.run(0.04, 1)
         np.testing.assert_array_equal(out[1][r], one.get_field(), err_msg=str(r))
         one.close()
+
+
+# Two-parity phi launches against half-sweeps.  6: the brick is the lattice, so
+# its facing rows are its own; 22, 34, 50: short last bricks and rows that leave
+# lanes of the last wavefront without a site; 64: one brick per CU
+@pytest.mark.parametrize("N,prec", [(6, 0), (6, 1), (22, 0), (34, 1), (50, 0), (64, 0), (64, 1)])
+@pytest.mark.parametrize("scounts", [(2, 3), (3, 1)])  # 3: a pair and one in place
+def test_two_parity_launches_keep_results(L, monkeypatch, N, prec, scounts):
+    print(f"[gpu-test] bricks {N} {prec} {scounts}", flush=True)
+    u = np.random.default_rng(N).normal(size=(N, N, N, 10)) * 0.5
+    out = []
+    for bricks in ("0", "1"):
+        monkeypatch.setenv("LGV_PHI_BRICKS", bricks)
+        ctx = L.Context(L.model_params(N, seed=5), precision=prec, scounts=scounts)
+        ctx.set_field(u)
+        ctx.run(0.04, 2)
+        ctx.set_phi_kernel(L.PHI_SITE)  # folds the counts, keeps the kernel
+        ctx.hb_phi_step(0.01)
+        ctx.run(0.04, 1)
+        out.append((ctx.get_field(), ctx.monitors(), ctx.rng_state().sweep_ctr))
+        ctx.close()
+    np.testing.assert_array_equal(out[0][0], out[1][0])
+    assert out[0][2] == out[1][2]
+    for k in ("down_counts", "up_counts", "up_yes", "up_no"):
+        assert out[0][1]["phi"][k] == out[1][1]["phi"][k], k
+
+
+def test_two_parity_launches_of_a_batch_keep_results(L, monkeypatch):
+    print("[gpu-test] bricks, batch", flush=True)
+    sizes = [34, 8, 8, 8, 22]
+    out = []
+    for bricks in ("0", "1"):
+        monkeypatch.setenv("LGV_PHI_BRICKS", bricks)
+        ctx = L.Context([L.model_params(N, seed=7 + i) for i, N in enumerate(sizes)])
+        for r, N in enumerate(sizes):
+            ctx.set_field(np.random.default_rng(r).normal(size=(N, N, N, 10)) * 0.5, r)
+        ctx.run(0.04, 2)
+        out.append([(ctx.get_field(r), ctx.monitors(r)["phi"]["up_yes"]) for r in range(5)])
+        ctx.close()
+    for r in range(5):
+        np.testing.assert_array_equal(out[0][r][0], out[1][r][0], err_msg=str(r))
+        assert out[0][r][1] == out[1][r][1]
+
+
+def test_sweep_counters_of_mixed_calls(L):
+    """Each call takes its streams from the counter that the calls before it
+    left, whether the host or the replicas hold it: the same call alone, on a
+    new context with that counter set, gives the same field."""
+    print("[gpu-test] sweep counters", flush=True)
+    N, dt = 12, 0.03
+    calls = ["phi", "phi", "ideal", "phi", "charge", "phi", "step", "phi", "run", "graph",
+             "phi", "set", "phi", "graph"]
+    takes = {"phi": 2, "ideal": 1, "charge": 7, "step": 22, "run": 44, "graph": 66, "set": 0}
+
+    def call(ctx, what):
+        if what == "phi":
+            ctx.hb_phi_step(dt)
+        elif what == "ideal":
+            ctx.ideal_step(dt)
+        elif what == "charge":
+            ctx.charge_step(dt)
+        elif what == "step":
+            ctx.step(dt)
+        elif what == "set":
+            ctx.set_rng_state(ctx.rng_state())
+        else:
+            ctx.use_graph(2 if what == "graph" else 0)
+            ctx.run(dt, 3 if what == "graph" else 2)
+            ctx.use_graph(0)
+
+    ctx = L.Context(L.model_params(N, seed=8))
+    ctx.set_field(np.random.default_rng(2).normal(size=(N, N, N, 10)) * 0.5)
+    counter = ctx.rng_state().sweep_ctr
+    for what in calls:
+        before, state = ctx.get_field(), ctx.rng_state()
+        assert state.sweep_ctr == counter, what
+        call(ctx, what)
+        one = L.Context(L.model_params(N, seed=8))
+        one.set_field(before)
+        one.set_rng_state(state)
+        call(one, what)
+        np.testing.assert_array_equal(ctx.get_field(), one.get_field(), err_msg=what)
+        one.close()
+        counter += takes[what]
+    assert ctx.rng_state().sweep_ctr == counter
+    ctx.close()
