@@ -117,10 +117,12 @@ struct lgv_ctx {
   // reallocated them: [replica][phi, charge]
   std::vector<std::array<lgv_monitor, 2>> mon_carry;
   EnergySlot *eslots = nullptr;
-  // Sweeps counted here and not yet in the replicas' sweep_ctr: a launch's
-  // counter offset starts from it, so that a lone phi sweep needs no launch to
-  // advance the state (six sweeps of 32^3: 70.8 -> 51.8 us).
+  // Counters and live-buffer flips of lone sweeps that are not in the replicas'
+  // state: the launches that follow start from them, so that such a sweep needs
+  // no launch of its own to advance the state (six phi sweeps of 32^3: 70.8 ->
+  // 51.8 us).
   uint64_t ctr = 0;
+  int flip = 0;
   double coef_hb = NAN, coef_charge = NAN, coef_ideal = NAN;
   double *d_aos = nullptr;
   int maxN = 0;
@@ -302,7 +304,9 @@ int64_t ideal_plane_blocks(const ReplicaParams &p, int cap) {
 // 435 with 25).  Depth: a block marches TZ planes and rotates one more on
 // either side, and the GPU holds `slots` blocks at a time.  A launch of up to
 // two rounds takes whole rounds of TZ planes, a longer one its blocks' share
-// and a tail; TZ of 16, 8, 4, and 2, 1 within one round, minimises that (FP64, TZ 16, 8, 4: 256^3
+// and a tail; TZ of 16, 8, 4, and 64, 32, 2, 1 within one round, minimises that
+// (256^3 FP64: TZ 64, 512 blocks, 532 us, 16 538; 320^3 has two rounds of 64,
+// 1145, and takes 16, 1112.  FP64, TZ 16, 8, 4: 256^3
 // 537, 546, 575 us; 240^3 558, 522, 523; 192^3 261, 245, 249; 144^3 140, 125,
 // 123; 100^3 63, 42, 38; 64^3 TZ 1 17 us, TZ 16 60).
 void resolve_ideal_tiles(lgv_ctx *c) {
@@ -323,15 +327,16 @@ void resolve_ideal_tiles(lgv_ctx *c) {
       p.tile_cap = 32;
     if (!c->fp32 && p.NH % 32 == 16 && p.NH > p.tile_cap) p.tile_cap = 16;
   }
-  int best = 16;
+  int best = 64;
   double best_cost = 1e300;
   const double tail = c->fp32 ? .15 : .25;
-  for (int tz = 16; tz >= 1; tz /= 2) {
+  for (int tz = 64; tz >= 1; tz /= 2) {
     int64_t blocks = 0;
     for (const ReplicaParams &p : c->hp)
       blocks += ideal_plane_blocks(p, p.tile_cap) * ((p.N + tz - 1) / tz);
     const double rounds = (double)blocks / slots;
     if (tz < 4 && rounds > 1.) break;
+    if (tz > 16 && rounds > 1.) continue;
     const double cost = (rounds <= 2. ? std::ceil(rounds) : rounds + tail) * (tz + .5);
     if (cost < best_cost) {
       best = tz;
@@ -701,16 +706,21 @@ int enqueue_charge(lgv_ctx *c, int off, int flip, hipStream_t st) {
   return 2;  // three flips of the charge buffers
 }
 
-// The sweeps counted on the host, for a launch sequence whose k_advance adds
-// them to the replicas' counters.
-int take_ctr(lgv_ctx *c) {
+// The counter and the flips held on the host, for a launch sequence whose
+// k_advance adds them to the replicas' state.
+int take_state(lgv_ctx *c, int &flip) {
   const int n = (int)c->ctr;
+  flip = c->flip;
   c->ctr = 0;
+  c->flip = 0;
   return n;
 }
-// Adds them by a launch of their own (before a graph, whose offsets start at 0).
-void flush_ctr(lgv_ctx *c) {
-  if (const int n = take_ctr(c)) launch_advance(c->nrep, c->dS, 0., 0, (uint64_t)n, 0, c->stream);
+// Adds them by a launch of their own: before a graph, whose offsets start at
+// 0, and before launches that read the live buffers by the state alone.
+void settle(lgv_ctx *c) {
+  int flip;
+  const int n = take_state(c, flip);
+  if (n) launch_advance(c->nrep, c->dS, 0., 0, (uint64_t)n, flip, c->stream);
 }
 
 // PV2HBSplit::step (Stepper.cxx:542-580); returns the number of stream
@@ -724,8 +734,7 @@ void flush_ctr(lgv_ctx *c) {
 // GPU on their own), and so do timed steps (events on one stream).  flip
 // returns the step's net live-buffer flip.
 int enqueue_step(lgv_ctx *c, int &flip) {
-  int off = take_ctr(c);
-  flip = 0;
+  int off = take_state(c, flip);
   bool charge_queued = false, join_event = false;
   c->timing_now = c->timing && c->timing_ctr++ % c->timing_every == 0;
   // a timed step keeps one stream (events on it bracket every launch)
@@ -1036,6 +1045,7 @@ int lgv_set_field(lgv_ctx *c, int r, const double *aos) {
   const int N = c->hp[r].N;
   const int64_t P = (int64_t)N * N * 10;  // doubles per z-plane
   const int slab = slab_planes(N);
+  settle(c);
   HIPCHECK(hipStreamSynchronize(c->stream));
   for (int z0 = 0; z0 < N; z0 += slab) {
     const int nz = std::min(slab, N - z0);
@@ -1055,6 +1065,7 @@ int lgv_get_field(lgv_ctx *c, int r, double *aos) {
   const int N = c->hp[r].N;
   const int64_t P = (int64_t)N * N * 10;  // doubles per z-plane
   const int slab = slab_planes(N);
+  settle(c);
   for (int z0 = 0; z0 < N; z0 += slab) {
     const int nz = std::min(slab, N - z0);
     launch_rb_to_aos(c->fp32, c->dP, c->dS, r, N, z0, nz, c->d_aos, c->stream);
@@ -1155,7 +1166,7 @@ int lgv_run(lgv_ctx *c, double dt, int nsteps) {
     }
     return check_launch();
   }
-  flush_ctr(c);
+  settle(c);
   if (!c->graph_exec || c->graph_dt != dt) {
     if ((rc = drop_graphs(c))) return rc;
     // graph_steps steps in one graph, and (when that is more than one) one
@@ -1194,8 +1205,9 @@ int lgv_ideal_step(lgv_ctx *c, double dt) {
   int rc = ensure_coeffs(c, c->coef_hb, c->coef_charge, dt);
   if (rc) return rc;
   c->timing_now = c->timing;  // single sweeps are always timed
-  const int off = take_ctr(c), flip = enqueue_ideal(c, off, 0);
-  launch_advance(c->nrep, c->dS, 0., 0, (uint64_t)off + 1, flip, c->stream);
+  if (c->ctr >> 20) settle(c);
+  c->flip ^= enqueue_ideal(c, (int)c->ctr, c->flip);
+  c->ctr += 1;
   return check_launch();
 }
 
@@ -1205,8 +1217,8 @@ int lgv_hb_phi_step(lgv_ctx *c, double dt) {
   int rc = ensure_coeffs(c, dt, c->coef_charge, c->coef_ideal);
   if (rc) return rc;
   c->timing_now = c->timing;  // single sweeps are always timed
-  if (c->ctr >> 20) flush_ctr(c);
-  enqueue_hb(c, (int)c->ctr, 0);  // in place: the live buffers stay
+  if (c->ctr >> 20) settle(c);
+  c->flip ^= enqueue_hb(c, (int)c->ctr, c->flip);
   c->ctr += 2;
   return check_launch();
 }
@@ -1217,8 +1229,9 @@ int lgv_charge_step(lgv_ctx *c, double dt) {
   int rc = ensure_coeffs(c, c->coef_hb, dt, c->coef_ideal);
   if (rc) return rc;
   c->timing_now = c->timing;  // single sweeps are always timed
-  const int off = take_ctr(c), flip = enqueue_charge(c, off, 0, c->stream);
-  launch_advance(c->nrep, c->dS, 0., 0, (uint64_t)off + 7, flip, c->stream);
+  if (c->ctr >> 20) settle(c);
+  c->flip ^= enqueue_charge(c, (int)c->ctr, c->flip, c->stream);
+  c->ctr += 7;
   return check_launch();
 }
 
@@ -1338,6 +1351,7 @@ int lgv_measure(lgv_ctx *c, int r, double *wall, double *wallphase, double *oavg
   HIPCHECK(hipSetDevice(c->device));
   const int N = c->hp[r].N;
   const MeasBuf mb(c->d_meas, N), h(c->h_meas, N);
+  settle(c);
   launch_measure(c->fp32, c->dP, c->dS, r, N, c->d_part, mb.wall, mb.wallphase, h.wall,
                  h.wallphase, c->stream);
   if ((rc = check_launch())) return rc;
@@ -1384,6 +1398,7 @@ int lgv_measure_full(lgv_ctx *c, int r, lgv_measurement *m) {
   HIPCHECK(hipSetDevice(c->device));
   const int N = c->hp[r].N, nk = N / 2 + 1;
   const MeasBuf mb(c->d_meas, N), h(c->h_meas, N);
+  settle(c);
   launch_measure(c->fp32, c->dP, c->dS, r, N, c->d_part, mb.wall, mb.wallphase, h.wall,
                  h.wallphase, c->stream);
   launch_wall_dft(N, mb.wall, mb.wallphase, h.wallk, h.wallphasek, c->stream);

@@ -189,4 +189,13 @@ def test_sweep_counters_of_mixed_calls(L):
         one.close()
         counter += takes[what]
     assert ctx.rng_state().sweep_ctr == counter
+    # and all of them with nothing read in between
+    one = L.Context(L.model_params(N, seed=8))
+    one.set_field(np.random.default_rng(2).normal(size=(N, N, N, 10)) * 0.5)
+    for what in calls:
+        call(one, what)
+    oavg = one.measure()[2]
+    np.testing.assert_array_equal(oavg, ctx.measure()[2])
+    np.testing.assert_array_equal(ctx.get_field(), one.get_field())
+    one.close()
     ctx.close()
