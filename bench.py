@@ -28,7 +28,8 @@ HBM_PEAK = 8.0e12  # MI355X HBM3E, B/s
 # Algorithmic bytes per site per launch, FP64 fields (halve for FP32):
 # ideal substep (k_ideal_fused) read 80 + write 80; phi half-sweep
 # (k_hb_march for large fields, k_hb_phi otherwise) read all phi 32 + write
-# one parity 16; charge direction (k_charge_march, both sub-sweeps of one
+# one parity 16, or half of a launch of both parities (k_hb_sweep for large FP64
+# fields, k_hb_brick for small lattices) read 16 + write 16; charge direction (k_charge_march, both sub-sweeps of one
 # direction) read 48 + write 48.
 ALG_BYTES = {"ideal": 160, "phi": 48, "charge": 96}
 KERNEL = {"ideal": "k_ideal_fused", "phi": "k_hb_march", "charge": "k_charge_march"}
@@ -52,11 +53,14 @@ MEASURED_TRAFFIC = {
 }
 
 
-def tables(fp32, march):
+def tables(fp32, march, pairs=0):
     """(algorithmic bytes per site per launch, kernel name, schedule bytes per
     site-update) for the precision's kernel schedule; march: the phi
-    half-sweep runs the z-march."""
+    half-sweep runs the z-march; pairs: Context.phi_pairs()."""
     sched = SCHEDULE_BYTES_PER_SITE_UPDATE_FP32 if fp32 else SCHEDULE_BYTES_PER_SITE_UPDATE
+    if pairs:
+        return (dict(ALG_BYTES, phi=32),
+                dict(KERNEL, phi="k_hb_sweep" if pairs == 2 else "k_hb_brick"), sched - 12 * 16)
     if march:
         return ALG_BYTES, KERNEL, sched
     return ALG_BYTES, dict(KERNEL, phi="k_hb_phi"), sched
@@ -313,7 +317,7 @@ def run_single(L, N, fp32, steps, warmup, graph=False, tune=True, ideal_tile=Non
     sites = N ** 3
     value = sites * steps / el
     march = ctx.phi_kernel() == L.PHI_MARCH
-    alg, kern, sched = tables(fp32, march)
+    alg, kern, sched = tables(fp32, march, ctx.phi_pairs())
     out = {
         "value": value, "ms_per_step": el * 1e3 / steps, "steps": steps, "warmup": warmup,
         "dtype": "f32-storage/f64-arith" if fp32 else "f64",
@@ -394,7 +398,7 @@ def run_batched(L, fp32, steps, warmup, tune=True, graph=True, graph_steps=10,
         seq_el += time.perf_counter() - t0
         c1.close()
     seq_value = sites * steps / seq_el
-    alg, kern, _ = tables(fp32, march)
+    alg, kern, _ = tables(fp32, march, ctx.phi_pairs())
     return {
         "value": value, "ms_per_step": el * 1e3 / steps, "steps": steps, "warmup": warmup,
         "dtype": "f32-storage/f64-arith" if fp32 else "f64",

@@ -192,12 +192,17 @@ int lgv_set_sweep_tiles(lgv_ctx *ctx, int replica, int hb_cap, int hb_tz, int ch
  * ModelG/Stepper.cxx:287-389): LGV_PHI_SITE one thread per site,
  * LGV_PHI_MARCH the z-march with the other parity's plane in LDS,
  * LGV_PHI_AUTO the size rule (the march from 7 million sites of all replicas
- * on).  Results do not depend on it; the autotuner picks
+ * on; and below 560000 sites, and FP64 fields from 2.9 million on, the pairs
+ * of sweeps of a step in launches of both parities, which the other two values
+ * leave out).  Results do not depend on it; the autotuner picks
  * it.  Monitor counts are kept across the change.  lgv_get_phi_kernel
  * reports the kernel in use (LGV_PHI_SITE or LGV_PHI_MARCH). */
 enum { LGV_PHI_AUTO = 0, LGV_PHI_SITE = 1, LGV_PHI_MARCH = 2 };
 int lgv_set_phi_kernel(lgv_ctx *ctx, int kernel);
 int lgv_get_phi_kernel(lgv_ctx *ctx, int *kernel);
+/* How pairs of phi sweeps of a step run: 0 as half-sweeps, 1 in launches of both
+ * parities over bricks, 2 in the march of both parities. */
+int lgv_get_phi_pairs(lgv_ctx *ctx, int *kernel);
 
 int lgv_synchronize(lgv_ctx *ctx);
 /* Device address of a replica's field storage (10 component planes, each

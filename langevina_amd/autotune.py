@@ -105,10 +105,10 @@ def _search(ctx, dt, steps, cls, apply, candidates):
 
 
 def autotune_sweeps(ctx, dt, march=None, steps=3, verbose=False):
-    """march None: first the phi half-sweep kernel, the per-site kernel or
-    the z-march, timed over whole steps (the march's lower traffic also
-    speeds up the kernels that follow it), the size rule's choice being the
-    incumbent; march True / False: keep the kernel in use and tune (or not)
+    """march None: first the phi kernel (the size rule's choice, the per-site
+    half-sweeps, the z-march), timed over whole steps (a kernel's lower traffic
+    also speeds up the kernels that follow it), the size rule's choice being
+    the incumbent; march True / False: keep the kernel in use and tune (or not)
     the march's tiles.  Then per size class, as autotune_ideal: the charge
     march (tile width x chunk) and, when the phi half-sweep runs the z-march,
     its tile width x z-chunk.  Returns {N: (hb_cap, hb_tz, chg_cap,
@@ -128,11 +128,9 @@ def autotune_sweeps(ctx, dt, march=None, steps=3, verbose=False):
         ctx.step(dt)
     if march is None:
         from .lgv import PHI_AUTO, PHI_MARCH, PHI_SITE
-        ctx.set_phi_kernel(PHI_AUTO)
-        inc = ctx.phi_kernel()
-        kernel, ms = _search(ctx, dt, 8 * steps, None, ctx.set_phi_kernel,
-                             [inc, PHI_SITE if inc == PHI_MARCH else PHI_MARCH])
-        march = kernel == PHI_MARCH
+        _, ms = _search(ctx, dt, 8 * steps, None, ctx.set_phi_kernel,
+                        [PHI_AUTO, PHI_SITE, PHI_MARCH])
+        march = ctx.phi_kernel() == PHI_MARCH
         if verbose:
             print(f"autotune phi kernel: {'march' if march else 'site'} {ms:.3f} ms/step",
                   flush=True)

@@ -84,6 +84,9 @@ struct TileRequest {
   int ideal_cap = 0, ideal_tz = 0, hb_cap = 0, hb_tz = 0, chg_cap = 0, chg_chunk = 0;
 };
 
+// The kernel of launches of both parities: k_hb_brick, k_hb_sweep.
+enum class TwoParity { kNone, kBricks, kMarch };
+
 struct lgv_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -103,16 +106,18 @@ struct lgv_ctx {
   ReplicaParams *dP = nullptr;
   ReplicaState *dS = nullptr;
   std::vector<void *> fields;
-  Plan plan_half, plan_full, plan_ideal, plan_charge, plan_hb, plan_brick;
+  Plan plan_half, plan_full, plan_ideal, plan_charge, plan_hb, plan_pair;
   bool wide = false;    // some plane is >= 4 GiB: kernels use 64-bit offsets
   uint64_t buffer_bytes = 0;  // one buffer's fields, all replicas
   int nt_stores = -1;  // non-temporal stores: -1 by the rule, 0 / 1 forced
   bool phi_march = false;  // the phi half-sweep runs the z-march kernel
   bool phi_march_auto = false;  // the size rule's choice (LGV_PHI_AUTO)
-  // the per-site kernel's sweeps come in pairs of two-parity launches
-  bool phi_bricks = false;
-  int brick_lds = 0;  // bytes of LDS of such a launch
-  MonSlot *mon_phi = nullptr, *mon_brick = nullptr, *mon_charge = nullptr, *mon_ideal = nullptr;
+  // pairs of phi sweeps run as out-of-place launches of both parities
+  // (LGV_PHI_AUTO), in the kernel that the size rule chose
+  bool phi_pairs = false;
+  TwoParity two_parity = TwoParity::kNone;
+  int brick_lds = 0;  // bytes of LDS of a launch in bricks
+  MonSlot *mon_phi = nullptr, *mon_pair = nullptr, *mon_charge = nullptr, *mon_ideal = nullptr;
   // monitor counts folded out of the per-block slots when a retile
   // reallocated them: [replica][phi, charge]
   std::vector<std::array<lgv_monitor, 2>> mon_carry;
@@ -442,11 +447,11 @@ int brick_rows(int N, int by, int bz) {
   return y * z + 2 * y + 2 * z;
 }
 
-// The bricks of the two-parity phi sweep: of the BY x BZ rows whose even sites
-// fit kBrickLds, those with the fewest decisions per CU, in wavefronts and
-// whole rounds of 256 blocks (64^3 FP64: 4 x 4 rows, 256 blocks, 24 wavefronts
-// against the 16 that have no facing rows).
-int build_brick_plan(lgv_ctx *c) {
+// The bricks of k_hb_brick: of the BY x BZ rows whose even sites fit kBrickLds,
+// those with the fewest decisions per CU, in wavefronts and whole rounds of 256
+// blocks (64^3 FP64: 4 x 4 rows, 256 blocks, 24 wavefronts against the 16 that
+// have no facing rows).  False: no brick fits.
+bool resolve_bricks(lgv_ctx *c) {
   const int esz = c->fp32 ? 4 : 8;
   int best_y = 0, best_z = 0;
   double best = 1e300;
@@ -459,7 +464,8 @@ int build_brick_plan(lgv_ctx *c) {
         fits = fits && rows * p.NH * 4 * esz <= kBrickLds;
         const double n = (double)((p.N + by - 1) / by) * ((p.N + bz - 1) / bz);
         blocks += n;
-        waves += n * ((rows * p.NH + 63) / 64 + (std::min(by, p.N) * std::min(bz, p.N) * p.NH + 63) / 64);
+        waves += n * ((rows * p.NH + 63) / 64 +
+                      (std::min(by, p.N) * std::min(bz, p.N) * p.NH + 63) / 64);
       }
       const double cost = waves / blocks * std::ceil(blocks / kCUs);
       if (fits && cost < best) {
@@ -468,18 +474,55 @@ int build_brick_plan(lgv_ctx *c) {
         best_z = bz;
       }
     }
-  if (!best_y) c->phi_bricks = false;  // rows longer than the LDS holds
-  if (!c->phi_bricks) return LGV_OK;
+  for (ReplicaParams &p : c->hp) {
+    p.pair_y = best_y;
+    p.pair_z = best_z;
+    c->brick_lds = std::max(c->brick_lds, brick_rows(p.N, best_y, best_z) * p.NH * 4 * esz);
+  }
+  return best_y != 0;
+}
+
+// The tiles of k_hb_sweep: as many rows as its threads hold (half-columns, with
+// a facing row on either side), and the depth TZ that minimises whole rounds of
+// one block per CU, each of TZ planes and about five planes' time for the two
+// more that it decides, its start and its end (256^3 FP64, per half-sweep: TZ
+// 52, one round of 215 blocks, 131 us; 24, two, 133; 16, three, 142; 8 160).
+// False: rows that are too long, or sides below kPairMarchSide.
+bool resolve_pair_march(lgv_ctx *c) {
+  for (ReplicaParams &p : c->hp) {
+    if (kPairBlock / p.NH < 3 || p.N < kPairMarchSide) return false;
+    p.pair_y = std::min(kPairBlock / p.NH - 2, p.N);
+  }
+  int best = 0;
+  double best_cost = 1e300;
+  for (int tz = 2; tz <= 64; tz++) {
+    int64_t blocks = 0;
+    for (const ReplicaParams &p : c->hp)
+      blocks += (int64_t)((p.N + p.pair_y - 1) / p.pair_y) * ((p.N + tz - 1) / tz);
+    const double cost = std::ceil((double)blocks / kCUs) * (tz + 5.);
+    if (cost < best_cost) {
+      best = tz;
+      best_cost = cost;
+    }
+  }
+  for (ReplicaParams &p : c->hp) p.pair_z = best;
+  return true;
+}
+
+// Blocks of the launches of both parities.
+int build_pair_plan(lgv_ctx *c) {
+  if (c->two_parity == TwoParity::kBricks && !resolve_bricks(c)) c->two_parity = TwoParity::kNone;
+  if (c->two_parity == TwoParity::kMarch && !resolve_pair_march(c))
+    c->two_parity = TwoParity::kNone;
+  if (c->two_parity == TwoParity::kNone) return LGV_OK;
   std::vector<PlanWork> work;
   bool wide = c->wide;
-  for (ReplicaParams &p : c->hp) {
-    p.brick_y = best_y;
-    p.brick_z = best_z;
-    c->brick_lds = std::max(c->brick_lds, brick_rows(p.N, best_y, best_z) * p.NH * 4 * esz);
-    const int64_t plane = (p.N + best_y - 1) / best_y;
-    work.push_back({plane * ((p.N + best_z - 1) / best_z), (double)plane});
+  for (const ReplicaParams &p : c->hp) {
+    wide = wide || 2 * (uint64_t)p.half * (c->fp32 ? 4 : 8) > 0xFFFFFFFFull;
+    const int64_t plane = (p.N + p.pair_y - 1) / p.pair_y;
+    work.push_back({plane * ((p.N + p.pair_z - 1) / p.pair_z), (double)plane});
   }
-  return build_plan(c->plan_brick, work, wide);
+  return build_plan(c->plan_pair, work, wide);
 }
 
 // Whether the x sub-sweeps of every replica run whole rows per wavefront
@@ -683,11 +726,15 @@ int enqueue_hb(lgv_ctx *c, int off, int flip) {
 // the in-place sweeps do), the others in place.
 void enqueue_phi_sweeps(lgv_ctx *c, int n, int off, int flip) {
   int i = 0;
-  if (c->phi_bricks && !use_march(c)) {
+  if (c->phi_pairs) {
     for (; i < n - n % 2; i++) {
       Timed tm(c, LGV_CLASS_PHI, 2);  // two half-sweeps
-      launch_hb_brick(c->fp32, c->plan_brick, c->brick_lds, c->dP, c->dS, off + 2 * i,
-                      flip ^ (i & 1), c->mon_brick, c->stream);
+      if (c->two_parity == TwoParity::kMarch)
+        launch_hb_sweep(c->fp32, c->plan_pair, c->dP, c->dS, off + 2 * i, flip ^ (i & 1),
+                        c->mon_pair, c->stream);
+      else
+        launch_hb_brick(c->fp32, c->plan_pair, c->brick_lds, c->dP, c->dS, off + 2 * i,
+                        flip ^ (i & 1), c->mon_pair, c->stream);
     }
   }
   for (; i < n; i++) enqueue_hb(c, off + 2 * i, flip);
@@ -961,9 +1008,13 @@ int lgv_create(const lgv_config *cfg, lgv_ctx **out) {
       return fail(LGV_ERR_ARG, "LGV_PHI_KERNEL=%s: expected site or march", pk);
     c->phi_march = k == "march";
   }
-  c->phi_bricks = buffer_bytes / (10 * esz) < kBrickSites;
-  // test hook: LGV_PHI_BRICKS=0/1 forces the two-parity launches off / on
-  if (const char *pb = getenv("LGV_PHI_BRICKS")) c->phi_bricks = atoi(pb) != 0;
+  const uint64_t sites = buffer_bytes / (10 * esz);
+  if (sites < kBrickSites) c->two_parity = TwoParity::kBricks;
+  if (!c->fp32 && sites >= kPairMarchSites) c->two_parity = TwoParity::kMarch;
+  // test hook: LGV_PHI_PAIRS=0/1/2 takes no launches of both parities, bricks,
+  // the march
+  if (const char *pb = getenv("LGV_PHI_PAIRS"))
+    c->two_parity = (TwoParity)std::min(std::max(atoi(pb), 0), 2);
   HIPCHECK(hipMalloc(&c->dS, c->nrep * sizeof(ReplicaState)));
   HIPCHECK(hipMemcpy(c->dS, hs.data(), c->nrep * sizeof(ReplicaState), hipMemcpyHostToDevice));
   int rc;
@@ -972,16 +1023,19 @@ int lgv_create(const lgv_config *cfg, lgv_ctx **out) {
   if ((rc = build_ideal_plan(c.get())) != LGV_OK) return rc;
   if ((rc = build_charge_plan(c.get())) != LGV_OK) return rc;
   if ((rc = build_hb_plan(c.get())) != LGV_OK) return rc;
-  if ((rc = build_brick_plan(c.get())) != LGV_OK) return rc;
+  if ((rc = build_pair_plan(c.get())) != LGV_OK) return rc;
+  // the hooks that force a half-sweep kernel or its stores leave out the others
+  c->phi_pairs =
+      c->two_parity != TwoParity::kNone && !getenv("LGV_PHI_KERNEL") && c->nt_stores < 0;
   // the parameters as the plans' tile rules left them
   HIPCHECK(hipMalloc(&c->dP, c->nrep * sizeof(ReplicaParams)));
   HIPCHECK(hipMemcpy(c->dP, c->hp.data(), c->nrep * sizeof(ReplicaParams),
                      hipMemcpyHostToDevice));
   HIPCHECK(hipMalloc(&c->mon_phi, hb_plan(c.get()).nblocks * sizeof(MonSlot)));
   HIPCHECK(hipMemset(c->mon_phi, 0, hb_plan(c.get()).nblocks * sizeof(MonSlot)));
-  if (c->phi_bricks) {
-    HIPCHECK(hipMalloc(&c->mon_brick, c->plan_brick.nblocks * sizeof(MonSlot)));
-    HIPCHECK(hipMemset(c->mon_brick, 0, c->plan_brick.nblocks * sizeof(MonSlot)));
+  if (c->two_parity != TwoParity::kNone) {
+    HIPCHECK(hipMalloc(&c->mon_pair, c->plan_pair.nblocks * sizeof(MonSlot)));
+    HIPCHECK(hipMemset(c->mon_pair, 0, c->plan_pair.nblocks * sizeof(MonSlot)));
   }
   HIPCHECK(hipMalloc(&c->mon_charge, c->plan_charge.nblocks * sizeof(MonSlot)));
   HIPCHECK(hipMemset(c->mon_charge, 0, c->plan_charge.nblocks * sizeof(MonSlot)));
@@ -1019,10 +1073,10 @@ int lgv_destroy(lgv_ctx *c) {
   note(hipFree(c->dP));
   note(hipFree(c->dS));
   for (Plan *pl : {&c->plan_half, &c->plan_full, &c->plan_ideal, &c->plan_charge, &c->plan_hb,
-                   &c->plan_brick}) {
+                   &c->plan_pair}) {
     for (int *q : {pl->blocks.rep, pl->blocks.local, pl->blocks.first}) note(hipFree(q));
   }
-  for (void *q : {(void *)c->mon_phi, (void *)c->mon_brick, (void *)c->mon_charge, (void *)c->mon_ideal,
+  for (void *q : {(void *)c->mon_phi, (void *)c->mon_pair, (void *)c->mon_charge, (void *)c->mon_ideal,
                   (void *)c->eslots, (void *)c->d_aos, (void *)c->d_part,
                   (void *)c->d_meas})
     note(hipFree(q));
@@ -1135,7 +1189,7 @@ static int realloc_monitors(lgv_ctx *c) {
   HIPCHECK(hipMemset(c->mon_phi, 0, hb_plan(c).nblocks * sizeof(MonSlot)));
   HIPCHECK(hipMalloc(&c->mon_charge, c->plan_charge.nblocks * sizeof(MonSlot)));
   HIPCHECK(hipMemset(c->mon_charge, 0, c->plan_charge.nblocks * sizeof(MonSlot)));
-  if (c->mon_brick) HIPCHECK(hipMemset(c->mon_brick, 0, c->plan_brick.nblocks * sizeof(MonSlot)));
+  if (c->mon_pair) HIPCHECK(hipMemset(c->mon_pair, 0, c->plan_pair.nblocks * sizeof(MonSlot)));
   return LGV_OK;
 }
 
@@ -1275,8 +1329,8 @@ int lgv_monitor_get(lgv_ctx *c, int r, lgv_monitor out[3]) {
   HIPCHECK(hipSetDevice(c->device));
   HIPCHECK(hipStreamSynchronize(c->stream));
   // phi half-sweeps, charge sweeps, two-parity phi sweeps
-  MonSlot *src[3] = {c->mon_phi, c->mon_charge, c->mon_brick};
-  const Plan *plan[3] = {&hb_plan(c), &c->plan_charge, &c->plan_brick};
+  MonSlot *src[3] = {c->mon_phi, c->mon_charge, c->mon_pair};
+  const Plan *plan[3] = {&hb_plan(c), &c->plan_charge, &c->plan_pair};
   for (int k = 0; k < 2; k++) out[k] = c->mon_carry[r][k];
   for (int k = 0; k < 3; k++) {
     if (!src[k]) continue;
@@ -1498,11 +1552,13 @@ int lgv_set_phi_kernel(lgv_ctx *c, int kernel) {
   if (kernel != LGV_PHI_AUTO && kernel != LGV_PHI_SITE && kernel != LGV_PHI_MARCH)
     return fail(LGV_ERR_ARG, "phi kernel %d: expected LGV_PHI_AUTO, _SITE or _MARCH", kernel);
   const bool march = kernel == LGV_PHI_AUTO ? c->phi_march_auto : kernel == LGV_PHI_MARCH;
-  if (march == c->phi_march) return LGV_OK;
+  const bool pairs = kernel == LGV_PHI_AUTO && c->two_parity != TwoParity::kNone;
+  if (march == c->phi_march && pairs == c->phi_pairs) return LGV_OK;
   HIPCHECK(hipSetDevice(c->device));
   HIPCHECK(hipStreamSynchronize(c->stream));
   if (int rm = fold_monitors(c)) return rm;
   c->phi_march = march;
+  c->phi_pairs = pairs;
   if (int rm = realloc_monitors(c)) return rm;
   HIPCHECK(hipDeviceSynchronize());
   return drop_graphs(c);
@@ -1514,13 +1570,19 @@ int lgv_get_phi_kernel(lgv_ctx *c, int *kernel) {
   return LGV_OK;
 }
 
+int lgv_get_phi_pairs(lgv_ctx *c, int *kernel) {
+  if (!c || !kernel) return fail(LGV_ERR_ARG, "null argument");
+  *kernel = c->phi_pairs ? (int)c->two_parity : 0;
+  return LGV_OK;
+}
+
 int lgv_monitor_reset(lgv_ctx *c) {
   if (!c) return fail(LGV_ERR_ARG, "null context");
   HIPCHECK(hipSetDevice(c->device));
   HIPCHECK(hipStreamSynchronize(c->stream));
   HIPCHECK(hipMemset(c->mon_phi, 0, hb_plan(c).nblocks * sizeof(MonSlot)));
   HIPCHECK(hipMemset(c->mon_charge, 0, c->plan_charge.nblocks * sizeof(MonSlot)));
-  if (c->mon_brick) HIPCHECK(hipMemset(c->mon_brick, 0, c->plan_brick.nblocks * sizeof(MonSlot)));
+  if (c->mon_pair) HIPCHECK(hipMemset(c->mon_pair, 0, c->plan_pair.nblocks * sizeof(MonSlot)));
   HIPCHECK(hipMemset(c->mon_ideal, 0, c->nrep * sizeof(MonSlot)));
   HIPCHECK(hipDeviceSynchronize());
   for (auto &cr : c->mon_carry) cr = {lgv_monitor{}, lgv_monitor{}};

@@ -9,8 +9,8 @@
 
 namespace lgv {
 
-constexpr int kBlock = 256;  // threads per block of every sweep kernel but k_hb_brick
-constexpr int kBrickBlock = 1024;
+constexpr int kBlock = 256;  // threads per block of every sweep kernel but these:
+constexpr int kPairBlock = 1024;  // k_hb_brick, k_hb_sweep
 
 // Read-only (for the kernels) description of one replica.  The step
 // coefficients (rdtg, rms, dt_ideal, tau) are computed on the host with the
@@ -32,7 +32,7 @@ struct ReplicaParams {
   int tile_cap, tile_tz;   // ideal-kernel tile (see ideal_tile)
   int hb_cap, hb_tz;       // phi-march tile (see hb_tile)
   int chg_cap, chg_chunk;  // charge-march tile (see charge_tile)
-  int brick_y, brick_z;    // rows of a brick of the two-parity phi sweep
+  int pair_y, pair_z;      // rows in y and planes of a block of both parities
 };
 
 // Device-written state of one replica (clock, counters, per-step data).
@@ -147,15 +147,29 @@ constexpr uint64_t kCacheBytes = 256ull << 20;
 // 2253 -> 2214, 256^3 2949 -> 2708.
 constexpr uint64_t kMarchSites = 7000000;
 
-// Below this many sites (all replicas) the per-site phi sweeps of a step run as
-// two-parity launches (k_hb_brick), in bricks that fit kBrickLds bytes of LDS
-// (two blocks of a CU).  Whole steps, half-sweeps -> two-parity launches: FP64
-// 16^3 100 -> 88 us, 32^3 106 -> 93, 64^3 151 -> 144, 80^3 231 -> 226, 84^3 248
-// -> 275, 5 x 48^3 230 -> 229; FP32 64^3 138 -> 128, 80^3 193 -> 189, 84^3 207
-// -> 209, 16 x 32^3 174 -> 165, 32 x 32^3 251 -> 246, 64 x 32^3 422 -> 457:
-// above, the facing rows' extra decisions cost more than the launches saved.
+// Pairs of phi sweeps run as launches of both parities, out of place (a pair
+// leaves the live buffer where it was), below the first number of sites (all
+// replicas) in bricks that fit kBrickLds bytes of LDS (k_hb_brick, two blocks of
+// a CU), and FP64 fields from the second on in the march k_hb_sweep.
+// Small lattices save launches.  Whole steps, half-sweeps -> bricks: FP64 16^3
+// 100 -> 88 us, 32^3 106 -> 93, 64^3 151 -> 144, 80^3 231 -> 226, 84^3 248 ->
+// 275, 5 x 48^3 230 -> 229; FP32 64^3 138 -> 128, 80^3 193 -> 189, 84^3 207 ->
+// 209, 16 x 32^3 174 -> 165, 32 x 32^3 251 -> 246, 64 x 32^3 422 -> 457: above,
+// the facing rows' extra decisions cost more than the launches saved.
+// Large FP64 lattices are bound by the bytes of a half-sweep, which reads both
+// parities and writes one; both parities in one pass read and write each value
+// once.  Half-sweeps -> k_hb_sweep: 128^3 628 -> 648 us, 140^3 938 -> 938, 144^3
+// 986 -> 967, 160^3 1267 -> 1176, 200^3 2509 -> 2414, 224^3 3221 -> 3057, 256^3
+// 4319 -> 4162 (three contexts at once 4444 -> 4135 a step), 300^3 9159 -> 8372.
+// FP32 fields move half the bytes and the march is bound by its decisions and
+// one barrier per plane: 256^3 2664 -> 2911 us, 160^3 FP32 likewise slower.
 constexpr uint64_t kBrickSites = 560000;
 constexpr int kBrickLds = 64 << 10;
+// In a batch, a replica below the side fills too few of a block's threads with
+// its rows: 96 x 48^3 3004 -> 3278, but 16 x 64^3 1167 -> 1144, 8 x 96^3 2026 ->
+// 1945, 2 x 160^3 2460 -> 2184.
+constexpr uint64_t kPairMarchSites = 2900000;
+constexpr int kPairMarchSide = 64;
 
 // A context of one lattice whose fields (one buffer) exceed this keeps the
 // charge sweep after the phi sweeps rather than beside them.
@@ -218,6 +232,8 @@ void launch_hb_phi(bool fp32, const Plan &plan, const ReplicaParams *P, ReplicaS
                    int ieo, int ctr_off, int flip, MonSlot *mon, hipStream_t st);
 void launch_hb_brick(bool fp32, const Plan &plan, int lds, const ReplicaParams *P,
                      ReplicaState *S, int ctr_off, int flip, MonSlot *mon, hipStream_t st);
+void launch_hb_sweep(bool fp32, const Plan &plan, const ReplicaParams *P, ReplicaState *S,
+                     int ctr_off, int flip, MonSlot *mon, hipStream_t st);
 void launch_hb_march(bool fp32, const Plan &plan, const ReplicaParams *P, ReplicaState *S,
                      int ieo, int ctr_off, int flip, MonSlot *mon, hipStream_t st);
 void launch_charge_march(bool fp32, const Plan &plan, const ReplicaParams *P, ReplicaState *S,

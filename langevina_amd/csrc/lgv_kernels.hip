@@ -179,8 +179,11 @@ struct ChargePlanes<T, false> {
 // the plane after next come and go with the register allocation).
 // W == true: 64-bit addresses.
 // NT: a value no other thread reads, not kept in the caches.
+// Offset kNone: no access (a load gives zero); with a buffer resource that lies
+// past its end, where the hardware neither reads nor writes.
 template <typename T, bool W>
 struct PhiPlanes {
+  static constexpr uint32_t kNone = 0xFFFFFFFFu / sizeof(T);
   GPlane<T, true> f[4];
   int64_t half_bytes;
   uint32_t plane;
@@ -196,15 +199,16 @@ struct PhiPlanes {
   }
   template <bool NT>
   __device__ __forceinline__ T ld(int l, int par, int z, uint32_t i) const {
-    return half(l, par).template get_raw<NT>((uint32_t)z * plane + i);
+    return i == kNone ? T(0) : half(l, par).template get_raw<NT>((uint32_t)z * plane + i);
   }
   template <bool NT>
   __device__ __forceinline__ void st(int l, int par, int z, uint32_t i, T v) const {
-    half(l, par).template put_raw<NT>((uint32_t)z * plane + i, v);
+    if (i != kNone) half(l, par).template put_raw<NT>((uint32_t)z * plane + i, v);
   }
 };
 template <typename T>
 struct PhiPlanes<T, false> {
+  static constexpr uint32_t kNone = 0xFFFFFFFFu / sizeof(T);
   __amdgpu_buffer_rsrc_t f[4];
   uint32_t half_bytes, plane_bytes;
   __device__ __forceinline__ PhiPlanes(const ReplicaParams &p, int cur) {
@@ -455,7 +459,7 @@ __device__ __forceinline__ int wrapz(int z, int N) { return z < 0 ? z + N : (z >
 // 4.6 us, of 64^3 8.6 -> 7.1, half of a launch; 100^3 15.9 -> 16.7: kBrickSites).
 // The first round of odd values is loaded before the even sites' decisions.
 template <typename T, bool W>
-__global__ __launch_bounds__(kBrickBlock) void k_hb_brick(const ReplicaParams *__restrict__ P,
+__global__ __launch_bounds__(kPairBlock) void k_hb_brick(const ReplicaParams *__restrict__ P,
                                                           const ReplicaState *__restrict__ S,
                                                           LaunchBlocks blk, int ctr_off, int flip,
                                                           MonSlot *__restrict__ mon) {
@@ -467,9 +471,9 @@ __global__ __launch_bounds__(kBrickBlock) void k_hb_brick(const ReplicaParams *_
   const ReplicaState &s = S[r];
   const int cur = s.cur_phi ^ (flip & 1), nxt = cur ^ 1;  // phi planes only
   const uint32_t N = p.N, NH = p.NH;
-  const int nby = (N + p.brick_y - 1) / p.brick_y;
-  const int y0 = b % nby * p.brick_y, z0 = b / nby * p.brick_z;
-  const int h = min(p.brick_y, (int)N - y0), d = min(p.brick_z, (int)N - z0);
+  const int nby = (N + p.pair_y - 1) / p.pair_y;
+  const int y0 = b % nby * p.pair_y, z0 = b / nby * p.pair_z;
+  const int h = min(p.pair_y, (int)N - y0), d = min(p.pair_z, (int)N - z0);
   // rows: the brick's, then the facing ones at y0 - 1, y0 + h, z0 - 1, z0 + d
   const int ni = h * d, fy0 = ni, fy1 = ni + d, fz0 = ni + 2 * d, fz1 = fz0 + h;
   const int rows = fz1 + h;
@@ -506,7 +510,7 @@ __global__ __launch_bounds__(kBrickBlock) void k_hb_brick(const ReplicaParams *_
   if (wave0 < odd) odd_load(wave0);
   // Every lane of a wavefront takes part in each of its rounds (the tallies
   // are the wavefront's): lanes past the end repeat the last site.
-  for (int i0 = wave0; i0 < comp; i0 += kBrickBlock) {
+  for (int i0 = wave0; i0 < comp; i0 += kPairBlock) {
     const bool in = i0 + lane < comp;
     const uint32_t i = in ? i0 + lane : comp - 1;
     const uint32_t rid = __umulhi(i, inv), xh = i - rid * NH;
@@ -541,7 +545,7 @@ __global__ __launch_bounds__(kBrickBlock) void k_hb_brick(const ReplicaParams *_
     }
   }
   __syncthreads();
-  for (int i0 = wave0; i0 < odd; i0 += kBrickBlock) {
+  for (int i0 = wave0; i0 < odd; i0 += kPairBlock) {
     const bool in = i0 + lane < odd;
     uint32_t rid, xh;
     int dy, dz;
@@ -554,7 +558,7 @@ __global__ __launch_bounds__(kBrickBlock) void k_hb_brick(const ReplicaParams *_
     double phi_o[4], heff[4], phi_n[4];
 #pragma unroll
     for (int l = 0; l < 4; l++) phi_o[l] = odd_o[l];
-    if (i0 + kBrickBlock < odd) odd_load(i0 + kBrickBlock);
+    if (i0 + kPairBlock < odd) odd_load(i0 + kPairBlock);
 #pragma unroll
     for (int l = 0; l < 4; l++) {
       const T *f = even + l * comp;
@@ -569,7 +573,153 @@ __global__ __launch_bounds__(kBrickBlock) void k_hb_brick(const ReplicaParams *_
       for (int l = 0; l < 4; l++) gplane<T, W>(p, nxt, l, 1).st(idx, phi_n[l]);
     }
   }
-  block_monitor_add<kBrickBlock>(slot, mt);
+  block_monitor_add<kPairBlock>(slot, mt);
+}
+
+// Both parities of EulerLangevinHB::step (Stepper.cxx:309-386) in one launch,
+// out of place, marching z: a block owns BY whole x rows of each plane and the
+// facing row on either side, one thread to a half-column.  Step k decides the
+// even sites of plane z0 - 1 + k (on the facing rows as well) from the odd
+// values of the planes around it, and then the odd sites of the plane before
+// from the even ones.  In LDS lie the odd values of this plane and the last one
+// and the new even values of the last two; one barrier per plane.
+// It reads and writes each value once where two half-sweeps read both parities
+// twice (counted at 256^3 FP64: 12 -> 8 bytes per component and site), for
+// which it decides the even sites of the facing rows and of two planes a chunk
+// twice.  256^3 FP64: 257 us for both parities (two half-sweeps 295), 4.9 us a
+// plane of a block; about 60 % of that are vector instructions (235 a decision,
+// 28 decisions a SIMD lane), the rest the barrier's skew and LDS reads.  Whole
+// rows need no ring in x; 16 wavefronts, of which a facing row's have half the
+// work, spread evenly over the four SIMDs.
+template <typename T, bool W>
+__global__ __launch_bounds__(kPairBlock) void k_hb_sweep(const ReplicaParams *__restrict__ P,
+                                                          const ReplicaState *__restrict__ S,
+                                                          LaunchBlocks blk, int ctr_off, int flip,
+                                                          MonSlot *__restrict__ mon) {
+  __shared__ T odd[2][4][kPairBlock], even[2][4][kPairBlock];
+  int r, b;
+  MonSlot *slot = mon + block_of(blk, r, b);
+  const ReplicaParams &p = P[r];
+  const ReplicaState &s = S[r];
+  const int cur = first_lane(s.cur_phi ^ (flip & 1));  // phi planes only
+  const int N = p.N, NH = p.NH;
+  const int nby = (N + p.pair_y - 1) / p.pair_y;
+  const int y0 = b % nby * p.pair_y, z0 = b / nby * p.pair_z;
+  const int h = min(p.pair_y, N - y0), tz = min(p.pair_z, N - z0);
+  const int t = threadIdx.x;
+  const int j = (int)__umulhi((uint32_t)t, 0xFFFFFFFFu / NH + 1), xh = t - j * NH;
+  const bool own = j < h + 2, inner = own && j >= 1 && j <= h;
+  const int y = wrapz(y0 - 1 + j, N);
+  const bool low = j == 0, outer = low || j == h + 1;  // rows that face the tile
+  constexpr uint32_t kNone = PhiPlanes<T, W>::kNone;
+  const uint32_t i_own = own ? (uint32_t)y * NH + xh : kNone;
+  const uint32_t i_out =
+      own && outer ? (uint32_t)wrapz(low ? y - 1 : y + 1, N) * NH + xh : kNone;
+  const uint32_t i_inner = inner ? i_own : kNone;
+  const int tu = outer && !low ? t : t + NH, td = low ? t : t - NH;  // rows above, below
+  const double mass = p.mass0 + p.dmassdt * s.t;
+  const double Lambda2 = 0.5 * (2. * 3. + mass);
+  const double lambda = p.lambda, H = p.H, rdtg = p.rdtg;
+  const uint64_t key_e = stream_key(p.base_key, s.sweep_ctr + ctr_off);
+  const uint64_t key_o = stream_key(p.base_key, s.sweep_ctr + ctr_off + 1);
+  const PhiPlanes<T, W> in(p, cur), out(p, cur ^ 1);
+  Tally mt;
+  auto ld4 = [&](int par, uint32_t i, int z, T v[4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int l = 0; l < 4; l++) v[l] = in.template ld<false>(l, par, z, i);
+  };
+  // the half-columns of row position c that hold x + 1 and x - 1 of a site with
+  // x = 2 c + o, as steps from the thread's own slot
+  auto step_up = [&](int o) __attribute__((always_inline)) {
+    return o ? (xh + 1 == NH ? 1 - NH : 1) : 0;
+  };
+  auto step_down = [&](int o) __attribute__((always_inline)) {
+    return o ? 0 : (xh == 0 ? NH - 1 : -1);
+  };
+  T o_next[4], o_far[4], e_old[4], e_far[4], o_out[4], o_outn[4];
+  int z = wrapz(z0 - 1, N);  // plane of step k
+  if (own) {
+    T a[4], c[4];
+    ld4(1, i_own, wrapz(z - 1, N), a);
+    ld4(1, i_own, z, c);
+    ld4(1, i_own, wrapz(z + 1, N), o_next);
+    ld4(0, i_own, z, e_old);
+    if (outer) ld4(1, i_out, z, o_out);
+#pragma unroll
+    for (int l = 0; l < 4; l++) {
+      odd[1][l][t] = a[l];
+      odd[0][l][t] = c[l];
+    }
+  }
+  const bool wave_inner = lanes(inner) != 0;
+  for (int k = 0; k < tz + 2; k++) {
+    const int q = k & 1, zn = wrapz(z + 1, N);
+    // every lane issues the same loads and stores, so that the wait for the
+    // loads at the end of the step leaves the stores in flight
+    const bool more = k < tz + 1;
+    ld4(1, more ? i_own : kNone, wrapz(zn + 1, N), o_far);
+    ld4(0, more ? i_own : kNone, zn, e_far);
+    ld4(1, more ? i_out : kNone, zn, o_outn);
+    __syncthreads();
+    T e_new[4], o_new[4];
+    const bool mid = k >= 1 && k <= tz;
+    if (own) {
+      const int o = (y + z) & 1;
+      double phi_o[4], heff[4], phi_n[4];
+      const int tp = t + step_up(o), tm = t + step_down(o);
+#pragma unroll
+      for (int l = 0; l < 4; l++) {
+        double up = (double)odd[q][l][tu], dn = (double)odd[q][l][td];
+        if (outer) (low ? dn : up) = (double)o_out[l];
+        heff[l] = ((double)odd[q][l][tp] + (double)odd[q][l][tm]) + (up + dn) +
+                  ((double)o_next[l] + (double)odd[q ^ 1][l][t]);
+        phi_o[l] = (double)e_old[l];
+      }
+      Xoro g = xoro_seeded(site_key(key_e, ((uint64_t)z * N + y) * N + 2 * xh + o));
+      hb_decide(phi_o, heff, Lambda2, lambda, H, rdtg, g, phi_n, mt, inner && mid);
+#pragma unroll
+      for (int l = 0; l < 4; l++) e_new[l] = (T)phi_n[l];
+    }
+#pragma unroll
+    for (int l = 0; l < 4; l++) out.template st<false>(l, 0, z, mid ? i_inner : kNone, e_new[l]);
+    const int zo = wrapz(z - 1, N);
+    if (k >= 2 && wave_inner && own) {
+      const int oo = (1 + y + zo) & 1;
+      const int up = t + step_up(oo), dn = t + step_down(oo);
+      double phi_o[4], heff[4], phi_n[4];
+#pragma unroll
+      for (int l = 0; l < 4; l++) {
+        heff[l] = ((double)even[q ^ 1][l][up] + (double)even[q ^ 1][l][dn]) +
+                  ((double)even[q ^ 1][l][tu] + (double)even[q ^ 1][l][td]) +
+                  ((double)e_new[l] + (double)even[q][l][t]);
+        phi_o[l] = (double)odd[q ^ 1][l][t];
+      }
+      Xoro go = xoro_seeded(site_key(key_o, ((uint64_t)zo * N + y) * N + 2 * xh + oo));
+      hb_decide(phi_o, heff, Lambda2, lambda, H, rdtg, go, phi_n, mt, inner);
+#pragma unroll
+      for (int l = 0; l < 4; l++) o_new[l] = (T)phi_n[l];
+    }
+#pragma unroll
+    for (int l = 0; l < 4; l++)
+      out.template st<false>(l, 1, zo, k >= 2 ? i_inner : kNone, o_new[l]);
+    // the slots of the next step: read by no other thread until the barrier
+    // (the even ones of two planes ago, the odd ones of the last plane)
+    if (own) {
+#pragma unroll
+      for (int l = 0; l < 4; l++) {
+        even[q][l][t] = e_new[l];
+        odd[q ^ 1][l][t] = o_next[l];
+      }
+    }
+#pragma unroll
+    for (int l = 0; l < 4; l++) {
+      o_next[l] = o_far[l];
+      e_old[l] = e_far[l];
+      o_out[l] = o_outn[l];
+    }
+    z = zn;
+  }
+  block_monitor_add<kPairBlock>(slot, mt);
 }
 
 // One parity of EulerLangevinHB::step (Stepper.cxx:309-386), in place, by
@@ -1895,10 +2045,19 @@ void launch_hb_phi(bool fp32, const Plan &plan, const ReplicaParams *P, ReplicaS
                ctr_off, flip, mon);
 }
 
+void launch_hb_sweep(bool fp32, const Plan &plan, const ReplicaParams *P, ReplicaState *S,
+                     int ctr_off, int flip, MonSlot *mon, hipStream_t st) {
+#define LGV_SWEEP(TT, WW) \
+  k_hb_sweep<TT, WW><<<plan.nblocks, kPairBlock, 0, st>>>(P, S, plan.blocks, ctr_off, flip, mon)
+  if (fp32) { if (plan.wide) LGV_SWEEP(float, true); else LGV_SWEEP(float, false); }
+  else { if (plan.wide) LGV_SWEEP(double, true); else LGV_SWEEP(double, false); }
+#undef LGV_SWEEP
+}
+
 void launch_hb_brick(bool fp32, const Plan &plan, int lds, const ReplicaParams *P,
                      ReplicaState *S, int ctr_off, int flip, MonSlot *mon, hipStream_t st) {
 #define LGV_BRICK(TT, WW) \
-  k_hb_brick<TT, WW><<<plan.nblocks, kBrickBlock, lds, st>>>(P, S, plan.blocks, ctr_off, flip, mon)
+  k_hb_brick<TT, WW><<<plan.nblocks, kPairBlock, lds, st>>>(P, S, plan.blocks, ctr_off, flip, mon)
   if (fp32) { if (plan.wide) LGV_BRICK(float, true); else LGV_BRICK(float, false); }
   else { if (plan.wide) LGV_BRICK(double, true); else LGV_BRICK(double, false); }
 #undef LGV_BRICK

@@ -62,6 +62,7 @@ EXPORTS = [
     "lgv_em_last_error", "lgv_em_create", "lgv_em_set_stream", "lgv_em_forward",
     "lgv_em_backward", "lgv_em_destroy", "lgv_em_series", "lgv_em_step",
     "lgv_em_step_noalloc", "lgv_set_phi_kernel", "lgv_get_phi_kernel",
+    "lgv_get_phi_pairs",
 ]
 
 # lgv_set_phi_kernel values
@@ -308,6 +309,13 @@ class Context:
         """The phi half-sweep kernel in use: PHI_SITE or PHI_MARCH."""
         k = C.c_int()
         _check(lib().lgv_get_phi_kernel(self.h, C.byref(k)))
+        return k.value
+
+    def phi_pairs(self):
+        """How pairs of phi sweeps run: 0 half-sweeps, 1 bricks, 2 the march
+        of both parities."""
+        k = C.c_int()
+        _check(lib().lgv_get_phi_pairs(self.h, C.byref(k)))
         return k.value
 
     def timing_enable(self, enable=True):

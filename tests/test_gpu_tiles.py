@@ -106,46 +106,52 @@ def test_phi_march_of_a_mixed_batch_keeps_results(L):
         one.close()
 
 
-# Two-parity phi launches against half-sweeps.  6: the brick is the lattice, so
-# its facing rows are its own; 22, 34, 50: short last bricks and rows that leave
-# lanes of the last wavefront without a site; 64: one brick per CU
-@pytest.mark.parametrize("N,prec", [(6, 0), (6, 1), (22, 0), (34, 1), (50, 0), (64, 0), (64, 1)])
+# Launches of both parities (1: bricks, 2: the march) against half-sweeps.  6:
+# the block's rows are the lattice, so its facing rows are its own; 22, 34, 50:
+# short last blocks and wavefronts with lanes that have no site or straddle
+# rows; 64: one brick per CU; 130: rows of 65, 13 of them a block
+@pytest.mark.parametrize("N,prec", [(6, 0), (6, 1), (22, 0), (34, 1), (50, 0), (64, 0), (64, 1),
+                                    (130, 0)])
 @pytest.mark.parametrize("scounts", [(2, 3), (3, 1)])  # 3: a pair and one in place
 def test_two_parity_launches_keep_results(L, monkeypatch, N, prec, scounts):
-    print(f"[gpu-test] bricks {N} {prec} {scounts}", flush=True)
+    print(f"[gpu-test] both parities {N} {prec} {scounts}", flush=True)
     u = np.random.default_rng(N).normal(size=(N, N, N, 10)) * 0.5
     out = []
-    for bricks in ("0", "1"):
-        monkeypatch.setenv("LGV_PHI_BRICKS", bricks)
+    for pairs, wide in (("0", "0"), ("1", "0"), ("1", "1"), ("2", "0"), ("2", "1")):
+        monkeypatch.setenv("LGV_PHI_PAIRS", pairs)
+        monkeypatch.setenv("LGV_FORCE_WIDE", wide)
         ctx = L.Context(L.model_params(N, seed=5), precision=prec, scounts=scounts)
         ctx.set_field(u)
         ctx.run(0.04, 2)
-        ctx.set_phi_kernel(L.PHI_SITE)  # folds the counts, keeps the kernel
+        ctx.set_phi_kernel(L.PHI_SITE)  # folds the counts, no pairs
         ctx.hb_phi_step(0.01)
+        ctx.set_phi_kernel(L.PHI_AUTO)
         ctx.run(0.04, 1)
         out.append((ctx.get_field(), ctx.monitors(), ctx.rng_state().sweep_ctr))
         ctx.close()
-    np.testing.assert_array_equal(out[0][0], out[1][0])
-    assert out[0][2] == out[1][2]
-    for k in ("down_counts", "up_counts", "up_yes", "up_no"):
-        assert out[0][1]["phi"][k] == out[1][1]["phi"][k], k
+    for got in out[1:]:
+        np.testing.assert_array_equal(out[0][0], got[0])
+        assert out[0][2] == got[2]
+        for k in ("down_counts", "up_counts", "up_yes", "up_no"):
+            assert out[0][1]["phi"][k] == got[1]["phi"][k], k
 
 
 def test_two_parity_launches_of_a_batch_keep_results(L, monkeypatch):
-    print("[gpu-test] bricks, batch", flush=True)
+    print("[gpu-test] both parities, batch", flush=True)
     sizes = [34, 8, 8, 8, 22]
     out = []
-    for bricks in ("0", "1"):
-        monkeypatch.setenv("LGV_PHI_BRICKS", bricks)
+    for pairs in ("0", "1", "2"):
+        monkeypatch.setenv("LGV_PHI_PAIRS", pairs)
         ctx = L.Context([L.model_params(N, seed=7 + i) for i, N in enumerate(sizes)])
         for r, N in enumerate(sizes):
             ctx.set_field(np.random.default_rng(r).normal(size=(N, N, N, 10)) * 0.5, r)
         ctx.run(0.04, 2)
         out.append([(ctx.get_field(r), ctx.monitors(r)["phi"]["up_yes"]) for r in range(5)])
         ctx.close()
-    for r in range(5):
-        np.testing.assert_array_equal(out[0][r][0], out[1][r][0], err_msg=str(r))
-        assert out[0][r][1] == out[1][r][1]
+    for got in out[1:]:
+        for r in range(5):
+            np.testing.assert_array_equal(out[0][r][0], got[r][0], err_msg=str(r))
+            assert out[0][r][1] == got[r][1]
 
 
 def test_sweep_counters_of_mixed_calls(L):
