@@ -380,6 +380,7 @@ def run_batched(L, fp32, steps, warmup, tune=True, graph=True, graph_steps=10,
     el = time.perf_counter() - t0
     value = sites * steps / el
     march = ctx.phi_kernel() == L.PHI_MARCH
+    pairs = ctx.phi_pairs()
     ctx.close()
     seq_el = 0.0
     for p in reps:
@@ -398,7 +399,7 @@ def run_batched(L, fp32, steps, warmup, tune=True, graph=True, graph_steps=10,
         seq_el += time.perf_counter() - t0
         c1.close()
     seq_value = sites * steps / seq_el
-    alg, kern, _ = tables(fp32, march, ctx.phi_pairs())
+    alg, kern, _ = tables(fp32, march, pairs)
     return {
         "value": value, "ms_per_step": el * 1e3 / steps, "steps": steps, "warmup": warmup,
         "dtype": "f32-storage/f64-arith" if fp32 else "f64",
