@@ -36,7 +36,8 @@ KERNEL = {"ideal": "k_ideal_fused", "phi": "k_hb_march", "charge": "k_charge_mar
 # Per site-update with one pass per dependency level of the reference
 # (12 phi half-sweeps of 48 B, 6 charge sub-sweeps of 96 B): 3*160 + 12*48 + 6*96.
 ALG_BYTES_PER_SITE_UPDATE = 1632
-# The same for this schedule: 3 ideal, 12 phi and 3 charge launches.
+# The same for this schedule: 3 ideal, 12 phi and 3 charge launches (tables: with
+# launches of both parities).
 SCHEDULE_BYTES_PER_SITE_UPDATE = 3 * 160 + 12 * 48 + 3 * 96  # 1344
 SCHEDULE_BYTES_PER_SITE_UPDATE_FP32 = SCHEDULE_BYTES_PER_SITE_UPDATE
 # HBM bytes per launch per site measured with rocprofv3 --pmc FETCH_SIZE and

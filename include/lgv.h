@@ -149,7 +149,8 @@ int lgv_measure(lgv_ctx *ctx, int replica, double *wall, double *wallphase,
  * timing, the charge sweep beside the phi sweeps where the context does so;
  * a timed step keeps one stream).  Enabling resets the totals; while
  * enabled, lgv_run issues kernels directly instead of replaying a graph.
- * The single sweeps (lgv_ideal_step, ...) are timed whenever enabled. */
+ * The single sweeps (lgv_ideal_step, ...) are timed whenever enabled.  Phi
+ * launches are counted in half-sweeps: one of both parities counts as two. */
 enum { LGV_CLASS_IDEAL = 0, LGV_CLASS_PHI = 1, LGV_CLASS_CHARGE = 2, LGV_CLASS_ENERGY = 3,
        LGV_NCLASS = 4 };
 int lgv_timing_enable(lgv_ctx *ctx, int enable);

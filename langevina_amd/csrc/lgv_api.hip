@@ -487,10 +487,10 @@ bool resolve_bricks(lgv_ctx *c) {
 // one block per CU, each of TZ planes and about five planes' time for the two
 // more that it decides, its start and its end (256^3 FP64, per half-sweep: TZ
 // 52, one round of 215 blocks, 131 us; 24, two, 133; 16, three, 142; 8 160).
-// False: rows that are too long, or sides below kPairMarchSide.
+// False: the rows are too long.
 bool resolve_pair_march(lgv_ctx *c) {
   for (ReplicaParams &p : c->hp) {
-    if (kPairBlock / p.NH < 3 || p.N < kPairMarchSide) return false;
+    if (kPairBlock / p.NH < 3) return false;
     p.pair_y = std::min(kPairBlock / p.NH - 2, p.N);
   }
   int best = 0;
@@ -947,7 +947,8 @@ int lgv_create(const lgv_config *cfg, lgv_ctx **out) {
   c->noise.resize(c->nrep);
   const size_t esz = c->fp32 ? sizeof(float) : sizeof(double);
   std::vector<PlanWork> whalf, wfull;
-  uint64_t buffer_bytes = 0;  // one buffer: 10 planes x 2 parities
+  uint64_t buffer_bytes = 0;
+  int minN = kMaxN;  // one buffer: 10 planes x 2 parities
   std::vector<ReplicaState> hs(c->nrep);
   for (int r = 0; r < c->nrep; r++) {
     const lgv_model_params &m = c->mp[r];
@@ -984,6 +985,7 @@ int lgv_create(const lgv_config *cfg, lgv_ctx **out) {
     // test hook: LGV_FORCE_WIDE=1 runs the 64-bit-offset kernels on any size
     if (const char *fw = getenv("LGV_FORCE_WIDE")) c->wide = c->wide || atoi(fw) != 0;
     c->maxN = std::max(c->maxN, N);
+    minN = std::min(minN, N);
   }
   c->buffer_bytes = buffer_bytes;
   c->phi_march_auto = buffer_bytes / (10 * esz) >= kMarchSites;
@@ -1010,7 +1012,8 @@ int lgv_create(const lgv_config *cfg, lgv_ctx **out) {
   }
   const uint64_t sites = buffer_bytes / (10 * esz);
   if (sites < kBrickSites) c->two_parity = TwoParity::kBricks;
-  if (!c->fp32 && sites >= kPairMarchSites) c->two_parity = TwoParity::kMarch;
+  if (!c->fp32 && sites >= kPairMarchSites && minN >= kPairMarchSide)
+    c->two_parity = TwoParity::kMarch;
   // test hook: LGV_PHI_PAIRS=0/1/2 takes no launches of both parities, bricks,
   // the march
   if (const char *pb = getenv("LGV_PHI_PAIRS"))

@@ -2,9 +2,10 @@
 //
 // Blocks are mapped to replicas through a launch plan, so one launch steps
 // many independent lattices.  Fields live in the red-black
-// structure-of-arrays layout of lgv_device.h, double-buffered: the
-// Metropolis sweeps update the live buffer in place (a checkerboard never
-// reads what it writes), the fused ideal substep writes the other buffer.
+// structure-of-arrays layout of lgv_device.h, double-buffered: the phi
+// half-sweeps update the live buffer in place (a checkerboard never reads what
+// it writes); the phi launches of both parities, the charge launches and the
+// fused ideal substep write the other buffer.
 // All FP arithmetic is FP64 (FP32 storage is widened on load and rounded
 // on store).  The Metropolis sweeps follow the reference's expression order
 // bit for bit; the library is built with -ffp-contract=off.
