@@ -516,13 +516,16 @@ int build_pair_plan(lgv_ctx *c) {
     c->two_parity = TwoParity::kNone;
   if (c->two_parity == TwoParity::kNone) return LGV_OK;
   std::vector<PlanWork> work;
-  bool wide = c->wide;
+  bool wide = c->wide, stream = c->buffer_bytes > 2 * kCacheBytes;
   for (const ReplicaParams &p : c->hp) {
     wide = wide || 2 * (uint64_t)p.half * (c->fp32 ? 4 : 8) > 0xFFFFFFFFull;
+    stream = stream && whole_rows(c, p.NH, p.NH, 64);
     const int64_t plane = (p.N + p.pair_y - 1) / p.pair_y;
     work.push_back({plane * ((p.N + p.pair_z - 1) / p.pair_z), (double)plane});
   }
-  return build_plan(c->plan_pair, work, wide);
+  const int rc = build_plan(c->plan_pair, work, wide);
+  c->plan_pair.stream = stream;
+  return rc;
 }
 
 // Whether the x sub-sweeps of every replica run whole rows per wavefront

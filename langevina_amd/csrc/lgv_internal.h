@@ -121,7 +121,7 @@ struct Plan {
   std::vector<int> first;  // host copy of blocks.first
 };
 
-// The phi march and the ideal kernel write their outputs with non-temporal
+// The phi marches and the ideal kernel write their outputs with non-temporal
 // stores where the outputs are next read by a later launch, after planes that
 // together exceed the last-level cache have been swept, so that caching them
 // only evicts lines that neighbouring tiles still read; and only where a tile's
@@ -134,6 +134,11 @@ struct Plan {
 // halves; FP64 208^3 94.5 -> 90.8 us, 224^3 119 -> 106, 256^3 170 -> 148,
 // FP32 384^3 302 -> 291, but 256^3 FP32 (phi planes of just 256 MB) 86 -> 92,
 // 280^3 FP64 (rows of 8.75 lines) 228 -> 242, 320^3 in tiles of 54 342 -> 394.
+// k_hb_sweep: fields above twice the cache, rows of whole 64-byte halves; its own
+// time changes little (256^3 128 -> 127 us, 224^3 87 -> 89), but the ideal and the
+// charge kernel after it find more of their planes (256^3 551 -> 537, 329 -> 322;
+// whole steps 192^3 1889 -> 1862, 224^3 3043 -> 3008, 256^3 4156 -> 4091; 160^3
+// 1166 -> 1173, 200^3, rows of 6.25 lines, 2415 -> 2427).
 constexpr uint64_t kCacheBytes = 256ull << 20;
 
 // From this many sites on (all replicas) the phi half-sweeps run the z-march:

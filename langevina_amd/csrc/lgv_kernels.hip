@@ -592,7 +592,7 @@ __global__ __launch_bounds__(kPairBlock) void k_hb_brick(const ReplicaParams *__
 // 28 decisions a SIMD lane), the rest the barrier's skew and LDS reads.  Whole
 // rows need no ring in x; 16 wavefronts, of which a facing row's have half the
 // work, spread evenly over the four SIMDs.
-template <typename T, bool W>
+template <typename T, bool W, bool NTS>
 __global__ __launch_bounds__(kPairBlock) void k_hb_sweep(const ReplicaParams *__restrict__ P,
                                                           const ReplicaState *__restrict__ S,
                                                           LaunchBlocks blk, int ctr_off, int flip,
@@ -682,7 +682,7 @@ __global__ __launch_bounds__(kPairBlock) void k_hb_sweep(const ReplicaParams *__
       for (int l = 0; l < 4; l++) e_new[l] = (T)phi_n[l];
     }
 #pragma unroll
-    for (int l = 0; l < 4; l++) out.template st<false>(l, 0, z, mid ? i_inner : kNone, e_new[l]);
+    for (int l = 0; l < 4; l++) out.template st<NTS>(l, 0, z, mid ? i_inner : kNone, e_new[l]);
     const int zo = wrapz(z - 1, N);
     if (k >= 2 && wave_inner && own) {
       const int oo = (1 + y + zo) & 1;
@@ -702,7 +702,7 @@ __global__ __launch_bounds__(kPairBlock) void k_hb_sweep(const ReplicaParams *__
     }
 #pragma unroll
     for (int l = 0; l < 4; l++)
-      out.template st<false>(l, 1, zo, k >= 2 ? i_inner : kNone, o_new[l]);
+      out.template st<NTS>(l, 1, zo, k >= 2 ? i_inner : kNone, o_new[l]);
     // the slots of the next step: read by no other thread until the barrier
     // (the even ones of two planes ago, the odd ones of the last plane)
     if (own) {
@@ -2048,10 +2048,11 @@ void launch_hb_phi(bool fp32, const Plan &plan, const ReplicaParams *P, ReplicaS
 
 void launch_hb_sweep(bool fp32, const Plan &plan, const ReplicaParams *P, ReplicaState *S,
                      int ctr_off, int flip, MonSlot *mon, hipStream_t st) {
-#define LGV_SWEEP(TT, WW) \
-  k_hb_sweep<TT, WW><<<plan.nblocks, kPairBlock, 0, st>>>(P, S, plan.blocks, ctr_off, flip, mon)
-  if (fp32) { if (plan.wide) LGV_SWEEP(float, true); else LGV_SWEEP(float, false); }
-  else { if (plan.wide) LGV_SWEEP(double, true); else LGV_SWEEP(double, false); }
+#define LGV_SWEEP(TT, WW, SS) \
+  k_hb_sweep<TT, WW, SS><<<plan.nblocks, kPairBlock, 0, st>>>(P, S, plan.blocks, ctr_off, flip, mon)
+  if (fp32) { if (plan.wide) LGV_SWEEP(float, true, false); else LGV_SWEEP(float, false, false); }
+  else if (plan.stream) { if (plan.wide) LGV_SWEEP(double, true, true); else LGV_SWEEP(double, false, true); }
+  else { if (plan.wide) LGV_SWEEP(double, true, false); else LGV_SWEEP(double, false, false); }
 #undef LGV_SWEEP
 }
 

@@ -68,17 +68,18 @@ def test_default_tiles_of_a_mixed_batch_keep_results(L):
 def test_phi_kernels_agree_on_default_tiles(L, N, prec):
     print(f"[gpu-test] phi kernels {N} {prec}", flush=True)
     u = np.random.default_rng(N).normal(size=(N, N, N, 10)) * 0.5
-    out = []
-    for kernel in (L.PHI_SITE, L.PHI_MARCH):
+    ref = None
+    for kernel in (L.PHI_SITE, L.PHI_MARCH, L.PHI_AUTO):
         ctx = L.Context(L.model_params(N, seed=5), precision=prec)
         ctx.set_phi_kernel(kernel)
         ctx.set_field(u)
         ctx.run(0.04, 1)
-        out.append((ctx.get_field(), ctx.monitors()["phi"]))
+        got, mon = ctx.get_field(), ctx.monitors()["phi"]
         ctx.close()
-    np.testing.assert_array_equal(out[0][0], out[1][0])
-    for k in ("down_counts", "up_counts", "up_yes", "up_no"):
-        assert out[0][1][k] == out[1][1][k], k
+        ref = ref or (got, mon)
+        np.testing.assert_array_equal(ref[0], got)
+        for k in ("down_counts", "up_counts", "up_yes", "up_no"):
+            assert ref[1][k] == mon[k], k
 
 
 def test_phi_march_of_a_mixed_batch_keeps_results(L):
