@@ -45,9 +45,9 @@ SCHEDULE_BYTES_PER_SITE_UPDATE_FP32 = SCHEDULE_BYTES_PER_SITE_UPDATE
 # copy-kernel calibration (bench.py --calibrate-copy); the summary of those
 # runs is profiles/modelg_256_hbm_traffic.md.
 MEASURED_TRAFFIC = {
-    ("k_ideal_fused", "fp64", 256): (97.39, 80.00),
+    ("k_ideal_fused", "fp64", 256): (97.56, 80.00),
     # half of a launch of both parities
-    ("k_hb_sweep", "fp64", 256): (19.63, 16.00),
+    ("k_hb_sweep", "fp64", 256): (18.90, 16.00),
     ("k_hb_march", "fp64", 256): (37.98, 16.01),
     ("k_charge_march", "fp64", 256): (52.05, 48.19),
     ("k_ideal_fused", "fp32", 256): (44.88, 40.00),

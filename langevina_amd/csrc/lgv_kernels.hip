@@ -585,13 +585,13 @@ __global__ __launch_bounds__(kPairBlock) void k_hb_brick(const ReplicaParams *__
 // from the even ones.  In LDS lie the odd values of this plane and the last one
 // and the new even values of the last two; one barrier per plane.
 // It reads and writes each value once where two half-sweeps read both parities
-// twice (counted at 256^3 FP64: 12 -> 8 bytes per component and site), for
+// twice (counted at 256^3 FP64: 70 bytes a site, the half-sweeps 108), for
 // which it decides the even sites of the facing rows and of two planes a chunk
-// twice.  256^3 FP64: 257 us for both parities (two half-sweeps 295), 4.9 us a
+// twice.  256^3 FP64: 256 us for both parities (two half-sweeps 295), 4.9 us a
 // plane of a block; about 60 % of that are vector instructions (235 a decision,
-// 28 decisions a SIMD lane), the rest the barrier's skew and LDS reads.  Whole
-// rows need no ring in x; 16 wavefronts, of which a facing row's have half the
-// work, spread evenly over the four SIMDs.
+// 28 wavefronts' decisions on four SIMDs), the rest the barrier's skew and LDS
+// reads.  Whole rows need no ring in x; the 16 wavefronts, of which a facing
+// row's have half the work, spread evenly over the SIMDs.
 template <typename T, bool W, bool NTS>
 __global__ __launch_bounds__(kPairBlock) void k_hb_sweep(const ReplicaParams *__restrict__ P,
                                                           const ReplicaState *__restrict__ S,
