@@ -46,7 +46,7 @@ struct ReplicaState {
 };
 
 // The tile fields of ReplicaParams hold what a launch uses: the caller's
-// request, or where that is 0 the choice of the rules below (resolve_tiles in
+// request, or where that is 0 the choice of the rules (the resolve_ functions in
 // lgv_api.hip, by replica size, storage type and the blocks of the launch).
 
 // Tile of the fused ideal kernel: TXH half-columns x TY rows in x-y,
