@@ -90,8 +90,8 @@ enum class TwoParity { kNone, kBricks, kMarch };
 struct lgv_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
-  // the charge sweep of a step runs on stream2, concurrently with the phi
-  // sweeps that follow the last ideal substep (see enqueue_step)
+  // the charge sweep of a step and the phi sweeps that follow the last ideal
+  // substep run concurrently, one of them on stream2 (see enqueue_step)
   hipStream_t stream2 = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   bool overlap = true;
@@ -711,15 +711,13 @@ int enqueue_ideal(lgv_ctx *c, int off, int flip) {
 // 256^3 116, 86.
 bool use_march(const lgv_ctx *c) { return c->phi_march; }
 const Plan &hb_plan(const lgv_ctx *c) { return use_march(c) ? c->plan_hb : c->plan_half; }
-int enqueue_hb(lgv_ctx *c, int off, int flip) {
+int enqueue_hb(lgv_ctx *c, int off, int flip, hipStream_t st) {
   for (int ieo = 0; ieo < 2; ieo++) {
     Timed tm(c, LGV_CLASS_PHI);
     if (use_march(c))
-      launch_hb_march(c->fp32, c->plan_hb, c->dP, c->dS, ieo, off + ieo, flip, c->mon_phi,
-                      c->stream);
+      launch_hb_march(c->fp32, c->plan_hb, c->dP, c->dS, ieo, off + ieo, flip, c->mon_phi, st);
     else
-      launch_hb_phi(c->fp32, c->plan_half, c->dP, c->dS, ieo, off + ieo, flip, c->mon_phi,
-                    c->stream);
+      launch_hb_phi(c->fp32, c->plan_half, c->dP, c->dS, ieo, off + ieo, flip, c->mon_phi, st);
   }
   return 0;  // in place
 }
@@ -727,20 +725,20 @@ int enqueue_hb(lgv_ctx *c, int off, int flip) {
 // n sweeps of EulerLangevinHB::step: pairs of out-of-place two-parity launches
 // where the context has them (a pair leaves the live buffer where it was, as
 // the in-place sweeps do), the others in place.
-void enqueue_phi_sweeps(lgv_ctx *c, int n, int off, int flip) {
+void enqueue_phi_sweeps(lgv_ctx *c, int n, int off, int flip, hipStream_t st) {
   int i = 0;
   if (c->phi_pairs) {
     for (; i < n - n % 2; i++) {
       Timed tm(c, LGV_CLASS_PHI, 2);  // two half-sweeps
       if (c->two_parity == TwoParity::kMarch)
         launch_hb_sweep(c->fp32, c->plan_pair, c->dP, c->dS, off + 2 * i, flip ^ (i & 1),
-                        c->mon_pair, c->stream);
+                        c->mon_pair, st);
       else
         launch_hb_brick(c->fp32, c->plan_pair, c->brick_lds, c->dP, c->dS, off + 2 * i,
-                        flip ^ (i & 1), c->mon_pair, c->stream);
+                        flip ^ (i & 1), c->mon_pair, st);
     }
   }
-  for (; i < n; i++) enqueue_hb(c, off + 2 * i, flip);
+  for (; i < n; i++) enqueue_hb(c, off + 2 * i, flip, st);
 }
 
 // ModelGChargeHB::step: the shuffle (counter off, drawn by every charge
@@ -774,44 +772,48 @@ void settle(lgv_ctx *c) {
 }
 
 // PV2HBSplit::step (Stepper.cxx:542-580); returns the number of stream
-// counters consumed, and those taken from the host's count.  The charge sweep reads and writes only the charges
-// and the phi sweeps only phi, so after the last ideal substep the charge
-// sweep runs on the second stream while the phi sweeps run on the first
+// counters consumed, and those taken from the host's count.  The charge sweep
+// reads and writes only the charges and the phi sweeps only phi, so after the
+// last ideal substep the two run side by side on the context's two streams
 // (fork and join by events, which a graph capture records as well).  Every
 // sweep keeps its counter (random streams) and its monitor slots, so the
 // result is the sequential one bit for bit.  Contexts of one lattice whose
 // fields exceed 600 MiB keep the sequential order (their launches fill the
-// GPU on their own), and so do timed steps (events on one stream).  flip
+// GPU on their own), and so do timed steps (events on one stream).  On the
+// stream the charge sweep, the longer of the two, follows the ideal launch
+// without an event's wait and the phi sweeps take the second stream (steps
+// with the charge sweep on the second stream -> on the first: 16^3 100 -> 92
+// us, 64^3 155 -> 144, 100^3 334 -> 341 but three contexts at once 310 -> 309,
+// 128^3 655 -> 637, 192^3 1896 -> 1874); in a graph the phi sweeps follow it
+// and the charge sweep branches off (64^3 145 -> 138, 128^3 646 -> 626).  flip
 // returns the step's net live-buffer flip.
-int enqueue_step(lgv_ctx *c, int &flip) {
+int enqueue_step(lgv_ctx *c, int &flip, bool capture = false) {
   int off = take_state(c, flip);
-  bool charge_queued = false, join_event = false;
   c->timing_now = c->timing && c->timing_ctr++ % c->timing_every == 0;
   // a timed step keeps one stream (events on it bracket every launch)
-  const bool fork = c->overlap && !c->timing_now && !c->onlydiffuse && !c->nodiffuse;
+  const bool overlap = c->overlap && !c->timing_now && !c->onlydiffuse && !c->nodiffuse;
+  bool forked = false, join_event = false;
+  hipStream_t phi = c->stream, charge = c->stream;
+  if (overlap) (capture ? charge : phi) = c->stream2;
   if (!c->onlydiffuse) {
     for (unsigned i1 = 0; i1 < c->s1; i1++) {
       flip ^= enqueue_ideal(c, off, flip);
       off += 1;
-      if (fork && i1 + 1 == c->s1 && hipEventRecord(c->ev_fork, c->stream) == hipSuccess &&
-          hipStreamWaitEvent(c->stream2, c->ev_fork, 0) == hipSuccess) {
-        // the phi sweeps that follow do not touch the charge bit of flip
-        flip ^= enqueue_charge(c, off + 2 * (int)c->s0, flip, c->stream2);
-        charge_queued = true;
-        join_event = hipEventRecord(c->ev_join, c->stream2) == hipSuccess;
-      }
-      enqueue_phi_sweeps(c, (int)c->s0, off, flip);
+      forked = overlap && i1 + 1 == c->s1 && hipEventRecord(c->ev_fork, c->stream) == hipSuccess &&
+               hipStreamWaitEvent(c->stream2, c->ev_fork, 0) == hipSuccess;
+      // the phi sweeps that follow do not touch the charge bit of flip
+      if (forked) flip ^= enqueue_charge(c, off + 2 * (int)c->s0, flip, charge);
+      enqueue_phi_sweeps(c, (int)c->s0, off, flip, forked ? phi : c->stream);
       off += 2 * (int)c->s0;
+      if (forked) join_event = hipEventRecord(c->ev_join, c->stream2) == hipSuccess;
     }
   }
   if (!c->nodiffuse) {
-    if (!charge_queued) {
-      flip ^= enqueue_charge(c, off, flip, c->stream);
-    } else if (!join_event || hipStreamWaitEvent(c->stream, c->ev_join, 0) != hipSuccess) {
-      (void)hipStreamSynchronize(c->stream2);  // join on the host instead
-    }
+    if (!forked) flip ^= enqueue_charge(c, off, flip, c->stream);
     off += 7;
   }
+  if (forked && (!join_event || hipStreamWaitEvent(c->stream, c->ev_join, 0) != hipSuccess))
+    (void)hipStreamSynchronize(c->stream2);  // join on the host instead
   return off;
 }
 
@@ -1237,7 +1239,7 @@ int lgv_run(lgv_ctx *c, double dt, int nsteps) {
       HIPCHECK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
       for (int i = 0; i < k; i++) {
         int flip;
-        const int n = enqueue_step(c, flip);
+        const int n = enqueue_step(c, flip, true);
         launch_advance(c->nrep, c->dS, dt, 1, (uint64_t)n, flip, c->stream);
       }
       HIPCHECK(hipStreamEndCapture(c->stream, &graph));
@@ -1278,7 +1280,7 @@ int lgv_hb_phi_step(lgv_ctx *c, double dt) {
   if (rc) return rc;
   c->timing_now = c->timing;  // single sweeps are always timed
   if (c->ctr >> 20) settle(c);
-  c->flip ^= enqueue_hb(c, (int)c->ctr, c->flip);
+  c->flip ^= enqueue_hb(c, (int)c->ctr, c->flip, c->stream);
   c->ctr += 2;
   return check_launch();
 }
