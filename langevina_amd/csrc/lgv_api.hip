@@ -777,9 +777,9 @@ void settle(lgv_ctx *c) {
 // last ideal substep the two run side by side on the context's two streams
 // (fork and join by events, which a graph capture records as well).  Every
 // sweep keeps its counter (random streams) and its monitor slots, so the
-// result is the sequential one bit for bit.  Contexts of one lattice whose
-// fields exceed 600 MiB keep the sequential order (their launches fill the
-// GPU on their own), and so do timed steps (events on one stream).  On the
+// result is the sequential one bit for bit.  Contexts of one large lattice
+// (kOverlapBytes) keep the sequential order (their launches fill the GPU on
+// their own), and so do timed steps (events on one stream).  On the
 // stream the charge sweep, the longer of the two, follows the ideal launch
 // without an event's wait and the phi sweeps take the second stream (steps
 // with the charge sweep on the second stream -> on the first: 16^3 100 -> 92
@@ -1001,13 +1001,6 @@ int lgv_create(const lgv_config *cfg, lgv_ctx **out) {
     if (!c->fp32) c->phi_march_auto = c->nt_stores;
   }
   c->phi_march = c->phi_march_auto;
-  // one lattice whose launches each fill the GPU many times over gains
-  // nothing from running the charge sweep beside the phi sweeps (256^3:
-  // 1 % slower); smaller and batched lattices do (128^3 FP64 2.53e9 ->
-  // 2.67e9 site-updates/s, the 96-replica FP32 batch +2 %)
-  c->overlap = !(cfg->nreplicas == 1 && buffer_bytes > kOverlapBytes);
-  // test hook: LGV_OVERLAP=0/1 forces the sequential / concurrent order
-  if (const char *ov = getenv("LGV_OVERLAP")) c->overlap = atoi(ov) != 0;
   // test hook: LGV_PHI_KERNEL=site/march forces the phi half-sweep kernel
   if (const char *pk = getenv("LGV_PHI_KERNEL")) {
     const std::string k(pk);
@@ -1023,6 +1016,14 @@ int lgv_create(const lgv_config *cfg, lgv_ctx **out) {
   // the march
   if (const char *pb = getenv("LGV_PHI_PAIRS"))
     c->two_parity = (TwoParity)std::min(std::max(atoi(pb), 0), 2);
+  // one lattice whose launches each fill the GPU many times over gains
+  // nothing from running the charge sweep beside the phi sweeps; smaller and
+  // batched lattices do (kOverlapBytes)
+  c->overlap = !(cfg->nreplicas == 1 &&
+                 buffer_bytes > (c->two_parity == TwoParity::kMarch ? kOverlapBytesPairMarch
+                                                                    : kOverlapBytes));
+  // test hook: LGV_OVERLAP=0/1 forces the sequential / concurrent order
+  if (const char *ov = getenv("LGV_OVERLAP")) c->overlap = atoi(ov) != 0;
   HIPCHECK(hipMalloc(&c->dS, c->nrep * sizeof(ReplicaState)));
   HIPCHECK(hipMemcpy(c->dS, hs.data(), c->nrep * sizeof(ReplicaState), hipMemcpyHostToDevice));
   int rc;

@@ -177,8 +177,13 @@ constexpr uint64_t kPairMarchSites = 2900000;
 constexpr int kPairMarchSide = 64;
 
 // A context of one lattice whose fields (one buffer) exceed this keeps the
-// charge sweep after the phi sweeps rather than beside them.
+// charge sweep after the phi sweeps rather than beside them; beside k_hb_sweep,
+// which does not fill the memory system, the charge sweep gains up to more.
+// Steps, after -> beside: 192^3 FP64 1913 -> 1876 us, 224^3 3019 -> 2965, 256^3
+// 4131 -> 4073 (three contexts at once 4106 -> 4114), 300^3 8361 -> 8457; 256^3
+// FP32 2703 -> 2702 (three contexts 2705 -> 2717).
 constexpr uint64_t kOverlapBytes = 600ull << 20;
+constexpr uint64_t kOverlapBytesPairMarch = 1300ull << 20;
 
 // Largest side: N^3 must fit 32-bit site indices.
 constexpr int kMaxN = 1536;

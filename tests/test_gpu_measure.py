@@ -8,10 +8,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.fixture(scope="module")
 def L():
-    import torch
-    if not torch.cuda.is_available():
-        pytest.skip("no GPU")
     import langevina_amd
+    langevina_amd.lib()
     return langevina_amd
 
 
