@@ -206,8 +206,12 @@ int lgv_get_phi_kernel(lgv_ctx *ctx, int *kernel);
 int lgv_get_phi_pairs(lgv_ctx *ctx, int *kernel);
 
 int lgv_synchronize(lgv_ctx *ctx);
-/* Device address of a replica's field storage (10 component planes, each
- * split into even and odd half-lattices) and its element size in bytes. */
+/* Device address of the first of a replica's two field buffers (10 component
+ * planes, each split into even and odd half-lattices) and its element size in
+ * bytes.  It holds the current fields of a new context and after
+ * lgv_set_field on one; ideal launches (all planes) and charge launches
+ * (charge planes) each write the other buffer, so after an odd number of them
+ * the current planes are in the second one, which lgv_get_field reads. */
 int lgv_field_device_ptr(lgv_ctx *ctx, int replica, void **ptr, int *elem_bytes);
 
 /* ------------------------------------------------------------------------

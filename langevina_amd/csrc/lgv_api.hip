@@ -1608,7 +1608,7 @@ int lgv_synchronize(lgv_ctx *c) {
 int lgv_field_device_ptr(lgv_ctx *c, int r, void **ptr, int *elem_bytes) {
   int rc = check_replica(c, r);
   if (rc) return rc;
-  *ptr = c->fields[r];
+  *ptr = c->hp[r].fields[0];
   *elem_bytes = c->fp32 ? 4 : 8;
   return LGV_OK;
 }

@@ -596,3 +596,41 @@ def test_concurrent_charge_sweep_matches_sequential(L, orc, monkeypatch, N, prec
     else:
         ulp = np.spacing(np.abs(lat.u).astype(np.float32)).astype(np.float64)
         assert (np.abs(ref[0] - lat.u) <= 4 * ulp).all()
+
+
+def device_planes(L, ctx, r):
+    """The planes [10][2][z][y][x / 2] at a replica's device address."""
+    import ctypes as C
+    ptr, esz = ctx.field_device_ptr(r)
+    N = ctx.N[r]
+    out = np.empty((10, 2, N, N, N // 2), dtype=f"f{esz}")
+    copy = L.lib().hipMemcpy  # of the runtime that the library is linked to
+    copy.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int]
+    assert copy(out.ctypes.data, ptr, out.nbytes, 2) == 0  # hipMemcpyDeviceToHost
+    return out
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+def test_field_pointer_of_each_replica(L, prec):
+    """Replicas of different sides: the planes at each one's address are its
+    fields, after set_field and after two steps (six ideal and six charge
+    launches, an even number of buffer changes)."""
+    log("field pointer", prec)
+    sizes = [16, 8, 12, 6]
+    ctx = L.Context([L.model_params(N, seed=2 + i, **PAR) for i, N in enumerate(sizes)],
+                    precision=prec)
+    for r, N in enumerate(sizes):
+        u = np.random.default_rng(r).normal(size=(N, N, N, 10))
+        ctx.set_field(u.astype(np.float32).astype(np.float64) if prec else u, r)
+    for steps in (0, 2):
+        if steps:
+            ctx.run(0.04, steps)
+        ctx.synchronize()
+        for r, N in enumerate(sizes):
+            got = device_planes(L, ctx, r)
+            u = ctx.get_field(r)
+            z, y, xh = np.indices((N, N, N // 2))
+            for par in (0, 1):
+                ref = u[z, y, 2 * xh + ((par + y + z) & 1)]
+                np.testing.assert_array_equal(got[:, par], np.moveaxis(ref, 3, 0), err_msg=str(N))
+    ctx.close()
