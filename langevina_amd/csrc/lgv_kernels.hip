@@ -341,8 +341,8 @@ __device__ void block_monitor_add(MonSlot *slot, const Tally &m, double unit = 1
 // precision is within 2e4 of (exp(x) - canonical(u)) 2^32 and its sign decides
 // where |D| > 2^16.  The double draw and the double exp decide the rest (3e-5
 // of the tests; with the earlier band of 1e-3 exp(x), a wavefront went there
-// at every tenth decision).  Lanes that are in `sure` (dS < 0, e >= 1) accept;
-// a NaN does not.
+// at every tenth decision), and for an e that is NaN.  Lanes that are in `sure`
+// (dS < 0, e >= 1) accept; a NaN dS does not.
 // The double test is out of line: inlined at every decision of a sweep
 // kernel its exp makes up a sizeable part of the kernel's code.
 __device__ __attribute__((noinline)) bool accept_exact(uint64_t u, double x) {
@@ -357,7 +357,7 @@ __device__ __forceinline__ uint64_t accept_draw(uint64_t u, float e, uint64_t su
   __asm__("" : "+v"(h));
   const float D = __builtin_fmaf(e, 0x1p32f, -(float)h);
   uint64_t accept = lanes(D > 0.f);
-  const uint64_t near = lanes(fabsf(D) <= 0x1p16f);
+  const uint64_t near = lanes(!(fabsf(D) > 0x1p16f));
   if (__builtin_expect(near != 0, 0)) {
     // the draw rebuilt from h (the same bits), so that u's top half need not
     // be kept beside h
@@ -892,14 +892,18 @@ __global__ __launch_bounds__(kBlock) void k_hb_march(const ReplicaParams *__rest
 // modelg_update_charge_pair (Stepper.cxx:419-441) for one component of one
 // pair, applied as nA + (-q), nB + q; counts the decision when count.
 // The constants of a charge sweep: the proposal width, the divisor d = 2 chi
-// of dS with its rounded reciprocal, and -log2(e) / d in single precision.
+// of dS with its rounded reciprocal, and -log2(e) / d in single precision.  That
+// is NaN, so that the double test decides, where dS d or 1 / d might leave the
+// range of single precision: within 2^-100 .. 2^100 a dS d that overflows is a
+// dS beyond 2^27, and one below 2^-126 a dS below 2^-26.
 struct ChargeK {
   double rms, d, inv;
   float l2;
 };
 __device__ __forceinline__ ChargeK charge_k(double rms, double chi) {
   const double d = 2. * chi, inv = 1. / d;
-  return {rms, d, inv, (float)(-0x1.71547652b82fep+0 * inv)};
+  const bool in_range = d >= 0x1p-100 && d <= 0x1p100;
+  return {rms, d, inv, in_range ? (float)(-0x1.71547652b82fep+0 * inv) : __builtin_nanf("")};
 }
 // x / d from the rounded reciprocal with one Markstein correction: q0 = x *
 // inv, the residual x - q0 d exact with one FMA, q0 + residual * inv rounded

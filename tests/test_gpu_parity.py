@@ -634,3 +634,20 @@ def test_field_pointer_of_each_replica(L, prec):
                 ref = u[z, y, 2 * xh + ((par + y + z) & 1)]
                 np.testing.assert_array_equal(got[:, par], np.moveaxis(ref, 3, 0), err_msg=str(N))
     ctx.close()
+
+
+# chi beyond the range of single precision, where -log2(e) / 2 chi or dS 2 chi
+# is no float
+@pytest.mark.parametrize("chi", [1e-44, 1e-37, 1e-30, 1e30, 1e37, 1e44])
+@pytest.mark.parametrize("N", [6, 16])
+def test_charge_sweep_of_extreme_susceptibilities(L, orc, N, chi):
+    log("charge, chi", chi, N)
+    ctx, lat = make_pair(L, orc, N, seed=7, chi=chi, scale=chi ** 0.5)
+    for dt in (0.04, 0.5):
+        ctx.charge_step(dt)
+        lat.charge_step(dt)
+        np.testing.assert_array_equal(ctx.get_field(), lat.u)
+    m_dev, m_orc = ctx.monitors()["charge"], lat.monitors()["charge"]
+    for k in ("down_counts", "up_counts", "up_yes", "up_no"):
+        assert m_dev[k] == m_orc[k], k
+    ctx.close()
