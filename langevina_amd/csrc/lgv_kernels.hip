@@ -1705,12 +1705,13 @@ __device__ __forceinline__ void site_obs(const T raw[10], double o[25]) {
   double n[4];
   if (phi2 > 100. * DBL_MIN) {
     // f / sigma from the reciprocal with one Markstein correction: the
-    // quotient rounded once, three instructions instead of ten
-    const double inv = 1. / sigma;
+    // quotient rounded once, three instructions instead of ten.  Where phi2
+    // overflows, inv = 0 and the residual takes a finite sigma: f / inf = 0.
+    const double inv = 1. / sigma, finite = fmin(sigma, DBL_MAX);
 #pragma unroll
     for (int l = 0; l < 4; l++) {
       const double q = f[l] * inv;
-      n[l] = fma(fma(-q, sigma, f[l]), inv, q);
+      n[l] = fma(fma(-q, finite, f[l]), inv, q);
     }
   } else {
     n[0] = 1; n[1] = 0; n[2] = 0; n[3] = 0;

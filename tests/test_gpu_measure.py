@@ -80,3 +80,26 @@ def test_walls_of_a_large_lattice(L):
     for d, (own, a, b) in enumerate(((g, h, k), (h, g, k), (k, g, h))):
         np.testing.assert_allclose(wall[d, 1], own + a.mean() + b.mean(), rtol=4e-16, atol=1e-14)
     np.testing.assert_array_equal(wall[:, 4], np.full((3, N), 2.0))
+
+
+def test_walls_of_n_where_the_square_of_phi_overflows(L):
+    """phi^2 = inf of finite phi: n = phi / inf = 0 there, and A', V' with it."""
+    print("[gpu-test] walls, overflow", flush=True)
+    N = 16
+    u = np.random.default_rng(3).normal(size=(N, N, N, 10))
+    for site in ((0, 0, 2), (3, 5, 7), (15, 15, 15)):
+        u[site][:4] = [1e200, -1e200, 5e199, 1e-3]
+    with np.errstate(over="ignore"):
+        obs = observables(u)
+    ctx = L.Context(L.model_params(N))
+    ctx.set_field(u)
+    wall, phase, _ = ctx.measure()
+    ctx.close()
+    walls = np.concatenate([wall, phase], axis=1)
+    for o, f in enumerate(obs):
+        if o in (10, 11, 24):  # phi^2, sigma: infinite
+            continue
+        for d, axes in enumerate(((0, 1), (0, 2), (1, 2))):
+            ref = f.sum(axis=axes, dtype=np.longdouble) / N ** 2
+            tol = 10 * np.finfo(float).eps * np.abs(f).mean(axis=axes) + 1e-300
+            assert (np.abs(walls[d, o] - ref) <= tol).all(), (d, o)
