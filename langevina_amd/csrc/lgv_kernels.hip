@@ -1743,20 +1743,6 @@ __device__ __forceinline__ void ksum_xor_merge(KSum &a, int o) {
   two_sum_add(a, b.s);
   a.c += b.c;
 }
-// The same for sums that start at a bias B, a power of two: while |x| stays
-// below |a.s|, Dekker's two-sum, three additions, gives the error exactly.  B
-// is 2^14 .. 2^15 times the largest magnitude of a first sample, so that holds
-// as long as the values and their sum stay below 2^13 times the sample's;
-// beyond that the additions round as plain FP64 ones.
-__device__ __forceinline__ void biased_add(KSum &a, double x) {
-  const double s = a.s + x;
-  a.c += x - (s - a.s);
-  a.s = s;
-}
-__device__ __forceinline__ double bias_of(double largest) {
-  const uint64_t e = (uint64_t)__double_as_longlong(largest) >> 52;  // largest >= 0
-  return largest > 0. ? __longlong_as_double((long long)((e < 1900 ? e + 15 : 1915) << 52)) : 1.;
-}
 
 // The three walls' slice sums in one pass over the fields (measurer.cxx:
 // 10-229).  A wavefront takes 64 columns (x, z), TX x TZ of them in use, and
@@ -1764,7 +1750,11 @@ __device__ __forceinline__ double bias_of(double largest) {
 // column summed over y in registers (from which the x and z walls follow), and
 // each row's sums over the columns (the y wall) are taken through the
 // wavefront's own LDS table, two lanes to an observable.  No wavefront waits
-// for another.  All sums are compensated.  Partial sums:
+// for another.  All sums are compensated, by a two-sum that holds for any order
+// of magnitudes (sums that started at a bias made from the first row's
+// magnitudes took three operations less an addition, 256^3 FP64 444 us against
+// 464, FP32 365 against 425, but were plain ones where a later row was larger).
+// Partial sums:
 //   px[(chunk, z tile)][25][N]  over the tile's planes and the chunk's rows,
 //   pz[(chunk, x tile)][25][N]  over the tile's columns and the chunk's rows,
 //   py[(x tile, z group)][25][N][nz > 1 ? 2 : 1]  over the columns of the
@@ -1831,24 +1821,8 @@ void k_measure_tile(const ReplicaParams *__restrict__ P, const ReplicaState *__r
     load(y0, raw[0]);
     if (y0 + 1 < y1) load(y0 + 1, raw[1]);
     KSum acc[25];
-    {
-      // the biases from the first row's largest magnitudes
-      double o[25];
-      observe(raw[0], o);
 #pragma unroll
-      for (int i = 0; i < 25; i++) q[i][lane] = o[i];
-      table_ready();
-      double m = 0.;
-      if (k < 25)
-        for (int i = s; i < kMeasureCols; i += 2) m = fmax(m, fabs(q[k][i]));
-      m = fmax(m, __shfl_xor(m, 1, 64));
-      table_ready();
-      if (k < 25 && s == 0) q[k][kMeasureCols] = bias_of(m);  // kept in the padding
-      table_ready();
-#pragma unroll
-      for (int i = 0; i < 25; i++) acc[i] = KSum{q[i][kMeasureCols], 0.};
-    }
-    const double yb = k < 25 ? q[k][kMeasureCols] : 1.;
+    for (int i = 0; i < 25; i++) acc[i] = KSum{0., 0.};
     auto take = [&](int y, T *r) __attribute__((always_inline)) {
       double o[25];
       observe(r, o);
@@ -1856,15 +1830,14 @@ void k_measure_tile(const ReplicaParams *__restrict__ P, const ReplicaState *__r
 #pragma unroll
       for (int i = 0; i < 25; i++) {
         q[i][lane] = o[i];
-        biased_add(acc[i], o[i]);
+        two_sum_add(acc[i], o[i]);
       }
       table_ready();
       if (k < 25) {
-        KSum a{yb, 0.};
+        KSum a{0., 0.};
         const double *row = &q[k][s];
 #pragma unroll
-        for (int i = 0; i < kMeasureCols; i += 2) biased_add(a, row[i]);
-        a.s -= yb;
+        for (int i = 0; i < kMeasureCols; i += 2) two_sum_add(a, row[i]);
         ksum_xor_merge(a, 1);
         if (s == 0) {
           double *w = yrow + ((int64_t)k * N + y) * yw;
@@ -1888,7 +1861,7 @@ void k_measure_tile(const ReplicaParams *__restrict__ P, const ReplicaState *__r
     }
     // the columns' sums over the chunk, then over the tile's planes / columns
 #pragma unroll
-    for (int i = 0; i < 25; i++) q[i][lane] = (acc[i].s - q[i][kMeasureCols]) + acc[i].c;
+    for (int i = 0; i < 25; i++) q[i][lane] = ksum_value(acc[i]);
     table_ready();
     double *xrow = px + (int64_t)(by * sh.ntz + bz) * 25 * N;
     if (tz == 0 && tx < tw) {

@@ -82,6 +82,60 @@ def test_walls_of_a_large_lattice(L):
     np.testing.assert_array_equal(wall[:, 4], np.full((3, N), 2.0))
 
 
+# Sides whose tiles and chunks are whole periods of the sign pattern below; 448:
+# a wavefront takes four z tiles in turn
+@pytest.mark.parametrize("N", [64, 128, 448])
+def test_sums_are_compensated_whatever_the_first_row_holds(L, N):
+    """Charges of +-2^16 that cancel in fours, plus noise of 2^-16, with rows
+    y = 0, 4, ... (the first of every chunk) that hold the noise alone, or
+    nothing: the walls in which the large values cancel inside a wavefront
+    keep only the noise."""
+    print(f"[gpu-test] compensated walls {N}", flush=True)
+    M, quantum = 2.0 ** 16, 2.0 ** -36  # M + k quantum is exact for |k| <= 2^20
+    i = np.arange(N)
+    p = np.array([0, 1, -1, 0], np.int64)[i % 4]
+    late = (i % 4 != 0).astype(np.int64)
+    one = np.ones(N, np.int64)
+    # sign(z) sign(y) sign(x) of component 4, 5, 6, 7, and whether its rows
+    # y = 0, 4, ... hold noise
+    signs = {4: (one, p, one, True), 5: (one, late, p, True), 6: (p, late, one, True),
+             7: (one, late, p, False)}
+    u = np.zeros((N, N, N, 10))
+    u[..., 0] = 1.0  # n = (1, 0, 0, 0): the A' and V' are the charges
+    rng = np.random.default_rng(N)
+    hi, lo, mag = {}, {}, {}
+    axes = ((0, 1), (0, 2), (1, 2))  # x, y, z walls of f[z, y, x]
+    for o, (sz, sy, sx, noise) in signs.items():
+        k = rng.integers(-2 ** 20, 2 ** 20 + 1, (N, N, N))
+        if not noise:
+            k *= late[None, :, None]
+        u[..., o] = sz[:, None, None] * sy[None, :, None] * sx[None, None, :] * M + k * quantum
+        for d, ax in enumerate(axes):
+            lo[o, d] = k.sum(axis=ax).astype(np.longdouble) * quantum
+            mag[o, d] = np.abs(k).sum(axis=ax) * quantum / N ** 2
+        for d, (a, b, own) in enumerate(((sz, sy, sx), (sz, sx, sy), (sy, sx, sz))):
+            hi[o, d] = (a.sum() * b.sum() * own).astype(np.longdouble) * M
+    ctx = L.Context(L.model_params(N))
+    ctx.set_field(u)
+    wall, phase, _ = ctx.measure()
+    ctx.close()
+    x, y, z = 0, 1, 2
+    cancels = {(4, x), (4, z), (5, y), (7, y)} | ({(6, y)} if N == 448 else set())
+    unit = 2.0 ** -53
+    for o in signs:
+        for d in (x, y, z):
+            ref = (hi[o, d] + lo[o, d]) / N ** 2
+            # at most four roundings: a column's sum over a chunk, a tile's sum,
+            # the wall's, and the division; the corrections themselves round
+            # in second order (chunks and rows of at most 224 terms)
+            tol = 4 * unit * mag[o, d] + unit ** 2 * N ** 2 * M
+            if (o, d) not in cancels:
+                tol = tol + 4 * unit * M
+            assert (np.abs(wall[d, o] - ref) <= tol).all(), (o, d)
+    np.testing.assert_array_equal(phase[:, 6:9], wall[:, 4:7])
+    np.testing.assert_array_equal(phase[:, 10], wall[:, 7])
+
+
 def test_walls_of_n_where_the_square_of_phi_overflows(L):
     """phi^2 = inf of finite phi: n = phi / inf = 0 there, and A', V' with it."""
     print("[gpu-test] walls, overflow", flush=True)
