@@ -189,25 +189,35 @@ constexpr uint64_t kOverlapBytesPairMarch = 1300ull << 20;
 constexpr int kMaxN = 1536;
 
 // Shape of the measurement pass (k_measure_tile): TX x TZ columns per
-// wavefront, nz tiles in z taken in turn, chunks of CY rows in y; ntx, ntz
-// tiles and nch chunks.  The partial sums hold 25 N (nch ntz + nch ntx + ntx ntz)
-// doubles (with nz > 1 2 ntx ntz / nz in place of ntx ntz), at most 50 max(2^19,
-// N^2): nz grows with N for that.  Chunks are halved until the launch has 2048
-// wavefronts, which is what the GPU holds (256^3 FP64: 471 us with 1024, 385
-// with 2048, 383 with 4096); small lattices stop at 16 N, where more
-// partial sums cost as much as the shorter chunks give.
+// wavefront, groups of nz tiles in z taken in turn, chunks of CY rows in y; ntx,
+// ntz tiles and nch chunks.  The partial sums hold 25 N (nch ntx + words
+// groups (nch + ntx)) doubles, at most 50 max(2^19, N^2).  While one tile a
+// wavefront fits that, chunks are halved until the launch has 2048 wavefronts,
+// which is what the GPU holds (256^3 FP64: 471 us with 1024, 385 with 2048, 383
+// with 4096); small lattices stop at 16 N, where more partial sums cost as much
+// as the shorter chunks give.  From N = 386 on nz and the chunk minimise the
+// rounds of wavefronts, each of nz tiles of CY rows and about four rows' time
+// for a tile's own sums (512^3 FP64: 512 wavefronts 7.5 ms, 2048 3.8).
 struct MeasureShape {
   int TX, TZ, nz, CY, ntx, ntz, nch;
 };
 constexpr int64_t kMeasurePart = int64_t(1) << 19;
+constexpr int kMeasureWaves = 2048;
 __host__ __device__ inline int64_t measure_part_limit(int N) {
   const int64_t n2 = (int64_t)N * N;
   return 50 * (n2 > kMeasurePart ? n2 : kMeasurePart);
 }
+__host__ __device__ inline int measure_groups(const MeasureShape &s) {
+  return (s.ntz + s.nz - 1) / s.nz;
+}
+__host__ __device__ inline int measure_words(const MeasureShape &s) { return s.nz > 1 ? 2 : 1; }
+__host__ __device__ inline int64_t measure_waves(const MeasureShape &s) {
+  return (int64_t)s.ntx * measure_groups(s) * s.nch;
+}
 __host__ __device__ inline int64_t measure_part(const MeasureShape &s, int N) {
-  const int64_t groups = (int64_t)s.ntx * ((s.ntz + s.nz - 1) / s.nz);
   return 25 * (int64_t)N *
-         ((int64_t)s.nch * (s.ntz + s.ntx) + (s.nz > 1 ? 2 : 1) * groups);
+         ((int64_t)s.nch * s.ntx +
+          (int64_t)measure_words(s) * measure_groups(s) * (s.nch + s.ntx));
 }
 inline MeasureShape measure_shape(int N) {
   MeasureShape s;
@@ -216,22 +226,33 @@ inline MeasureShape measure_shape(int N) {
   s.TZ = 64 / s.TX;
   if (s.TZ > N) s.TZ = N;
   s.ntz = (N + s.TZ - 1) / s.TZ;
-  s.nz = 1;
+  s.nz = s.nch = 1;
   s.CY = N;
-  s.nch = 1;
-  while (measure_part(s, N) > measure_part_limit(N)) s.nz *= 2;
-  const int64_t waves = N < 128 ? 16 * N : 2048;
-  // more chunks while the launch leaves the GPU idle and the sums have room
-  while (s.CY > 1) {
-    MeasureShape h = s;
-    h.CY = (s.CY + 1) / 2;
-    h.nch = (N + h.CY - 1) / h.CY;
-    if ((int64_t)s.ntx * ((s.ntz + s.nz - 1) / s.nz) * s.nch >= waves ||
-        measure_part(h, N) > measure_part_limit(N))
-      break;
-    s = h;
+  if (measure_part(s, N) <= measure_part_limit(N)) {
+    const int64_t waves = N < 128 ? 16 * N : kMeasureWaves;
+    while (s.CY > 1 && measure_waves(s) < waves) {
+      MeasureShape h = s;
+      h.CY = (s.CY + 1) / 2;
+      h.nch = (N + h.CY - 1) / h.CY;
+      if (measure_part(h, N) > measure_part_limit(N)) break;
+      s = h;
+    }
+    return s;
   }
-  return s;
+  MeasureShape best = s;
+  int64_t best_cost = INT64_MAX;
+  for (s.nz = 2; s.nz < 2 * s.ntz; s.nz *= 2)
+    for (s.CY = 4; s.CY < N + 4; s.CY += 4) {
+      s.nch = (N + s.CY - 1) / s.CY;
+      if (measure_part(s, N) > measure_part_limit(N)) continue;
+      const int64_t rounds = (measure_waves(s) + kMeasureWaves - 1) / kMeasureWaves;
+      const int64_t cost = rounds * s.nz * (s.CY + 4);
+      if (cost < best_cost) {
+        best_cost = cost;
+        best = s;
+      }
+    }
+  return best;
 }
 
 // Kernel launchers (lgv_kernels.hip).  fp32 selects the storage type.

@@ -1754,11 +1754,11 @@ __device__ __forceinline__ void ksum_xor_merge(KSum &a, int o) {
 // of magnitudes (sums that started at a bias made from the first row's
 // magnitudes took three operations less an addition, 256^3 FP64 444 us against
 // 464, FP32 365 against 425, but were plain ones where a later row was larger).
-// Partial sums:
-//   px[(chunk, z tile)][25][N]  over the tile's planes and the chunk's rows,
+// Partial sums, (sum, correction) pairs where a wavefront takes the nz > 1 z
+// tiles of a group in turn:
+//   px[(chunk, z group)][25][N][words]  over the group's planes, the chunk's rows,
 //   pz[(chunk, x tile)][25][N]  over the tile's columns and the chunk's rows,
-//   py[(x tile, z group)][25][N][nz > 1 ? 2 : 1]  over the columns of the
-//     group's nz z tiles, which one wavefront takes in turn (sum, correction).
+//   py[(x tile, z group)][25][N][words]  over the group's columns.
 // What bounds it is bytes in flight: two rows' loads ahead of the sums at two
 // wavefronts per SIMD keep 80 KB per CU under way.
 constexpr int kMeasureCols = 64;
@@ -1780,7 +1780,7 @@ void k_measure_tile(const ReplicaParams *__restrict__ P, const ReplicaState *__r
   const int wave = first_lane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
   MeasureTable &q = tab[wave];
   int b = (int)blockIdx.x * (kBlock / 64) + wave;
-  const int ngz = (sh.ntz + sh.nz - 1) / sh.nz;
+  const int ngz = measure_groups(sh);
   if (b >= sh.ntx * ngz * sh.nch) return;  // whole wavefronts; no barrier follows
   const int bx = b % sh.ntx;
   b /= sh.ntx;
@@ -1788,8 +1788,22 @@ void k_measure_tile(const ReplicaParams *__restrict__ P, const ReplicaState *__r
   const int tx = lane % sh.TX, tz = lane / sh.TX;
   const int x0 = bx * sh.TX, tw = min(sh.TX, N - x0);
   const int y0 = by * sh.CY, y1 = min(y0 + sh.CY, N);
-  const int yw = sh.nz > 1 ? 2 : 1;
-  double *yrow = py + (int64_t)(bx * ngz + gz) * 25 * N * yw;
+  const int words = measure_words(sh);
+  double *xrow = px + (int64_t)(by * ngz + gz) * 25 * N * words;
+  double *yrow = py + (int64_t)(bx * ngz + gz) * 25 * N * words;
+  // adds a tile's sum to the group's, which this lane alone reads and writes
+  auto put = [&](double *w, KSum a, int bz) __attribute__((always_inline)) {
+    if (words == 1) {
+      w[0] = ksum_value(a);
+    } else {
+      if (bz > gz * sh.nz) {
+        two_sum_add(a, w[0]);
+        a.c += w[1];
+      }
+      w[0] = a.s;
+      w[1] = a.c;
+    }
+  };
   // this lane's part in the table's row sums: row k, entries s, s + 2, ...
   const int k = lane >> 1, s = lane & 1;
   // the table is written and read by one wavefront: its LDS operations stay
@@ -1839,19 +1853,7 @@ void k_measure_tile(const ReplicaParams *__restrict__ P, const ReplicaState *__r
 #pragma unroll
         for (int i = 0; i < kMeasureCols; i += 2) two_sum_add(a, row[i]);
         ksum_xor_merge(a, 1);
-        if (s == 0) {
-          double *w = yrow + ((int64_t)k * N + y) * yw;
-          if (yw == 1) {
-            w[0] = ksum_value(a);
-          } else {
-            if (bz > gz * sh.nz) {  // the group's earlier tiles: this lane's own stores
-              two_sum_add(a, w[0]);
-              a.c += w[1];
-            }
-            w[0] = a.s;
-            w[1] = a.c;
-          }
-        }
+        if (s == 0) put(yrow + ((int64_t)k * N + y) * words, a, bz);
       }
       table_ready();
     };
@@ -1863,12 +1865,11 @@ void k_measure_tile(const ReplicaParams *__restrict__ P, const ReplicaState *__r
 #pragma unroll
     for (int i = 0; i < 25; i++) q[i][lane] = ksum_value(acc[i]);
     table_ready();
-    double *xrow = px + (int64_t)(by * sh.ntz + bz) * 25 * N;
     if (tz == 0 && tx < tw) {
       for (int i = 0; i < 25; i++) {
         KSum a{0., 0.};
         for (int r = 0; r < th; r++) two_sum_add(a, q[i][r * sh.TX + tx]);
-        xrow[(int64_t)i * N + x] = ksum_value(a);
+        put(xrow + ((int64_t)i * N + x) * words, a, bz);
       }
     }
     double *zrow = pz + (int64_t)(by * sh.ntx + bx) * 25 * N;
@@ -1902,19 +1903,19 @@ __global__ __launch_bounds__(64 * kReduceGroups) void k_measure_reduce(int N, Me
   const int lane = threadIdx.x & 63, g = threadIdx.x >> 6;
   const int k = blockIdx.x / nb % 25, d = blockIdx.x / nb / 25;
   const int n = (blockIdx.x % nb) * 64 + lane;
-  const int ngz = (sh.ntz + sh.nz - 1) / sh.nz;
-  const int entries = d == 0 ? sh.nch * sh.ntz : (d == 1 ? sh.ntx * ngz : sh.nch * sh.ntx);
+  const int ngz = measure_groups(sh);
+  const int entries = d == 0 ? sh.nch * ngz : (d == 1 ? sh.ntx * ngz : sh.nch * sh.ntx);
   const int64_t stride = 25 * (int64_t)N, at = (int64_t)k * N + n;
   KSum acc{0., 0.};
   if (n < N) {
-    if (d == 1 && sh.nz > 1) {
+    const double *src = d == 0 ? px : (d == 1 ? py : pz);
+    if (d != 2 && measure_words(sh) == 2) {
 #pragma unroll 8
       for (int e = g; e < entries; e += kReduceGroups) {
-        two_sum_add(acc, py[(e * stride + at) * 2]);
-        acc.c += py[(e * stride + at) * 2 + 1];
+        two_sum_add(acc, src[(e * stride + at) * 2]);
+        acc.c += src[(e * stride + at) * 2 + 1];
       }
     } else {
-      const double *src = d == 0 ? px : (d == 1 ? py : pz);
 #pragma unroll 8
       for (int e = g; e < entries; e += kReduceGroups) two_sum_add(acc, src[e * stride + at]);
     }
@@ -2113,9 +2114,9 @@ void launch_measure(bool fp32, const ReplicaParams *P, const ReplicaState *S, in
                     int N, double *part, double *wall, double *wallphase, double *host_wall,
                     double *host_wallphase, hipStream_t st) {
   const MeasureShape sh = measure_shape(N);
-  double *px = part, *pz = px + (int64_t)sh.nch * sh.ntz * 25 * N,
+  double *px = part, *pz = px + (int64_t)sh.nch * measure_groups(sh) * measure_words(sh) * 25 * N,
          *py = pz + (int64_t)sh.nch * sh.ntx * 25 * N;
-  const unsigned tiles = (unsigned)(sh.ntx * ((sh.ntz + sh.nz - 1) / sh.nz) * sh.nch);
+  const unsigned tiles = (unsigned)measure_waves(sh);
   const unsigned blocks = nblk(tiles, kBlock / 64);  // a wavefront to a tile
   if (fp32) k_measure_tile<float><<<blocks, kBlock, 0, st>>>(P, S, replica, sh, px, py, pz);
   else k_measure_tile<double><<<blocks, kBlock, 0, st>>>(P, S, replica, sh, px, py, pz);

@@ -1,0 +1,48 @@
+"""The host's rules that choose shapes by size (langevina_amd/csrc/lgv_internal.h),
+compiled as they stand: what they give over the whole range of sides."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HIP_INCLUDE = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include")
+
+
+@pytest.fixture(scope="module")
+def rule(tmp_path_factory):
+    """rule(body): runs a C++ main body with the header and returns the rows
+    of numbers it prints."""
+    def run(body):
+        d = tmp_path_factory.mktemp("rules")
+        src, exe = d / "rules.cpp", d / "rules"
+        src.write_text('#include <cstdio>\n#include "lgv_internal.h"\nusing namespace lgv;\n'
+                       "int main() {\n" + body + "\n}\n")
+        subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I", HIP_INCLUDE,
+                        "-I", os.path.join(ROOT, "include"),
+                        "-I", os.path.join(ROOT, "langevina_amd", "csrc"), str(src), "-o",
+                        str(exe)], check=True, capture_output=True, text=True)
+        out = subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout
+        return [[int(v) for v in line.split()] for line in out.splitlines()]
+    return run
+
+
+def test_measurement_fills_the_gpu_at_every_side(rule):
+    rows = rule("""
+  for (int N = 4; N <= kMaxN; N += 2) {
+    const MeasureShape s = measure_shape(N);
+    printf("%d %d %d %d %d %d %d %d %lld %lld\\n", N, s.TX, s.TZ, s.nz, s.CY, s.ntx, s.ntz, s.nch,
+           (long long)measure_part(s, N), (long long)measure_part_limit(N));
+  }""")
+    assert len(rows) == (1536 - 4) // 2 + 1
+    for N, TX, TZ, nz, CY, ntx, ntz, nch, part, limit in rows:
+        assert TX * TZ <= 64 and nz >= 1 and CY >= 1, N
+        for n, tiles, size in ((N, ntx, TX), (N, ntz, TZ), (N, nch, CY)):
+            assert (tiles - 1) * size < n <= tiles * size, N
+        assert part <= limit == 50 * max(2 ** 19, N * N), N
+        # wavefronts: what the GPU holds, of a lattice that has them, or nearly
+        # that with no second round of a few
+        waves = ntx * -(-ntz // nz) * nch
+        assert waves >= (1700 if N >= 128 else min(16 * N, ntx * ntz * N)), (N, waves)
+        if nz > 1:
+            assert -(-waves // 2048) * 2048 <= 1.25 * waves, (N, waves)
