@@ -482,16 +482,16 @@ bool resolve_bricks(lgv_ctx *c) {
   return best_y != 0;
 }
 
-// The tiles of k_hb_sweep: as many rows as its threads hold (half-columns, with
-// a facing row on either side), and the depth TZ that minimises whole rounds of
-// one block per CU, each of TZ planes and about five planes' time for the two
-// more that it decides, its start and its end (256^3 FP64, per half-sweep: TZ
-// 52, one round of 215 blocks, 131 us; 24, two, 133; 16, three, 142; 8 160).
+// The tiles of k_hb_sweep: as many rows as its threads hold (pair_march_rows),
+// and the depth TZ that minimises whole rounds of one block per CU, each of TZ
+// planes and about five planes' time for the two more that it decides, its start
+// and its end (256^3 FP64, per half-sweep: TZ 52, one round of 215 blocks, 131
+// us; 24, two, 133; 16, three, 142; 8 160).
 // False: the rows are too long.
 bool resolve_pair_march(lgv_ctx *c) {
   for (ReplicaParams &p : c->hp) {
-    if (kPairBlock / p.NH < 3) return false;
-    p.pair_y = std::min(kPairBlock / p.NH - 2, p.N);
+    p.pair_y = pair_march_rows(p.N);
+    if (!p.pair_y) return false;
   }
   int best = 0;
   double best_cost = 1e300;

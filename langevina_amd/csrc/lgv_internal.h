@@ -175,6 +175,15 @@ constexpr int kBrickLds = 64 << 10;
 // 1945, 2 x 160^3 2460 -> 2184.
 constexpr uint64_t kPairMarchSites = 2900000;
 constexpr int kPairMarchSide = 64;
+// Rows that a block of k_hb_sweep owns: its threads less a facing row on either
+// side; 0: the rows are too long for it.  A block of one row (sides above 512)
+// decides three sites for each it keeps: step 514^3 FP64 56.1 ms, half-sweeps
+// 49.9; 528^3 54.7, 48.5; 576^3 63.9, 56.4; of two rows 480^3 33.6, 33.7; 512^3
+// 35.8, 36.8; 410^3 24.7, 25.4.
+inline int pair_march_rows(int N) {
+  const int rows = kPairBlock / (N / 2) - 2;
+  return rows < 2 ? 0 : rows < N ? rows : N;
+}
 
 // A context of one lattice whose fields (one buffer) exceed this keeps the
 // charge sweep after the phi sweeps rather than beside them; beside k_hb_sweep,

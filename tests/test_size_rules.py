@@ -46,3 +46,11 @@ def test_measurement_fills_the_gpu_at_every_side(rule):
         assert waves >= (1700 if N >= 128 else min(16 * N, ntx * ntz * N)), (N, waves)
         if nz > 1:
             assert -(-waves // 2048) * 2048 <= 1.25 * waves, (N, waves)
+
+
+def test_a_block_of_both_parities_owns_two_rows_or_none(rule):
+    rows = rule("""
+  for (int N = 4; N <= kMaxN; N += 2) printf("%d %d\\n", N, pair_march_rows(N));""")
+    for N, own in rows:
+        threads = (own + 2) * (N // 2)
+        assert own == 0 if N > 512 else 2 <= own <= N and threads <= 1024, N
