@@ -283,15 +283,6 @@ int free_plan(Plan &plan) {
 
 constexpr int kCUs = 256;  // MI355X
 
-// Width of an x tile of at most cap half-columns that splits a row of NH
-// evenly: with a fixed width of 32 or 64 the last tile of a row whose length
-// is no multiple of it is mostly empty (NH = 75 in tiles of 64: 59 % of the
-// lanes at work; in two of 38, 99 %).
-int even_width(int NH, int cap) {
-  const int n = (NH + cap - 1) / cap;
-  return (NH + n - 1) / n;
-}
-
 // Blocks of one z plane of the ideal kernel with tiles of width cap.
 int64_t ideal_plane_blocks(const ReplicaParams &p, int cap) {
   int TXH, TY, TZ;
@@ -541,8 +532,8 @@ bool charge_rows(const lgv_ctx *c) {
   return rows;
 }
 
-// The charge march's tiles where the caller asked for none.  Width: an even
-// split of the row into at most 64 half-columns.  Chunk: a chunk of C sites
+// The charge march's tiles where the caller asked for none.  Width:
+// charge_width.  Chunk: a chunk of C sites
 // updates C/2 + 1 first-parity pairs for its C/2 second-parity ones, and the
 // GPU holds `slots` blocks at a time, so a launch takes about ceil(blocks /
 // slots) rounds of C/2 + 1.5 pairs; C of 16, 8, 4, 2 minimises that.  Measured
@@ -553,7 +544,7 @@ bool charge_rows(const lgv_ctx *c) {
 void resolve_charge_tiles(lgv_ctx *c) {
   for (int r = 0; r < c->nrep; r++) {
     ReplicaParams &p = c->hp[r];
-    p.chg_cap = c->tiles[r].chg_cap ? c->tiles[r].chg_cap : even_width(p.NH, 64);
+    p.chg_cap = c->tiles[r].chg_cap ? c->tiles[r].chg_cap : charge_width(p.NH, c->fp32);
   }
   const int slots = kCUs * (!c->fp32 && charge_rows(c) ? 3 : 4);
   int best = 16;

@@ -141,6 +141,31 @@ struct Plan {
 // 1166 -> 1173, 200^3, rows of 6.25 lines, 2415 -> 2427).
 constexpr uint64_t kCacheBytes = 256ull << 20;
 
+// Width of an x tile of at most cap half-columns that splits a row of NH
+// evenly: with a fixed width of 32 or 64 the last tile of a row whose length
+// is no multiple of it is mostly empty (NH = 75 in tiles of 64: 59 % of the
+// lanes at work; in two of 38, 99 %).
+inline int even_width(int NH, int cap) {
+  const int n = (NH + cap - 1) / cap;
+  return (NH + n - 1) / n;
+}
+
+// Width of the charge march's tiles: an even split of the row into at most 64.
+// Where a replica's fields exceed the last-level cache and its rows are whole
+// 64-byte units, tiles are too, or neighbouring tiles share a unit of every row
+// and plane: 64, or 48 where that takes no more tiles (a block then has five
+// lines instead of four).  Three launches, FP64, even -> 48 / 64: 176^3 475 ->
+// 434 / 455 us, 272^3 1654 -> 1379 / 1413, 320^3 2614 -> 2213 / 2076, 352^3 3390
+// -> 2829 / 2698, 528^3 9764 -> 10640 / 9563; FP32 224^3 575 -> 610 / 543, 480^3
+// 5301 -> - / 4753; below the cache FP64 144^3 251 -> 264 / 298, FP32 160^3 209 ->
+// 225 / 298.
+inline int charge_width(int NH, bool fp32) {
+  const int esz = fp32 ? 4 : 8;
+  const uint64_t bytes = 80 * (uint64_t)NH * NH * NH * esz;  // ten planes of (2 NH)^3
+  if (NH <= 64 || bytes <= kCacheBytes || NH * esz % 64 != 0) return even_width(NH, 64);
+  return (NH + 47) / 48 == (NH + 63) / 64 ? 48 : 64;
+}
+
 // From this many sites on (all replicas) the phi half-sweeps run the z-march:
 // it reads each value of the other parity once per launch where the
 // one-thread-per-site kernel reads it up to four times, which costs that

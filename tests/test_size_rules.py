@@ -54,3 +54,19 @@ def test_a_block_of_both_parities_owns_two_rows_or_none(rule):
     for N, own in rows:
         threads = (own + 2) * (N // 2)
         assert own == 0 if N > 512 else 2 <= own <= N and threads <= 1024, N
+
+
+def test_charge_tiles_of_large_lattices_are_whole_units(rule):
+    """Where the fields exceed the 256 MiB cache and a row is whole 64-byte units,
+    a tile is too, with most lanes at work; elsewhere rows split evenly."""
+    rows = rule("""
+  for (int N = 4; N <= kMaxN; N += 2)
+    for (int f = 0; f < 2; f++) printf("%d %d %d\\n", N, f, charge_width(N / 2, f));""")
+    for N, fp32, w in rows:
+        NH, esz = N // 2, 4 if fp32 else 8
+        n = -(-NH // w)
+        if NH > 64 and 10 * N ** 3 * esz > 2 ** 28 and NH * esz % 64 == 0:
+            assert w in (48, 64) and w * esz % 64 == 0, (N, fp32)
+            assert n == -(-NH // 64), (N, fp32)
+        else:
+            assert w <= 64 and n == -(-NH // 64) and w * n - NH < n, (N, fp32)
