@@ -281,23 +281,8 @@ int free_plan(Plan &plan) {
   return LGV_OK;
 }
 
-constexpr int kCUs = 256;  // MI355X
-
-// Blocks of one z plane of the ideal kernel with tiles of width cap.
-int64_t ideal_plane_blocks(const ReplicaParams &p, int cap) {
-  int TXH, TY, TZ;
-  ideal_tile(p.N, cap, 1, TXH, TY, TZ);
-  return (int64_t)((p.NH + TXH - 1) / TXH) * ((p.N + TY - 1) / TY);
-}
-
-// The ideal kernel's tiles where the caller asked for none.  Width: 32
-// half-columns where they divide the row (whole 128-byte lines of every
-// component: 256^3 FP64 541 us against 560 with 64) or need fewer tiles than
-// the alternative; 16 for FP64 rows of several tiles that those divide (160^3
-// 174 -> 148 us, 224^3 443 -> 398; a FP32 row of 16 is half a line); otherwise
-// the widest even split that the kernel's plane grid holds (every ring column
-// costs a line per row and component: 200^3 FP64 329 us with 50, 390 with 34,
-// 435 with 25).  Depth: a block marches TZ planes and rotates one more on
+// The ideal kernel's tiles where the caller asked for none.  Width:
+// ideal_width.  Depth: a block marches TZ planes and rotates one more on
 // either side, and the GPU holds `slots` blocks at a time.  A launch of up to
 // two rounds takes whole rounds of TZ planes, a longer one its blocks' share
 // and a tail; TZ of 16, 8, 4, and 64, 32, 2, 1 within one round, minimises that
@@ -306,22 +291,10 @@ int64_t ideal_plane_blocks(const ReplicaParams &p, int cap) {
 // 537, 546, 575 us; 240^3 558, 522, 523; 192^3 261, 245, 249; 144^3 140, 125,
 // 123; 100^3 63, 42, 38; 64^3 TZ 1 17 us, TZ 16 60).
 void resolve_ideal_tiles(lgv_ctx *c) {
-  const int slots = kCUs * (c->fp32 ? 3 : 2);
+  const int slots = ideal_slots(c->fp32);
   for (int r = 0; r < c->nrep; r++) {
     ReplicaParams &p = c->hp[r];
-    p.tile_cap = c->tiles[r].ideal_cap;
-    if (p.tile_cap) continue;
-    for (int cap = 64; cap >= 32 || !p.tile_cap; cap--) {
-      int TXH, TY, TZ;
-      ideal_tile(p.N, even_width(p.NH, cap), 1, TXH, TY, TZ);
-      if ((TY + 2) * (2 * TXH + 2) <= ideal_lds(c->fp32)) {
-        p.tile_cap = TXH;
-        break;
-      }
-    }
-    if (p.NH % 32 == 0 || ideal_plane_blocks(p, 32) < ideal_plane_blocks(p, p.tile_cap))
-      p.tile_cap = 32;
-    if (!c->fp32 && p.NH % 32 == 16 && p.NH > p.tile_cap) p.tile_cap = 16;
+    p.tile_cap = c->tiles[r].ideal_cap ? c->tiles[r].ideal_cap : ideal_width(p.N, c->fp32);
   }
   int best = 64;
   double best_cost = 1e300;
@@ -329,7 +302,7 @@ void resolve_ideal_tiles(lgv_ctx *c) {
   for (int tz = 64; tz >= 1; tz /= 2) {
     int64_t blocks = 0;
     for (const ReplicaParams &p : c->hp)
-      blocks += ideal_plane_blocks(p, p.tile_cap) * ((p.N + tz - 1) / tz);
+      blocks += ideal_plane_blocks(p.N, p.tile_cap) * ((p.N + tz - 1) / tz);
     const double rounds = (double)blocks / slots;
     if (tz < 4 && rounds > 1.) break;
     if (tz > 16 && rounds > 1.) continue;
@@ -361,7 +334,7 @@ int build_ideal_plan(lgv_ctx *c) {
     ideal_tile(p.N, p.tile_cap, p.tile_tz, TXH, TY, TZ);
     if ((TY + 2) * (2 * TXH + 2) > ideal_lds(c->fp32))
       return fail(LGV_ERR_ARG, "replica %d: ideal tile %dx%d exceeds the LDS plane", r, TXH, TY);
-    stream = stream && whole_rows(c, p.NH, TXH, 128);
+    stream = stream && whole_rows(c, p.NH, TXH, ideal_unit(p.N, c->fp32));
     const int64_t plane = (int64_t)((p.NH + TXH - 1) / TXH) * ((p.N + TY - 1) / TY);
     work.push_back({plane * ((p.N + TZ - 1) / TZ), (double)plane});
   }

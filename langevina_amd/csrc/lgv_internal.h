@@ -9,6 +9,7 @@
 
 namespace lgv {
 
+constexpr int kCUs = 256;  // MI355X
 constexpr int kBlock = 256;  // threads per block of every sweep kernel but these:
 constexpr int kPairBlock = 1024;  // k_hb_brick, k_hb_sweep
 
@@ -127,9 +128,12 @@ struct Plan {
 // only evicts lines that neighbouring tiles still read; and only where a tile's
 // rows are whole lines (a non-temporal store of part of a line costs more than
 // a cached one).  Ideal: fields (one buffer) above twice the cache, rows and
-// tile rows of whole 128-byte lines; FP64 192^3 263 -> 259 us, 224^3 449 ->
-// 437, 256^3 556 -> 534, FP32 256^3 324 -> 318, but 208^3 FP64 (rows of 6.5
-// lines) 384 -> 413, 200^3 308 -> 377, 288^3 FP32 644 -> 956.  Phi march: phi
+// tile rows of whole 128-byte lines, or of whole 64-byte halves of FP64 lattices
+// that alone exceed it (ideal_unit); FP64 192^3 263 -> 259 us, 224^3 449 ->
+// 437, 256^3 556 -> 534, FP32 256^3 324 -> 318; rows of 6.5 lines, 208^3, in
+// tiles of 56 356 -> 337, of broken units, 52, 384 -> 413; 200^3, rows of 12.5
+// halves, 308 -> 377; FP32 rows of halves 288^3 522 -> 536, in tiles of 36 644 ->
+// 956.  Phi march: phi
 // planes (one buffer) above the cache, rows and tile rows of whole 64-byte
 // halves; FP64 208^3 94.5 -> 90.8 us, 224^3 119 -> 106, 256^3 170 -> 148,
 // FP32 384^3 302 -> 291, but 256^3 FP32 (phi planes of just 256 MB) 86 -> 92,
@@ -148,6 +152,63 @@ constexpr uint64_t kCacheBytes = 256ull << 20;
 inline int even_width(int NH, int cap) {
   const int n = (NH + cap - 1) / cap;
   return (NH + n - 1) / n;
+}
+
+// The ideal kernel: blocks that the GPU holds at a time, and blocks of one z
+// plane with tiles of width cap.
+inline int ideal_slots(bool fp32) { return kCUs * (fp32 ? 3 : 2); }
+inline int64_t ideal_plane_blocks(int N, int cap) {
+  int TXH, TY, TZ;
+  ideal_tile(N, cap, 1, TXH, TY, TZ);
+  return (int64_t)((N / 2 + TXH - 1) / TXH) * ((N + TY - 1) / TY);
+}
+// Whether a lattice's fields alone exceed twice the cache.
+inline bool ideal_large(int N, bool fp32) {
+  return 10 * (uint64_t)N * N * N * (fp32 ? 4 : 8) > 2 * kCacheBytes;
+}
+// The unit in bytes whose multiples rows and tile rows have to be for
+// non-temporal stores (see kCacheBytes).
+inline int ideal_unit(int N, bool fp32) { return !fp32 && ideal_large(N, fp32) ? 64 : 128; }
+// The width of its tiles where the caller asked for none: 32 half-columns where
+// they divide the row (whole 128-byte lines of every component: 256^3 FP64 541
+// us against 560 with 64) or need fewer tiles than the alternative; 16 for FP64
+// rows of several tiles that those divide (160^3 174 -> 148 us, 224^3 443 ->
+// 398; a FP32 row of 16 is half a line).  Rows of whole 64-byte units of a large
+// lattice take such tiles: FP32 32 (288^3 583 -> 520, 480^3 2440 -> 2350), FP64
+// the width with most lanes at work (TY rows of NH half-columns in nt tiles), on
+// a tie the fewest, then the narrowest tiles (208^3 369 -> 337, 240^3 535 -> 490,
+// 272^3 865 -> 715, 304^3 1160 -> 1010, 368^3 2107 -> 1780, 400^3 2640 -> 2320).
+// Otherwise the widest even split that the kernel's plane grid holds (every ring
+// column costs a line per row and component: 200^3 FP64 329 us with 50, 390 with
+// 34, 435 with 25).
+inline int ideal_width(int N, bool fp32) {
+  const int NH = N / 2;
+  if (NH > 64 && ideal_large(N, fp32) && NH % 16 == (fp32 ? 0 : 8)) {
+    if (fp32) return 32;
+    int best = 0, best_ty = 0, best_nt = 1;
+    for (int cap = 32; cap <= 64; cap += 8) {
+      const int TY = kBlock / cap, nt = (NH + cap - 1) / cap;
+      const int gain = TY * best_nt - best_ty * nt;
+      if (gain > 0 || (gain == 0 && nt < best_nt)) {
+        best = cap;
+        best_ty = TY;
+        best_nt = nt;
+      }
+    }
+    return best;
+  }
+  int width = 0;
+  for (int cap = 64; cap >= 32 || !width; cap--) {
+    int TXH, TY, TZ;
+    ideal_tile(N, even_width(NH, cap), 1, TXH, TY, TZ);
+    if ((TY + 2) * (2 * TXH + 2) <= ideal_lds(fp32)) {
+      width = TXH;
+      break;
+    }
+  }
+  if (NH % 32 == 0 || ideal_plane_blocks(N, 32) < ideal_plane_blocks(N, width)) width = 32;
+  if (!fp32 && NH % 32 == 16 && NH > width) width = 16;
+  return width;
 }
 
 // Width of the charge march's tiles: an even split of the row into at most 64.

@@ -70,3 +70,24 @@ def test_charge_tiles_of_large_lattices_are_whole_units(rule):
             assert n == -(-NH // 64), (N, fp32)
         else:
             assert w <= 64 and n == -(-NH // 64) and w * n - NH < n, (N, fp32)
+
+
+def test_ideal_tiles_of_large_lattices_are_whole_units(rule):
+    """Where a lattice's fields exceed twice the 256 MiB cache and a row is whole
+    64-byte units, an ideal tile's rows are too (and FP64 ones are then stored
+    past the caches); every tile fits the kernel's plane grid."""
+    rows = rule("""
+  for (int N = 4; N <= kMaxN; N += 2)
+    for (int f = 0; f < 2; f++) {
+      const int w = ideal_width(N, f);
+      int TXH, TY, TZ;
+      ideal_tile(N, w, 1, TXH, TY, TZ);
+      printf("%d %d %d %d %d %d %d\\n", N, f, w, TXH, TY, ideal_lds(f), ideal_unit(N, f));
+    }""")
+    for N, fp32, w, TXH, TY, lds, unit in rows:
+        NH, esz = N // 2, 4 if fp32 else 8
+        assert (TY + 2) * (2 * TXH + 2) <= lds and TXH == min(w, NH), (N, fp32)
+        large = 10 * N ** 3 * esz > 2 ** 29
+        assert unit == (64 if large and not fp32 else 128), (N, fp32)
+        if large and NH * esz % 64 == 0:
+            assert w * esz % 64 == 0, (N, fp32, w)
