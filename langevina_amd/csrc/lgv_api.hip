@@ -295,6 +295,7 @@ void resolve_ideal_tiles(lgv_ctx *c) {
   for (int r = 0; r < c->nrep; r++) {
     ReplicaParams &p = c->hp[r];
     p.tile_cap = c->tiles[r].ideal_cap ? c->tiles[r].ideal_cap : ideal_width(p.N, c->fp32);
+    p.tile_alt = ideal_alternates(p.N, p.tile_cap, c->fp32);
   }
   int best = 64;
   double best_cost = 1e300;

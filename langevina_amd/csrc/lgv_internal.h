@@ -31,6 +31,7 @@ struct ReplicaParams {
   double tau_ideal;   // dt_ideal / 2.0
   uint64_t base_key;
   int tile_cap, tile_tz;   // ideal-kernel tile (see ideal_tile)
+  int tile_alt;            // its odd z chunks march downwards (see ideal_alternates)
   int hb_cap, hb_tz;       // phi-march tile (see hb_tile)
   int chg_cap, chg_chunk;  // charge-march tile (see charge_tile)
   int pair_y, pair_z;      // rows in y and planes of a block of both parities
@@ -209,6 +210,17 @@ inline int ideal_width(int N, bool fp32) {
   if (NH % 32 == 0 || ideal_plane_blocks(N, 32) < ideal_plane_blocks(N, width)) width = 32;
   if (!fp32 && NH % 32 == 16 && NH > width) width = 16;
   return width;
+}
+
+// Whether the ideal kernel's odd z chunks march downwards.  Two neighbouring
+// chunks that run at the same time then start, or end, at their common boundary
+// together, and the planes that each reads from the other are still in the XCD's
+// L2 (256^3 FP64 545 -> 530 us, 240^3 554 -> 534).  They do where the GPU holds
+// the blocks of both; otherwise the planes a chunk ends with are the first that
+// the next one, marching the same way, reads (512^3 FP64 4230 -> 4110 us, 528^3
+// 5100 -> 4950, 576^3 5950 -> 5850).
+inline bool ideal_alternates(int N, int cap, bool fp32) {
+  return 2 * ideal_plane_blocks(N, cap) <= ideal_slots(fp32);
 }
 
 // Width of the charge march's tiles: an even split of the row into at most 64.

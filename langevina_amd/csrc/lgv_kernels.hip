@@ -1399,11 +1399,10 @@ void k_ideal_fused(const ReplicaParams *__restrict__ P, const ReplicaState *__re
     }
   };
 
-  // Odd chunks march downwards: two neighbouring chunks then start, or end, at
-  // their common boundary at the same time, and the planes that each reads
-  // from the other are still in the XCD's L2 (256^3 FP64 555 -> 540 us, 200^3
-  // 320 -> 308).  Below, planes "z-1" and "z+1" are those behind and ahead of z.
-  const int dz = bz & 1 ? -1 : 1, zs = bz & 1 ? z0 + tz - 1 : z0;
+  // Odd chunks march downwards where tile_alt says so.  Below, planes "z-1" and
+  // "z+1" are those behind and ahead of z.
+  const bool down = bz & p.tile_alt;
+  const int dz = down ? -1 : 1, zs = down ? z0 + tz - 1 : z0;
   rotate_own(wrapz(zs - dz, N), nex, chn);
   if (own) {
 #pragma unroll

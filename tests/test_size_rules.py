@@ -91,3 +91,17 @@ def test_ideal_tiles_of_large_lattices_are_whole_units(rule):
         assert unit == (64 if large and not fp32 else 128), (N, fp32)
         if large and NH * esz % 64 == 0:
             assert w * esz % 64 == 0, (N, fp32, w)
+
+
+def test_ideal_chunks_alternate_where_neighbours_run_together(rule):
+    rows = rule("""
+  for (int N = 4; N <= kMaxN; N += 2)
+    for (int f = 0; f < 2; f++) {
+      const int w = ideal_width(N, f);
+      printf("%d %d %lld %d %d\\n", N, f, (long long)ideal_plane_blocks(N, w), ideal_slots(f),
+             ideal_alternates(N, w, f));
+    }""")
+    for N, fp32, plane, slots, alternate in rows:
+        assert alternate == (2 * plane <= slots), (N, fp32)
+        assert alternate or N > 256, (N, fp32)
+        assert not alternate or N < 512, (N, fp32)
