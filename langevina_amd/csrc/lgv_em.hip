@@ -25,40 +25,13 @@
 
 #include "lgv.h"
 #include "lgv_device.h"
+#include "lgv_em_tile.h"
 
 using namespace lgv;
 
 namespace {
 
-constexpr int kEmBlock = 256;
 constexpr uint64_t kEmTag = 0x4000000000000000ULL;
-
-// Tile of the two stencil marches: TX sites in x by TY rows in y, chunks of
-// TZ planes in z.  A block's plane (tile plus a one-site ring, no corners)
-// sits in LDS; each thread keeps its own column's planes z-1, z, z+1 in
-// registers.  TX splits the row evenly into at most 64.  A block marches TZ
-// planes after loading two, and the GPU holds about 1024 blocks: TZ of 8, 4, 2,
-// 1 minimises the rounds of TZ + 2 planes (per step with 8 -> with the rule's:
-// 33^3 Gaussian noise 24 -> 7.5 us (TZ 1), 64^3 15 -> 8.8 (TZ 1); 128^3 keeps 8).
-constexpr int kEmGrid = 400;  // (TY+2)(TX+2) <= 6 * 66
-__host__ __device__ inline int em_div(int a, int b) { return (a + b - 1) / b; }
-__host__ __device__ inline void em_tile(int N, int &TX, int &TY, int &TZ) {
-  TX = em_div(N, em_div(N, 64));
-  TY = kEmBlock / TX;
-  if (TY > N) TY = N;
-  const int tiles = em_div(N, TX) * em_div(N, TY);
-  TZ = 8;
-  for (int tz = 4; tz >= 1; tz /= 2)
-    if (em_div(tiles * em_div(N, tz), 1024) * (tz + 2) <
-        em_div(tiles * em_div(N, TZ), 1024) * (TZ + 2))
-      TZ = tz;
-  if (TZ > N) TZ = N;
-}
-__host__ __device__ inline int em_blocks(int N) {
-  int TX, TY, TZ;
-  em_tile(N, TX, TY, TZ);
-  return em_div(N, TX) * em_div(N, TY) * em_div(N, TZ);
-}
 
 struct GradSlot {
   double m2_s, m2_c, h_s, h_c, l_s, l_c;
@@ -214,11 +187,9 @@ struct EmMarch {
     tw = min(TX, N - x0);
     th = min(TY, N - y0);
     tz = min(TZ, N - z0);
-    // odd chunks march downwards: two neighbouring chunks then start, or end,
-    // at their common boundary at the same time, and the plane that each
-    // reads from the other is still in the XCD's L2
-    dz = bz & 1 ? -1 : 1;
-    zs = bz & 1 ? z0 + tz - 1 : z0;
+    const bool down = (bz & 1) && em_alternates(N, TX, TY);
+    dz = down ? -1 : 1;
+    zs = down ? z0 + tz - 1 : z0;
     GW = tw + 2;
     const int t = threadIdx.x;
     tx = t % TX;

@@ -1,5 +1,5 @@
-"""The host's rules that choose shapes by size (langevina_amd/csrc/lgv_internal.h),
-compiled as they stand: what they give over the whole range of sides."""
+"""The rules that choose shapes by size (langevina_amd/csrc/lgv_internal.h and
+lgv_em_tile.h), compiled as they stand: what they give over the whole range of sides."""
 import os
 import subprocess
 
@@ -16,7 +16,7 @@ def rule(tmp_path_factory):
     def run(body):
         d = tmp_path_factory.mktemp("rules")
         src, exe = d / "rules.cpp", d / "rules"
-        src.write_text('#include <cstdio>\n#include "lgv_internal.h"\nusing namespace lgv;\n'
+        src.write_text('#include <cstdio>\n#include "lgv_em_tile.h"\n#include "lgv_internal.h"\nusing namespace lgv;\n'
                        "int main() {\n" + body + "\n}\n")
         subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I", HIP_INCLUDE,
                         "-I", os.path.join(ROOT, "include"),
@@ -105,3 +105,30 @@ def test_ideal_chunks_alternate_where_neighbours_run_together(rule):
         assert alternate == (2 * plane <= slots), (N, fp32)
         assert alternate or N > 256, (N, fp32)
         assert not alternate or N < 512, (N, fp32)
+
+
+def test_euler_maruyama_tiles(rule):
+    """Rows of whole 64-byte units are split into such tiles; every tile fits the
+    kernels' plane and its ring the block's threads; a step of a side up to 256
+    fits the 8192 slots of the call without a handle."""
+    rows = rule("""
+  for (int N = 4; N <= 1024; N++) {
+    int TX, TY, TZ;
+    em_tile(N, TX, TY, TZ);
+    printf("%d %d %d %d %d %d\\n", N, TX, TY, TZ, em_blocks(N), em_alternates(N, TX, TY));
+  }""")
+    for N, TX, TY, TZ, blocks, alternate in rows:
+        assert (TY + 2) * (TX + 2) <= 400 and TX * TY <= 256 and 2 * (TX + TY) <= 256, N
+        assert 1 <= TZ <= N and TX <= N and TY <= N, N
+        even = -(-N // -(-N // 64))
+        lanes = min(N, 256 // TX) / -(-N // TX)
+        if N >= 100 and N % 8 == 0:
+            assert TX in (48, 64) or (TX == even and lanes > 1.1 * max(5 / -(-N // 48),
+                                                                      4 / -(-N // 64))), N
+            assert lanes >= 0.9 * (256 // even) / -(-N // even), N
+        else:
+            assert TX == even, N
+        plane = -(-N // TX) * -(-N // TY)
+        assert blocks == plane * -(-N // TZ), N
+        assert N > 256 or blocks <= 8192, N
+        assert alternate == (2 * plane <= 1024), N
