@@ -474,21 +474,25 @@ bool resolve_pair_march(lgv_ctx *c) {
   return true;
 }
 
-// Blocks of the launches of both parities.
+// Blocks of the launches of both parities, which exist where 32-bit offsets reach
+// a component's pair of half-planes (the march FP64 only); other contexts, which
+// no size rule sends there, run half-sweeps.
 int build_pair_plan(lgv_ctx *c) {
-  if (c->two_parity == TwoParity::kBricks && !resolve_bricks(c)) c->two_parity = TwoParity::kNone;
-  if (c->two_parity == TwoParity::kMarch && !resolve_pair_march(c))
+  bool reach = !(c->fp32 && c->two_parity == TwoParity::kMarch);
+  for (const ReplicaParams &p : c->hp)
+    reach = reach && 2 * (uint64_t)p.half * (c->fp32 ? 4 : 8) <= 0xFFFFFFFFull;
+  if (!reach || (c->two_parity == TwoParity::kBricks && !resolve_bricks(c)) ||
+      (c->two_parity == TwoParity::kMarch && !resolve_pair_march(c)))
     c->two_parity = TwoParity::kNone;
   if (c->two_parity == TwoParity::kNone) return LGV_OK;
   std::vector<PlanWork> work;
-  bool wide = c->wide, stream = c->buffer_bytes > 2 * kCacheBytes;
+  bool stream = c->buffer_bytes > 2 * kCacheBytes;
   for (const ReplicaParams &p : c->hp) {
-    wide = wide || 2 * (uint64_t)p.half * (c->fp32 ? 4 : 8) > 0xFFFFFFFFull;
     stream = stream && whole_rows(c, p.NH, p.NH, 64);
     const int64_t plane = (p.N + p.pair_y - 1) / p.pair_y;
     work.push_back({plane * ((p.N + p.pair_z - 1) / p.pair_z), (double)plane});
   }
-  const int rc = build_plan(c->plan_pair, work, wide);
+  const int rc = build_plan(c->plan_pair, work, false);
   c->plan_pair.stream = stream;
   return rc;
 }
@@ -696,7 +700,7 @@ void enqueue_phi_sweeps(lgv_ctx *c, int n, int off, int flip, hipStream_t st) {
     for (; i < n - n % 2; i++) {
       Timed tm(c, LGV_CLASS_PHI, 2);  // two half-sweeps
       if (c->two_parity == TwoParity::kMarch)
-        launch_hb_sweep(c->fp32, c->plan_pair, c->dP, c->dS, off + 2 * i, flip ^ (i & 1),
+        launch_hb_sweep(c->plan_pair, c->dP, c->dS, off + 2 * i, flip ^ (i & 1),
                         c->mon_pair, st);
       else
         launch_hb_brick(c->fp32, c->plan_pair, c->brick_lds, c->dP, c->dS, off + 2 * i,

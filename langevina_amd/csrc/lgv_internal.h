@@ -370,8 +370,8 @@ void launch_hb_phi(bool fp32, const Plan &plan, const ReplicaParams *P, ReplicaS
                    int ieo, int ctr_off, int flip, MonSlot *mon, hipStream_t st);
 void launch_hb_brick(bool fp32, const Plan &plan, int lds, const ReplicaParams *P,
                      ReplicaState *S, int ctr_off, int flip, MonSlot *mon, hipStream_t st);
-void launch_hb_sweep(bool fp32, const Plan &plan, const ReplicaParams *P, ReplicaState *S,
-                     int ctr_off, int flip, MonSlot *mon, hipStream_t st);
+void launch_hb_sweep(const Plan &plan, const ReplicaParams *P, ReplicaState *S, int ctr_off,
+                     int flip, MonSlot *mon, hipStream_t st);
 void launch_hb_march(bool fp32, const Plan &plan, const ReplicaParams *P, ReplicaState *S,
                      int ieo, int ctr_off, int flip, MonSlot *mon, hipStream_t st);
 void launch_charge_march(bool fp32, const Plan &plan, const ReplicaParams *P, ReplicaState *S,

@@ -459,7 +459,7 @@ __device__ __forceinline__ int wrapz(int z, int N) { return z < 0 ? z + N : (z >
 // count more than deciding the facing rows again (a half-sweep of 32^3 6.6 ->
 // 4.6 us, of 64^3 8.6 -> 7.1, half of a launch; 100^3 15.9 -> 16.7: kBrickSites).
 // The first round of odd values is loaded before the even sites' decisions.
-template <typename T, bool W>
+template <typename T>
 __global__ __launch_bounds__(kPairBlock) void k_hb_brick(const ReplicaParams *__restrict__ P,
                                                           const ReplicaState *__restrict__ S,
                                                           LaunchBlocks blk, int ctr_off, int flip,
@@ -506,7 +506,7 @@ __global__ __launch_bounds__(kPairBlock) void k_hb_brick(const ReplicaParams *__
     int dy, dz;
     const uint32_t idx = odd_site(i0, rid, xh, dy, dz);
 #pragma unroll
-    for (int l = 0; l < 4; l++) odd_o[l] = gplane<T, W>(p, cur, l, 1).raw(idx);
+    for (int l = 0; l < 4; l++) odd_o[l] = gplane<T, false>(p, cur, l, 1).raw(idx);
   };
   if (wave0 < odd) odd_load(wave0);
   // Every lane of a wavefront takes part in each of its rounds (the tallies
@@ -531,10 +531,10 @@ __global__ __launch_bounds__(kPairBlock) void k_hb_brick(const ReplicaParams *__
     double phi_o[4], heff[4], phi_n[4];
 #pragma unroll
     for (int l = 0; l < 4; l++) {
-      const GPlane<T, W> f = gplane<T, W>(p, cur, l, 1);
+      const GPlane<T, false> f = gplane<T, false>(p, cur, l, 1);
       heff[l] = (f.ld(nb[0]) + f.ld(nb[1])) + (f.ld(nb[2]) + f.ld(nb[3])) +
                 (f.ld(nb[4]) + f.ld(nb[5]));
-      phi_o[l] = gplane<T, W>(p, cur, l, 0).ld(row + xh);
+      phi_o[l] = gplane<T, false>(p, cur, l, 0).ld(row + xh);
     }
     const bool mine = in && (int)rid < ni;
     Xoro g = xoro_seeded(site_key(key_e, (uint64_t)rowi * N + x));
@@ -542,7 +542,7 @@ __global__ __launch_bounds__(kPairBlock) void k_hb_brick(const ReplicaParams *__
 #pragma unroll
     for (int l = 0; l < 4; l++) {
       even[l * comp + i] = (T)phi_n[l];
-      if (mine) gplane<T, W>(p, nxt, l, 0).st(row + xh, phi_n[l]);
+      if (mine) gplane<T, false>(p, nxt, l, 0).st(row + xh, phi_n[l]);
     }
   }
   __syncthreads();
@@ -571,7 +571,7 @@ __global__ __launch_bounds__(kPairBlock) void k_hb_brick(const ReplicaParams *__
     hb_decide(phi_o, heff, Lambda2, lambda, H, rdtg, g, phi_n, mt, in);
     if (in) {
 #pragma unroll
-      for (int l = 0; l < 4; l++) gplane<T, W>(p, nxt, l, 1).st(idx, phi_n[l]);
+      for (int l = 0; l < 4; l++) gplane<T, false>(p, nxt, l, 1).st(idx, phi_n[l]);
     }
   }
   block_monitor_add<kPairBlock>(slot, mt);
@@ -592,11 +592,12 @@ __global__ __launch_bounds__(kPairBlock) void k_hb_brick(const ReplicaParams *__
 // 28 wavefronts' decisions on four SIMDs), the rest the barrier's skew and LDS
 // reads.  Whole rows need no ring in x; the 16 wavefronts, of which a facing
 // row's have half the work, spread evenly over the SIMDs.
-template <typename T, bool W, bool NTS>
+template <bool NTS>
 __global__ __launch_bounds__(kPairBlock) void k_hb_sweep(const ReplicaParams *__restrict__ P,
                                                           const ReplicaState *__restrict__ S,
                                                           LaunchBlocks blk, int ctr_off, int flip,
                                                           MonSlot *__restrict__ mon) {
+  using T = double;  // FP32 fields run half-sweeps (see kPairMarchSites)
   __shared__ T odd[2][4][kPairBlock], even[2][4][kPairBlock];
   int r, b;
   MonSlot *slot = mon + block_of(blk, r, b);
@@ -612,7 +613,7 @@ __global__ __launch_bounds__(kPairBlock) void k_hb_sweep(const ReplicaParams *__
   const bool own = j < h + 2, inner = own && j >= 1 && j <= h;
   const int y = wrapz(y0 - 1 + j, N);
   const bool low = j == 0, outer = low || j == h + 1;  // rows that face the tile
-  constexpr uint32_t kNone = PhiPlanes<T, W>::kNone;
+  constexpr uint32_t kNone = PhiPlanes<T, false>::kNone;
   const uint32_t i_own = own ? (uint32_t)y * NH + xh : kNone;
   const uint32_t i_out =
       own && outer ? (uint32_t)wrapz(low ? y - 1 : y + 1, N) * NH + xh : kNone;
@@ -623,7 +624,7 @@ __global__ __launch_bounds__(kPairBlock) void k_hb_sweep(const ReplicaParams *__
   const double lambda = p.lambda, H = p.H, rdtg = p.rdtg;
   const uint64_t key_e = stream_key(p.base_key, s.sweep_ctr + ctr_off);
   const uint64_t key_o = stream_key(p.base_key, s.sweep_ctr + ctr_off + 1);
-  const PhiPlanes<T, W> in(p, cur), out(p, cur ^ 1);
+  const PhiPlanes<T, false> in(p, cur), out(p, cur ^ 1);
   Tally mt;
   auto ld4 = [&](int par, uint32_t i, int z, T v[4]) __attribute__((always_inline)) {
 #pragma unroll
@@ -1341,11 +1342,6 @@ void k_ideal_fused(const ReplicaParams *__restrict__ P, const ReplicaState *__re
   // read 1.92x its algorithmic bytes (the re-reads miss the 4 MB L2).
   constexpr bool kCarry = sizeof(T) == 8;
   __shared__ T chq[kCarry ? 1 : 2][kCarry ? 1 : 6][kCarry ? 1 : kBlock];
-  // The raw fields of the thread's first ring site of plane z+1 are loaded
-  // before the kick of plane z, so that their latency overlaps the kick
-  // (FP32: ten registers more, which the waves-per-SIMD bound of 3 holds at
-  // 168 with three spilled; 256^3 FP32 347 -> 329 us, 2 waves 360 us)
-  constexpr bool kEarlyRing = true;
   // The thread's two own sites of a plane are indexed by parity (pp), not by
   // x offset: a parity's plane base is the same for every lane, so the loads
   // and stores use one scalar base and 32-bit offsets.  The site of parity pp
@@ -1391,7 +1387,7 @@ void k_ideal_fused(const ReplicaParams *__restrict__ P, const ReplicaState *__re
 #pragma unroll
       for (int c = 0; c < 4; c++) lds[c][pos] = f[c];
     };
-    if (!kEarlyRing && t < nh) ring_fill(rgx, rgy, rpos);
+    // the second pass of a ring of more sites than threads
     for (int j = t + kBlock; j < nh; j += kBlock) {
       int gx, gy, pos;
       ring_site(j, gx, gy, pos);
@@ -1421,7 +1417,7 @@ void k_ideal_fused(const ReplicaParams *__restrict__ P, const ReplicaState *__re
         else chq[s][c][t] = chn[s][c];
       }
   }
-  if (kEarlyRing && t < nh) {
+  if (t < nh) {
     double f[10];
     load_site<T, W>(p, cur, rgx, rgy, zs, f);
     rotate_site_fast(f, f + 4, f + 7, h);
@@ -1433,8 +1429,12 @@ void k_ideal_fused(const ReplicaParams *__restrict__ P, const ReplicaState *__re
     const int z = zs + k * dz;
     const int zn = wrapz(z + dz, N);
     rotate_own(zn, nex, chn);
-    T rraw[10];  // the ring site's raw fields of plane z+1, as stored
-    const bool ring1 = kEarlyRing && t < nh && k + 1 < tz;
+    // The raw fields, as stored, of the thread's first ring site of plane z+1
+    // are loaded before the kick of plane z, so that their latency overlaps the
+    // kick (FP32: ten registers more, which the waves-per-SIMD bound of 3 holds
+    // at 168 with three spilled; 256^3 FP32 347 -> 329 us, 2 waves 360 us)
+    T rraw[10];
+    const bool ring1 = t < nh && k + 1 < tz;
     if (ring1) {
       const uint32_t ri = ((uint32_t)zn * N + rgy) * NH + (rgx >> 1);
       const int rpar = (rgx + rgy + zn) & 1;
@@ -2024,23 +2024,20 @@ void launch_hb_phi(bool fp32, const Plan &plan, const ReplicaParams *P, ReplicaS
                ctr_off, flip, mon);
 }
 
-void launch_hb_sweep(bool fp32, const Plan &plan, const ReplicaParams *P, ReplicaState *S,
-                     int ctr_off, int flip, MonSlot *mon, hipStream_t st) {
-#define LGV_SWEEP(TT, WW, SS) \
-  k_hb_sweep<TT, WW, SS><<<plan.nblocks, kPairBlock, 0, st>>>(P, S, plan.blocks, ctr_off, flip, mon)
-  if (fp32) { if (plan.wide) LGV_SWEEP(float, true, false); else LGV_SWEEP(float, false, false); }
-  else if (plan.stream) { if (plan.wide) LGV_SWEEP(double, true, true); else LGV_SWEEP(double, false, true); }
-  else { if (plan.wide) LGV_SWEEP(double, true, false); else LGV_SWEEP(double, false, false); }
-#undef LGV_SWEEP
+void launch_hb_sweep(const Plan &plan, const ReplicaParams *P, ReplicaState *S, int ctr_off,
+                     int flip, MonSlot *mon, hipStream_t st) {
+  if (plan.stream)
+    k_hb_sweep<true><<<plan.nblocks, kPairBlock, 0, st>>>(P, S, plan.blocks, ctr_off, flip, mon);
+  else
+    k_hb_sweep<false><<<plan.nblocks, kPairBlock, 0, st>>>(P, S, plan.blocks, ctr_off, flip, mon);
 }
 
 void launch_hb_brick(bool fp32, const Plan &plan, int lds, const ReplicaParams *P,
                      ReplicaState *S, int ctr_off, int flip, MonSlot *mon, hipStream_t st) {
-#define LGV_BRICK(TT, WW) \
-  k_hb_brick<TT, WW><<<plan.nblocks, kPairBlock, lds, st>>>(P, S, plan.blocks, ctr_off, flip, mon)
-  if (fp32) { if (plan.wide) LGV_BRICK(float, true); else LGV_BRICK(float, false); }
-  else { if (plan.wide) LGV_BRICK(double, true); else LGV_BRICK(double, false); }
-#undef LGV_BRICK
+  if (fp32)
+    k_hb_brick<float><<<plan.nblocks, kPairBlock, lds, st>>>(P, S, plan.blocks, ctr_off, flip, mon);
+  else
+    k_hb_brick<double><<<plan.nblocks, kPairBlock, lds, st>>>(P, S, plan.blocks, ctr_off, flip, mon);
 }
 
 void launch_hb_march(bool fp32, const Plan &plan, const ReplicaParams *P, ReplicaState *S,
