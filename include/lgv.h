@@ -193,9 +193,10 @@ int lgv_set_sweep_tiles(lgv_ctx *ctx, int replica, int hb_cap, int hb_tz, int ch
  * ModelG/Stepper.cxx:287-389): LGV_PHI_SITE one thread per site,
  * LGV_PHI_MARCH the z-march with the other parity's plane in LDS,
  * LGV_PHI_AUTO the size rule (the march from 7 million sites of all replicas
- * on; and below 560000 sites, and FP64 fields from 2.9 million on, the pairs
- * of sweeps of a step in launches of both parities, which the other two values
- * leave out).  Results do not depend on it; the autotuner picks
+ * on, 7.5 million of one FP64 lattice; and below 560000 sites, and FP64 lattices
+ * of sides 64 to 512 from 2.9 million sites on, the pairs of sweeps of a step in
+ * launches of both parities, which the other two values leave out).  Results do
+ * not depend on it; the autotuner picks
  * it.  Monitor counts are kept across the change.  lgv_get_phi_kernel
  * reports the kernel in use (LGV_PHI_SITE or LGV_PHI_MARCH). */
 enum { LGV_PHI_AUTO = 0, LGV_PHI_SITE = 1, LGV_PHI_MARCH = 2 };

@@ -674,7 +674,7 @@ int enqueue_ideal(lgv_ctx *c, int off, int flip) {
 // EulerLangevinHB::step (counters off, off+1 for the two parities), one
 // in-place launch per parity: the z-march with the other parity's plane in
 // LDS or the one-thread-per-site kernel, by the size rule (the march from
-// kMarchSites on) unless lgv_set_phi_kernel chose.  Per half-sweep, site
+// phi_march_sites on) unless lgv_set_phi_kernel chose.  Per half-sweep, site
 // against march, FP64: 64^3 8.9, 9.5 us; 100^3 16.8, 15.5; 160^3 42, 44; 192^3
 // 67, 66; 224^3 147, 109; 256^3 221, 147; FP32: 160^3 33, 33; 224^3 79, 70;
 // 256^3 116, 86.
@@ -962,7 +962,7 @@ int lgv_create(const lgv_config *cfg, lgv_ctx **out) {
     minN = std::min(minN, N);
   }
   c->buffer_bytes = buffer_bytes;
-  c->phi_march_auto = buffer_bytes / (10 * esz) >= kMarchSites;
+  c->phi_march_auto = buffer_bytes / (10 * esz) >= phi_march_sites(c->fp32, cfg->nreplicas);
   // test hook: LGV_NT_STORES=0/1 forces the store mode on any size, and with
   // FP64 fields the phi kernel that goes with it (1: the march)
   if (const char *nt = getenv("LGV_NT_STORES")) {

@@ -248,7 +248,14 @@ inline int charge_width(int NH, bool fp32) {
 // 180^3 2058 -> 2070, 192^3 2124 -> 2082, 224^3 3840 -> 3636, 256^3 5006 ->
 // 4371; FP32 128^3 410 -> 411, 180^3 1219 -> 1229, 192^3 1328 -> 1304, 224^3
 // 2253 -> 2214, 256^3 2949 -> 2708.
+// One FP64 lattice runs half-sweeps only as lone calls and as the last of an odd
+// number, without a step's other kernels in the cache: two of them, site ->
+// march, 192^3 123 -> 132 us, 200^3 139 -> 142, 204^3 181 -> 165 (a batch of 60 x
+// 48^3 144 -> 127).
 constexpr uint64_t kMarchSites = 7000000;
+inline uint64_t phi_march_sites(bool fp32, int nreplicas) {
+  return fp32 || nreplicas > 1 ? kMarchSites : 7500000;
+}
 
 // Pairs of phi sweeps run as launches of both parities, out of place (a pair
 // leaves the live buffer where it was), below the first number of sites (all

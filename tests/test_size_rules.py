@@ -132,3 +132,13 @@ def test_euler_maruyama_tiles(rule):
         assert blocks == plane * -(-N // TZ), N
         assert N > 256 or blocks <= 8192, N
         assert alternate == (2 * plane <= 1024), N
+
+
+def test_half_sweeps_of_one_fp64_lattice_march_from_196_on(rule):
+    rows = rule("""
+  printf("%lld %lld %lld\\n", (long long)phi_march_sites(false, 1),
+         (long long)phi_march_sites(true, 1), (long long)phi_march_sites(false, 60));""")
+    one64, one32, batch64 = rows[0]
+    assert 194 ** 3 < one64 <= 200 ** 3
+    assert 180 ** 3 < one32 <= 192 ** 3
+    assert batch64 == one32
