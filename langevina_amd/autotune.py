@@ -110,8 +110,9 @@ def autotune_sweeps(ctx, dt, march=None, steps=3, verbose=False):
     also speeds up the kernels that follow it), the size rule's choice being
     the incumbent; march True / False: keep the kernel in use and tune (or not)
     the march's tiles.  Then per size class, as autotune_ideal: the charge
-    march (tile width x chunk) and, when the phi half-sweep runs the z-march,
-    its tile width x z-chunk.  Returns {N: (hb_cap, hb_tz, chg_cap,
+    march (tile width x chunk) and, when the phi half-sweep runs the z-march and
+    a step's sweeps are half-sweeps, its tile width x z-chunk (no launch of both
+    parities depends on that tile).  Returns {N: (hb_cap, hb_tz, chg_cap,
     chg_chunk)} (0 = default); ctx.phi_kernel() reports the kernel."""
     sizes = sorted(set(ctx.N))
     chosen = {N: [0, 0, 0, 0] for N in sizes}
@@ -134,6 +135,7 @@ def autotune_sweeps(ctx, dt, march=None, steps=3, verbose=False):
         if verbose:
             print(f"autotune phi kernel: {'march' if march else 'site'} {ms:.3f} ms/step",
                   flush=True)
+    pairs = ctx.phi_pairs() and ctx.scounts[0] > 1
     for N in sizes:
         cands, seen = [(0, 0)], set()
         for cap in CHARGE_CAPS:
@@ -146,7 +148,7 @@ def autotune_sweeps(ctx, dt, march=None, steps=3, verbose=False):
         chosen[N][2:] = [cap, ch]
         if verbose:
             print(f"autotune charge N={N}: cap={cap} chunk={ch} {ms * 1e3:.1f} us", flush=True)
-        if not march:
+        if not march or pairs:
             continue
         cands, seen = [(0, 0)], set()
         for cap in HB_CAPS:

@@ -179,7 +179,7 @@ class Context:
         cfg.nreplicas = len(replicas)
         cfg.replicas = C.cast(self._params, C.POINTER(ModelParams))
         cfg.precision = precision
-        cfg.scounts[0], cfg.scounts[1] = scounts
+        cfg.scounts[0], cfg.scounts[1] = self.scounts = tuple(scounts)
         cfg.nodiffuse, cfg.onlydiffuse = int(nodiffuse), int(onlydiffuse)
         cfg.track_energy = int(track_energy)
         cfg.device = device
