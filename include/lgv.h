@@ -181,6 +181,8 @@ int lgv_monitor_reset(lgv_ctx *ctx);
  * at most txh_cap half-columns (2..64) in x, 256/txh rows in y, tz planes
  * per z-chunk.  Results do not depend on it; the autotuner picks it. */
 int lgv_set_ideal_tile(lgv_ctx *ctx, int replica, int txh_cap, int tz);
+/* The tile in use: the one set, or the library's own choice. */
+int lgv_get_ideal_tile(lgv_ctx *ctx, int replica, int *txh_cap, int *tz);
 /* Tiles of the two Metropolis sweep kernels for one replica (replica < 0:
  * all): the phi z-march (at most hb_cap half-columns, 4..64, x 256/hb_cap
  * rows, chunks of hb_tz planes) and the charge march (at most chg_cap

@@ -14,8 +14,8 @@ import time
 from .lgv import _check, lib
 
 CAPS = (8, 16, 32, 64)
-# short z chunks give a small lattice (one 64^3 replica: 32 blocks with the
-# default tile) more blocks than the march's depth costs it
+# short z chunks give a small lattice (one 64^3 replica: 32 blocks of 32
+# half-columns and 16 planes) more blocks than the march's depth costs it
 TZS = (1, 2, 4, 8, 16, 32, 64)
 CHARGE_CAPS = (16, 32, 64)
 CHARGE_CHUNKS = (2, 4, 8, 16, 32)
@@ -167,7 +167,8 @@ def autotune_sweeps(ctx, dt, march=None, steps=3, verbose=False):
 def autotune_ideal(ctx, dt, steps=3, cache_path=None, verbose=False):
     """Greedy per size class: for each distinct N among the context's
     replicas, try every (cap, tz) with the other classes fixed and keep the
-    fastest, starting from the default (32, 16).  Steps taken while tuning
+    fastest, starting from the tile in use (on a new context the library's own
+    choice, which a candidate replaces only when faster by MARGIN).  Steps taken while tuning
     advance the replicas' state like any other steps.
     Returns {N: (cap, tz, ms_per_ideal_launch)}."""
     cache = {}
@@ -201,8 +202,9 @@ def autotune_ideal(ctx, dt, steps=3, cache_path=None, verbose=False):
             for _ in range(WARMUP):
                 ctx.step(dt)
             warmed = True
-        cands = [(32, 16)] + [(cap, tz) for cap in ideal_caps(N) for tz in TZS
-                              if tz <= N and (cap, tz) != (32, 16)]
+        in_use = ctx.ideal_tile(reps[0])
+        cands = [in_use] + [(cap, tz) for cap in ideal_caps(N) for tz in TZS
+                            if tz <= N and (cap, tz) != in_use]
         (cap, tz), ms = _search(ctx, dt, steps, "ideal", apply, cands)
         if verbose:
             print(f"autotune ideal N={N}: cap={cap} tz={tz} {ms * 1e3:.1f} us", flush=True)

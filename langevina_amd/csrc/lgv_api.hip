@@ -1490,6 +1490,15 @@ int lgv_set_ideal_tile(lgv_ctx *c, int r, int txh_cap, int tz) {
   return LGV_OK;
 }
 
+int lgv_get_ideal_tile(lgv_ctx *c, int r, int *txh_cap, int *tz) {
+  int rc = check_replica(c, r);
+  if (rc) return rc;
+  if (!txh_cap || !tz) return fail(LGV_ERR_ARG, "null argument");
+  *txh_cap = c->hp[r].tile_cap;
+  *tz = c->hp[r].tile_tz;
+  return LGV_OK;
+}
+
 int lgv_set_sweep_tiles(lgv_ctx *c, int r, int hb_cap, int hb_tz, int chg_cap,
                         int chg_chunk) {
   if (!c) return fail(LGV_ERR_ARG, "null context");

@@ -62,7 +62,7 @@ EXPORTS = [
     "lgv_em_last_error", "lgv_em_create", "lgv_em_set_stream", "lgv_em_forward",
     "lgv_em_backward", "lgv_em_destroy", "lgv_em_series", "lgv_em_step",
     "lgv_em_step_noalloc", "lgv_set_phi_kernel", "lgv_get_phi_kernel",
-    "lgv_get_phi_pairs",
+    "lgv_get_phi_pairs", "lgv_get_ideal_tile",
 ]
 
 # lgv_set_phi_kernel values
@@ -115,6 +115,7 @@ def lib():
     L.lgv_set_mass.argtypes = [ctx, C.c_int, C.c_double, C.c_double]
     L.lgv_monitor_reset.argtypes = [ctx]
     L.lgv_set_ideal_tile.argtypes = [ctx, C.c_int, C.c_int, C.c_int]
+    L.lgv_get_ideal_tile.argtypes = [ctx, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int)]
     L.lgv_set_sweep_tiles.argtypes = [ctx, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int]
     L.lgv_synchronize.argtypes = [ctx]
     L.lgv_field_device_ptr.argtypes = [ctx, C.c_int, C.POINTER(C.c_void_p), C.POINTER(C.c_int)]
@@ -300,6 +301,12 @@ class Context:
 
     def synchronize(self):
         _check(lib().lgv_synchronize(self.h))
+
+    def ideal_tile(self, replica=0):
+        """(width cap, planes per z chunk) of the ideal kernel's tile in use."""
+        cap, tz = C.c_int(), C.c_int()
+        _check(lib().lgv_get_ideal_tile(self.h, replica, C.byref(cap), C.byref(tz)))
+        return cap.value, tz.value
 
     def set_phi_kernel(self, kernel):
         """PHI_AUTO (size rule), PHI_SITE or PHI_MARCH for the phi half-sweeps."""

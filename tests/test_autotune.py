@@ -15,6 +15,10 @@ class Recorder:
         self.pairs_auto, self.kernel = pairs, PHI_AUTO
         self.sweep, self.ideal = [], []
         self.timed = 0
+        self.tile = (56, 8)
+
+    def ideal_tile(self, replica=0):
+        return self.tile
 
     def step(self, dt):
         pass
@@ -60,3 +64,13 @@ def test_march_tiles_are_tuned_where_steps_run_half_sweeps(tuner, pairs, scounts
     ctx = Recorder(256, pairs, scounts)
     tuner.autotune_sweeps(ctx, 0.04)
     assert any(t[:2] != (0, 0) for t in ctx.sweep)
+
+
+def test_the_ideal_tile_in_use_is_the_incumbent(tuner, monkeypatch):
+    """No tile is faster than another: the context keeps the one it had."""
+    monkeypatch.setattr(tuner, "_class_ms", lambda *a: 1.0)
+    ctx = Recorder(208, pairs=0)
+    chosen = tuner.autotune_ideal(ctx, 0.04)
+    assert chosen[208] == (56, 8, 1.0)
+    assert ctx.ideal[0] == ctx.ideal[-1] == (56, 8)
+    assert len(set(ctx.ideal)) == len(ctx.ideal) // 2  # each candidate once a round
