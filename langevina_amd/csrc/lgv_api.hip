@@ -945,6 +945,7 @@ int lgv_create(const lgv_config *cfg, lgv_ctx **out) {
     p.lambda = m.lambda;
     p.H = m.H;
     p.chi = m.chi;
+    p.chg_l2 = charge_l2(m.chi);
     const double hx = (double)(m.LX > 0 ? m.LX : N) / N;
     p.axx = std::pow(1. / hx, 2);
     const uint32_t s32 = rank0_seed(m.seed);

@@ -34,8 +34,20 @@ struct ReplicaParams {
   int tile_alt;            // its odd z chunks march downwards (see ideal_alternates)
   int hb_cap, hb_tz;       // phi-march tile (see hb_tile)
   int chg_cap, chg_chunk;  // charge-march tile (see charge_tile)
+  float chg_l2;            // see charge_l2
   int pair_y, pair_z;      // rows in y and planes of a block of both parities
 };
+
+// -log2(e) / (2 chi) in single precision, with which the charge sweep forms
+// exp(-dS) from dS 2 chi.  NaN, so that the double test decides, where that or
+// dS 2 chi might leave the range of single precision: within 2^-100 .. 2^100 a
+// dS 2 chi that overflows is a dS beyond 2^27, and one below 2^-126 a dS below
+// 2^-26.
+inline float charge_l2(double chi) {
+  const double d = 2. * chi;
+  return d >= 0x1p-100 && d <= 0x1p100 ? (float)(-0x1.71547652b82fep+0 * (1. / d))
+                                       : __builtin_nanf("");
+}
 
 // Device-written state of one replica (clock, counters, per-step data).
 struct ReplicaState {

@@ -894,18 +894,16 @@ __global__ __launch_bounds__(kBlock) void k_hb_march(const ReplicaParams *__rest
 // modelg_update_charge_pair (Stepper.cxx:419-441) for one component of one
 // pair, applied as nA + (-q), nB + q; counts the decision when count.
 // The constants of a charge sweep: the proposal width, the divisor d = 2 chi
-// of dS with its rounded reciprocal, and -log2(e) / d in single precision.  That
-// is NaN, so that the double test decides, where dS d or 1 / d might leave the
-// range of single precision: within 2^-100 .. 2^100 a dS d that overflows is a
-// dS beyond 2^27, and one below 2^-126 a dS below 2^-26.
+// of dS with its rounded reciprocal, and -log2(e) / d in single precision (NaN
+// where that won't do: charge_l2; formed here, it cost 0.3 of the 37.5 us of
+// three launches at 64^3).
 struct ChargeK {
   double rms, d, inv;
   float l2;
 };
-__device__ __forceinline__ ChargeK charge_k(double rms, double chi) {
-  const double d = 2. * chi, inv = 1. / d;
-  const bool in_range = d >= 0x1p-100 && d <= 0x1p100;
-  return {rms, d, inv, in_range ? (float)(-0x1.71547652b82fep+0 * inv) : __builtin_nanf("")};
+__device__ __forceinline__ ChargeK charge_k(const ReplicaParams &p) {
+  const double d = 2. * p.chi;
+  return {p.rms, d, 1. / d, p.chg_l2};
 }
 // x / d from the rounded reciprocal with one Markstein correction: q0 = x *
 // inv, the residual x - q0 d exact with one FMA, q0 + residual * inv rounded
@@ -970,7 +968,7 @@ __device__ __forceinline__ void charge_line(const ReplicaParams &p, const Charge
     ii[k] = (zz * N + yy) * NH + (xx >> 1);
     lin[k] = (zz * N + yy) * N + xx;
   }
-  const ChargeK ck = charge_k(p.rms, p.chi);
+  const ChargeK ck = charge_k(p);
   Xoro gL = xoro_seeded(site_key(k1, lin[0]));
   Xoro gB = xoro_seeded(site_key(k1, lin[2]));
   Xoro gA = xoro_seeded(site_key(k2, lin[1]));
@@ -1018,7 +1016,7 @@ __device__ __forceinline__ void charge_row_wave(const ReplicaParams &p, const Ch
   static_assert(H == 1 || H == 2, "rows of up to 128 half-columns");
   const uint32_t N = p.N, NH = p.NH;
   const uint32_t row = z * N + y;
-  const ChargeK ck = charge_k(p.rms, p.chi);
+  const ChargeK ck = charge_k(p);
   // a1: updated A'_h; r: updated L_{h+1} from lane + 1; l0: lane 0's updated
   // L (H = 2 only); all as stored (T), which is how the second sub-sweep reads
   // them, so that FP32 fields hold and shuffle half the registers
@@ -1087,7 +1085,7 @@ __device__ __forceinline__ void charge_column(const ReplicaParams &p, const Char
                                               int dir, int e1, int e2, uint32_t x, uint32_t q, int c0,
                                               int c1, uint64_t k1, uint64_t k2, Tally &m) {
   const int N = p.N, NH = p.NH;
-  const ChargeK ck = charge_k(p.rms, p.chi);
+  const ChargeK ck = charge_k(p);
   // index / linear site of position m along the column
   auto at = [&](int m, uint32_t &ii, uint32_t &lin) __attribute__((always_inline)) {
     const uint32_t row = dir == 2 ? (uint32_t)m * N + q : q * N + (uint32_t)m;

@@ -142,3 +142,20 @@ def test_half_sweeps_of_one_fp64_lattice_march_from_196_on(rule):
     assert 194 ** 3 < one64 <= 200 ** 3
     assert 180 ** 3 < one32 <= 192 ** 3
     assert batch64 == one32
+
+
+def test_charge_factor_is_a_float_or_nan(rule):
+    """-log2(e) / 2 chi: NaN outside 2^-100 .. 2^100, else within a float's
+    rounding (relative error in units of 2^-26)."""
+    rows = rule("""
+  for (int e = -1000; e <= 1000; e++)
+    for (int m = 8; m < 16; m++) {
+      const double chi = __builtin_ldexp((double)m, e - 4), l2 = charge_l2(chi);
+      const double ref = -1.4426950408889634 / (2. * chi);
+      printf("%d %d %d %d\\n", e, m, l2 != l2,
+             l2 != l2 ? 0 : (int)(67108864. * __builtin_fabs(l2 / ref - 1.)));
+    }""")
+    for e, m, nan, err in rows:
+        d = m * 2.0 ** (e - 3)
+        assert nan == (not 2.0 ** -100 <= d <= 2.0 ** 100), (e, m)
+        assert err <= 4, (e, m)
