@@ -84,3 +84,41 @@ def test_kept_and_recomputed_states_give_the_same_gradients(torch, nsteps, ckpt)
     for grad, par in got[1:]:
         np.testing.assert_array_equal(grad, got[0][0])
         np.testing.assert_array_equal(par, got[0][1])
+
+
+# Rows of whole 64-byte units in tiles of 64 and 48 sites: 104: 64 and 40; 136: 48,
+# 48, 40; 240: five of 48; 352: six of 64, the last of 32, every chunk marched upwards
+WHOLE = [104, 136, 240, 352]
+
+
+@pytest.mark.parametrize("N", WHOLE)
+def test_tiles_of_whole_units_give_the_drift(torch, N):
+    test_the_difference_of_two_runs_is_the_drift(torch, N, 0)
+
+
+@pytest.mark.parametrize("N", WHOLE)
+def test_tiles_of_whole_units_give_the_adjoint(torch, N):
+    """Two steps, the loss phibar_0 of the last state: the gradient is
+    J(phi_0) J(phi_1) e_0 / V with the one-step Jacobian J, which is symmetric."""
+    print(f"[gpu-test] em adjoint tiles {N}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(N)
+    phi0 = torch.randn((4, N, N, N), generator=g, device="cuda", dtype=torch.float64)
+    phi1, grad = torch.empty_like(phi0), torch.empty_like(phi0)
+    torch.cuda.synchronize()
+    h = stepper(N, 2, 2, 0)
+    h.forward(phi0.data_ptr(), 1)
+    h.backward(grad.data_ptr())
+    h.step(phi0.data_ptr(), phi1.data_ptr(), 0)
+    torch.cuda.synchronize()
+    h.close()
+    gdt, big = PAR["gamma"] * PAR["dt"], 0.
+    lam = torch.zeros_like(phi0)
+    lam[0] = 1. / N ** 3
+    for phi in (phi1, phi0):
+        lap = sum(torch.roll(lam, s, d) for d in (1, 2, 3) for s in (1, -1)) - 6 * lam
+        lam = lam - gdt * (-lap + PAR["m2"] * lam + PAR["lam"] * (
+            (phi ** 2).sum(0) * lam + 2 * phi * (phi * lam).sum(0)))
+        big = max(big, (phi ** 2).sum(0).max().item())
+    # a dozen operations a step on terms of up to (1 + gdt 3 lambda |phi|^2) / V
+    tol = 64 * np.finfo(float).eps * (1 + 3 * gdt * PAR["lam"] * big) ** 2 / N ** 3
+    assert (grad - lam).abs().max().item() <= tol

@@ -204,3 +204,30 @@ def test_sweep_counters_of_mixed_calls(L):
     np.testing.assert_array_equal(ctx.get_field(), one.get_field())
     one.close()
     ctx.close()
+
+
+# Lattices large enough for tiles of whole 64-byte units, against tiles of 16: 176:
+# charge tiles of 48 and 40; 208: charge 64 and 40, ideal 56 and 48 stored past the
+# caches; 224 FP32: charge 64 and 48; 272: ideal and charge 48, 48, 40; 288 FP32:
+# ideal four of 32 and 16; 336: against ideal tiles of 40, whose chunks do not
+# alternate
+@pytest.mark.parametrize("N,prec,tile", [(176, 0, (16, 8)), (208, 0, (16, 8)), (224, 1, (16, 8)),
+                                         (272, 0, (16, 8)), (288, 1, (16, 8)), (336, 0, (40, 8))])
+def test_tiles_of_whole_units_keep_results(L, N, prec, tile):
+    print(f"[gpu-test] whole-unit tiles {N} {prec}", flush=True)
+    from langevina_amd.autotune import set_ideal_tile, set_sweep_tiles
+    u = np.random.default_rng(N).normal(size=(N, N, N, 10)) * 0.5
+    out = []
+    for fixed in (False, True):
+        ctx = L.Context(L.model_params(N, seed=3), precision=prec)
+        if fixed:
+            set_ideal_tile(ctx, 0, *tile)
+            set_sweep_tiles(ctx, 0, 0, 0, 16, 8)
+        ctx.set_field(u)
+        ctx.run(0.04, 2)
+        out.append((ctx.get_field(), ctx.monitors()["charge"], ctx.ideal_tile()))
+        ctx.close()
+    assert out[0][2] != out[1][2] == tile
+    np.testing.assert_array_equal(out[0][0], out[1][0])
+    for k in ("down_counts", "up_counts", "up_yes", "up_no"):
+        assert out[0][1][k] == out[1][1][k], k
