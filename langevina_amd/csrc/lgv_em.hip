@@ -175,9 +175,8 @@ struct EmMarch {
   int tx, ty, x, y;
   bool own, halo;
   int hx, hy, hpos, pos;
-  __device__ explicit EmMarch(int n) : N(n) {
-    int TX, TY, TZ;
-    em_tile(N, TX, TY, TZ);
+  __device__ EmMarch(int n, const EmTile &tile) : N(n) {
+    const int TX = tile.TX, TY = tile.TY, TZ = tile.TZ;
     const int ntx = (N + TX - 1) / TX, nty = (N + TY - 1) / TY;
     int bx, by, bz;
     yband_tile(blockIdx.x, ntx, nty, bx, by, bz);
@@ -187,7 +186,7 @@ struct EmMarch {
     tw = min(TX, N - x0);
     th = min(TY, N - y0);
     tz = min(TZ, N - z0);
-    const bool down = (bz & 1) && em_alternates(N, TX, TY);
+    const bool down = (bz & 1) && tile.alternate;
     dz = down ? -1 : 1;
     zs = down ? z0 + tz - 1 : z0;
     GW = tw + 2;
@@ -225,13 +224,13 @@ struct EmMarch {
 template <int NS, bool GAUSS>
 __global__ __launch_bounds__(kEmBlock) void k_em_step(const double *__restrict__ in,
                                                       double *__restrict__ out, int N,
-                                                      double m2, double lam, double H,
+                                                      EmTile tile, double m2, double lam, double H,
                                                       double gdt, double amp, uint64_t skey,
                                                       double *slots, EmMerge prev) {
   __shared__ double Q[2][4][kEmGrid];
   const int64_t V = (int64_t)N * N * N;
   if (prev.slots && blockIdx.x == 0) em_merge(prev, V);
-  const EmMarch m(N);
+  const EmMarch m(N, tile);
   KSum acc[NS > 0 ? NS : 1];
   for (int i = 0; i < NS; i++) acc[i] = KSum{0., 0.};
   double cm[4], cc[4], cp[4];  // own column behind z, at z, ahead of z
@@ -288,9 +287,9 @@ __global__ __launch_bounds__(kEmBlock) void k_em_step(const double *__restrict__
 // The observable sums of a state without stepping it (the measurement
 // before the first step); the same blocks and slots as k_em_step.
 __global__ __launch_bounds__(kEmBlock) void k_em_observe(const double *__restrict__ in, int N,
-                                                         double *slots) {
+                                                         EmTile tile, double *slots) {
   const int64_t V = (int64_t)N * N * N;
-  const EmMarch m(N);
+  const EmMarch m(N, tile);
   KSum acc[kObsSums];
   for (int i = 0; i < kObsSums; i++) acc[i] = KSum{0., 0.};
   if (m.own) {
@@ -314,12 +313,13 @@ __global__ __launch_bounds__(kEmBlock) void k_em_merge(EmMerge m, int64_t V) { e
 __global__ __launch_bounds__(kEmBlock) void k_em_adjoint(const double *__restrict__ phi,
                                                          const double *__restrict__ lin,
                                                          double *__restrict__ lout, int N,
-                                                         double m2, double lam, double gdt,
+                                                         EmTile tile, double m2, double lam,
+                                                         double gdt,
                                                          double dl,
                                                          GradSlot *__restrict__ slots) {
   __shared__ double Q[2][4][kEmGrid];
   const int64_t V = (int64_t)N * N * N;
-  const EmMarch m(N);
+  const EmMarch m(N, tile);
   KSum ga{0., 0.}, gb{0., 0.}, gc{0., 0.};  // d/d m2, d/d H, d/d lambda
   double lm[4], lc[4], lp[4];  // lam_in of the own column behind z, at z, ahead
   if (m.own) {
@@ -451,8 +451,8 @@ void launch_step(int NS, const lgv_em_params &p, uint64_t base, int nblocks, con
   const double amp = std::sqrt(2.0 * gdt);
   const uint64_t skey = stream_key(base, kEmTag | (uint64_t)n);
   auto launch = [&](auto kernel) {
-    kernel<<<nblocks, kEmBlock, 0, st>>>(in, out, p.N, p.m2, p.lambda, p.H, gdt, amp, skey,
-                                         slots, prev);
+    kernel<<<nblocks, kEmBlock, 0, st>>>(in, out, p.N, em_tile(p.N), p.m2, p.lambda, p.H, gdt,
+                                         amp, skey, slots, prev);
   };
   if (p.noise_kind)
     launch(NS == 0 ? k_em_step<0, true> : (NS == 1 ? k_em_step<1, true> : k_em_step<kObsSums, true>));
@@ -681,8 +681,8 @@ int lgv_em_backward(lgv_em *h, double *grad_phi0, double grad_params[3]) {
         dl = (1.0 / W + (double)h->V * 2.0 * (h->phibar_host[n] - (double)mean) / W) /
              (double)h->V;
       k_em_adjoint<<<h->nblocks, kEmBlock, 0, h->stream>>>(
-          n == n0 ? first : h->seg + (int64_t)(n - n0) * 4 * h->V, lam, nxt, h->p.N, h->p.m2, h->p.lambda, gdt,
-          dl, h->gslots);
+          n == n0 ? first : h->seg + (int64_t)(n - n0) * 4 * h->V, lam, nxt, h->p.N,
+          em_tile(h->p.N), h->p.m2, h->p.lambda, gdt, dl, h->gslots);
       std::swap(lam, nxt);
     }
   }
@@ -717,7 +717,7 @@ int lgv_em_series(lgv_em *h, const double *phi0, int every, double *phi_final,
   // steps, inside the step launch that produces the state
   // (slots of parity 1, merged by step 0's launch)
   double *slots = h->part + (size_t)h->nblocks * kPartStride;
-  k_em_observe<<<h->nblocks, kEmBlock, 0, h->stream>>>(phi0, h->p.N, slots);
+  k_em_observe<<<h->nblocks, kEmBlock, 0, h->stream>>>(phi0, h->p.N, em_tile(h->p.N), slots);
   EMCHECK(hipGetLastError());
   const EmMerge row0{slots, kObsSums, h->nblocks, nullptr, h->rows};
   int rc;

@@ -13,7 +13,7 @@ constexpr int kEmSlots = 1024;  // blocks that the GPU holds at a time, about
 // sits in LDS; each thread keeps its own column's planes z-1, z, z+1 in
 // registers.
 constexpr int kEmGrid = 400;  // (TY+2)(TX+2) <= 6 * 66
-__host__ __device__ inline int em_div(int a, int b) { return (a + b - 1) / b; }
+inline int em_div(int a, int b) { return (a + b - 1) / b; }
 
 // TX: an even split of the row into at most 64.  From N = 100 on, where rows are
 // whole 64-byte units, 64 or 48 instead, so that tiles are whole units too,
@@ -24,7 +24,7 @@ __host__ __device__ inline int em_div(int a, int b) { return (a + b - 1) / b; }
 // 368^3 862 / 1766 -> 786 / 1501, 772 / 1504; 288^3 393 / 799 -> 349 / 680, 388 /
 // 744; 200^3 with Gaussian noise 196 / 313 -> -, 217 / 320; 72^3 15.0 / 28.4 ->
 // 16.5 / 30.8, 16.4 / 29.1.
-__host__ __device__ inline int em_width(int N) {
+inline int em_width(int N) {
   const int even = em_div(N, em_div(N, 64));
   if (N < 100 || N % 8 != 0) return even;
   const int n48 = em_div(N, 48), n64 = em_div(N, 64);
@@ -38,7 +38,7 @@ __host__ __device__ inline int em_width(int N) {
 // A block marches TZ planes after loading two: TZ of 8, 4, 2, 1 minimises the
 // rounds of TZ + 2 planes (per step with 8 -> with the rule's: 33^3 Gaussian
 // noise 24 -> 7.5 us (TZ 1), 64^3 15 -> 8.8 (TZ 1); 128^3 keeps 8).
-__host__ __device__ inline void em_tile(int N, int &TX, int &TY, int &TZ) {
+inline void em_tile(int N, int &TX, int &TY, int &TZ) {
   TX = em_width(N);
   TY = kEmBlock / TX;
   if (TY > N) TY = N;
@@ -50,7 +50,7 @@ __host__ __device__ inline void em_tile(int N, int &TX, int &TY, int &TZ) {
       TZ = tz;
   if (TZ > N) TZ = N;
 }
-__host__ __device__ inline int em_blocks(int N) {
+inline int em_blocks(int N) {
   int TX, TY, TZ;
   em_tile(N, TX, TY, TZ);
   return em_div(N, TX) * em_div(N, TY) * em_div(N, TZ);
@@ -60,8 +60,21 @@ __host__ __device__ inline int em_blocks(int N) {
 // their common boundary at the same time, and the plane that each reads from
 // the other is still in the XCD's L2.  Where the GPU does not hold the blocks of
 // two neighbouring chunks at a time, all march upwards.
-__host__ __device__ inline bool em_alternates(int N, int TX, int TY) {
+inline bool em_alternates(int N, int TX, int TY) {
   return 2 * em_div(N, TX) * em_div(N, TY) <= kEmSlots;
+}
+
+// The tile of a launch, from the host: worked out in the kernels it is a chain
+// of divisions before the first load (64^3 10.8 us a step, 11.5 so).
+struct EmTile {
+  int TX, TY, TZ;
+  bool alternate;
+};
+inline EmTile em_tile(int N) {
+  EmTile t;
+  em_tile(N, t.TX, t.TY, t.TZ);
+  t.alternate = em_alternates(N, t.TX, t.TY);
+  return t;
 }
 
 }  // namespace lgv

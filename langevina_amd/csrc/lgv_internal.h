@@ -30,8 +30,11 @@ struct ReplicaParams {
   double dt_ideal;    // dt / scounts[1]
   double tau_ideal;   // dt_ideal / 2.0
   uint64_t base_key;
-  int tile_cap, tile_tz;   // ideal-kernel tile (see ideal_tile)
-  int tile_alt;            // its odd z chunks march downwards (see ideal_alternates)
+  // ideal-kernel tile (see ideal_tile), and whether its odd z chunks march
+  // downwards (see ideal_alternates); short, so that the kernel's parameters stay
+  // within two scalar cache lines (64^3 13.8 us, 14.5 with a third)
+  int16_t tile_cap, tile_alt;
+  int tile_tz;
   int hb_cap, hb_tz;       // phi-march tile (see hb_tile)
   int chg_cap, chg_chunk;  // charge-march tile (see charge_tile)
   float chg_l2;            // see charge_l2
