@@ -295,7 +295,6 @@ void resolve_ideal_tiles(lgv_ctx *c) {
   for (int r = 0; r < c->nrep; r++) {
     ReplicaParams &p = c->hp[r];
     p.tile_cap = c->tiles[r].ideal_cap ? c->tiles[r].ideal_cap : ideal_width(p.N, c->fp32);
-    p.tile_alt = ideal_alternates(p.N, p.tile_cap, c->fp32);
   }
   int best = 64;
   double best_cost = 1e300;
@@ -328,9 +327,10 @@ bool whole_rows(const lgv_ctx *c, int NH, int TXH, int bytes) {
 int build_ideal_plan(lgv_ctx *c) {
   resolve_ideal_tiles(c);
   std::vector<PlanWork> work;
-  bool stream = c->buffer_bytes > 2 * kCacheBytes;
+  bool stream = c->buffer_bytes > 2 * kCacheBytes, alternate = true;
   for (int r = 0; r < c->nrep; r++) {
     const ReplicaParams &p = c->hp[r];
+    alternate = alternate && ideal_alternates(p.N, p.tile_cap, c->fp32);
     int TXH, TY, TZ;
     ideal_tile(p.N, p.tile_cap, p.tile_tz, TXH, TY, TZ);
     if ((TY + 2) * (2 * TXH + 2) > ideal_lds(c->fp32))
@@ -344,6 +344,7 @@ int build_ideal_plan(lgv_ctx *c) {
   if (rc) return rc;
   rc = build_plan(c->plan_ideal, work, c->wide);
   c->plan_ideal.stream = c->nt_stores < 0 ? stream : c->nt_stores;
+  c->plan_ideal.alternate = alternate;
   return rc;
 }
 

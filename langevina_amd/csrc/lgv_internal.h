@@ -30,15 +30,11 @@ struct ReplicaParams {
   double dt_ideal;    // dt / scounts[1]
   double tau_ideal;   // dt_ideal / 2.0
   uint64_t base_key;
-  // ideal-kernel tile (see ideal_tile), and whether its odd z chunks march
-  // downwards (see ideal_alternates); short, so that the kernel's parameters stay
-  // within two scalar cache lines (64^3 13.8 us, 14.5 with a third)
-  int16_t tile_cap, tile_alt;
-  int tile_tz;
+  int tile_cap, tile_tz;   // ideal-kernel tile (see ideal_tile)
   int hb_cap, hb_tz;       // phi-march tile (see hb_tile)
   int chg_cap, chg_chunk;  // charge-march tile (see charge_tile)
-  float chg_l2;            // see charge_l2
   int pair_y, pair_z;      // rows in y and planes of a block of both parities
+  float chg_l2;            // see charge_l2
 };
 
 // -log2(e) / (2 chi) in single precision, with which the charge sweep forms
@@ -134,6 +130,10 @@ struct Plan {
                         // is >= 4 GiB
   bool stream = false;  // outputs written with non-temporal stores (see kCacheBytes)
   bool far = false;     // some replica's charge planes span >= 4 GiB (charge launch)
+  // ideal launch: every replica's odd z chunks march downwards (see
+  // ideal_alternates); an argument of the launch: read with a replica's tile, it
+  // cost a step of 64^3 0.5 us
+  bool alternate = true;
   bool xwave = false;   // charge launch: every replica has N = 128 or 256 (x rows per wave)
   std::vector<int> first;  // host copy of blocks.first
 };

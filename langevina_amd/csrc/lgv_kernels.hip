@@ -1291,7 +1291,7 @@ __device__ __forceinline__ void load_site(const ReplicaParams &p, int cur, int x
 template <typename T, bool W, bool NTS>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 3 : 1)))
 void k_ideal_fused(const ReplicaParams *__restrict__ P, const ReplicaState *__restrict__ S,
-                   LaunchBlocks blk, int flip) {
+                   LaunchBlocks blk, int flip, int alternate) {
   __shared__ double lds[4][ideal_lds(sizeof(T) == 4)];
   // rotated phi of plane z-1 at the thread's own sites: thread-private slots
   __shared__ double lprv[2][4][kBlock];
@@ -1394,9 +1394,9 @@ void k_ideal_fused(const ReplicaParams *__restrict__ P, const ReplicaState *__re
     }
   };
 
-  // Odd chunks march downwards where tile_alt says so.  Below, planes "z-1" and
+  // With `alternate` (0 or 1) odd chunks march downwards.  Below, planes "z-1" and
   // "z+1" are those behind and ahead of z.
-  const bool down = bz & p.tile_alt;
+  const bool down = bz & alternate;
   const int dz = down ? -1 : 1, zs = down ? z0 + tz - 1 : z0;
   rotate_own(wrapz(zs - dz, N), nex, chn);
   if (own) {
@@ -2064,7 +2064,7 @@ void launch_charge_march(bool fp32, const Plan &plan, const ReplicaParams *P, Re
 
 void launch_ideal(bool fp32, const Plan &plan, const ReplicaParams *P, ReplicaState *S,
                   int flip, hipStream_t st) {
-  LGV_DISPATCH_S(k_ideal_fused, plan.nblocks, st, P, S, plan.blocks, flip);
+  LGV_DISPATCH_S(k_ideal_fused, plan.nblocks, st, P, S, plan.blocks, flip, (int)plan.alternate);
 }
 
 void launch_energy(bool fp32, const Plan &plan, const ReplicaParams *P,
